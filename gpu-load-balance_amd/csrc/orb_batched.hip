@@ -169,12 +169,26 @@ __global__ void k_b_init(orb_cell *heap, uint8_t *exists, uint8_t *sub, int64_t 
     if (i < 2) status[i] = 0;
 }
 
-// Level record of entry i from the device heap (small cells are marked
-// for the subtree kernel, cells inside a finished subtree are skipped);
-// returns its chunk count.
+// Which kernels a level's launches hold, for its cell records: cells of at
+// most sub_max keys (and kSmallLeaves leaves) go to the subtree kernel, cells
+// of at most cell_max keys to k_b_cell (0: not launched), the others to the
+// chunk kernels.  A level without chunk kernels (chunks = 0, chosen from the
+// sizes the host expects) leaves a larger cell alone and counts it in the
+// build's pass counter 0; the host then runs the levels again with every
+// kernel (again = 1), which skips the cells that are split already.
+struct LevelMode {
+    uint32_t sub_max, cell_max;
+    int32_t chunks, again;
+};
+constexpr int kFlagBlock = 3;  // CellRec.flags: the cell goes to k_b_cell
+
+// Level record of entry i from the device heap (cells inside a finished
+// subtree, and cells that a left-alone ancestor has not made yet, are
+// skipped); returns its chunk count.
 __device__ inline uint32_t level_rec(const LevelEntry *entries, int32_t i, const orb_cell *heap,
-                                     const uint32_t *ranges, const uint8_t *sub, int use_subtree,
-                                     uint32_t sub_max, CellRec *recs)
+                                     const uint8_t *exists, const uint32_t *ranges,
+                                     const uint8_t *sub, const LevelMode mode, CellRec *recs,
+                                     int32_t *level_passes)
 {
     const LevelEntry en = entries[i];
     const int32_t id = en.id;
@@ -198,10 +212,19 @@ __device__ inline uint32_t level_rec(const LevelEntry *entries, int32_t i, const
     r.st = en.st;
     r.lmax = en.lmax;
     const uint32_t n = r.end - r.begin;
-    if (sub[g]) r.flags = 1;
-    else if (use_subtree && en.sub_ok && n <= sub_max && cl.nLeafCells <= kSmallLeaves)
+    const int64_t gl = (int64_t)en.hb + left_child_id(id);
+    if (sub[g] || !exists[g] || (mode.again && exists[gl])) {
+        r.flags = 1;
+    } else if (mode.sub_max && en.sub_ok && n <= mode.sub_max && cl.nLeafCells <= kSmallLeaves) {
         r.flags = 2;
-    else r.flags = 0;
+    } else if (mode.cell_max && n <= mode.cell_max) {
+        r.flags = kFlagBlock;
+    } else if (mode.chunks) {
+        r.flags = 0;
+    } else {
+        r.flags = 1;
+        atomicAdd(&level_passes[en.lp & ~63], 1);
+    }
     recs[i] = r;
     return r.flags ? 0u : (n + (uint32_t)kChunk - 1u) / (uint32_t)kChunk;
 }
@@ -221,9 +244,9 @@ __device__ inline void level_finals(uint32_t fb0, const PendingFinalDev &fin,
 }
 
 __global__ void k_b_recs(const LevelEntry *entries, int32_t nCells, const orb_cell *heap,
-                         const uint32_t *ranges, const uint8_t *sub, int use_subtree,
-                         uint32_t sub_max, CellRec *recs, uint32_t *nchunks, uint32_t rec_blocks,
-                         PendingFinalDev fin)
+                         const uint8_t *exists, const uint32_t *ranges, const uint8_t *sub,
+                         LevelMode mode, CellRec *recs, uint32_t *nchunks, int32_t *level_passes,
+                         uint32_t rec_blocks, PendingFinalDev fin)
 {
     if (blockIdx.x >= rec_blocks) {  // uniform
         level_finals(rec_blocks, fin, ranges);
@@ -232,7 +255,7 @@ __global__ void k_b_recs(const LevelEntry *entries, int32_t nCells, const orb_ce
     int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i > nCells) return;
     nchunks[i] = i == nCells ? 0u
-                             : level_rec(entries, i, heap, ranges, sub, use_subtree, sub_max, recs);
+                             : level_rec(entries, i, heap, exists, ranges, sub, mode, recs, level_passes);
 }
 
 // A level of fewer than kRecsScan cells in one block of kRecsScan threads,
@@ -242,9 +265,9 @@ __global__ void k_b_recs(const LevelEntry *entries, int32_t nCells, const orb_ce
 constexpr int kRecsScan = 1024;
 __global__ __launch_bounds__(kRecsScan) void k_b_recs_scan(
     const LevelEntry *__restrict__ entries, int32_t nCells, const orb_cell *__restrict__ heap,
-    const uint32_t *__restrict__ ranges, const uint8_t *__restrict__ sub, int use_subtree,
-    uint32_t sub_max, CellRec *__restrict__ recs, uint32_t *__restrict__ first,
-    PendingFinalDev fin)
+    const uint8_t *__restrict__ exists, const uint32_t *__restrict__ ranges,
+    const uint8_t *__restrict__ sub, LevelMode mode, CellRec *__restrict__ recs,
+    uint32_t *__restrict__ first, int32_t *__restrict__ level_passes, PendingFinalDev fin)
 {
     if (blockIdx.x > 0) {  // uniform: the previous level's row swaps
         level_finals(1u, fin, ranges);
@@ -254,7 +277,7 @@ __global__ __launch_bounds__(kRecsScan) void k_b_recs_scan(
     __shared__ uint32_t wsum[kW];
     const int t = threadIdx.x, lane = t & 63, w = t >> 6;
     const uint32_t v =
-        t < nCells ? level_rec(entries, t, heap, ranges, sub, use_subtree, sub_max, recs) : 0u;
+        t < nCells ? level_rec(entries, t, heap, exists, ranges, sub, mode, recs, level_passes) : 0u;
     const uint32_t inc = wave_inclusive_scan(v);
     if (lane == 63) wsum[w] = inc;
     __syncthreads();
@@ -815,16 +838,6 @@ __device__ inline RoundOut replay_round(const T *P, float lo, float hi, float ta
     }
     return replay_path<T>(nle, [&](int j) { return P[j]; }, lo, hi, target, passes0, lane,
                           trace_row);
-}
-
-// A wave-uniform value of lane src.
-__device__ inline uint32_t lane_value(uint32_t v, int src)
-{
-    return (uint32_t)__builtin_amdgcn_readlane((int)v, src);
-}
-__device__ inline uint64_t lane_value(uint64_t v, int src)
-{
-    return (uint64_t)lane_value((uint32_t)v, src) | ((uint64_t)lane_value((uint32_t)(v >> 32), src) << 32);
 }
 
 // replay_round with the round's prefix sums in registers, not in LDS: lane l
@@ -2205,6 +2218,317 @@ __global__ __launch_bounds__(kSubBlock) void k_b_subtree(const CellRec *recs, in
 }
 
 // ---------------------------------------------------------------------------
+// one level of a mid-sized cell by one block
+// ---------------------------------------------------------------------------
+// A cell too large for the subtree kernel but of at most kRows * kThreads keys
+// takes its whole level in one block: the cut-axis keys are read
+// once into registers (kRows per lane: wave w holds the contiguous part
+// [w * 64 * rows, (w + 1) * 64 * rows), 64 consecutive keys a row), every
+// histogram round, the stopper masks and the pair lists come from there, and
+// x, y, z (and the payload) are swapped in place.  The chunk path reads the
+// keys twice and takes 16 dependent launches a level; what bounds this kernel
+// is the swap's memory traffic on levels that fill the chip (12 B read and
+// written per key, 4 B more for the keys) and its own serial phases on levels
+// of few cells.  Measured: a level of 4096 cells of 16384 keys 451 us (chunk
+// path 530), one of two 32768-key cells 45 us, of four 16384-key cells 34 us
+// (chunk path 85).
+//
+// rows is a multiple of 4, so a wave's part is whole 256-key groups; keys
+// past the cell's end are +INF in their lane (never below a cut, never an
+// R-stopper) and are masked out of the L-stopper words.
+//
+// Latency decides on levels of few cells: 1024 threads a cell.  Levels that
+// fill the chip take 512-thread blocks of twice the rows, two to a CU, so that
+// one block's barriers and replays lie under the other's traffic.
+constexpr int kCellRowsMax = 40;
+constexpr uint32_t kCellSmall = 20u * 1024u, kCellLarge = 40u * 1024u;  // the two capacities
+constexpr int32_t kCellManyCells = 256;  // more than a cell per CU
+static_assert(kCellRowsMax <= 64 && kCellLarge <= 65536u, "a mask word per lane, 16-bit positions");
+
+template <int kThreads, int kRows, int kArrays>
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4, 4))) void k_b_cell(CellRec *recs, int32_t nCells, orb_cell *heap,
+                                                       uint8_t *exists, uint32_t *ranges, float *x,
+                                                       float *y, float *z, uint32_t *pid,
+                                                       uint32_t *wgt, int le_cmp, uint64_t *trace,
+                                                       int32_t *level_passes, int32_t *status)
+{
+    static_assert(kRows % 4 == 0 && kRows <= kCellRowsMax, "whole groups, a mask word per lane");
+    constexpr int kWaves = kThreads / 64;
+    constexpr uint32_t kCap = (uint32_t)kRows * kThreads;
+    constexpr int kBatch = 4;  // pairs per thread in flight
+    // a swapped pair's two positions differ and no position is in two pairs:
+    // at most n / 2 pairs
+    __shared__ uint16_t slist[2][kCap / 2];
+    __shared__ uint32_t hist[kBins];
+    __shared__ uint32_t s_cnt[2][kWaves];
+    __shared__ float s_lr[2];
+    __shared__ int32_t s_pf[2];
+    __shared__ uint32_t s_K, s_i;
+    const int t = threadIdx.x, lane = t & 63, w = (int)uniform((uint32_t)t >> 6);
+    for (int32_t c = blockIdx.x; c < nCells; c += gridDim.x) {
+        if (uniform((uint32_t)recs[c].flags) != (uint32_t)kFlagBlock) continue;
+        const CellRec &rec = recs[c];  // this block alone writes it, at the search's end
+        const uint32_t begin = uniform(rec.begin), n = uniform(rec.end) - begin;
+        const int axis = (int)uniform((uint32_t)rec.axis);
+        const int32_t id = (int32_t)uniform((uint32_t)rec.id), hb = (int32_t)uniform((uint32_t)rec.hb);
+        if (n > kCap || axis < 0 || axis > 2) {
+            // the level records hand over neither; refuse anything else
+            if (t == 0) report_error(status + rec.st, rec.lp & 63, kErrSplit, id);
+            continue;
+        }
+        const uint32_t rows = 4u * ((n + 4u * kThreads - 1u) / (4u * kThreads));
+        const uint32_t wb = 64u * rows * (uint32_t)w;
+        const uint32_t len = wb < n ? (n - wb < 64u * rows ? n - wb : 64u * rows) : 0u;
+        const float *const key = axis_ptr(x, y, z, axis) + begin;
+        float v[kRows];
+        // f(row) over the rows in use, unrolled (v stays in registers), a
+        // uniform branch per four rows
+        auto each_row = [&](auto f) __attribute__((always_inline)) {
+            // a value of its own: otherwise the compiler keeps every group's
+            // comparison in scalar registers from one sweep to the next
+            uint32_t used = rows;
+            asm volatile("" : "+s"(used));
+            static_for<0, kRows / 4>([&](auto gc) __attribute__((always_inline)) {
+                constexpr int g = decltype(gc)::value;
+                if (4u * (uint32_t)g < used)
+                    static_for<4 * g, 4 * g + 4>(
+                        [&](auto jc) __attribute__((always_inline)) { f(jc); });
+                __builtin_amdgcn_sched_barrier(0);
+            });
+        };
+        {
+            const __amdgpu_buffer_rsrc_t kr = __builtin_amdgcn_make_buffer_rsrc(
+                const_cast<float *>(key), 0, (int)(n * 4u), 0x00020000);
+            each_row([&](auto jc) __attribute__((always_inline)) {
+                constexpr int j = decltype(jc)::value;
+                v[j] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
+                    kr, (int)((wb + 64u * (uint32_t)j + (uint32_t)lane) * 4u), 0, 0));
+            });
+        }
+        for (int q = t; q < kBins; q += kThreads) hist[q] = 0u;
+        if (len < 64u * rows) {  // wave-uniform: the cell's end lies in (or before) this part
+            each_row([&](auto jc) __attribute__((always_inline)) {
+                constexpr int j = decltype(jc)::value;
+                if (64u * (uint32_t)j + (uint32_t)lane >= len) v[j] = INFINITY;
+            });
+        }
+        __syncthreads();
+        // ---- the bisection controller in rounds of 8 passes (orbit.cpp:149-231)
+        const float target = difference_target(n, (int32_t)uniform((uint32_t)rec.nLeaf));
+        uint64_t *trow = trace ? trace + ((size_t)hb + id) * ORB_MAX_PASSES : nullptr;
+        float lo = uniform(rec.margin_l), hi = uniform(rec.margin_r);
+        int32_t passes = 0;
+        bool found = false;
+        while (true) {
+            const float width = hi - lo;
+            const float scale = width > 0.0f ? (float)kBins / width : 0.0f;
+            const float lim = 0.5f - bin_tolerance(lo, hi, scale);
+            uint32_t below = 0;  // wave-uniform; keys above the margins are in no prefix sum
+            uint64_t slow = 0ull;  // this lane's rows too close to a bin edge for the estimate
+            each_row([&](auto jc) __attribute__((always_inline)) {
+                constexpr int j = decltype(jc)::value;
+                const bool lt = v[j] < lo, in = !lt && !(v[j] > hi);
+                below += (uint32_t)__popcll(__ballot(lt));
+                const float ef = (v[j] - lo) * scale;
+                const int bin = (int)__builtin_amdgcn_fmed3f(ef, 0.0f, 255.5f);
+                const bool est = fabsf(__builtin_amdgcn_fractf(ef) - 0.5f) < lim;
+                if (in && est) atomicAdd(&hist[bin], 1u);
+                slow |= in && !est ? 1ull << j : 0ull;
+            });
+            while (__ballot(slow != 0ull)) {
+                // exact bins of the slow keys (about 1 in 2000 of a first
+                // round; every one where coordinates sit on a grid), read
+                // again: four rows a step, their loads in flight together
+                float sv[4];
+                bool on[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    on[u] = slow != 0ull;
+                    const uint32_t row = on[u] ? (uint32_t)__builtin_ctzll(slow) : 0u;
+                    slow &= slow - 1ull;  // 0 stays 0
+                    sv[u] = on[u] ? key[wb + 64u * row + (uint32_t)lane] : 0.0f;
+                }
+#pragma unroll
+                for (int u = 0; u < 4; ++u)
+                    if (on[u])
+                        atomicAdd(&hist[le_cmp ? bin_walk<1>(sv[u], lo, hi) : bin_walk<0>(sv[u], lo, hi)],
+                                  1u);
+            }
+            if (lane == 0 && below) atomicAdd(&hist[0], below);
+            __syncthreads();
+            if (w == 0) {
+                const uint4 h4 = reinterpret_cast<const uint4 *>(hist)[lane];
+                reinterpret_cast<uint4 *>(hist)[lane] = make_uint4(0u, 0u, 0u, 0u);
+                const uint32_t s0 = h4.x, s1 = s0 + h4.y, s2 = s1 + h4.z, s3 = s2 + h4.w;
+                const uint32_t base = wave_inclusive_scan(s3) - s3;
+                // P[4 lane + 1 + q] (P[j] = keys in bins below j)
+                const uint32_t pv[4] = {base + s0, base + s1, base + s2, base + s3};
+                const RoundOut ro = replay_round_lanes(pv, lo, hi, target, passes, lane, trow);
+                if (lane == 0) {
+                    s_lr[0] = ro.L;
+                    s_lr[1] = ro.R;
+                    s_pf[0] = ro.passes;
+                    s_pf[1] = ro.found ? 1 : 0;
+                }
+            }
+            __syncthreads();
+            lo = uniform(s_lr[0]);
+            hi = uniform(s_lr[1]);
+            passes = (int32_t)uniform((uint32_t)s_pf[0]);
+            found = uniform((uint32_t)s_pf[1]) != 0u;
+            if (found || passes >= ORB_MAX_PASSES) break;
+        }
+        // ---- Hoare (partition.cpp:28-60): stopper words, a word per lane
+        const float cut = cell_cut(lo, hi);
+        uint64_t mineL = 0ull, mineR = 0ull;
+        each_row([&](auto jc) __attribute__((always_inline)) {
+            constexpr int j = decltype(jc)::value;
+            constexpr uint32_t p0 = 64u * (uint32_t)j;
+            const uint64_t valid =
+                p0 >= len ? 0ull : (len - p0 >= 64u ? ~0ull : (1ull << (len - p0)) - 1ull);
+            const uint64_t mL = __ballot(!(v[j] < cut)) & valid;
+            const uint64_t mR = __ballot(!(v[j] > cut)) & valid;
+            mineL = lane == j ? mL : mineL;
+            mineR = lane == j ? mR : mineR;
+        });
+        const uint32_t cL = (uint32_t)__popcll(mineL), cR = (uint32_t)__popcll(mineR);
+        const uint32_t iL = wave_inclusive_scan(cL), iR = wave_inclusive_scan(cR);
+        if (lane == 63) {
+            s_cnt[0][w] = iL;
+            s_cnt[1][w] = iR;
+        }
+        __syncthreads();
+        // the waves' stopper counts, wave q in lane q, and their prefix sums
+        const uint32_t wL = lane < kWaves ? s_cnt[0][lane] : 0u;
+        const uint32_t wR = lane < kWaves ? s_cnt[1][lane] : 0u;
+        const uint32_t pL = wave_inclusive_scan(wL) - wL, pR = wave_inclusive_scan(wR) - wR;
+        const uint32_t TL = lane_value(pL + wL, 63), TR = lane_value(pR + wR, 63);
+        const bool bad = n == 0u || TL == 0u;  // the reference's loop leaves the cell
+        // With A(p) the L-stoppers before position p and B(p) the R-stoppers
+        // at or after it (A grows, B shrinks), K = max over p of
+        // min(A(p), B(p)) and i = the last p with A(p) <= K <= B(p).  Both lie
+        // in one word: the last whose start has A <= B, resp. A <= K <= B.
+        const uint32_t aL = lane_value(pL, w), aR = lane_value(pR, w);
+        const uint32_t xA = aL + iL - cL, xB = TR - (aR + iR - cR);  // A and B at this lane's word
+        if (t == (kWaves > 1 ? 64 : 0))  // the cell's margins, its passes, its children
+            finish_round(rec, c, RoundOut{lo, hi, passes, found, 0}, found ? 1 : 0, recs, heap,
+                         level_passes, exists, status);
+        // A and B at bit `lane` of word q of this wave, and just after it
+        auto at_bit = [&](int q, uint32_t &a0, uint32_t &b0, uint32_t &a1, uint32_t &b1) {
+            const uint64_t mL = lane_value(mineL, q), mR = lane_value(mineR, q);
+            a0 = lane_value(xA, q) + __builtin_amdgcn_mbcnt_hi(
+                     (uint32_t)(mL >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mL, 0u));
+            b0 = lane_value(xB, q) - __builtin_amdgcn_mbcnt_hi(
+                     (uint32_t)(mR >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mR, 0u));
+            a1 = a0 + (uint32_t)((mL >> lane) & 1ull);
+            b1 = b0 - (uint32_t)((mR >> lane) & 1ull);
+        };
+        if (!bad) {
+            const uint64_t mk = __ballot(lane < kWaves && pL + pR <= TR);
+            if (w == 63 - __clzll((long long)mk)) {  // A <= B at the start of this wave's part
+                const uint64_t mw = __ballot((uint32_t)lane < rows && xA <= xB);
+                uint32_t a0, b0, a1, b1;
+                at_bit(63 - __clzll((long long)mw), a0, b0, a1, b1);
+                // the maximum over the word's positions, and the word's end
+                const uint32_t k0 = a0 < b0 ? a0 : b0, k1 = a1 < b1 ? a1 : b1;
+                const uint32_t best = wave_max(k0 > k1 ? k0 : k1);
+                if (lane == 0) s_K = best;
+            }
+        }
+        __syncthreads();
+        const int64_t lid = left_child_id(id), rid = right_child_id(id);
+        if (bad || rid >= (int32_t)uniform((uint32_t)rec.capr)) {
+            if (t == 0) report_error(status + rec.st, rec.lp & 63, kErrPartition, id);
+            continue;  // uniform
+        }
+        const uint32_t K = uniform(s_K);
+        {
+            const uint64_t mk = __ballot(lane < kWaves && pL <= K && K + pR <= TR);
+            if (w == 63 - __clzll((long long)mk)) {
+                const uint64_t mw = __ballot((uint32_t)lane < rows && xA <= K && K <= xB);
+                const int q = 63 - __clzll((long long)mw);
+                uint32_t a0, b0, a1, b1;
+                at_bit(q, a0, b0, a1, b1);
+                const uint64_t mb = __ballot(a0 <= K && K <= b0);
+                if (lane == 0) s_i = wb + 64u * (uint32_t)q + 63u - (uint32_t)__clzll((long long)mb);
+            }
+        }
+        {
+            // the pairs' positions: L_t at t, R_t at t
+            const uint32_t xL = iL - cL, xR = iR - cR;
+            each_row([&](auto jc) __attribute__((always_inline)) {
+                constexpr int j = decltype(jc)::value;
+                const uint32_t pos = wb + 64u * (uint32_t)j + (uint32_t)lane;
+                const uint64_t mL = lane_value(mineL, j), mR = lane_value(mineR, j);
+                const uint32_t oL = aL + lane_value(xL, j), oR = aR + lane_value(xR, j);
+                if (oL < K && mL) {  // uniform
+                    const uint32_t idx = oL + __builtin_amdgcn_mbcnt_hi(
+                        (uint32_t)(mL >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mL, 0u));
+                    if (((mL >> lane) & 1ull) && idx < K) slist[0][idx] = (uint16_t)pos;
+                }
+                if (oR + (uint32_t)__popcll(mR) + K > TR && mR) {  // uniform
+                    const uint32_t idx = oR + __builtin_amdgcn_mbcnt_hi(
+                        (uint32_t)(mR >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mR, 0u));
+                    if (((mR >> lane) & 1ull) && idx + K >= TR) slist[1][TR - 1u - idx] = (uint16_t)pos;
+                }
+            });
+        }
+        __syncthreads();
+        const uint32_t i = uniform(s_i);
+        const CellArrays<true> ca(x, y, z, pid, wgt, begin);
+        const int na = ca.count;  // uniform, at most kArrays
+        for (uint32_t j0 = (uint32_t)t; j0 < K + (uint32_t)t; j0 += kThreads * kBatch) {
+            uint32_t pa[kBatch], pb[kBatch];
+            uint32_t va[kArrays][kBatch] = {}, vb[kArrays][kBatch] = {};
+#pragma unroll
+            for (int u = 0; u < kBatch; ++u) {
+                const uint32_t jj = j0 + (uint32_t)(u * kThreads);
+                pa[u] = jj < K ? 4u * slist[0][jj] : 0u;
+                pb[u] = jj < K ? 4u * slist[1][jj] : 0u;
+            }
+#pragma unroll
+            for (int arr = 0; arr < kArrays; ++arr) {
+                if (arr >= na) break;
+#pragma unroll
+                for (int u = 0; u < kBatch; ++u) {
+                    if (j0 + (uint32_t)(u * kThreads) < K) {
+                        va[arr][u] = ca.load(arr, pa[u]);
+                        vb[arr][u] = ca.load(arr, pb[u]);
+                    }
+                }
+            }
+#pragma unroll
+            for (int arr = 0; arr < kArrays; ++arr) {
+                if (arr >= na) break;
+#pragma unroll
+                for (int u = 0; u < kBatch; ++u) {
+                    if (j0 + (uint32_t)(u * kThreads) < K) {
+                        ca.store(arr, pa[u], vb[arr][u]);
+                        ca.store(arr, pb[u], va[arr][u]);
+                    }
+                }
+            }
+        }
+        __syncthreads();  // every pair is in place before the last row swap
+        if (t < na && i != n - 1u) {
+            // Hoare's last step (partition.cpp:61-62), an array per lane
+            const uint32_t a = ca.load(t, 4u * i), b = ca.load(t, 4u * (n - 1u));
+            ca.store(t, 4u * i, b);
+            ca.store(t, 4u * (n - 1u), a);
+        }
+        if (t == 0) {
+            const int64_t gl = hb + lid, gr = hb + rid;
+            ranges[2 * gl] = begin;
+            ranges[2 * gl + 1] = begin + i;
+            ranges[2 * gr] = begin + i;
+            ranges[2 * gr + 1] = begin + n;
+        }
+        // (the next cell's first barrier stands before it rewrites any LDS
+        // that a wave still reads here)
+    }
+}
+
+// ---------------------------------------------------------------------------
 // orchestration
 // ---------------------------------------------------------------------------
 static int ensure_state(Ctx &c, int32_t levels_mode, bool *complete)
@@ -2283,13 +2607,17 @@ int enqueue_level(Ctx &c, const LevelEntry *entries, int32_t nCells, orb_cell *h
                   uint8_t *exists, uint8_t *sub, uint16_t *chunk_hist, uint32_t *cell_hist,
                   uint64_t *trace, int32_t *level_passes, int32_t *status, bool any_subtree,
                   bool full_cover, int32_t level, uint64_t *chunk_hist_w, uint64_t *cell_hist_w,
-                  const PendingFinal *fin_in, bool defer_final)
+                  const PendingFinal *fin_in, bool defer_final, const LevelKernels &kernels)
 {
     if (c.weighted && (!chunk_hist_w || !cell_hist_w)) return ORB_ERR_STATE;
     if (!c.weighted && (c.sel.n < (size_t)c.stride || c.sel_lists.n < (size_t)c.max_chunks + 1))
         return ORB_ERR_STATE;  // rounds 3 and 4 gather into these
     const int32_t sub_max = subtree_max_keys(c);
     const bool use_subtree = any_subtree && c.part == ORB_PART_HOARE && sub_max > 0;
+    if ((kernels.cell_max || !kernels.chunks) && (c.part != ORB_PART_HOARE || c.weighted))
+        return ORB_ERR_STATE;
+    const LevelMode mode{use_subtree ? (uint32_t)sub_max : 0u, kernels.cell_max,
+                         kernels.chunks ? 1 : 0, kernels.again ? 1 : 0};
     const int32_t cgroup = cell_group(nCells);
     // Chunk order: the first round walks the level's chunks from the last, so
     // it starts with the chunks the previous level's swap wrote last (still in
@@ -2314,19 +2642,20 @@ int enqueue_level(Ctx &c, const LevelEntry *entries, int32_t nCells, orb_cell *h
     if (nCells < kRecsScan) {
         const unsigned gf = (unsigned)((fin.nCells + kRecsScan - 1) / kRecsScan);
         hipLaunchKernelGGL(k_b_recs_scan, dim3(1 + gf), dim3(kRecsScan), 0, c.stream, entries, nCells,
-                           heap, c.ranges.p, sub, use_subtree ? 1 : 0, (uint32_t)sub_max, c.recs.p,
-                           c.cell_first.p, fin);
+                           heap, exists, c.ranges.p, sub, mode, c.recs.p, c.cell_first.p,
+                           level_passes, fin);
         ORB_HIP(hipGetLastError());
     } else {
         unsigned g1 = (unsigned)((nCells + 1 + kBlock - 1) / kBlock);
         const unsigned gf = (unsigned)((fin.nCells + kBlock - 1) / kBlock);
         hipLaunchKernelGGL(k_b_recs, dim3(g1 + gf), dim3(kBlock), 0, c.stream, entries, nCells, heap,
-                           c.ranges.p, sub, use_subtree ? 1 : 0, (uint32_t)sub_max, c.recs.p,
-                           c.cell_nchunks.p, g1, fin);
+                           exists, c.ranges.p, sub, mode, c.recs.p, c.cell_nchunks.p, level_passes,
+                           g1, fin);
         ORB_HIP(hipGetLastError());
-        ORB_TRY(scan_exclusive_u32(c, c.cell_nchunks.p, c.cell_first.p, (size_t)nCells + 1));
+        if (kernels.chunks)
+            ORB_TRY(scan_exclusive_u32(c, c.cell_nchunks.p, c.cell_first.p, (size_t)nCells + 1));
     }
-    {
+    if (kernels.chunks) {
         // the chunk table, and the first round's candidate tables (not used
         // by weighted builds)
         const int tb = timing_mark(c);
@@ -2363,6 +2692,19 @@ int enqueue_level(Ctx &c, const LevelEntry *entries, int32_t nCells, orb_cell *h
                            status, c.ids(), c.weights(), group);
         ORB_HIP(hipGetLastError());
     }
+    if (kernels.cell_max) {
+        const bool payload = c.ids() != nullptr;
+        const bool large = kernels.cell_max > kCellSmall, many = nCells > kCellManyCells;
+        auto cell = large  ? (payload ? k_b_cell<1024, 40, 4> : k_b_cell<1024, 40, 3>)
+                    : many ? (payload ? k_b_cell<512, 40, 4> : k_b_cell<512, 40, 3>)
+                           : (payload ? k_b_cell<1024, 20, 4> : k_b_cell<1024, 20, 3>);
+        hipLaunchKernelGGL(cell, dim3((unsigned)std::min<int32_t>(nCells, 65536)),
+                           dim3(!large && many ? 512 : 1024), 0, c.stream, c.recs.p, nCells, heap,
+                           exists, c.ranges.p, c.x(), c.y(), c.z(), c.ids(), c.weights(), le, trace,
+                           level_passes, status);
+        ORB_HIP(hipGetLastError());
+    }
+    if (!kernels.chunks) return ORB_OK;
     const unsigned gq = chunk_grid(c);
     const unsigned gr = (unsigned)((gq + kReduceRows - 1) / kReduceRows);  // a block per 64-row tile
     const unsigned gw = (unsigned)((nCells + 3) / 4);
@@ -2466,28 +2808,56 @@ int enqueue_level(Ctx &c, const LevelEntry *entries, int32_t nCells, orb_cell *h
     return ORB_OK;
 }
 
+// The kernels of a level whose cells are expected to hold lo to hi keys
+// (counts within the termination rule's +-2 a split of the exact shares, four
+// a level allowed for).  k_b_cell takes a level of cells that fit its
+// registers in two launches where the chunk path needs sixteen and reads the
+// keys once, not twice; a level whose every cell fits it or the subtree kernel
+// goes without the chunk kernels.
+static LevelKernels level_kernels(const Ctx &c, int32_t level, int64_t lo, int64_t hi, bool all_sub)
+{
+    LevelKernels k;
+    if (c.part != ORB_PART_HOARE || c.weighted || lo < 0) return k;
+    hi += 4 * (int64_t)level;
+    lo -= 4 * (int64_t)level;
+    if (all_sub) {
+        k.chunks = false;
+        return k;
+    }
+    if (lo <= (int64_t)kCellLarge) k.cell_max = hi <= (int64_t)kCellSmall ? kCellSmall : kCellLarge;
+    k.chunks = hi > (int64_t)kCellLarge;
+    return k;
+}
+
 // All launches of one batched build, in stream order; no allocation, no
-// host synchronisation, no memset: the sequence can be captured.
-static int enqueue_build(Ctx &c, int32_t levels_mode)
+// host synchronisation, no memset: the sequence can be captured.  again: the
+// levels once more over a build whose launches left cells alone (LevelMode),
+// with every kernel and without the fresh start.
+static int enqueue_build(Ctx &c, int32_t levels_mode, bool again)
 {
     BatchedState &b = *c.batched;
     uint64_t *trace = c.trace ? b.trace.p : nullptr;
     const int64_t trace_n = c.trace ? c.cap * ORB_MAX_PASSES : 0;
     const orb_cell root = cell_root(c.d);
-    hipLaunchKernelGGL(k_b_init, dim3(1024), dim3(kBlock), 0, c.stream, b.heap.p, b.exists.p,
-                       b.sub.p, (int64_t)c.cap, root, trace, trace_n, b.level_passes.p, c.ranges.p,
-                       (uint32_t)c.n, c.status.p);
-    ORB_HIP(hipGetLastError());
+    if (again) {
+        ORB_TRY(launch_zero_u32(c.stream, reinterpret_cast<uint32_t *>(b.level_passes.p), 1));
+    } else {
+        hipLaunchKernelGGL(k_b_init, dim3(1024), dim3(kBlock), 0, c.stream, b.heap.p, b.exists.p,
+                           b.sub.p, (int64_t)c.cap, root, trace, trace_n, b.level_passes.p,
+                           c.ranges.p, (uint32_t)c.n, c.status.p);
+        ORB_HIP(hipGetLastError());
+    }
     const int32_t lmax = levels_mode == ORB_LEVELS_REFERENCE ? b.D - 1 : b.D;
-    // chunks each level expects, for the chunk kernels' grids: cells split
-    // by count, so a level's cell sizes follow from n and d (orb_level_shape,
-    // within the termination rule's +-2 a split); below a level whose every
-    // cell goes to the subtree kernel nothing is left.  Weighted builds split
-    // by weight: unknown.
+    // the cell sizes each level expects: cells split by count, so they follow
+    // from n and d (orb_level_shape, within the termination rule's +-2 a
+    // split).  They give the chunk kernels' grids and the level's kernels;
+    // where every cell of a level is expected to finish in the subtree
+    // kernel, the build ends there.  Weighted builds split by weight: unknown.
     c.level_chunk_hint.assign((size_t)lmax + 2, -1);
-    if (!c.weighted) {
+    std::vector<LevelKernels> kernels((size_t)lmax + 2);
+    int32_t last = lmax;
+    if (!c.weighted && !again) {
         const int32_t sub_max = subtree_max_keys(c);
-        bool done = false;
         for (int32_t l = 1; l <= lmax; ++l) {
             int64_t lo = 0, hi = 0;
             const int cells = orb_level_shape(c.n, c.d, l, &lo, &hi);
@@ -2495,14 +2865,18 @@ static int enqueue_build(Ctx &c, int32_t levels_mode)
             const int64_t max_leaf = ((int64_t)c.d + (int64_t(1) << (l - 1)) - 1) >> (l - 1);
             const bool all_sub = b.complete && c.part == ORB_PART_HOARE && sub_max > 0 &&
                                  hi + 4 * l <= sub_max && max_leaf <= kSmallLeaves;
-            c.level_chunk_hint[(size_t)l] = (done || all_sub) ? 0 : c.n / kChunk + cells + 1;
-            done = done || all_sub;
+            c.level_chunk_hint[(size_t)l] = c.n / kChunk + cells + 1;
+            kernels[(size_t)l] = level_kernels(c, l, cells > 0 ? lo : -1, hi, all_sub);
+            if (all_sub) {
+                last = l;
+                break;
+            }
         }
     }
     // a level's last Hoare row swaps run in the next level's first launch;
     // the last level's at the end
     PendingFinal fin;
-    for (int32_t l = 1; l <= lmax; ++l) {
+    for (int32_t l = 1; l <= last; ++l) {
         const int32_t nCells = b.level_n[(size_t)l];
         if (nCells == 0) continue;
         const int tlevel = timing_mark(c);
@@ -2514,14 +2888,18 @@ static int enqueue_build(Ctx &c, int32_t levels_mode)
         const int64_t few = c.n * (int64_t)b.level_min_leaf[(size_t)l] / (c.d > 0 ? c.d : 1);
         const bool may_sub = few <= 4 * (int64_t)subtree_max_keys(c);
         const LevelEntry *entries = b.level_ids.p + b.level_off[(size_t)l];
+        LevelKernels k = kernels[(size_t)l];
+        k.again = again;
         ORB_TRY(enqueue_level(c, entries, nCells, b.heap.p, b.exists.p, b.sub.p, b.chunk_hist.p,
                               b.cell_hist.p, trace, b.level_passes.p, c.status.p,
                               b.complete && may_sub, b.level_cover[(size_t)l] != 0, l,
-                              b.chunk_hist_w.p, b.cell_hist_w.p, &fin, true));
+                              b.chunk_hist_w.p, b.cell_hist_w.p, &fin, true, k));
         fin.entries = entries;
-        fin.nCells = c.part == ORB_PART_HOARE ? nCells : 0;
+        fin.nCells = c.part == ORB_PART_HOARE && k.chunks ? nCells : 0;
         ORB_TRY(timing_pair(c, tlevel, kTimeLevel + l));
     }
+    for (int32_t l = last + 1; l <= lmax; ++l)  // nothing left: their time is the marks'
+        if (b.level_n[(size_t)l]) ORB_TRY(timing_pair(c, timing_mark(c), kTimeLevel + l));
     if (fin.nCells > 0) ORB_TRY(launch_hoare_final(c, fin.nCells));
     return particles_home(c);  // in-stream: the capture ends where it began
 }
@@ -2550,7 +2928,7 @@ int build_batched(Ctx &c, int32_t levels_mode, orb_build_info *info)
         if (!b.exec || sig != b.gsig) {
             drop_graph(b);
             ORB_HIP(hipStreamBeginCapture(c.stream, hipStreamCaptureModeThreadLocal));
-            int rc = enqueue_build(c, levels_mode);
+            int rc = enqueue_build(c, levels_mode, false);
             hipGraph_t g = nullptr;
             hipError_t e = hipStreamEndCapture(c.stream, &g);
             if (rc < 0) {
@@ -2564,17 +2942,27 @@ int build_batched(Ctx &c, int32_t levels_mode, orb_build_info *info)
         }
         ORB_HIP(hipGraphLaunch(b.exec, c.stream));
     } else {
-        ORB_TRY(enqueue_build(c, levels_mode));
+        ORB_TRY(enqueue_build(c, levels_mode, false));
     }
     c.table_ids.clear();
 
     // status and pass counts come back now; the tree stays in HBM until a
     // getter asks for it (batched_pull_results)
-    ORB_HIP(hipMemcpyAsync(c.hstatus.p, c.status.p, 2 * sizeof(int32_t), hipMemcpyDeviceToHost,
-                           c.stream));
-    ORB_HIP(hipMemcpyAsync(b.hpasses.p, b.level_passes.p, 64 * sizeof(int32_t),
-                           hipMemcpyDeviceToHost, c.stream));
-    ORB_HIP(hipStreamSynchronize(c.stream));
+    auto pull_status = [&]() -> int {
+        ORB_HIP(hipMemcpyAsync(c.hstatus.p, c.status.p, 2 * sizeof(int32_t), hipMemcpyDeviceToHost,
+                               c.stream));
+        ORB_HIP(hipMemcpyAsync(b.hpasses.p, b.level_passes.p, 64 * sizeof(int32_t),
+                               hipMemcpyDeviceToHost, c.stream));
+        ORB_HIP(hipStreamSynchronize(c.stream));
+        return ORB_OK;
+    };
+    ORB_TRY(pull_status());
+    if (b.hpasses.p[0] > 0) {
+        // cells larger than their level's kernels expected (keys that tie at
+        // a cut do not split evenly) were left alone: the rest of the build
+        ORB_TRY(enqueue_build(c, levels_mode, true));
+        ORB_TRY(pull_status());
+    }
     c.results_on_device = true;
     ORB_TRY(timing_collect(c));
     const int32_t lmax = levels_mode == ORB_LEVELS_REFERENCE ? b.D - 1 : b.D;

@@ -387,7 +387,8 @@ struct CellRec {
     float margin_l;     // cutMarginLeft
     float margin_r;     // cutMarginRight
     int32_t id;         // heap id
-    int32_t flags;      // batched form: 0 active, 1 inside a finished subtree, 2 small (subtree kernel)
+    int32_t flags;      // batched form: 0 active (chunk kernels), 1 not taken on this level (inside a
+                        // finished subtree, ...), 2 subtree kernel, 3 k_b_cell
     int32_t passes;     // batched form: bisection passes so far
     // where the cell's build keeps its state (several builds can share a
     // launch): heap/range/flag index = hb + id, the build's heap capacity,
@@ -611,6 +612,14 @@ struct PendingFinal {
     const LevelEntry *entries = nullptr;
     int32_t nCells = 0;
 };
+// The kernels a level of the batched form launches beside the subtree
+// kernel: the chunk path, and k_b_cell for cells of at most cell_max keys (0:
+// none).  again: only cells that are not split yet.
+struct LevelKernels {
+    bool chunks = true;
+    uint32_t cell_max = 0;
+    bool again = false;
+};
 // one level step of the batched form over `entries` (device array)
 // (chunk_hist_w, cell_hist_w: the weighted rounds' rows, when c.weighted;
 // fin_in: the previous level's due row swaps, run in this level's first
@@ -620,7 +629,7 @@ int enqueue_level(Ctx &c, const LevelEntry *entries, int32_t nCells, orb_cell *h
                   uint64_t *trace, int32_t *level_passes, int32_t *status, bool any_subtree,
                   bool full_cover, int32_t level, uint64_t *chunk_hist_w = nullptr,
                   uint64_t *cell_hist_w = nullptr, const PendingFinal *fin_in = nullptr,
-                  bool defer_final = false);
+                  bool defer_final = false, const LevelKernels &kernels = LevelKernels());
 int preallocate_scratch(Ctx &c);
 // level tables for nCells cells and (at least) `chunks` chunks
 int ensure_level_capacity(Ctx &c, int64_t nCells, int64_t chunks = 0);

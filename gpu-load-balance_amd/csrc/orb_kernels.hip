@@ -979,39 +979,6 @@ __global__ __launch_bounds__(kBlock) void k_hoare_masks_window(
     }
 }
 
-__device__ inline uint32_t lo32(uint64_t v) { return (uint32_t)v; }
-__device__ inline uint32_t hi32(uint64_t v) { return (uint32_t)(v >> 32); }
-
-// Last k in [lo, hi) with pred(k), given pred(lo) and pred true then false
-// over [lo, hi): a 64-way search, one ballot per step.  Every lane calls
-// pred on every step (with lo where its probe is out of range), so pred
-// may shuffle.
-template <class Pred>
-__device__ inline uint32_t wave_last_true(uint32_t lo, uint32_t hi, Pred pred)
-{
-    const int lane = threadIdx.x & 63;
-    while (hi - lo > 1u) {
-        const uint32_t span = hi - lo;
-        const bool dense = span <= 65u;
-        auto probe = [&](uint32_t j) {
-            return dense ? lo + 1u + j : lo + (uint32_t)(((uint64_t)(j + 1u) * span) / 65u);
-        };
-        const uint32_t k = probe((uint32_t)lane);
-        const bool valid = k < hi;
-        const bool pr = pred(valid ? k : lo) && valid;
-        const uint64_t m = __ballot(pr);
-        if (m == 0ull) {
-            hi = probe(0u);
-        } else {
-            const uint32_t j = 63u - (uint32_t)__clzll((long long)m);
-            const uint32_t kn = j < 63u ? probe(j + 1u) : hi;
-            lo = probe(j);
-            hi = kn < hi ? kn : hi;
-        }
-    }
-    return lo;
-}
-
 // A chunk's mask of one side, word `lane` in each lane, with the exclusive
 // prefix of the words' popcounts.
 __device__ inline void load_mask(const uint64_t *masks, uint32_t q, int side, uint64_t &word,
@@ -1021,34 +988,6 @@ __device__ inline void load_mask(const uint64_t *masks, uint32_t q, int side, ui
     word = masks[(size_t)q * (2 * kMaskWords) + (size_t)side * kMaskWords + (uint32_t)lane];
     const uint32_t c = (uint32_t)__popcll(word);
     ex = wave_inclusive_scan(c) - c;
-}
-
-// Chunk position (0..4095) of the set bit of rank r of a mask held as by
-// load_mask.  Each lane asks for its own r (below the mask's popcount); all
-// lanes call (shuffles).
-__device__ inline uint32_t wave_select(uint64_t word, uint32_t ex, uint32_t r)
-{
-    int k = 0;  // the last word whose prefix is <= r holds the bit
-#pragma unroll
-    for (int s = 32; s > 0; s >>= 1) {
-        const uint32_t e = (uint32_t)__shfl((int)ex, k + s, 64);
-        if (e <= r) k += s;
-    }
-    const uint32_t wl = (uint32_t)__shfl((int)(uint32_t)word, k, 64);
-    const uint32_t wh = (uint32_t)__shfl((int)(uint32_t)(word >> 32), k, 64);
-    uint32_t rr = r - (uint32_t)__shfl((int)ex, k, 64);
-    uint64_t wd = ((uint64_t)wh << 32) | wl;
-    uint32_t bit = 0;
-#pragma unroll
-    for (int s = 32; s > 0; s >>= 1) {
-        const uint32_t c = (uint32_t)__popcll(wd & ((1ull << s) - 1ull));
-        if (rr >= c) {
-            rr -= c;
-            bit += (uint32_t)s;
-            wd >>= s;
-        }
-    }
-    return 64u * (uint32_t)k + bit;
 }
 
 // The chunk offsets of one cell: side 0 counts L-stoppers, side 1
@@ -1194,66 +1133,6 @@ __device__ inline void side_range(int side, const SwapUnit &u, uint32_t TR, uint
 // Swaps m pairs: positions sl[j] and sr[j] (cell-local) for j < m, with
 // kSwapBatch pairs per thread in flight (all loads, then all stores).
 constexpr int kSwapBatch = 8;
-
-// Particle arrays seen from a cell's first particle: x, y, z, then the
-// payload arrays that move with them (ids, weights), whichever are on, in
-// that order (`count` of them).  Narrow: raw buffer accesses with 32-bit
-// byte offsets over one descriptor per array (one address register per
-// access; the cell holds fewer than 2^30 particles).  Wide: plain 64-bit
-// addressing.
-template <bool kNarrow>
-struct CellArrays;
-
-template <>
-struct CellArrays<true> {
-    __amdgpu_buffer_rsrc_t a[5];
-    int count;
-    __device__ CellArrays(float *x, float *y, float *z, uint32_t *pid, uint32_t *w, uint32_t begin)
-    {
-        // raw buffer, 32-bit data format, no range limit below 4 GiB
-        a[0] = __builtin_amdgcn_make_buffer_rsrc(x + begin, 0, -1, 0x00020000);
-        a[1] = __builtin_amdgcn_make_buffer_rsrc(y + begin, 0, -1, 0x00020000);
-        a[2] = __builtin_amdgcn_make_buffer_rsrc(z + begin, 0, -1, 0x00020000);
-        uint32_t *p3 = pid ? pid : w, *p4 = pid ? w : nullptr;
-        a[3] = __builtin_amdgcn_make_buffer_rsrc(p3 ? p3 + begin : nullptr, 0, -1, 0x00020000);
-        a[4] = __builtin_amdgcn_make_buffer_rsrc(p4 ? p4 + begin : nullptr, 0, -1, 0x00020000);
-        count = 3 + (pid ? 1 : 0) + (w ? 1 : 0);
-    }
-    using Off = uint32_t;
-    __device__ uint32_t load(int arr, Off o) const
-    {
-        return __builtin_amdgcn_raw_buffer_load_b32(a[arr], (int)o, 0, 0);
-    }
-    __device__ void store(int arr, Off o, uint32_t v) const
-    {
-        __builtin_amdgcn_raw_buffer_store_b32(v, a[arr], (int)o, 0, 0);
-    }
-};
-
-template <>
-struct CellArrays<false> {
-    char *a[5];
-    int count;
-    __device__ CellArrays(float *x, float *y, float *z, uint32_t *pid, uint32_t *w, uint32_t begin)
-    {
-        a[0] = reinterpret_cast<char *>(x + begin);
-        a[1] = reinterpret_cast<char *>(y + begin);
-        a[2] = reinterpret_cast<char *>(z + begin);
-        uint32_t *p3 = pid ? pid : w, *p4 = pid ? w : nullptr;
-        a[3] = reinterpret_cast<char *>(p3 ? p3 + begin : nullptr);
-        a[4] = reinterpret_cast<char *>(p4 ? p4 + begin : nullptr);
-        count = 3 + (pid ? 1 : 0) + (w ? 1 : 0);
-    }
-    using Off = uint64_t;
-    __device__ uint32_t load(int arr, Off o) const
-    {
-        return *reinterpret_cast<const uint32_t *>(a[arr] + o);
-    }
-    __device__ void store(int arr, Off o, uint32_t v) const
-    {
-        *reinterpret_cast<uint32_t *>(a[arr] + o) = v;
-    }
-};
 
 // kArrays: the most arrays this instantiation moves (3 without payload, up
 // to 5 with ids and weights): the register arrays are sized by it.

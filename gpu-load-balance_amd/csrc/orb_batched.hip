@@ -171,14 +171,15 @@ __global__ void k_b_init(orb_cell *heap, uint8_t *exists, uint8_t *sub, int64_t 
 
 // Which kernels a level's launches hold, for its cell records: cells of at
 // most sub_max keys (and kSmallLeaves leaves) go to the subtree kernel, cells
-// of at most cell_max keys to k_b_cell (0: not launched), the others to the
-// chunk kernels.  A level without chunk kernels (chunks = 0, chosen from the
-// sizes the host expects) leaves a larger cell alone and counts it in the
-// build's pass counter 0; the host then runs the levels again with every
-// kernel (again = 1), which skips the cells that are split already.
+// of at most cell_max keys to k_b_cell (0: not launched), cells of at most
+// chunk_max keys to the chunk kernels.  A level whose kernels do not take
+// every size (chosen from the sizes the host expects) leaves a larger cell
+// alone and counts it in the build's pass counter 0; the host then runs the
+// levels again with the chunk path (again = 1), which skips the cells that
+// are split already.
 struct LevelMode {
-    uint32_t sub_max, cell_max;
-    int32_t chunks, again;
+    uint32_t sub_max, cell_max, chunk_max;
+    int32_t again;
 };
 constexpr int kFlagBlock = 3;  // CellRec.flags: the cell goes to k_b_cell
 
@@ -219,7 +220,7 @@ __device__ inline uint32_t level_rec(const LevelEntry *entries, int32_t i, const
         r.flags = 2;
     } else if (mode.cell_max && n <= mode.cell_max) {
         r.flags = kFlagBlock;
-    } else if (mode.chunks) {
+    } else if (n <= mode.chunk_max) {
         r.flags = 0;
     } else {
         r.flags = 1;
@@ -261,13 +262,16 @@ __global__ void k_b_recs(const LevelEntry *entries, int32_t nCells, const orb_ce
 // A level of fewer than kRecsScan cells in one block of kRecsScan threads,
 // a cell per thread: the cell records and the exclusive scan of their chunk
 // counts into first[] (first[nCells] = the level's chunks), in place of a
-// record launch and a scan launch.
+// record launch and a scan launch.  kFill (levels of few chunks): the block
+// also fills the chunk records and clears the cells' key counters.
 constexpr int kRecsScan = 1024;
+template <bool kFill>
 __global__ __launch_bounds__(kRecsScan) void k_b_recs_scan(
     const LevelEntry *__restrict__ entries, int32_t nCells, const orb_cell *__restrict__ heap,
     const uint8_t *__restrict__ exists, const uint32_t *__restrict__ ranges,
-    const uint8_t *__restrict__ sub, LevelMode mode, CellRec *__restrict__ recs,
-    uint32_t *__restrict__ first, int32_t *__restrict__ level_passes, PendingFinalDev fin)
+    const uint8_t *__restrict__ sub, LevelMode mode, CellRec *recs,
+    uint32_t *__restrict__ first, int32_t *__restrict__ level_passes, uint4 *chunk_desc,
+    uint32_t max_chunks, unsigned long long *sel_lists, PendingFinalDev fin)
 {
     if (blockIdx.x > 0) {  // uniform: the previous level's row swaps
         level_finals(1u, fin, ranges);
@@ -275,6 +279,9 @@ __global__ __launch_bounds__(kRecsScan) void k_b_recs_scan(
     }
     constexpr int kW = kRecsScan / 64;
     __shared__ uint32_t wsum[kW];
+    __shared__ uint32_t s_first[kFill ? kRecsScan : 1], s_begin[kFill ? kRecsScan : 1];
+    __shared__ uint32_t s_end[kFill ? kRecsScan : 1];
+    __shared__ int32_t s_axis[kFill ? kRecsScan : 1];
     const int t = threadIdx.x, lane = t & 63, w = t >> 6;
     const uint32_t v =
         t < nCells ? level_rec(entries, t, heap, exists, ranges, sub, mode, recs, level_passes) : 0u;
@@ -284,6 +291,26 @@ __global__ __launch_bounds__(kRecsScan) void k_b_recs_scan(
     uint32_t pre = 0;
     for (int i = 0; i < w; ++i) pre += wsum[i];
     if (t <= nCells) first[t] = pre + inc - v;  // t = nCells: the level's chunk count
+    if constexpr (kFill) {
+        if (t <= nCells) s_first[t] = pre + inc - v;
+        if (t < nCells) {
+            const CellRec &r = recs[t];  // this thread's own
+            s_begin[t] = r.begin;
+            s_end[t] = r.end;
+            s_axis[t] = r.axis >= 0 && r.axis <= 2 ? r.axis : (int32_t)kChunkIdle;
+            if (v) sel_lists[pre + inc - v] = 0ull;
+        }
+        __syncthreads();
+        uint32_t total = s_first[nCells];
+        if (total > max_chunks) total = max_chunks;
+        for (uint32_t q = (uint32_t)t; q < total; q += kRecsScan) {
+            // every chunk of the table is searched (other cells have none)
+            const uint32_t cell = chunk_to_cell(s_first, nCells, q);
+            const uint32_t cb = s_begin[cell] + (q - s_first[cell]) * (uint32_t)kChunk, ce = s_end[cell];
+            chunk_desc[q] = make_uint4(cb, ce - cb < (uint32_t)kChunk ? ce : cb + (uint32_t)kChunk,
+                                       cell, (uint32_t)s_axis[cell]);
+        }
+    }
 }
 
 // in-order index t in [1, 255] of the depth-8 candidate tree on [lo, hi]
@@ -2529,6 +2556,458 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4, 4))
 }
 
 // ---------------------------------------------------------------------------
+// levels of few chunks whose cells are too large for k_b_cell
+// ---------------------------------------------------------------------------
+// A level of at most kMidLevelChunks chunks, its cells at most kMidChunks
+// chunks each, is bound by its launches, not by memory: the chunk path takes
+// 16 of them, 4-7 us each however little they do.  Here it takes five:
+//   k_b_recs_scan<true>  cell records, chunk table, the cells' key counters
+//   k_m_hist             round 1 per chunk, added to the cell's row (atomics:
+//                        few blocks share a row)
+//   k_m_window           every block replays round 1 from its cell's row (a
+//                        1 KB read in place of two launches), then takes the
+//                        window pass and appends its window keys to the cell's list
+//   k_m_tail             a block per cell: round 1 again, the later rounds over
+//                        the listed keys, the stopper masks, K, i and the swap plan
+//   k_hoare_swap
+// The same rounds, masks and plan as the chunk path's.  The five top levels of
+// 2^20 keys (1 to 16 cells): 53 us a level, from 89.  Past kMidLevelChunks the
+// atomics on the cells' rows and the tail's chunks per block cost what the
+// launches save (2^23 keys: within 5% of the chunk path).
+constexpr int kMidChunks = 512;         // per cell: k_m_tail's tables
+constexpr int64_t kMidLevelChunks = 2048;
+
+// Round 1 of a chunk's cell from the cell's row of counts (bins of every key
+// of the cell), by a whole wave.
+__device__ inline RoundOut replay_row(const uint32_t *row, const CellRec &r, int lane,
+                                      uint64_t *trace_row)
+{
+    const uint4 h4 = reinterpret_cast<const uint4 *>(row)[lane];
+    const uint32_t s0 = h4.x, s1 = s0 + h4.y, s2 = s1 + h4.z, s3 = s2 + h4.w;
+    const uint32_t base = wave_inclusive_scan(s3) - s3;
+    // P[4 lane + 1 + q] (P[j] = keys in bins below j)
+    const uint32_t pv[4] = {base + s0, base + s1, base + s2, base + s3};
+    const float target = difference_target(uniform(r.end) - uniform(r.begin),
+                                           (int32_t)uniform((uint32_t)r.nLeaf));
+    return replay_round_lanes(pv, uniform(r.margin_l), uniform(r.margin_r), target, 0, lane, trace_row);
+}
+
+// Round 1: as k_b_hist, without a candidate table (the exact bin of a key
+// near a bin edge comes from the walk) and with the chunk's row added to the
+// cell's.
+template <int LE>
+__global__ __launch_bounds__(kBlock) void k_m_hist(const CellRec *__restrict__ recs, int32_t nCells,
+                                                   const uint32_t *__restrict__ first,
+                                                   const uint4 *__restrict__ chunk_desc,
+                                                   uint32_t max_chunks, const float *__restrict__ x,
+                                                   const float *__restrict__ y,
+                                                   const float *__restrict__ z,
+                                                   uint32_t *__restrict__ cell_hist)
+{
+    constexpr int kW = kBlock / 64;
+    constexpr int kPerWave = kMaskWords / kW;  // 16 loads of 64 keys
+    __shared__ uint32_t hist[kW][kBins];
+    const int t = threadIdx.x, lane = t & 63, w = (int)uniform((uint32_t)t >> 6);
+    const uint32_t sb = (uint32_t)(w * kPerWave * 64);
+    const uint32_t total = first[nCells];
+    for (uint32_t q = blockIdx.x;; q += gridDim.x) {
+        const uint4 d = chunk_record(chunk_desc, q, max_chunks);
+        const uint32_t b = uniform(d.x), e = uniform(d.y), cell = uniform(d.z);
+        const uint32_t axis = uniform(d.w);
+        keep_values(b, e, cell, axis);
+        if (q >= total) break;
+        if (axis > 2u) continue;  // uniform: the cell is not searched
+        float v[kPerWave];
+        issue_chunk_loads(x, y, z, true, d, sb, lane, v);
+        const float lo = uniform(recs[cell].margin_l), hi = uniform(recs[cell].margin_r);
+#pragma unroll
+        for (int u = 0; u < kW; ++u) hist[u][t] = 0u;
+        __syncthreads();
+        const float width = hi - lo;
+        const float scale = width > 0.0f ? (float)kBins / width : 0.0f;
+        const float lim = 0.5f - bin_tolerance(lo, hi, scale);
+        const float limx = lim > 0.25f ? lim : -1.0f;  // as k_b_hist
+        const uint32_t len = e - b;
+        static_for<0, kPerWave>([&](auto jc) __attribute__((always_inline)) {
+            constexpr int j = decltype(jc)::value;
+            const bool ok = sb + 64u * (uint32_t)j + (uint32_t)lane < len;
+            const float ef = __builtin_amdgcn_fmed3f((v[j] - lo) * scale, -0.5f, 255.5f);
+            int bin = (int)ef;
+            const bool slow = ok && !(fabsf(__builtin_amdgcn_fractf(ef) - 0.5f) < limx);
+            if (__ballot(slow)) {  // wave-uniform; rare
+                if (slow) bin = bin_walk<LE>(v[j], lo, hi);
+            }
+            if (ok) atomicAdd(&hist[w][bin], 1u);
+        });
+        __syncthreads();
+        const uint32_t sum = hist[0][t] + hist[1][t] + hist[2][t] + hist[3][t];
+        if (sum) atomicAdd(&cell_hist[(size_t)cell * kBins + t], sum);
+        __syncthreads();  // the next chunk rewrites hist
+    }
+}
+
+// Window pass: as k_b_hist_window, from round 1's outcome, without binning:
+// the keys below and above the margins are counted, the keys inside go to the
+// chunk quarter's slots of `pack` (in position order, for the masks) and to
+// the cell's list in `sel` (in any order, for the rounds), whose counter
+// (keys | keys below << 32) takes one atomic a chunk.  A cell whose cut round
+// 1 found has that cut as its window.
+__global__ __launch_bounds__(kBlock) void k_m_window(
+    const CellRec *__restrict__ recs, int32_t nCells, const uint32_t *__restrict__ first,
+    const uint4 *__restrict__ chunk_desc, uint32_t max_chunks, const float *__restrict__ x,
+    const float *__restrict__ y, const float *__restrict__ z, const uint32_t *__restrict__ cell_hist,
+    float *__restrict__ pack, uint64_t *__restrict__ masks, float *__restrict__ sel,
+    unsigned long long *__restrict__ sel_lists)
+{
+    constexpr int kW = kBlock / 64;
+    constexpr int kPerWave = kMaskWords / kW;
+    __shared__ float wkeys[kW][kChunk / kW];  // each wave's window keys, packed
+    __shared__ uint32_t s_n[kW], s_below[kW], s_base;
+    __shared__ uint64_t words[kW][2][kPerWave];
+    const int t = threadIdx.x, lane = t & 63, w = (int)uniform((uint32_t)t >> 6);
+    const uint64_t lanes_below = lane == 0 ? 0ull : (~0ull >> (64 - lane));
+    const uint32_t sb = (uint32_t)(w * kPerWave * 64);
+    const uint32_t total = first[nCells];
+    for (uint32_t q = blockIdx.x;; q += gridDim.x) {
+        const uint4 d = chunk_record(chunk_desc, q, max_chunks);
+        const uint32_t b = uniform(d.x), e = uniform(d.y), cell = uniform(d.z);
+        const uint32_t axis = uniform(d.w);
+        keep_values(b, e, cell, axis);
+        if (q >= total) break;
+        if (axis > 2u) continue;  // uniform: the cell is not searched
+        float v[kPerWave];
+        issue_chunk_loads(x, y, z, true, d, sb, lane, v);
+        const CellRec &r = recs[cell];
+        const uint32_t begin = uniform(r.begin), f = uniform(first[cell]);
+        const RoundOut ro = replay_row(cell_hist + (size_t)cell * kBins, r, lane, nullptr);
+        const float cut = cell_cut(ro.L, ro.R);
+        const float lo = uniform(ro.found ? cut : ro.L), hi = uniform(ro.found ? cut : ro.R);
+        const uint32_t len = e - b;
+        uint32_t below = 0, packed = 0;  // wave-uniform
+        float *dst = pack + b + sb;
+        float *wk = wkeys[w];
+        static_for<0, kPerWave>([&](auto jc) __attribute__((always_inline)) {
+            constexpr int j = decltype(jc)::value;
+            const uint32_t p0 = sb + 64u * (uint32_t)j;  // chunk position of lane 0
+            const uint64_t valid =
+                p0 >= len ? 0ull : (len - p0 >= 64u ? ~0ull : (1ull << (len - p0)) - 1ull);
+            const uint64_t mB = __ballot(v[j] < lo) & valid;
+            const uint64_t mG = __ballot(v[j] > hi) & valid;
+            const uint64_t mW = valid & ~mB & ~mG;
+            below += (uint32_t)__popcll(mB);
+            if (lane == 0) {  // staged by one lane, as in k_b_hist_window
+                words[w][0][j] = mG;
+                words[w][1][j] = mW;
+            }
+            if (mW) {  // wave-uniform: most loads have no key in the window
+                if ((mW >> lane) & 1ull) {
+                    const uint32_t slot = packed + (uint32_t)__popcll(mW & lanes_below);
+                    dst[slot] = v[j];
+                    wk[slot] = v[j];
+                }
+                packed += (uint32_t)__popcll(mW);
+            }
+        });
+        if (lane == 0) {
+            s_n[w] = packed;
+            s_below[w] = below;
+        }
+        __syncthreads();
+        if (t == 0) {
+            const uint32_t ns = s_n[0] + s_n[1] + s_n[2] + s_n[3];
+            const uint32_t nb = s_below[0] + s_below[1] + s_below[2] + s_below[3];
+            s_base = ns || nb ? (uint32_t)atomicAdd(&sel_lists[f], (unsigned long long)ns |
+                                                                       ((unsigned long long)nb << 32))
+                              : 0u;
+        }
+        uint64_t *mq = masks + (size_t)q * (2 * kMaskWords) + w * kPerWave;
+        if (lane < kPerWave) {
+            mq[lane] = words[w][0][lane];
+            mq[kMaskWords + lane] = words[w][1][lane];
+        }
+        __syncthreads();
+        // the cell's list: from its first particle on (it holds at most the cell's keys)
+        uint32_t at = begin + s_base;
+        for (int u = 0; u < w; ++u) at += s_n[u];
+        for (uint32_t k = (uint32_t)lane; k < packed; k += 64u) sel[at + k] = wk[k];
+        __syncthreads();  // the next chunk rewrites the tables
+    }
+}
+
+// The rest of a cell's search and its split, a block per cell: round 1's
+// outcome, the later rounds over the listed keys (those inside the margins),
+// the cell's record and children, the stopper masks of its chunks from the
+// window pass's words and packed keys, the chunks' stopper offsets, K and i
+// as in k_b_cell (the crossing chunk, its word, its bit), the children's
+// ranges, and each chunk's swap unit as k_hoare_plan makes it.
+constexpr int kTailBlock = 1024;
+__global__ __launch_bounds__(kTailBlock) void k_m_tail(
+    CellRec *recs, int32_t nCells, const uint32_t *__restrict__ first, uint32_t *cell_hist,
+    const float *__restrict__ sel, const unsigned long long *__restrict__ sel_lists,
+    const float *__restrict__ pack, uint64_t *masks, uint64_t *chunk_pre, SplitRec *splits,
+    SwapPlan *plan, uint32_t *ranges, orb_cell *heap, uint8_t *exists, int le_cmp, uint64_t *trace,
+    int32_t *level_passes, int32_t *status)
+{
+    constexpr int kW = kTailBlock / 64;
+    __shared__ uint32_t hist[kBins];
+    __shared__ uint32_t preL[kMidChunks + 1], preR[kMidChunks + 1];
+    __shared__ uint64_t s_sum[kW];
+    __shared__ uint32_t s_cnt[kW];
+    __shared__ float s_lr[2];
+    __shared__ int32_t s_pf[2];
+    __shared__ uint32_t s_K, s_i, s_ks;
+    const int t = threadIdx.x, lane = t & 63, w = (int)uniform((uint32_t)t >> 6);
+    for (int32_t c = blockIdx.x; c < nCells; c += gridDim.x) {
+        const CellRec &rec = recs[c];  // this block alone writes it
+        if (uniform((uint32_t)rec.flags) != 0u) {
+            if (t == 0) splits[c] = SplitRec{0u, 0u, 0u, 0u};
+            continue;  // uniform
+        }
+        const uint32_t begin = uniform(rec.begin), n = uniform(rec.end) - begin;
+        const int32_t id = (int32_t)uniform((uint32_t)rec.id), hb = (int32_t)uniform((uint32_t)rec.hb);
+        const uint32_t f = uniform(first[c]), nch = uniform(first[c + 1]) - f;
+        if (nch > (uint32_t)kMidChunks) {
+            // the level records hand over at most kMidChunks; refuse anything else
+            if (t == 0) {
+                report_error(status + rec.st, rec.lp & 63, kErrSplit, id);
+                splits[c] = SplitRec{0u, 0u, 0u, 0u};
+            }
+            continue;
+        }
+        uint64_t *trow = trace ? trace + ((size_t)hb + id) * ORB_MAX_PASSES : nullptr;
+        uint32_t *row = cell_hist + (size_t)c * kBins;
+        const RoundOut r1 = replay_row(row, rec, lane, w == 0 ? trow : nullptr);
+        float lo = uniform(r1.L), hi = uniform(r1.R);
+        int32_t passes = r1.passes;
+        bool found = r1.found;
+        const unsigned long long list = n ? sel_lists[f] : 0ull;
+        const uint32_t m = uniform((uint32_t)list) < n ? uniform((uint32_t)list) : n;
+        const uint32_t nbelow = uniform((uint32_t)(list >> 32));
+        const float target = difference_target(n, (int32_t)uniform((uint32_t)rec.nLeaf));
+        if (t < kBins) hist[t] = 0u;
+        __syncthreads();  // every wave has read the row
+        if (t < kBins) row[t] = 0u;  // the next level adds to zero
+        while (!found && passes < ORB_MAX_PASSES) {
+            const float width = hi - lo;
+            const float scale = width > 0.0f ? (float)kBins / width : 0.0f;
+            const float lim = 0.5f - bin_tolerance(lo, hi, scale);
+            uint32_t below = 0;  // wave-uniform
+            for (uint32_t k0 = 0; k0 < m; k0 += 4u * kTailBlock) {
+                float v[4];
+                bool in[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    const uint32_t k = k0 + (uint32_t)(u * kTailBlock + t);
+                    in[u] = k < m;
+                    v[u] = in[u] ? sel[begin + k] : 0.0f;
+                }
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    const bool lt = in[u] && v[u] < lo, on = in[u] && !(v[u] < lo) && !(v[u] > hi);
+                    below += (uint32_t)__popcll(__ballot(lt));
+                    if (!on) continue;
+                    int bin;
+                    if (!bin_estimate(v[u], lo, scale, lim, bin))
+                        bin = le_cmp ? bin_walk<1>(v[u], lo, hi) : bin_walk<0>(v[u], lo, hi);
+                    atomicAdd(&hist[bin], 1u);
+                }
+            }
+            if (lane == 0 && below) atomicAdd(&hist[0], below);
+            if (t == 0 && nbelow) atomicAdd(&hist[0], nbelow);  // the keys below the window
+            __syncthreads();
+            if (w == 0) {
+                const uint4 h4 = reinterpret_cast<const uint4 *>(hist)[lane];
+                reinterpret_cast<uint4 *>(hist)[lane] = make_uint4(0u, 0u, 0u, 0u);
+                const uint32_t s0 = h4.x, s1 = s0 + h4.y, s2 = s1 + h4.z, s3 = s2 + h4.w;
+                const uint32_t base = wave_inclusive_scan(s3) - s3;
+                const uint32_t pv[4] = {base + s0, base + s1, base + s2, base + s3};
+                const RoundOut ro = replay_round_lanes(pv, lo, hi, target, passes, lane, trow);
+                if (lane == 0) {
+                    s_lr[0] = ro.L;
+                    s_lr[1] = ro.R;
+                    s_pf[0] = ro.passes;
+                    s_pf[1] = ro.found ? 1 : 0;
+                }
+            }
+            __syncthreads();
+            lo = uniform(s_lr[0]);
+            hi = uniform(s_lr[1]);
+            passes = (int32_t)uniform((uint32_t)s_pf[0]);
+            found = uniform((uint32_t)s_pf[1]) != 0u;
+        }
+        const float cut = cell_cut(lo, hi);
+        // ---- stopper masks: a wave per kPer chunks, a word per lane
+        constexpr int kPer = 4;
+        for (uint32_t k0 = (uint32_t)(w * kPer); k0 < nch; k0 += (uint32_t)(kW * kPer)) {
+            uint64_t G[kPer], W[kPer];
+            float v0[kPer];
+            const float *pk[kPer];
+#pragma unroll
+            for (int u = 0; u < kPer; ++u) {
+                const uint32_t k = k0 + (uint32_t)u < nch ? k0 + (uint32_t)u : nch - 1u;
+                const uint64_t *mq = masks + (size_t)(f + k) * (2 * kMaskWords);
+                G[u] = mq[lane];
+                W[u] = mq[kMaskWords + lane];
+            }
+#pragma unroll
+            for (int u = 0; u < kPer; ++u) {
+                const uint32_t k = k0 + (uint32_t)u < nch ? k0 + (uint32_t)u : nch - 1u;
+                const uint32_t cw = (uint32_t)__popcll(W[u]);
+                const uint32_t ex = wave_inclusive_scan(cw) - cw;
+                const int q0 = lane & ~15;  // first word of this lane's quarter
+                const uint32_t rank = ex - (uint32_t)__shfl((int)ex, q0, 64);
+                pk[u] = pack + begin + k * (uint32_t)kChunk + 64u * (uint32_t)q0 + rank;
+                v0[u] = W[u] ? *pk[u] : 0.0f;
+            }
+#pragma unroll
+            for (int u = 0; u < kPer; ++u) {
+                const uint32_t k = k0 + (uint32_t)u;
+                if (k >= nch) break;  // uniform
+                const uint32_t p0 = k * (uint32_t)kChunk + 64u * (uint32_t)lane;
+                const uint64_t valid =
+                    p0 >= n ? 0ull : (n - p0 >= 64u ? ~0ull : (1ull << (n - p0)) - 1ull);
+                uint64_t L = G[u], R = valid & ~G[u] & ~W[u], wd = W[u];
+                float vk = v0[u];
+                const float *at = pk[u];
+                while (wd) {
+                    const uint32_t bit = (uint32_t)__builtin_ctzll(wd);
+                    wd &= wd - 1ull;
+                    L |= (!(vk < cut) ? 1ull : 0ull) << bit;
+                    R |= (!(vk > cut) ? 1ull : 0ull) << bit;
+                    if (wd) vk = *++at;
+                }
+                uint64_t *mq = masks + (size_t)(f + k) * (2 * kMaskWords);
+                mq[lane] = L;
+                mq[kMaskWords + lane] = R;
+                const uint32_t nl = wave_sum((uint32_t)__popcll(L));
+                const uint32_t nr = wave_sum((uint32_t)__popcll(R));
+                if (lane == 0) {
+                    preL[k] = nl;
+                    preR[k] = nr;
+                }
+            }
+        }
+        __syncthreads();
+        // ---- the chunks' stopper offsets, a chunk per thread
+        const uint64_t mine = (uint32_t)t < nch ? (uint64_t)preL[t] | ((uint64_t)preR[t] << 32) : 0ull;
+        const uint64_t inc = wave_inclusive_scan(mine);
+        if (lane == 63) s_sum[w] = inc;
+        __syncthreads();
+        const uint64_t ws = lane < kW ? s_sum[lane] : 0ull;
+        const uint64_t wp = wave_inclusive_scan(ws);
+        const uint64_t all = lane_value(wp, 63);
+        const uint64_t off = inc - mine + lane_value(wp, w) - lane_value(ws, w);
+        const uint32_t TL = lo32(all), TR = hi32(all);
+        if ((uint32_t)t <= nch && t <= kMidChunks) {
+            preL[t] = lo32(off);
+            preR[t] = hi32(off);
+            chunk_pre[f + (uint32_t)c + (uint32_t)t] = off;
+        }
+        if (t == 64)  // the cell's margins, its passes, its children
+            finish_round(rec, c, RoundOut{lo, hi, passes, found, 0}, found ? 1 : 0, recs, heap,
+                         level_passes, exists, status);
+        const int64_t lid = left_child_id(id), rid = right_child_id(id);
+        if (n == 0u || TL == 0u || rid >= (int64_t)(int32_t)uniform((uint32_t)rec.capr)) {
+            // empty cell or no key >= cut: the reference's loop leaves the cell
+            if (t == 0) {
+                report_error(status + rec.st, rec.lp & 63, kErrPartition, id);
+                splits[c] = SplitRec{0u, 0u, 0u, 0u};  // the swap skips the cell
+            }
+            for (uint32_t k = (uint32_t)t; k < nch; k += kTailBlock)
+                reinterpret_cast<uint4 *>(plan + f + k)[0] = make_uint4(~0u, 0u, 0u, 0u);
+            __syncthreads();  // the next cell rewrites the tables
+            continue;  // uniform
+        }
+        // ---- K and i (see k_b_cell); A and B at this thread's chunk
+        const uint32_t cA = lo32(off), cB = TR - hi32(off);
+        auto last_chunk = [&](bool pred) {  // the last chunk where pred holds (true, then false)
+            const uint64_t mb = __ballot((uint32_t)t < nch && pred);
+            if (lane == 0) s_cnt[w] = (uint32_t)__popcll(mb);
+            __syncthreads();
+            if (t == 0) {
+                uint32_t k = 0;
+                for (int u = 0; u < kW; ++u) k += s_cnt[u];
+                s_ks = k - 1u;  // it holds at chunk 0
+            }
+            __syncthreads();
+        };
+        // A and B at bit `lane` of the word of chunk k that pred(A, B) picks
+        // (the last whose start it holds at), and just after it
+        auto at_bit = [&](uint32_t k, auto pred, uint32_t &q, uint32_t &a0, uint32_t &b0,
+                          uint32_t &a1, uint32_t &b1) {
+            const uint64_t *mq = masks + (size_t)(f + k) * (2 * kMaskWords);
+            const uint64_t L = mq[lane], R = mq[kMaskWords + lane];
+            const uint32_t cL = (uint32_t)__popcll(L), cR = (uint32_t)__popcll(R);
+            const uint32_t xA = preL[k] + wave_inclusive_scan(cL) - cL;
+            const uint32_t xB = TR - (preR[k] + wave_inclusive_scan(cR) - cR);
+            q = 63u - (uint32_t)__clzll((long long)__ballot(pred(xA, xB)));
+            const uint64_t mL = lane_value(L, (int)q), mR = lane_value(R, (int)q);
+            a0 = lane_value(xA, (int)q) + (uint32_t)__builtin_amdgcn_mbcnt_hi(
+                     (uint32_t)(mL >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mL, 0u));
+            b0 = lane_value(xB, (int)q) - (uint32_t)__builtin_amdgcn_mbcnt_hi(
+                     (uint32_t)(mR >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mR, 0u));
+            a1 = a0 + (uint32_t)((mL >> lane) & 1ull);
+            b1 = b0 - (uint32_t)((mR >> lane) & 1ull);
+        };
+        last_chunk(cA <= cB);
+        if (w == 0) {
+            uint32_t q, a0, b0, a1, b1;
+            at_bit(s_ks, [](uint32_t a, uint32_t b) { return a <= b; }, q, a0, b0, a1, b1);
+            const uint32_t k0 = a0 < b0 ? a0 : b0, k1 = a1 < b1 ? a1 : b1;
+            const uint32_t best = wave_max(k0 > k1 ? k0 : k1);
+            if (lane == 0) s_K = best;
+        }
+        __syncthreads();
+        const uint32_t K = uniform(s_K);
+        last_chunk(cA <= K && K <= cB);
+        if (w == 0) {
+            const uint32_t k = s_ks;
+            uint32_t q, a0, b0, a1, b1;
+            at_bit(k, [&](uint32_t a, uint32_t b) { return a <= K && K <= b; }, q, a0, b0, a1, b1);
+            const uint64_t mb = __ballot(a0 <= K && K <= b0);
+            if (lane == 0)
+                s_i = k * (uint32_t)kChunk + 64u * q + 63u - (uint32_t)__clzll((long long)mb);
+        }
+        __syncthreads();
+        const uint32_t i = uniform(s_i);
+        // ---- the swap plan, a chunk per thread (k_hoare_plan)
+        if ((uint32_t)t < nch) {
+            const uint32_t kc = (uint32_t)t;
+            const int owner = 2ull * i >= (uint64_t)n ? 0 : 1;
+            const uint32_t t0 = owner ? TR - preR[kc + 1] : preL[kc];
+            uint32_t t1 = owner ? TR - preR[kc] : preL[kc + 1];
+            if (t1 > K) t1 = K;
+            uint4 p0 = make_uint4(~0u, 0u, 0u, 0u), p1 = make_uint4(0u, 0u, 0u, 0u);
+            if (t0 < t1) {
+                // the first partner chunk: the last k with at(partner, k) <= ap0
+                const uint32_t *pre = owner ? preL : preR;
+                const uint32_t ap0 = owner ? t0 : TR - t1;
+                uint32_t a = 0, b = nch - 1u;
+                while (a < b) {
+                    const uint32_t mid = (a + b + 1u) >> 1;
+                    if (pre[mid] <= ap0) a = mid;
+                    else b = mid - 1u;
+                }
+                p0 = make_uint4(t0 | ((uint32_t)owner << 31), t1, TR, begin);
+                p1 = make_uint4(f, nch, a, f + (uint32_t)c);
+            }
+            uint4 *dst = reinterpret_cast<uint4 *>(plan + f + kc);
+            dst[0] = p0;
+            dst[1] = p1;
+        }
+        if (t == 0) {
+            splits[c] = SplitRec{TL, TR, K, i};
+            const int64_t gl = hb + lid, gr = hb + rid;
+            ranges[2 * gl] = begin;
+            ranges[2 * gl + 1] = begin + i;
+            ranges[2 * gr] = begin + i;
+            ranges[2 * gr + 1] = begin + n;
+        }
+        __syncthreads();  // the next cell rewrites the tables
+    }
+}
+
+// ---------------------------------------------------------------------------
 // orchestration
 // ---------------------------------------------------------------------------
 static int ensure_state(Ctx &c, int32_t levels_mode, bool *complete)
@@ -2614,10 +3093,14 @@ int enqueue_level(Ctx &c, const LevelEntry *entries, int32_t nCells, orb_cell *h
         return ORB_ERR_STATE;  // rounds 3 and 4 gather into these
     const int32_t sub_max = subtree_max_keys(c);
     const bool use_subtree = any_subtree && c.part == ORB_PART_HOARE && sub_max > 0;
-    if ((kernels.cell_max || !kernels.chunks) && (c.part != ORB_PART_HOARE || c.weighted))
+    if ((kernels.cell_max || kernels.chunks != kChunksAll) && (c.part != ORB_PART_HOARE || c.weighted))
         return ORB_ERR_STATE;
+    const bool mid = kernels.chunks == kChunksMid;
+    if (mid && nCells >= kRecsScan) return ORB_ERR_STATE;  // one block fills its tables
     const LevelMode mode{use_subtree ? (uint32_t)sub_max : 0u, kernels.cell_max,
-                         kernels.chunks ? 1 : 0, kernels.again ? 1 : 0};
+                         kernels.chunks == kChunksAll ? ~0u
+                                                      : (mid ? (uint32_t)(kMidChunks * kChunk) : 0u),
+                         kernels.again ? 1 : 0};
     const int32_t cgroup = cell_group(nCells);
     // Chunk order: the first round walks the level's chunks from the last, so
     // it starts with the chunks the previous level's swap wrote last (still in
@@ -2641,9 +3124,11 @@ int enqueue_level(Ctx &c, const LevelEntry *entries, int32_t nCells, orb_cell *h
     }
     if (nCells < kRecsScan) {
         const unsigned gf = (unsigned)((fin.nCells + kRecsScan - 1) / kRecsScan);
-        hipLaunchKernelGGL(k_b_recs_scan, dim3(1 + gf), dim3(kRecsScan), 0, c.stream, entries, nCells,
-                           heap, exists, c.ranges.p, sub, mode, c.recs.p, c.cell_first.p,
-                           level_passes, fin);
+        hipLaunchKernelGGL(mid ? k_b_recs_scan<true> : k_b_recs_scan<false>, dim3(1 + gf),
+                           dim3(kRecsScan), 0, c.stream, entries, nCells, heap, exists, c.ranges.p, sub,
+                           mode, c.recs.p, c.cell_first.p, level_passes, c.chunk_desc.p,
+                           (uint32_t)c.max_chunks,
+                           reinterpret_cast<unsigned long long *>(c.sel_lists.p), fin);
         ORB_HIP(hipGetLastError());
     } else {
         unsigned g1 = (unsigned)((nCells + 1 + kBlock - 1) / kBlock);
@@ -2652,10 +3137,10 @@ int enqueue_level(Ctx &c, const LevelEntry *entries, int32_t nCells, orb_cell *h
                            exists, c.ranges.p, sub, mode, c.recs.p, c.cell_nchunks.p, level_passes,
                            g1, fin);
         ORB_HIP(hipGetLastError());
-        if (kernels.chunks)
+        if (kernels.chunks == kChunksAll)
             ORB_TRY(scan_exclusive_u32(c, c.cell_nchunks.p, c.cell_first.p, (size_t)nCells + 1));
     }
-    if (kernels.chunks) {
+    if (kernels.chunks == kChunksAll) {
         // the chunk table, and the first round's candidate tables (not used
         // by weighted builds)
         const int tb = timing_mark(c);
@@ -2704,8 +3189,30 @@ int enqueue_level(Ctx &c, const LevelEntry *entries, int32_t nCells, orb_cell *h
                            level_passes, status);
         ORB_HIP(hipGetLastError());
     }
-    if (!kernels.chunks) return ORB_OK;
+    if (kernels.chunks == kChunksNone) return ORB_OK;
     const unsigned gq = chunk_grid(c);
+    if (mid) {
+        const int tb = timing_mark(c);
+        unsigned long long *lists = reinterpret_cast<unsigned long long *>(c.sel_lists.p);
+        hipLaunchKernelGGL(le ? k_m_hist<1> : k_m_hist<0>, dim3(gq), dim3(kBlock), 0, c.stream,
+                           c.recs.p, nCells, c.cell_first.p, c.chunk_desc.p, (uint32_t)c.max_chunks,
+                           c.x(), c.y(), c.z(), cell_hist);
+        hipLaunchKernelGGL(k_m_window, dim3(gq), dim3(kBlock), 0, c.stream, c.recs.p, nCells,
+                           c.cell_first.p, c.chunk_desc.p, (uint32_t)c.max_chunks, c.x(), c.y(), c.z(),
+                           cell_hist, c.packed.p, c.masks.p, c.sel.p, lists);
+        ORB_HIP(hipGetLastError());
+        ORB_TRY(timing_pair(c, tb, kTimeCount));
+        const int tp = timing_mark(c);
+        hipLaunchKernelGGL(k_m_tail, dim3((unsigned)std::max<int32_t>(nCells, 1)), dim3(kTailBlock), 0,
+                           c.stream, c.recs.p, nCells, c.cell_first.p, cell_hist, c.sel.p, lists,
+                           c.packed.p, c.masks.p, c.chunk_pre.p, c.splits.p,
+                           reinterpret_cast<SwapPlan *>(c.swap_plan.p), c.ranges.p, heap, exists, le,
+                           trace, level_passes, status);
+        ORB_HIP(hipGetLastError());
+        ORB_TRY(launch_hoare_swap(c, nCells, 0));
+        ORB_TRY(timing_pair(c, tp, kTimePartition));
+        return defer_final ? ORB_OK : launch_hoare_final(c, nCells);
+    }
     const unsigned gr = (unsigned)((gq + kReduceRows - 1) / kReduceRows);  // a block per 64-row tile
     const unsigned gw = (unsigned)((nCells + 3) / 4);
     if (c.weighted) {
@@ -2814,18 +3321,23 @@ int enqueue_level(Ctx &c, const LevelEntry *entries, int32_t nCells, orb_cell *h
 // registers in two launches where the chunk path needs sixteen and reads the
 // keys once, not twice; a level whose every cell fits it or the subtree kernel
 // goes without the chunk kernels.
-static LevelKernels level_kernels(const Ctx &c, int32_t level, int64_t lo, int64_t hi, bool all_sub)
+static LevelKernels level_kernels(const Ctx &c, int32_t level, int32_t cells, int64_t lo, int64_t hi,
+                                  bool all_sub)
 {
     LevelKernels k;
-    if (c.part != ORB_PART_HOARE || c.weighted || lo < 0) return k;
+    if (c.part != ORB_PART_HOARE || c.weighted || cells <= 0) return k;
     hi += 4 * (int64_t)level;
     lo -= 4 * (int64_t)level;
     if (all_sub) {
-        k.chunks = false;
+        k.chunks = kChunksNone;
         return k;
     }
     if (lo <= (int64_t)kCellLarge) k.cell_max = hi <= (int64_t)kCellSmall ? kCellSmall : kCellLarge;
-    k.chunks = hi > (int64_t)kCellLarge;
+    if (hi <= (int64_t)kCellLarge)
+        k.chunks = kChunksNone;
+    else if (hi <= (int64_t)kMidChunks * kChunk && c.n / kChunk + cells <= kMidLevelChunks &&
+             cells < kRecsScan)
+        k.chunks = kChunksMid;
     return k;
 }
 
@@ -2866,7 +3378,7 @@ static int enqueue_build(Ctx &c, int32_t levels_mode, bool again)
             const bool all_sub = b.complete && c.part == ORB_PART_HOARE && sub_max > 0 &&
                                  hi + 4 * l <= sub_max && max_leaf <= kSmallLeaves;
             c.level_chunk_hint[(size_t)l] = c.n / kChunk + cells + 1;
-            kernels[(size_t)l] = level_kernels(c, l, cells > 0 ? lo : -1, hi, all_sub);
+            kernels[(size_t)l] = level_kernels(c, l, cells, lo, hi, all_sub);
             if (all_sub) {
                 last = l;
                 break;
@@ -2895,7 +3407,7 @@ static int enqueue_build(Ctx &c, int32_t levels_mode, bool again)
                               b.complete && may_sub, b.level_cover[(size_t)l] != 0, l,
                               b.chunk_hist_w.p, b.cell_hist_w.p, &fin, true, k));
         fin.entries = entries;
-        fin.nCells = c.part == ORB_PART_HOARE && k.chunks ? nCells : 0;
+        fin.nCells = c.part == ORB_PART_HOARE && k.chunks != kChunksNone ? nCells : 0;
         ORB_TRY(timing_pair(c, tlevel, kTimeLevel + l));
     }
     for (int32_t l = last + 1; l <= lmax; ++l)  // nothing left: their time is the marks'

@@ -427,6 +427,23 @@ struct SplitRec {
     uint32_t i;         // split index (cell-local)
 };
 
+// Each chunk's swap unit, planned once per level by a thread per chunk (so
+// that a swap block starts from one load instead of the chain chunk ->
+// cell -> split and offsets -> a search for the first partner chunk): the
+// owner side and pairs [t0, t1), the cell's R-stopper total, first
+// particle, first chunk and chunk count, the first partner chunk
+// (cell-relative), and where the cell's chunk offsets start in chunk_pre (f
+// of a level-wide scan; f + cell where each cell has a table of its own, one
+// entry longer than its chunks).  t0o = ~0 marks a chunk with no pairs to swap.
+struct SwapPlan {
+    uint32_t t0o;  // t0 | owner << 31
+    uint32_t t1;
+    uint32_t TR;
+    uint32_t begin;
+    uint32_t f, nch, kp, fo;
+};
+static_assert(sizeof(SwapPlan) == 32, "two 16-byte loads");
+
 // ---------------------------------------------------------------------------
 // the context (the PST leaf's LocalData, src/services/pst.h:6-41)
 // ---------------------------------------------------------------------------
@@ -588,6 +605,7 @@ struct HistCounts {
 };
 int launch_hoare(Ctx &c, int32_t nCells, int32_t *status = nullptr,
                  const HistCounts *hc = nullptr, int rev = 0, bool defer_final = false);
+int launch_hoare_swap(Ctx &c, int32_t nCells, int rev);  // from the planned units
 int launch_hoare_final(Ctx &c, int32_t nCells);  // rows i and n-1 of the level's cells
 int launch_stopper_counts(Ctx &c, int32_t nCells, bool le_only, const HistCounts *hc = nullptr);
 int invalidate_stamps(Ctx &c, int32_t nCells);
@@ -613,10 +631,12 @@ struct PendingFinal {
     int32_t nCells = 0;
 };
 // The kernels a level of the batched form launches beside the subtree
-// kernel: the chunk path, and k_b_cell for cells of at most cell_max keys (0:
+// kernel: the chunk path (kChunksAll), its form for levels of few chunks
+// (kChunksMid) or neither, and k_b_cell for cells of at most cell_max keys (0:
 // none).  again: only cells that are not split yet.
+enum { kChunksNone = 0, kChunksMid = 1, kChunksAll = 2 };
 struct LevelKernels {
-    bool chunks = true;
+    int32_t chunks = kChunksAll;
     uint32_t cell_max = 0;
     bool again = false;
 };

@@ -358,7 +358,7 @@ int ensure_level_capacity(Ctx &c, int64_t nCells, int64_t chunks)
     ORB_TRY(c.stamps.alloc(m));
     ORB_TRY(c.chunk_ltle.alloc(c.max_chunks + 1));
     ORB_TRY(c.chunk_cnt.alloc(c.max_chunks + 1));
-    ORB_TRY(c.chunk_pre.alloc(c.max_chunks + 1));
+    ORB_TRY(c.chunk_pre.alloc(c.max_chunks + m + 2));  // a level-wide scan, or a table per cell
     ORB_TRY(c.masks.alloc(2 * (size_t)kMaskWords * (size_t)c.max_chunks));
     ORB_TRY(c.cell_cand.alloc((size_t)m * kBins));
     ORB_TRY(c.splits.alloc(m));
@@ -1184,21 +1184,6 @@ __device__ inline void swap_pairs(const uint32_t *sl, const uint32_t *sr, uint32
 // block scan ranks both, and every stopper whose index the unit uses goes
 // to its slot (L index t -> t - t0, R index j -> TR - 1 - j - t0).  Later
 // rounds continue on the partner side only, chunk by chunk.
-// Each chunk's swap unit, planned once per level by a thread per chunk (so
-// that a swap block starts from one load instead of the chain chunk ->
-// cell -> split and offsets -> a search for the first partner chunk): the
-// owner side and pairs [t0, t1), the cell's R-stopper total, first
-// particle, first chunk and chunk count, and the first partner chunk
-// (cell-relative).  t0o = ~0 marks a chunk with no pairs to swap.
-struct SwapPlan {
-    uint32_t t0o;  // t0 | owner << 31
-    uint32_t t1;
-    uint32_t TR;
-    uint32_t begin;
-    uint32_t f, nch, kp, pad;
-};
-static_assert(sizeof(SwapPlan) == 32, "two 16-byte loads");
-
 __global__ __launch_bounds__(kBlock) void k_hoare_plan(const CellRec *__restrict__ recs,
                                                        int32_t nCells,
                                                        const uint32_t *__restrict__ first,
@@ -1230,12 +1215,12 @@ __global__ __launch_bounds__(kBlock) void k_hoare_plan(const CellRec *__restrict
                     if (co.at(sp, mid) <= ap0) lo = mid;
                     else hi = mid - 1u;
                 }
-                pl = SwapPlan{u.t0 | ((uint32_t)u.owner << 31), u.t1, s.TR, r.begin, f, nch, lo, 0u};
+                pl = SwapPlan{u.t0 | ((uint32_t)u.owner << 31), u.t1, s.TR, r.begin, f, nch, lo, f};
             }
         }
         uint4 *dst = reinterpret_cast<uint4 *>(plan + q);
         dst[0] = make_uint4(pl.t0o, pl.t1, pl.TR, pl.begin);
-        dst[1] = make_uint4(pl.f, pl.nch, pl.kp, 0u);
+        dst[1] = make_uint4(pl.f, pl.nch, pl.kp, pl.fo);
     }
 }
 
@@ -1263,7 +1248,7 @@ __global__ __launch_bounds__(kBlock) void k_hoare_swap(const uint32_t *first,
         u.t0 = p0.x & 0x7fffffffu;
         u.t1 = p0.y;
         const uint32_t TR = p0.z, begin = p0.w, f = p1.x, nch = p1.y, kc = q - f;
-        const CellOffsets co{chunk_pre + f, chunk_pre[f]};
+        const CellOffsets co{chunk_pre + p1.w, chunk_pre[p1.w]};
         const int so = u.owner, sp = 1 - so;
         uint32_t ao0, ao1, ap0, ap1;
         side_range(so, u, TR, ao0, ao1);
@@ -1437,6 +1422,30 @@ __global__ void k_sum_swap_pairs(const CellRec *recs, const SplitRec *splits, in
     if ((threadIdx.x & 63) == 0 && k) atomicAdd(acc, k);
 }
 
+int launch_hoare_swap(Ctx &c, int32_t nCells, int rev)
+{
+    if (c.timing && c.swap_pairs.p) {
+        const unsigned gs = (unsigned)((nCells + kBlock - 1) / kBlock);
+        hipLaunchKernelGGL(k_sum_swap_pairs, dim3(gs < 1024 ? gs : 1024), dim3(kBlock), 0, c.stream,
+                           c.recs.p, c.splits.p, nCells, c.swap_pairs.p);
+        ORB_HIP(hipGetLastError());
+    }
+    // byte offsets inside any cell fit 32 bits below 2^30 particles; the
+    // payload-free instantiation keeps the fewest registers
+    const bool narrow = c.stride < (int64_t(1) << 30);
+    const int arrays = 3 + (c.ids() ? 1 : 0) + (c.weights() ? 1 : 0);
+    auto swap = narrow ? (arrays == 3 ? k_hoare_swap<true, 3>
+                          : arrays == 4 ? k_hoare_swap<true, 4> : k_hoare_swap<true, 5>)
+                       : (arrays == 3 ? k_hoare_swap<false, 3>
+                          : arrays == 4 ? k_hoare_swap<false, 4> : k_hoare_swap<false, 5>);
+    const int ts = timing_mark(c);
+    hipLaunchKernelGGL(swap, dim3(chunk_grid(c)), dim3(kBlock), 0, c.stream, c.cell_first.p, nCells,
+                       c.chunk_pre.p, c.masks.p, reinterpret_cast<const SwapPlan *>(c.swap_plan.p),
+                       c.x(), c.y(), c.z(), c.ids(), c.weights(), rev);
+    ORB_HIP(hipGetLastError());
+    return timing_pair(c, ts, kTimeSwap);
+}
+
 int launch_hoare(Ctx &c, int32_t nCells, int32_t *status, const HistCounts *hc, int rev,
                  bool defer_final)
 {
@@ -1460,31 +1469,12 @@ int launch_hoare(Ctx &c, int32_t nCells, int32_t *status, const HistCounts *hc, 
                        c.stream, c.recs.p, nCells, c.cell_first.p, c.chunk_pre.p, c.masks.p,
                        c.splits.p, c.ranges.p, status, cgroup);
     ORB_HIP(hipGetLastError());
-    if (c.timing && c.swap_pairs.p) {
-        const unsigned gs = (unsigned)((nCells + kBlock - 1) / kBlock);
-        hipLaunchKernelGGL(k_sum_swap_pairs, dim3(gs < 1024 ? gs : 1024), dim3(kBlock), 0, c.stream,
-                           c.recs.p, c.splits.p, nCells, c.swap_pairs.p);
-        ORB_HIP(hipGetLastError());
-    }
-    // byte offsets inside any cell fit 32 bits below 2^30 particles; the
-    // payload-free instantiation keeps the fewest registers
-    const bool narrow = c.stride < (int64_t(1) << 30);
-    const int arrays = 3 + (c.ids() ? 1 : 0) + (c.weights() ? 1 : 0);
-    auto swap = narrow ? (arrays == 3 ? k_hoare_swap<true, 3>
-                          : arrays == 4 ? k_hoare_swap<true, 4> : k_hoare_swap<true, 5>)
-                       : (arrays == 3 ? k_hoare_swap<false, 3>
-                          : arrays == 4 ? k_hoare_swap<false, 4> : k_hoare_swap<false, 5>);
     SwapPlan *plan = reinterpret_cast<SwapPlan *>(c.swap_plan.p);
     hipLaunchKernelGGL(k_hoare_plan, dim3(grid_for((size_t)c.max_chunks, 16384)), dim3(kBlock), 0,
                        c.stream, c.recs.p, nCells, c.cell_first.p, c.chunk_cell.p, c.chunk_pre.p,
                        c.splits.p, plan);
     ORB_HIP(hipGetLastError());
-    const int ts = timing_mark(c);
-    hipLaunchKernelGGL(swap, dim3(gq), dim3(kBlock), 0, c.stream, c.cell_first.p, nCells,
-                       c.chunk_pre.p, c.masks.p, plan, c.x(), c.y(), c.z(), c.ids(), c.weights(),
-                       rev);
-    ORB_HIP(hipGetLastError());
-    ORB_TRY(timing_pair(c, ts, kTimeSwap));
+    ORB_TRY(launch_hoare_swap(c, nCells, rev));
     // the last row swaps: here, or (batched builds) in the next level's first
     // launch, which reads no particle
     return defer_final ? ORB_OK : launch_hoare_final(c, nCells);

@@ -1,7 +1,7 @@
-"""Levels whose cells one block takes whole (keys in registers): sizes at the
-edges of its capacities, of its waves' parts and of the 64-key rows, both
-block shapes, ids, ties, and cells larger than the level expected, against the
-CPU oracle, bit for bit."""
+"""Levels whose cells one block takes whole (keys in registers), and levels of
+few chunks: sizes at the edges of their capacities, of the waves' parts, of
+the 64-key rows and of the chunks, both block shapes, ids, ties, and cells
+larger than the level expected, against the CPU oracle, bit for bit."""
 import numpy as np
 import pytest
 from gpu_helpers import assert_heaps_equal, bin_edge_keys, fbits
@@ -49,6 +49,15 @@ def test_one_cell(orb, oracle, n, cmp):
     assert check(orb, oracle, inputs.clustered(n, n_spheres=5, a=0.05, seed=n), 2, cmp=cmp, ids=True)
 
 
+# levels of few chunks: partial last chunks, one chunk more or less, the largest
+# cell of their tables (512 chunks less what the level rule keeps free) and one past it
+@pytest.mark.parametrize("n,d", [(40961, 2), (65537, 3), (8 * 4096 * 64 - 1, 5), (2097148, 2), (2097149, 2),
+                                 (1500007, 30)])
+@pytest.mark.parametrize("cmp", [0, 1])
+def test_few_chunks(orb, oracle, n, d, cmp):
+    assert check(orb, oracle, inputs.clustered(n, n_spheres=9, a=0.03, seed=d), d, cmp=cmp, ids=n < 100000)
+
+
 # no subtree kernel: every level of every size, down to cells of two leaves of
 # a few keys; d = 1024 has more than 256 cells on its last levels
 @pytest.mark.parametrize("n,d", [(1, 1), (300, 2), (5000, 7), (70001, 64), (131072, 1024), (200003, 1000)])
@@ -56,15 +65,17 @@ def test_every_level(orb, oracle, n, d):
     assert check(orb, oracle, oracle.generate(n), d, ids=True, subtree=0)
 
 
-@pytest.mark.parametrize("keys", ["grid", "edges", "one_value"])
+@pytest.mark.parametrize("keys", ["grid", "edges", "one_value", "sorted"])
 @pytest.mark.parametrize("cmp", [0, 1])
-def test_ties(orb, oracle, keys, cmp):
+@pytest.mark.parametrize("n", [30011, 150001])
+def test_ties(orb, oracle, keys, cmp, n):
     rng = np.random.default_rng(5)
-    n = 30011
     if keys == "grid":
         xyz = inputs.quantized(n, levels=9, seed=3)
     elif keys == "edges":
         xyz = tuple(bin_edge_keys(n, rng) for _ in range(3))
+    elif keys == "sorted":  # the window's keys lie side by side
+        xyz = tuple(np.sort(a) for a in oracle.generate(n))
     else:  # every x the same: one side of the first cut is empty
         xyz = (np.full(n, 0.125, np.float32),) + oracle.generate(n)[1:]
     check(orb, oracle, xyz, 8, cmp=cmp, subtree=0)

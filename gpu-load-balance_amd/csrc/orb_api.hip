@@ -163,7 +163,8 @@ static int prepare(Ctx &c, const orb_cell *cells, int32_t nCells)
 static int timed_count(Ctx &c, int32_t nCells, bool skip_found, const float *axis)
 {
     if (c.timing) ORB_HIP(hipEventRecord(c.ev[0], c.stream));
-    ORB_TRY(launch_count(c, nCells, skip_found, axis, c.timing ? c.ev[1] : nullptr));
+    // the sums go straight to the pinned counts: 8 B a cell
+    ORB_TRY(launch_count(c, nCells, skip_found, axis, c.hcnt.p, c.timing ? c.ev[1] : nullptr));
     return ORB_OK;
 }
 
@@ -185,8 +186,6 @@ static int count_service(Ctx &c, const orb_cell *cells, int32_t nCells, uint32_t
     ORB_TRY(prepare(c, cells, nCells));
     if (nCells == 0) return 0;
     ORB_TRY(timed_count(c, nCells, lt_skip_found, axis));
-    ORB_HIP(hipMemcpyAsync(c.hcnt.p, c.cnt.p, 2 * sizeof(uint32_t) * (size_t)nCells,
-                           hipMemcpyDeviceToHost, c.stream));
     ORB_HIP(hipStreamSynchronize(c.stream));
     ORB_TRY(finish_timed_count(c));
     for (int32_t i = 0; i < nCells; ++i) {
@@ -228,9 +227,7 @@ static int count_sizes(Ctx &c, const orb_cell *cells, int32_t nCells, uint32_t *
     if (nCells > 0 && !out) return ORB_ERR_ARG;
     ORB_TRY(prepare(c, cells, nCells));
     if (nCells == 0) return 0;
-    ORB_TRY(launch_cell_sizes(c, nCells, c.cnt.p));
-    ORB_HIP(hipMemcpyAsync(c.hcnt.p, c.cnt.p, sizeof(uint32_t) * (size_t)nCells,
-                           hipMemcpyDeviceToHost, c.stream));
+    ORB_TRY(launch_cell_sizes(c, nCells, c.hcnt.p));
     ORB_HIP(hipStreamSynchronize(c.stream));
     std::memcpy(out, c.hcnt.p, sizeof(uint32_t) * (size_t)nCells);
     return (int)(nCells * sizeof(uint32_t));
@@ -509,14 +506,12 @@ int orb_finalize(orb_ctx *ctx)
     c->hcnt_w.release();
     c->ranges.release();
     c->swap_pairs.release();
-    c->dcells.release();
     c->recs.release();
     c->cell_nchunks.release();
     c->cell_first.release();
     c->chunk_cell.release();
     c->chunk_desc.release();
     c->total_chunks.release();
-    c->cnt.release();
     c->stamps.release();
     c->chunk_ltle.release();
     c->chunk_cnt.release();

@@ -2572,8 +2572,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4, 4))
 //   k_hoare_swap
 // The same rounds, masks and plan as the chunk path's.  The five top levels of
 // 2^20 keys (1 to 16 cells): 53 us a level, from 89.  Past kMidLevelChunks the
-// atomics on the cells' rows and the tail's chunks per block cost what the
-// launches save (2^23 keys: within 5% of the chunk path).
+// atomics on the cells' rows and the chunks each tail block walks grow, and the
+// chunk path's launches are no longer what bounds a level.
 constexpr int kMidChunks = 512;         // per cell: k_m_tail's tables
 constexpr int64_t kMidLevelChunks = 2048;
 
@@ -3071,7 +3071,7 @@ static std::vector<uint64_t> graph_signature(const Ctx &c, const BatchedState &b
                           c.cell_nchunks.p, c.cell_first.p, c.chunk_cell.p, c.chunk_desc.p,
                           c.chunk_ltle.p, c.chunk_cnt.p, c.chunk_pre.p, c.scan_partials.p,
                           c.packed.p, c.masks.p, c.cell_cand.p, c.splits.p, c.chunk_comp.p,
-                          c.sel.p, c.sel_lists.p, c.swap_plan.p, c.status.p, c.stamps.p, c.cnt.p, b.level_ids.p, b.heap.p, b.exists.p,
+                          c.sel.p, c.sel_lists.p, c.swap_plan.p, c.status.p, c.stamps.p, b.level_ids.p, b.heap.p, b.exists.p,
                           b.sub.p, b.chunk_hist.p, b.cell_hist.p, b.trace.p, b.level_passes.p,
                           c.wt.p, c.wt_tmp.p, b.chunk_hist_w.p, b.cell_hist_w.p};
     for (const void *p : bufs) s.push_back((uint64_t)(uintptr_t)p);

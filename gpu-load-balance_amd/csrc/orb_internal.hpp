@@ -400,6 +400,15 @@ struct CellRec {
     int32_t lmax;
 };
 
+// What the services' kernels need of a caller's cell.
+struct CellIn {
+    int32_t id;
+    float cut;       // getCut()
+    int32_t axis;
+    int32_t found;
+};
+static_assert(sizeof(CellIn) == 16, "one load");
+
 // One cell of a level step: the build it belongs to and where that build's
 // state lives (see CellRec).
 struct LevelEntry {
@@ -482,7 +491,6 @@ struct Ctx {
     // level tables (sized for the widest level)
     int64_t max_level_cells = 0;
     int64_t max_chunks = 0;
-    DevBuf<orb_cell> dcells;
     DevBuf<CellRec> recs;
     DevBuf<uint32_t> cell_nchunks;   // [cells+1]
     DevBuf<uint32_t> cell_first;     // [cells+1] exclusive scan
@@ -490,7 +498,6 @@ struct Ctx {
     DevBuf<uint4> chunk_desc;        // [max_chunks] first key, end, cell, axis (kChunkIdle:
                                      // the cell is not searched this level)
     DevBuf<uint32_t> total_chunks;   // [1]
-    DevBuf<uint32_t> cnt;            // [cells][2] lt, le
     DevBuf<CountStamp> stamps;       // [cells] cut/axis of the chunk counts
     DevBuf<uint32_t> chunk_ltle;     // [max_chunks+1] packed lt | le<<16 per chunk
     DevBuf<uint64_t> chunk_cnt;      // [max_chunks+1] packed (nL | nR<<32)
@@ -513,8 +520,8 @@ struct Ctx {
     DevBuf<uint32_t> ids_dev;        // [cells]
 
     // host staging
-    PinBuf<orb_cell> hcells;
-    PinBuf<uint32_t> hcnt;
+    PinBuf<CellIn> hcells;           // read by the record kernel
+    PinBuf<uint32_t> hcnt;           // [cells][2] lt, le, written by the count kernels
     PinBuf<int32_t> hstatus;
     PinBuf<uint32_t> hranges;
     std::vector<int32_t> table_ids;  // ids of the current chunk table
@@ -581,8 +588,10 @@ unsigned chunk_grid(const Ctx &c);
 int upload_level(Ctx &c, const orb_cell *cells, int32_t nCells);
 // scanned: cell_first already holds the exclusive scan of the chunk counts
 int build_chunk_table(Ctx &c, int32_t nCells, bool with_stamps = true, bool scanned = false);
+// Count pass; the per-cell (lt, le) sums go to cnt ([cells][2], device or
+// pinned memory).
 int launch_count(Ctx &c, int32_t nCells, bool lt_skip_found, const float *axis_override,
-                 hipEvent_t after_count = nullptr);
+                 uint32_t *cnt, hipEvent_t after_count = nullptr);
 // Weighted count pass into c.cnt_w ([cells][2]: weight < cut, <= cut; with
 // total_only both are the cell's weight); skip_found leaves found cells out.
 int launch_count_w(Ctx &c, int32_t nCells, bool skip_found, bool total_only);

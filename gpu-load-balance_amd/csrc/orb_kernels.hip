@@ -290,8 +290,13 @@ int scan_exclusive_u64(Ctx &c, const uint64_t *in, uint64_t *out, size_t m, cons
 // ---------------------------------------------------------------------------
 // level records and the chunk table (ServiceCopyCells, copyCells.cu:10-64)
 // ---------------------------------------------------------------------------
-__global__ void k_level_recs(const orb_cell *cells, int32_t nCells, const uint32_t *ranges,
-                             CellRec *recs, uint32_t *nchunks, int32_t cap)
+// The services' kernels read four words of a cell (CellIn); the kernel takes
+// them from the pinned staging buffer itself, 16 B a cell over PCIe: 512 cells
+// cost less than the copy command and its gap did (the count service of 512
+// cells 83 -> 71 us), and no device copy of the cells is kept.
+__global__ void k_level_recs(const CellIn *__restrict__ cells, int32_t nCells,
+                             const uint32_t *__restrict__ ranges, CellRec *__restrict__ recs,
+                             uint32_t *__restrict__ nchunks, int32_t cap)
 {
     int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i > nCells) return;
@@ -299,18 +304,19 @@ __global__ void k_level_recs(const orb_cell *cells, int32_t nCells, const uint32
         nchunks[nCells] = 0u;
         return;
     }
-    const orb_cell &cl = cells[i];
+    const uint4 in = reinterpret_cast<const uint4 *>(cells)[i];
+    const int32_t id = (int32_t)in.x;
     CellRec r;
-    r.begin = ranges[2 * (size_t)cl.id];
-    r.end = ranges[2 * (size_t)cl.id + 1];
+    r.begin = ranges[2 * (size_t)id];
+    r.end = ranges[2 * (size_t)id + 1];
     if (r.end < r.begin) r.end = r.begin;
-    r.cut = cell_get_cut(cl);
-    r.axis = cl.cutAxis;
-    r.found = cl.foundCut ? 1 : 0;
-    r.nLeaf = cl.nLeafCells;
-    r.margin_l = cl.cutMarginLeft;
-    r.margin_r = cl.cutMarginRight;
-    r.id = cl.id;
+    r.cut = __uint_as_float(in.y);
+    r.axis = (int32_t)in.z;
+    r.found = (int32_t)in.w;
+    r.nLeaf = 0;  // the bisection's own fields: not used by the services
+    r.margin_l = 0.0f;
+    r.margin_r = 0.0f;
+    r.id = id;
     r.flags = 0;
     r.passes = 0;
     r.hb = 0;
@@ -348,13 +354,11 @@ int ensure_level_capacity(Ctx &c, int64_t nCells, int64_t chunks)
     const int64_t level_chunks = c.n / kChunk + m + 1;
     int64_t mc = level_chunks > c.max_chunks ? level_chunks : c.max_chunks;
     c.max_chunks = chunks > mc ? chunks : mc;
-    ORB_TRY(c.dcells.alloc(m));
     ORB_TRY(c.recs.alloc(m));
     ORB_TRY(c.cell_nchunks.alloc(m + 1));
     ORB_TRY(c.cell_first.alloc(m + 1));
     ORB_TRY(c.chunk_cell.alloc(c.max_chunks));
     ORB_TRY(c.chunk_desc.alloc(c.max_chunks));
-    ORB_TRY(c.cnt.alloc(2 * m));
     ORB_TRY(c.stamps.alloc(m));
     ORB_TRY(c.chunk_ltle.alloc(c.max_chunks + 1));
     ORB_TRY(c.chunk_cnt.alloc(c.max_chunks + 1));
@@ -376,14 +380,14 @@ int upload_level(Ctx &c, const orb_cell *cells, int32_t nCells)
     ORB_TRY(ensure_level_capacity(c, nCells));
     // the previous upload may still be reading the pinned staging buffer
     if (c.ev_upload) ORB_HIP(hipEventSynchronize(c.ev_upload));
-    std::memcpy(c.hcells.p, cells, sizeof(orb_cell) * (size_t)nCells);
-    ORB_HIP(hipMemcpyAsync(c.dcells.p, c.hcells.p, sizeof(orb_cell) * (size_t)nCells,
-                           hipMemcpyHostToDevice, c.stream));
-    if (c.ev_upload) ORB_HIP(hipEventRecord(c.ev_upload, c.stream));
+    for (int32_t i = 0; i < nCells; ++i)
+        c.hcells.p[i] = CellIn{cells[i].id, cell_get_cut(cells[i]), cells[i].cutAxis,
+                               cells[i].foundCut ? 1 : 0};
     unsigned g = (unsigned)((nCells + 1 + kBlock - 1) / kBlock);
-    hipLaunchKernelGGL(k_level_recs, dim3(g), dim3(kBlock), 0, c.stream, c.dcells.p, nCells,
+    hipLaunchKernelGGL(k_level_recs, dim3(g), dim3(kBlock), 0, c.stream, c.hcells.p, nCells,
                        c.ranges.p, c.recs.p, c.cell_nchunks.p, (int32_t)c.cap);
     ORB_HIP(hipGetLastError());
+    if (c.ev_upload) ORB_HIP(hipEventRecord(c.ev_upload, c.stream));
     return ORB_OK;
 }
 
@@ -463,42 +467,40 @@ __device__ inline void count_range(const float *key, uint32_t b, uint32_t e, flo
     }
 }
 
-__device__ inline void k_count_chunk(uint32_t q, const CellRec *recs, int32_t nCells,
-                                                  const uint32_t *first, const uint32_t *chunk_cell,
-                                                  const float *x, const float *y, const float *z,
-                                                  const float *axisT, int skip_found,
-                                                  uint32_t *chunk_ltle)
+// A block reaches its keys after two dependent loads: the chunk's record with
+// the chunk count, then the cell's (the record's axis word is not used: cells
+// find their cuts while the table stands).
+__global__ __launch_bounds__(kBlock) void k_count(const CellRec *__restrict__ recs, int32_t nCells,
+                                                  const uint32_t *__restrict__ first,
+                                                  const uint4 *__restrict__ chunk_desc,
+                                                  uint32_t max_chunks, const float *__restrict__ x,
+                                                  const float *__restrict__ y,
+                                                  const float *__restrict__ z,
+                                                  const float *__restrict__ axisT, int skip_found,
+                                                  uint32_t *__restrict__ chunk_ltle)
 {
     __shared__ uint32_t sm[4];
-    uint32_t cell, b, e;
-    if (!chunk_range(q, first, nCells, chunk_cell, recs, cell, b, e)) return;
-    const CellRec r = recs[cell];
-    if (skip_found && r.found) return;
-    if (r.axis < 0 || r.axis > 2) {  // no cut axis: nothing is left of the cut
-        if (threadIdx.x == 0) chunk_ltle[q] = 0u;
-        return;
-    }
-    const float *key = axisT ? axisT : axis_ptr(x, y, z, r.axis);
-    uint32_t lt = 0, le = 0;
-    count_range(key, b, e, r.cut, lt, le);
-    // both counts <= 4096: one packed word, one reduction
-    uint32_t packed = block_sum(lt | (le << 16), sm);
-    if (threadIdx.x == 0) chunk_ltle[q] = packed;
-}
-
-__global__ __launch_bounds__(kBlock) void k_count(const CellRec *recs, int32_t nCells,
-                                                  const uint32_t *first, const uint32_t *chunk_cell,
-                                                  const float *x, const float *y, const float *z,
-                                                  const float *axisT, int skip_found,
-                                                  uint32_t *chunk_ltle)
-{
     const uint32_t total = first[nCells];  // the caller keeps it within the table
-    for (uint32_t q = blockIdx.x; q < total; q += gridDim.x) {
-        k_count_chunk(q, recs, nCells, first, chunk_cell, x, y, z, axisT, skip_found, chunk_ltle);
-        __syncthreads();  // the next chunk reuses this block's LDS
+    for (uint32_t q = blockIdx.x;; q += gridDim.x) {
+        const uint4 d = chunk_record(chunk_desc, q, max_chunks);
+        const uint32_t b = uniform(d.x), e = uniform(d.y), cell = uniform(d.z);
+        keep_values(b, e, cell, 0u);  // the record, in flight with total
+        if (q >= total) break;
+        const CellRec &r = recs[cell];
+        const int axis = (int)uniform((uint32_t)r.axis);
+        const float cut = uniform(r.cut);
+        if (skip_found && uniform((uint32_t)r.found)) continue;
+        if (axis < 0 || axis > 2) {  // no cut axis: nothing is left of the cut
+            if (threadIdx.x == 0) chunk_ltle[q] = 0u;
+            continue;
+        }
+        uint32_t lt = 0, le = 0;
+        count_range(axisT ? axisT : axis_ptr(x, y, z, axis), b, e, cut, lt, le);
+        // both counts <= 4096: one packed word, one reduction
+        const uint32_t packed = block_sum(lt | (le << 16), sm);
+        if (threadIdx.x == 0) chunk_ltle[q] = packed;
     }
 }
-
 
 // Per-cell sums of the chunk slots; stamps the cut and axis the counts were
 // taken at (a later partition at the same cut reuses the chunk slots).  One
@@ -575,17 +577,17 @@ int invalidate_stamps(Ctx &c, int32_t nCells)
 }
 
 int launch_count(Ctx &c, int32_t nCells, bool skip_found, const float *axis_override,
-                 hipEvent_t after_count)
+                 uint32_t *cnt, hipEvent_t after_count)
 {
     hipLaunchKernelGGL(k_count, dim3(chunk_grid(c)), dim3(kBlock), 0, c.stream,
-                       c.recs.p, nCells, c.cell_first.p, c.chunk_cell.p, c.x(), c.y(), c.z(),
-                       axis_override, skip_found ? 1 : 0, c.chunk_ltle.p);
+                       c.recs.p, nCells, c.cell_first.p, c.chunk_desc.p, (uint32_t)c.max_chunks, c.x(),
+                       c.y(), c.z(), axis_override, skip_found ? 1 : 0, c.chunk_ltle.p);
     ORB_HIP(hipGetLastError());
     if (after_count) ORB_HIP(hipEventRecord(after_count, c.stream));
     unsigned g = (unsigned)(nCells < 65536 ? nCells : 65536);
     hipLaunchKernelGGL(k_cell_totals, dim3(g), dim3(kBlock), 0, c.stream, c.recs.p, nCells,
                        c.cell_first.p, c.chunk_ltle.p, skip_found ? 1 : 0,
-                       axis_override ? 0 : 1, c.cnt.p, c.stamps.p);
+                       axis_override ? 0 : 1, cnt, c.stamps.p);
     ORB_HIP(hipGetLastError());
     return ORB_OK;
 }
@@ -688,8 +690,8 @@ int launch_count_explicit(hipStream_t s, const CellRec *recs, int32_t nCells, co
     hipLaunchKernelGGL(k_fill_chunks, dim3(grid_for((size_t)max_chunks, 16384)), dim3(kBlock), 0, s,
                        first, nCells, recs, chunk_cell, chunk_desc, max_chunks);
     hipLaunchKernelGGL(k_count, dim3(chunk_blocks > 0 ? chunk_blocks : 1u), dim3(kBlock), 0, s, recs,
-                       nCells, first, chunk_cell, x, y, z, (const float *)nullptr, skip_found ? 1 : 0,
-                       chunk_ltle);
+                       nCells, first, chunk_desc, max_chunks, x, y, z, (const float *)nullptr,
+                       skip_found ? 1 : 0, chunk_ltle);
     const unsigned g = (unsigned)(nCells < 65536 ? nCells : 65536);
     hipLaunchKernelGGL(k_cell_totals, dim3(g), dim3(kBlock), 0, s, recs, nCells, first, chunk_ltle,
                        skip_found ? 1 : 0, 0, cnt, stamps);

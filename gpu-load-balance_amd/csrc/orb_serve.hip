@@ -555,13 +555,11 @@ int orb_server_destroy(orb_server *o)
     c.status.release();
     c.hstatus.release();
     c.hranges.release();
-    c.dcells.release();
     c.recs.release();
     c.cell_nchunks.release();
     c.cell_first.release();
     c.chunk_cell.release();
     c.chunk_desc.release();
-    c.cnt.release();
     c.stamps.release();
     c.chunk_ltle.release();
     c.chunk_cnt.release();

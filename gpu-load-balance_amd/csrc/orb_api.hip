@@ -107,11 +107,8 @@ int timing_collect(Ctx &c, bool reuse_events)
 
 static int reset_ranges(Ctx &c)
 {
-    ORB_TRY(launch_zero_u32(c.stream, c.ranges.p, 2 * (size_t)c.cap));
-    c.hranges.p[0] = 0;
-    c.hranges.p[1] = (uint32_t)c.n;
-    ORB_HIP(hipMemcpyAsync(c.ranges.p, c.hranges.p, 2 * sizeof(uint32_t), hipMemcpyHostToDevice,
-                           c.stream));
+    c.ranges_on_host = false;
+    ORB_TRY(launch_root_range(c.stream, c.ranges.p, c.cap, (uint32_t)c.n));
     ORB_HIP(hipStreamSynchronize(c.stream));
     c.table_ids.clear();
     return ORB_OK;
@@ -205,6 +202,7 @@ static int partition_service(Ctx &c, const orb_cell *cells, int32_t nCells, bool
     if (nCells == 0) return 0;
     for (int32_t i = 0; i < nCells; ++i)
         if (right_child_id(cells[i].id) >= c.cap) return ORB_ERR_ARG;
+    c.ranges_on_host = false;
     ORB_TRY(clear_status(c));
     if (c.timing) ORB_HIP(hipEventRecord(c.ev[0], c.stream));
     if (hoare) ORB_TRY(launch_hoare(c, nCells));
@@ -462,7 +460,7 @@ int orb_init(orb_ctx **out, int64_t nParticles, int32_t d, bool generate, orb_me
     if ((rc = c.packed.alloc((size_t)c.stride)) < 0) return fail(rc);
     if ((rc = c.status.alloc(2)) < 0) return fail(rc);
     if ((rc = c.hstatus.alloc(2)) < 0) return fail(rc);
-    if ((rc = c.hranges.alloc(2 * (size_t)c.cap)) < 0) return fail(rc);
+    if ((rc = c.hranges.alloc(host_tree_words(c.cap))) < 0) return fail(rc);
     if ((rc = ensure_level_capacity(c, (c.cap + 1) / 2)) < 0) return fail(rc);
     if (generate && nParticles > 0) {
         PinBuf<float> h;
@@ -857,8 +855,9 @@ int orb_get_heap(orb_ctx *ctx, orb_cell *heap, int64_t cap)
     Ctx *c = C(ctx);
     if (!c || !heap || cap < c->cap) return ORB_ERR_ARG;
     if (c->results_on_device) ORB_TRY(batched_pull_results(*c));
-    std::memset(heap, 0, sizeof(orb_cell) * (size_t)cap);
-    if (!c->heap.empty()) std::memcpy(heap, c->heap.data(), sizeof(orb_cell) * c->heap.size());
+    const size_t held = c->heap.size();
+    if (held) std::memcpy(heap, c->heap.data(), sizeof(orb_cell) * held);
+    std::memset(heap + held, 0, sizeof(orb_cell) * ((size_t)cap - held));
     return ORB_OK;
 }
 
@@ -876,11 +875,15 @@ int orb_get_ranges(orb_ctx *ctx, uint32_t *ranges, int64_t cap)
 {
     Ctx *c = C(ctx);
     if (!c || !ranges || cap < c->cap) return ORB_ERR_ARG;
-    std::memset(ranges, 0, 2 * sizeof(uint32_t) * (size_t)cap);
-    ORB_HIP(hipMemcpyAsync(c->hranges.p, c->ranges.p, 2 * sizeof(uint32_t) * (size_t)c->cap,
-                           hipMemcpyDeviceToHost, c->stream));
-    ORB_HIP(hipStreamSynchronize(c->stream));
+    // a small tree comes back whole, in one wait
+    if (c->results_on_device && c->cap <= kHostTreeCells) ORB_TRY(batched_pull_results(*c));
+    if (!c->ranges_on_host) {
+        ORB_HIP(hipMemcpyAsync(c->hranges.p, c->ranges.p, 2 * sizeof(uint32_t) * (size_t)c->cap,
+                               hipMemcpyDeviceToHost, c->stream));
+        ORB_HIP(hipStreamSynchronize(c->stream));
+    }
     std::memcpy(ranges, c->hranges.p, 2 * sizeof(uint32_t) * (size_t)c->cap);
+    std::memset(ranges + 2 * c->cap, 0, 2 * sizeof(uint32_t) * (size_t)(cap - c->cap));
     return ORB_OK;
 }
 

@@ -169,6 +169,16 @@ __global__ void k_b_init(orb_cell *heap, uint8_t *exists, uint8_t *sub, int64_t 
     if (i < 2) status[i] = 0;
 }
 
+// End of a build: its status pair and pass counters into pinned memory (two
+// copy commands less).
+__global__ void k_b_done(const int32_t *status, const int32_t *level_passes, int32_t *hstatus,
+                         int32_t *hpasses)
+{
+    const int t = threadIdx.x;
+    hpasses[t] = level_passes[t];
+    if (t < 2) hstatus[t] = status[t];
+}
+
 // Which kernels a level's launches hold, for its cell records: cells of at
 // most sub_max keys (and kSmallLeaves leaves) go to the subtree kernel, cells
 // of at most cell_max keys to k_b_cell (0: not launched), cells of at most
@@ -3073,7 +3083,7 @@ static std::vector<uint64_t> graph_signature(const Ctx &c, const BatchedState &b
                           c.packed.p, c.masks.p, c.cell_cand.p, c.splits.p, c.chunk_comp.p,
                           c.sel.p, c.sel_lists.p, c.swap_plan.p, c.status.p, c.stamps.p, b.level_ids.p, b.heap.p, b.exists.p,
                           b.sub.p, b.chunk_hist.p, b.cell_hist.p, b.trace.p, b.level_passes.p,
-                          c.wt.p, c.wt_tmp.p, b.chunk_hist_w.p, b.cell_hist_w.p};
+                          c.wt.p, c.wt_tmp.p, b.chunk_hist_w.p, b.cell_hist_w.p, c.hstatus.p, b.hpasses.p};
     for (const void *p : bufs) s.push_back((uint64_t)(uintptr_t)p);
     s.push_back((uint64_t)c.tune_chunk_blocks.size());
     for (int32_t v : c.tune_chunk_blocks) s.push_back((uint64_t)(int64_t)v);
@@ -3413,6 +3423,9 @@ static int enqueue_build(Ctx &c, int32_t levels_mode, bool again)
     for (int32_t l = last + 1; l <= lmax; ++l)  // nothing left: their time is the marks'
         if (b.level_n[(size_t)l]) ORB_TRY(timing_pair(c, timing_mark(c), kTimeLevel + l));
     if (fin.nCells > 0) ORB_TRY(launch_hoare_final(c, fin.nCells));
+    hipLaunchKernelGGL(k_b_done, dim3(1), dim3(64), 0, c.stream, c.status.p, b.level_passes.p,
+                       c.hstatus.p, b.hpasses.p);
+    ORB_HIP(hipGetLastError());
     return particles_home(c);  // in-stream: the capture ends where it began
 }
 
@@ -3458,22 +3471,16 @@ int build_batched(Ctx &c, int32_t levels_mode, orb_build_info *info)
     }
     c.table_ids.clear();
 
-    // status and pass counts come back now; the tree stays in HBM until a
-    // getter asks for it (batched_pull_results)
-    auto pull_status = [&]() -> int {
-        ORB_HIP(hipMemcpyAsync(c.hstatus.p, c.status.p, 2 * sizeof(int32_t), hipMemcpyDeviceToHost,
-                               c.stream));
-        ORB_HIP(hipMemcpyAsync(b.hpasses.p, b.level_passes.p, 64 * sizeof(int32_t),
-                               hipMemcpyDeviceToHost, c.stream));
-        ORB_HIP(hipStreamSynchronize(c.stream));
-        return ORB_OK;
-    };
-    ORB_TRY(pull_status());
+    // status and pass counts are in the pinned words once the stream is done
+    // (k_b_done); the tree stays in HBM until a getter asks for it
+    // (batched_pull_results)
+    c.ranges_on_host = false;
+    ORB_HIP(hipStreamSynchronize(c.stream));
     if (b.hpasses.p[0] > 0) {
         // cells larger than their level's kernels expected (keys that tie at
         // a cut do not split evenly) were left alone: the rest of the build
         ORB_TRY(enqueue_build(c, levels_mode, true));
-        ORB_TRY(pull_status());
+        ORB_HIP(hipStreamSynchronize(c.stream));
     }
     c.results_on_device = true;
     ORB_TRY(timing_collect(c));
@@ -3498,10 +3505,15 @@ int batched_pull_results(Ctx &c)
     BatchedState &b = *c.batched;
     c.heap.resize((size_t)c.cap);
     c.exists.resize((size_t)c.cap);
-    ORB_HIP(hipMemcpyAsync(c.heap.data(), b.heap.p, sizeof(orb_cell) * (size_t)c.cap,
+    const bool small = c.cap <= kHostTreeCells;
+    orb_cell *heap = small ? reinterpret_cast<orb_cell *>(c.hranges.p + 2 * c.cap) : c.heap.data();
+    uint8_t *exists = small ? reinterpret_cast<uint8_t *>(heap + c.cap) : c.exists.data();
+    if (small)
+        ORB_HIP(hipMemcpyAsync(c.hranges.p, c.ranges.p, 2 * sizeof(uint32_t) * (size_t)c.cap,
+                               hipMemcpyDeviceToHost, c.stream));
+    ORB_HIP(hipMemcpyAsync(heap, b.heap.p, sizeof(orb_cell) * (size_t)c.cap,
                            hipMemcpyDeviceToHost, c.stream));
-    ORB_HIP(hipMemcpyAsync(c.exists.data(), b.exists.p, (size_t)c.cap, hipMemcpyDeviceToHost,
-                           c.stream));
+    ORB_HIP(hipMemcpyAsync(exists, b.exists.p, (size_t)c.cap, hipMemcpyDeviceToHost, c.stream));
     if (c.trace && b.trace.p) {
         c.trace_counts.resize((size_t)c.cap * ORB_MAX_PASSES);
         ORB_HIP(hipMemcpyAsync(c.trace_counts.data(), b.trace.p,
@@ -3509,6 +3521,11 @@ int batched_pull_results(Ctx &c)
                                c.stream));
     }
     ORB_HIP(hipStreamSynchronize(c.stream));
+    if (small) {
+        std::memcpy(c.heap.data(), heap, sizeof(orb_cell) * (size_t)c.cap);
+        std::memcpy(c.exists.data(), exists, (size_t)c.cap);
+        c.ranges_on_host = true;
+    }
     c.results_on_device = false;
     return ORB_OK;
 }

@@ -523,7 +523,8 @@ struct Ctx {
     PinBuf<CellIn> hcells;           // read by the record kernel
     PinBuf<uint32_t> hcnt;           // [cells][2] lt, le, written by the count kernels
     PinBuf<int32_t> hstatus;
-    PinBuf<uint32_t> hranges;
+    PinBuf<uint32_t> hranges;        // [cap][2], then for small trees the heap and the flags
+    bool ranges_on_host = false;     // hranges holds the current map
     std::vector<int32_t> table_ids;  // ids of the current chunk table
     int32_t table_cells = 0;
 
@@ -567,6 +568,16 @@ struct Ctx {
     uint32_t *weights() const { return weighted ? (in_tmp ? wt_tmp.p : wt.p) : nullptr; }
     uint32_t *other_weights() const { return weighted ? (in_tmp ? wt.p : wt_tmp.p) : nullptr; }
 };
+
+// A tree of at most kHostTreeCells heap slots comes back through pinned memory
+// (61 B a slot, 4 MB at most, allocated with the context): ranges, heap and
+// flags in one wait, where copies into pageable memory wait one by one.
+constexpr int64_t kHostTreeCells = int64_t(1) << 16;
+inline size_t host_tree_words(int64_t cap)
+{
+    const size_t n = (size_t)cap;
+    return cap <= kHostTreeCells ? 2 * n + (sizeof(orb_cell) * n + n + 3) / 4 : 2 * n;
+}
 
 // timing helpers (orb_api.hip): marks are -1 when timing is off
 enum { kTimeCount = 0, kTimePartition = 1, kTimeOther = 2, kTimeSwap = 3, kTimeLevel = 100 /* + level */ };
@@ -623,6 +634,8 @@ int launch_stable_le(Ctx &c, int32_t nCells, int32_t *status = nullptr, bool ful
 int ensure_stable_buffers(Ctx &c);
 int launch_copy_u32(hipStream_t s, const uint32_t *src, uint32_t *dst, size_t n);
 int launch_iota(hipStream_t s, uint32_t *p, size_t n);
+// range(0) = [0, n), every other range empty
+int launch_root_range(hipStream_t s, uint32_t *ranges, int64_t cap, uint32_t n);
 // raises the status pair to kErrInputWord if x, y or z hold a NaN
 int launch_find_nan(hipStream_t s, const float *x, const float *y, const float *z, size_t n,
                     int32_t *status_pair);

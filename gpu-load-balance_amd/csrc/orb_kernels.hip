@@ -238,6 +238,19 @@ int launch_iota(hipStream_t s, uint32_t *p, size_t n)
     return ORB_OK;
 }
 
+__global__ void k_root_range(uint32_t *ranges, int64_t cap, uint32_t n)
+{
+    int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    for (; i < 2 * cap; i += (int64_t)gridDim.x * blockDim.x) ranges[i] = i == 1 ? n : 0u;
+}
+
+int launch_root_range(hipStream_t s, uint32_t *ranges, int64_t cap, uint32_t n)
+{
+    hipLaunchKernelGGL(k_root_range, dim3(grid_for(2 * (size_t)cap)), dim3(kBlock), 0, s, ranges, cap, n);
+    ORB_HIP(hipGetLastError());
+    return ORB_OK;
+}
+
 // Non-finite input check: NaN compares false both ways, so it is neither
 // below nor above any cut, which the histogram rounds cannot count the way
 // the reference's comparisons treat it.  Builds refuse such input: any NaN

@@ -519,6 +519,7 @@ int orb_finalize(orb_ctx *ctx)
     c->masks.release();
     c->cell_cand.release();
     c->splits.release();
+    c->round_state.release();
     c->chunk_comp.release();
     c->sel.release();
     c->sel_lists.release();

@@ -1406,6 +1406,55 @@ __global__ __launch_bounds__(kBlock) void k_b_finish_block(CellRec *recs, int32_
 // cell (no window packing), so a row's total is the chunk's weight and a
 // cell histogram's total the cell's weight.
 // ---------------------------------------------------------------------------
+// The weights of a chunk (record dd) as issue_chunk_loads reads its keys: past
+// the chunk's end 0.
+template <int kPerWave>
+__device__ inline void issue_weight_loads(const uint32_t *wgt, uint4 dd, uint32_t sb, int lane,
+                                          uint32_t (&wv)[kPerWave])
+{
+    const uint32_t b = uniform(dd.x), e = uniform(dd.y);
+    const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint32_t *>(wgt) + b, 0, (int)((e - b) * 4u), 0x00020000);
+#pragma unroll
+    for (int j = 0; j < kPerWave; ++j)
+        wv[j] = __builtin_amdgcn_raw_buffer_load_b32(
+            wr, (int)((sb + (uint32_t)lane) * 4u + 256u * (uint32_t)j), 0, 0);
+}
+
+template <int LE>
+__device__ inline int bin_walk(float v, float lo, float hi);
+
+// A wave's keys and weights into the block's row of weight sums: keys outside
+// the margins add up in registers (as atomics they would share two words) and
+// keys of weight 0, those past the chunk's end among them, add nothing.
+template <int LE, int kPerWave>
+__device__ inline void bin_weights(const float (&v)[kPerWave], const uint32_t (&wv)[kPerWave], float lo,
+                                   float hi, unsigned long long *hist, int lane)
+{
+    const float width = hi - lo;
+    const float scale = width > 0.0f ? (float)kBins / width : 0.0f;
+    const float lim = 0.5f - bin_tolerance(lo, hi, scale);
+    uint64_t below = 0ull, above = 0ull;
+    static_for<0, kPerWave>([&](auto jc) __attribute__((always_inline)) {
+        constexpr int j = decltype(jc)::value;
+        const float vj = v[j];
+        const bool lt = vj < lo, gt = vj > hi;
+        below += lt ? wv[j] : 0u;
+        above += gt ? wv[j] : 0u;
+        if (!lt && !gt && wv[j]) {
+            int bin;
+            if (!bin_estimate(vj, lo, scale, lim, bin)) bin = bin_walk<LE>(vj, lo, hi);
+            atomicAdd(&hist[bin], (unsigned long long)wv[j]);
+        }
+    });
+    below = wave_sum(below);
+    above = wave_sum(above);
+    if (lane == 0) {
+        if (below) atomicAdd(&hist[0], (unsigned long long)below);
+        if (above) atomicAdd(&hist[kBins - 1], (unsigned long long)above);
+    }
+}
+
 template <int LE>
 __global__ __launch_bounds__(kBlock) void k_bw_hist(
     const CellRec *__restrict__ recs, int32_t nCells, const uint32_t *__restrict__ first,
@@ -1413,9 +1462,10 @@ __global__ __launch_bounds__(kBlock) void k_bw_hist(
     const float *__restrict__ y, const float *__restrict__ z, const uint32_t *__restrict__ wgt,
     uint64_t *__restrict__ chunk_hist_w)
 {
-    __shared__ float cand[kBins + 1];
     __shared__ unsigned long long hist[kBins];
-    const int t = threadIdx.x;
+    constexpr int kPerWave = kMaskWords / (kBlock / 64);  // 16 loads of 64 keys and weights
+    const int t = threadIdx.x, lane = t & 63, w = (int)uniform((uint32_t)t >> 6);
+    const uint32_t sb = (uint32_t)(w * kPerWave * 64);
     const uint32_t total = first[nCells];
     for (uint32_t q = blockIdx.x;; q += gridDim.x) {
         const uint4 d = chunk_record(chunk_desc, q, max_chunks);
@@ -1426,31 +1476,17 @@ __global__ __launch_bounds__(kBlock) void k_bw_hist(
         if (axis > 2u) continue;  // uniform: the cell is not searched
         const CellRec &r = recs[cell];
         if (r.found) continue;    // uniform: an earlier round found the cut
+        float v[kPerWave];
+        issue_chunk_loads(x, y, z, true, d, sb, lane, v);
+        uint32_t wv[kPerWave];
+        issue_weight_loads(wgt, d, sb, lane, wv);
         const float lo = uniform(r.margin_l), hi = uniform(r.margin_r);
-        store_cands(cand, t ? candidate(t, lo, hi) : -INFINITY);
         hist[t] = 0ull;
         __syncthreads();
-        const float width = hi - lo;
-        const float scale = width > 0.0f ? (float)kBins / width : 0.0f;
-        const float lim = 0.5f - bin_tolerance(lo, hi, scale);
-        const float *key = axis_ptr(x, y, z, (int)axis);
-        for (uint32_t p = b + (uint32_t)t; p < e; p += kBlock) {
-            const float v = key[p];
-            const unsigned long long wv = wgt[p];
-            int bin;
-            if (v < lo) {
-                bin = 0;                  // below every candidate
-            } else if (v > hi) {
-                bin = kBins - 1;          // above every candidate
-            } else if (!bin_estimate(v, lo, scale, lim, bin)) {
-                int tj;
-                bin = bin_of<LE>(cand, v, lo, scale, tj);
-            }
-            atomicAdd(&hist[bin], wv);
-        }
+        bin_weights<LE>(v, wv, lo, hi, hist, lane);
         __syncthreads();
         chunk_hist_w[(size_t)q * kBins + t] = hist[t];
-        __syncthreads();  // the next chunk rewrites cand and hist
+        __syncthreads();  // the next chunk rewrites hist
     }
 }
 
@@ -1481,17 +1517,27 @@ __global__ __launch_bounds__(kBlock) void k_bw_reduce(const CellRec *recs, int32
         __syncthreads();
         int32_t cur = -1;
         unsigned long long acc = 0;
-        for (uint32_t u = 0; u < nrows; ++u) {
-            const int32_t cl = scell[u];
-            if (cl != cur) {
-                if (cur >= 0 && acc)
-                    atomicAdd(reinterpret_cast<unsigned long long *>(cell_hist_w) +
-                                  (size_t)cur * kBins + t,
-                              acc);
-                cur = cl;
-                acc = 0;
+        for (uint32_t u0 = 0; u0 < nrows; u0 += 16u) {
+            // 16 rows' loads in flight: 22 -> 11.5 us a launch at 2^24 keys
+            // against one row after another
+            uint64_t v[16];
+#pragma unroll
+            for (uint32_t u = 0; u < 16u; ++u)
+                v[u] = u0 + u < nrows && scell[u0 + u] >= 0
+                           ? chunk_hist_w[(size_t)(q0 + u0 + u) * kBins + t] : 0ull;
+#pragma unroll
+            for (uint32_t u = 0; u < 16u; ++u) {
+                const int32_t cl = u0 + u < nrows ? scell[u0 + u] : cur;
+                if (cl != cur) {
+                    if (cur >= 0 && acc)
+                        atomicAdd(reinterpret_cast<unsigned long long *>(cell_hist_w) +
+                                      (size_t)cur * kBins + t,
+                                  acc);
+                    cur = cl;
+                    acc = 0;
+                }
+                acc += v[u];
             }
-            if (cl >= 0) acc += chunk_hist_w[(size_t)(q0 + u) * kBins + t];
         }
         if (cur >= 0 && acc)
             atomicAdd(reinterpret_cast<unsigned long long *>(cell_hist_w) + (size_t)cur * kBins + t,
@@ -2744,17 +2790,151 @@ __global__ __launch_bounds__(kBlock) void k_m_window(
     }
 }
 
+// ---------------------------------------------------------------------------
+// weighted levels of few chunks
+// ---------------------------------------------------------------------------
+// The weighted rounds bin every key of a searching cell in each of the four
+// rounds (a weight histogram needs every key).  On a level of few chunks
+// every block replays the round before from its cell's row of weight sums,
+// starting from the margins the block of the cell's first chunk left in the
+// round before that (state[round parity]), then bins its chunk and adds its
+// row to the cell's row of this round: one launch a round where the chunk path
+// takes three.  k_mw_masks replays the last round and writes the stopper
+// masks, k_m_tail<true> takes the split and the plan.
+struct RoundState {
+    float L, R;
+    int32_t passes, found;
+};
+
+// The state after `round` rounds: the state before it and its row.  Every wave
+// that calls it gets it; trace_row (the round's left weights) where wanted.
+__device__ inline RoundState weighted_state(const CellRec &r, uint32_t cell, int32_t nCells, int round,
+                                            const RoundState *state, const uint64_t *rows, int lane,
+                                            uint64_t *trace_row)
+{
+    RoundState s{uniform(r.margin_l), uniform(r.margin_r), 0, 0};
+    if (round == 0) return s;
+    if (round > 1) {
+        const RoundState p = state[(size_t)((round - 1) & 1) * (size_t)nCells + cell];
+        s = RoundState{uniform(p.L), uniform(p.R), (int32_t)uniform((uint32_t)p.passes),
+                       (int32_t)uniform((uint32_t)p.found)};
+        if (s.found) return s;
+    }
+    const uint64_t *row = rows + ((size_t)(round - 1) * (size_t)nCells + cell) * kBins;
+    const ulonglong2 a = reinterpret_cast<const ulonglong2 *>(row)[2 * lane];
+    const ulonglong2 b2 = reinterpret_cast<const ulonglong2 *>(row)[2 * lane + 1];
+    const uint64_t s0 = a.x, s1 = s0 + a.y, s2 = s1 + b2.x, s3 = s2 + b2.y;
+    const uint64_t base = wave_inclusive_scan(s3) - s3;
+    const uint64_t pv[4] = {base + s0, base + s1, base + s2, base + s3};
+    const uint64_t weight = lane_value(pv[3], 63);  // every key of the cell was binned
+    const float target = difference_target_w(weight, (int32_t)uniform((uint32_t)r.nLeaf));
+    const RoundOut ro = replay_round_lanes(pv, s.L, s.R, target, s.passes, lane, trace_row);
+    return RoundState{uniform(ro.L), uniform(ro.R), ro.passes, ro.found ? 1 : 0};
+}
+
+template <int LE>
+__global__ __launch_bounds__(kBlock) void k_mw_hist(
+    const CellRec *__restrict__ recs, int32_t nCells, const uint32_t *__restrict__ first,
+    const uint4 *__restrict__ chunk_desc, uint32_t max_chunks, const float *__restrict__ x,
+    const float *__restrict__ y, const float *__restrict__ z, const uint32_t *__restrict__ wgt,
+    int round, RoundState *state, uint64_t *rows, uint64_t *trace)
+{
+    constexpr int kW = kBlock / 64;
+    constexpr int kPerWave = kMaskWords / kW;  // 16 loads of 64 keys and weights
+    __shared__ unsigned long long hist[kBins];
+    const int t = threadIdx.x, lane = t & 63, w = (int)uniform((uint32_t)t >> 6);
+    const uint32_t sb = (uint32_t)(w * kPerWave * 64);
+    const uint32_t total = first[nCells];
+    for (uint32_t q = blockIdx.x;; q += gridDim.x) {
+        const uint4 d = chunk_record(chunk_desc, q, max_chunks);
+        const uint32_t b = uniform(d.x), e = uniform(d.y), cell = uniform(d.z);
+        const uint32_t axis = uniform(d.w);
+        keep_values(b, e, cell, axis);
+        if (q >= total) break;
+        if (axis > 2u) continue;  // uniform: the cell is not searched
+        float v[kPerWave];
+        issue_chunk_loads(x, y, z, true, d, sb, lane, v);
+        uint32_t wv[kPerWave];
+        issue_weight_loads(wgt, d, sb, lane, wv);
+        const CellRec &r = recs[cell];
+        const bool lead = q == uniform(first[cell]);  // the cell's first chunk keeps its state
+        uint64_t *trow = trace && lead && w == 0
+                             ? trace + ((size_t)r.hb + r.id) * ORB_MAX_PASSES : nullptr;
+        const RoundState s = weighted_state(r, cell, nCells, round, state, rows, lane, trow);
+        if (lead && t == 0) state[(size_t)(round & 1) * (size_t)nCells + cell] = s;
+        if (s.found) continue;  // uniform
+        hist[t] = 0ull;
+        __syncthreads();
+        bin_weights<LE>(v, wv, s.L, s.R, hist, lane);
+        __syncthreads();
+        if (hist[t])
+            atomicAdd(reinterpret_cast<unsigned long long *>(rows) +
+                          ((size_t)round * (size_t)nCells + cell) * kBins + t, hist[t]);
+        __syncthreads();  // the next chunk rewrites hist
+    }
+}
+
+// The stopper masks of each chunk at its cell's cut (the state after the last
+// round, which the block of the cell's first chunk leaves for k_m_tail).
+__global__ __launch_bounds__(kBlock) void k_mw_masks(
+    const CellRec *__restrict__ recs, int32_t nCells, const uint32_t *__restrict__ first,
+    const uint4 *__restrict__ chunk_desc, uint32_t max_chunks, const float *__restrict__ x,
+    const float *__restrict__ y, const float *__restrict__ z, RoundState *state,
+    const uint64_t *__restrict__ rows, uint64_t *__restrict__ masks, uint64_t *trace)
+{
+    constexpr int kW = kBlock / 64;
+    constexpr int kPerWave = kMaskWords / kW;
+    const int t = threadIdx.x, lane = t & 63, w = (int)uniform((uint32_t)t >> 6);
+    const uint32_t sb = (uint32_t)(w * kPerWave * 64);
+    const uint32_t total = first[nCells];
+    for (uint32_t q = blockIdx.x;; q += gridDim.x) {
+        const uint4 d = chunk_record(chunk_desc, q, max_chunks);
+        const uint32_t b = uniform(d.x), e = uniform(d.y), cell = uniform(d.z);
+        const uint32_t axis = uniform(d.w);
+        keep_values(b, e, cell, axis);
+        if (q >= total) break;
+        if (axis > 2u) continue;
+        float v[kPerWave];
+        issue_chunk_loads(x, y, z, true, d, sb, lane, v);
+        const CellRec &r = recs[cell];
+        const bool lead = q == uniform(first[cell]);
+        uint64_t *trow = trace && lead && w == 0
+                             ? trace + ((size_t)r.hb + r.id) * ORB_MAX_PASSES : nullptr;
+        const RoundState s = weighted_state(r, cell, nCells, kRounds, state, rows, lane, trow);
+        if (lead && t == 0) state[(size_t)(kRounds & 1) * (size_t)nCells + cell] = s;
+        const float cut = cell_cut(s.L, s.R);
+        const uint32_t len = e - b;
+        uint64_t mineL = 0ull, mineR = 0ull;
+        static_for<0, kPerWave>([&](auto jc) __attribute__((always_inline)) {
+            constexpr int j = decltype(jc)::value;
+            const bool in = sb + 64u * (uint32_t)j + (uint32_t)lane < len;
+            const uint64_t mL = __ballot(in && !(v[j] < cut));
+            const uint64_t mR = __ballot(in && !(v[j] > cut));
+            mineL = lane == j ? mL : mineL;
+            mineR = lane == j ? mR : mineR;
+        });
+        uint64_t *mq = masks + (size_t)q * (2 * kMaskWords) + w * kPerWave;
+        if (lane < kPerWave) {
+            mq[lane] = mineL;
+            mq[kMaskWords + lane] = mineR;
+        }
+    }
+}
+
 // The rest of a cell's search and its split, a block per cell: round 1's
 // outcome, the later rounds over the listed keys (those inside the margins),
 // the cell's record and children, the stopper masks of its chunks from the
 // window pass's words and packed keys, the chunks' stopper offsets, K and i
 // as in k_b_cell (the crossing chunk, its word, its bit), the children's
-// ranges, and each chunk's swap unit as k_hoare_plan makes it.
+// ranges, and each chunk's swap unit as k_hoare_plan makes it.  WEIGHTED: the
+// search and the masks are done (state, k_mw_masks); the chunks' counts come
+// from the masks.
 constexpr int kTailBlock = 1024;
+template <bool WEIGHTED>
 __global__ __launch_bounds__(kTailBlock) void k_m_tail(
     CellRec *recs, int32_t nCells, const uint32_t *__restrict__ first, uint32_t *cell_hist,
     const float *__restrict__ sel, const unsigned long long *__restrict__ sel_lists,
-    const float *__restrict__ pack, uint64_t *masks, uint64_t *chunk_pre, SplitRec *splits,
+    const float *__restrict__ pack, const RoundState *__restrict__ state, uint64_t *rows, uint64_t *masks, uint64_t *chunk_pre, SplitRec *splits,
     SwapPlan *plan, uint32_t *ranges, orb_cell *heap, uint8_t *exists, int le_cmp, uint64_t *trace,
     int32_t *level_passes, int32_t *status)
 {
@@ -2784,116 +2964,147 @@ __global__ __launch_bounds__(kTailBlock) void k_m_tail(
             }
             continue;
         }
-        uint64_t *trow = trace ? trace + ((size_t)hb + id) * ORB_MAX_PASSES : nullptr;
-        uint32_t *row = cell_hist + (size_t)c * kBins;
-        const RoundOut r1 = replay_row(row, rec, lane, w == 0 ? trow : nullptr);
-        float lo = uniform(r1.L), hi = uniform(r1.R);
-        int32_t passes = r1.passes;
-        bool found = r1.found;
-        const unsigned long long list = n ? sel_lists[f] : 0ull;
-        const uint32_t m = uniform((uint32_t)list) < n ? uniform((uint32_t)list) : n;
-        const uint32_t nbelow = uniform((uint32_t)(list >> 32));
-        const float target = difference_target(n, (int32_t)uniform((uint32_t)rec.nLeaf));
-        if (t < kBins) hist[t] = 0u;
-        __syncthreads();  // every wave has read the row
-        if (t < kBins) row[t] = 0u;  // the next level adds to zero
-        while (!found && passes < ORB_MAX_PASSES) {
-            const float width = hi - lo;
-            const float scale = width > 0.0f ? (float)kBins / width : 0.0f;
-            const float lim = 0.5f - bin_tolerance(lo, hi, scale);
-            uint32_t below = 0;  // wave-uniform
-            for (uint32_t k0 = 0; k0 < m; k0 += 4u * kTailBlock) {
-                float v[4];
-                bool in[4];
-#pragma unroll
-                for (int u = 0; u < 4; ++u) {
-                    const uint32_t k = k0 + (uint32_t)(u * kTailBlock + t);
-                    in[u] = k < m;
-                    v[u] = in[u] ? sel[begin + k] : 0.0f;
-                }
-#pragma unroll
-                for (int u = 0; u < 4; ++u) {
-                    const bool lt = in[u] && v[u] < lo, on = in[u] && !(v[u] < lo) && !(v[u] > hi);
-                    below += (uint32_t)__popcll(__ballot(lt));
-                    if (!on) continue;
-                    int bin;
-                    if (!bin_estimate(v[u], lo, scale, lim, bin))
-                        bin = le_cmp ? bin_walk<1>(v[u], lo, hi) : bin_walk<0>(v[u], lo, hi);
-                    atomicAdd(&hist[bin], 1u);
-                }
+        float lo = uniform(rec.margin_l), hi = uniform(rec.margin_r);
+        int32_t passes = 0;
+        bool found = false;
+        if constexpr (WEIGHTED) {
+            if (nch) {
+                const RoundState s = state[(size_t)(kRounds & 1) * (size_t)nCells + c];
+                lo = uniform(s.L);
+                hi = uniform(s.R);
+                passes = (int32_t)uniform((uint32_t)s.passes);
+                found = uniform((uint32_t)s.found) != 0u;
+            } else {
+                // no chunk carried the rounds of an empty cell: its first pass
+                // finds 0 of 0
+                passes = 1;
+                found = true;
+                if (trace && t == 0) trace[((size_t)hb + id) * ORB_MAX_PASSES] = 0ull;
             }
-            if (lane == 0 && below) atomicAdd(&hist[0], below);
-            if (t == 0 && nbelow) atomicAdd(&hist[0], nbelow);  // the keys below the window
-            __syncthreads();
-            if (w == 0) {
-                const uint4 h4 = reinterpret_cast<const uint4 *>(hist)[lane];
-                reinterpret_cast<uint4 *>(hist)[lane] = make_uint4(0u, 0u, 0u, 0u);
-                const uint32_t s0 = h4.x, s1 = s0 + h4.y, s2 = s1 + h4.z, s3 = s2 + h4.w;
-                const uint32_t base = wave_inclusive_scan(s3) - s3;
-                const uint32_t pv[4] = {base + s0, base + s1, base + s2, base + s3};
-                const RoundOut ro = replay_round_lanes(pv, lo, hi, target, passes, lane, trow);
-                if (lane == 0) {
-                    s_lr[0] = ro.L;
-                    s_lr[1] = ro.R;
-                    s_pf[0] = ro.passes;
-                    s_pf[1] = ro.found ? 1 : 0;
-                }
-            }
-            __syncthreads();
-            lo = uniform(s_lr[0]);
-            hi = uniform(s_lr[1]);
-            passes = (int32_t)uniform((uint32_t)s_pf[0]);
-            found = uniform((uint32_t)s_pf[1]) != 0u;
-        }
-        const float cut = cell_cut(lo, hi);
-        // ---- stopper masks: a wave per kPer chunks, a word per lane
-        constexpr int kPer = 4;
-        for (uint32_t k0 = (uint32_t)(w * kPer); k0 < nch; k0 += (uint32_t)(kW * kPer)) {
-            uint64_t G[kPer], W[kPer];
-            float v0[kPer];
-            const float *pk[kPer];
-#pragma unroll
-            for (int u = 0; u < kPer; ++u) {
-                const uint32_t k = k0 + (uint32_t)u < nch ? k0 + (uint32_t)u : nch - 1u;
+            for (int q = t; q < kRounds * kBins; q += kTailBlock)  // the next level adds to zero
+                rows[((size_t)(q / kBins) * (size_t)nCells + c) * kBins + q % kBins] = 0ull;
+            for (uint32_t k = (uint32_t)w; k < nch; k += kW) {
                 const uint64_t *mq = masks + (size_t)(f + k) * (2 * kMaskWords);
-                G[u] = mq[lane];
-                W[u] = mq[kMaskWords + lane];
-            }
-#pragma unroll
-            for (int u = 0; u < kPer; ++u) {
-                const uint32_t k = k0 + (uint32_t)u < nch ? k0 + (uint32_t)u : nch - 1u;
-                const uint32_t cw = (uint32_t)__popcll(W[u]);
-                const uint32_t ex = wave_inclusive_scan(cw) - cw;
-                const int q0 = lane & ~15;  // first word of this lane's quarter
-                const uint32_t rank = ex - (uint32_t)__shfl((int)ex, q0, 64);
-                pk[u] = pack + begin + k * (uint32_t)kChunk + 64u * (uint32_t)q0 + rank;
-                v0[u] = W[u] ? *pk[u] : 0.0f;
-            }
-#pragma unroll
-            for (int u = 0; u < kPer; ++u) {
-                const uint32_t k = k0 + (uint32_t)u;
-                if (k >= nch) break;  // uniform
-                const uint32_t p0 = k * (uint32_t)kChunk + 64u * (uint32_t)lane;
-                const uint64_t valid =
-                    p0 >= n ? 0ull : (n - p0 >= 64u ? ~0ull : (1ull << (n - p0)) - 1ull);
-                uint64_t L = G[u], R = valid & ~G[u] & ~W[u], wd = W[u];
-                float vk = v0[u];
-                const float *at = pk[u];
-                while (wd) {
-                    const uint32_t bit = (uint32_t)__builtin_ctzll(wd);
-                    wd &= wd - 1ull;
-                    L |= (!(vk < cut) ? 1ull : 0ull) << bit;
-                    R |= (!(vk > cut) ? 1ull : 0ull) << bit;
-                    if (wd) vk = *++at;
-                }
-                uint64_t *mq = masks + (size_t)(f + k) * (2 * kMaskWords);
-                mq[lane] = L;
-                mq[kMaskWords + lane] = R;
-                const uint32_t nl = wave_sum((uint32_t)__popcll(L));
-                const uint32_t nr = wave_sum((uint32_t)__popcll(R));
+                const uint32_t nl = wave_sum((uint32_t)__popcll(mq[lane]));
+                const uint32_t nr = wave_sum((uint32_t)__popcll(mq[kMaskWords + lane]));
                 if (lane == 0) {
                     preL[k] = nl;
                     preR[k] = nr;
+                }
+            }
+        } else {
+            uint64_t *trow = trace ? trace + ((size_t)hb + id) * ORB_MAX_PASSES : nullptr;
+            uint32_t *row = cell_hist + (size_t)c * kBins;
+            const RoundOut r1 = replay_row(row, rec, lane, w == 0 ? trow : nullptr);
+            lo = uniform(r1.L);
+            hi = uniform(r1.R);
+            passes = r1.passes;
+            found = r1.found;
+            const unsigned long long list = n ? sel_lists[f] : 0ull;
+            const uint32_t m = uniform((uint32_t)list) < n ? uniform((uint32_t)list) : n;
+            const uint32_t nbelow = uniform((uint32_t)(list >> 32));
+            const float target = difference_target(n, (int32_t)uniform((uint32_t)rec.nLeaf));
+            if (t < kBins) hist[t] = 0u;
+            __syncthreads();  // every wave has read the row
+            if (t < kBins) row[t] = 0u;  // the next level adds to zero
+            while (!found && passes < ORB_MAX_PASSES) {
+                const float width = hi - lo;
+                const float scale = width > 0.0f ? (float)kBins / width : 0.0f;
+                const float lim = 0.5f - bin_tolerance(lo, hi, scale);
+                uint32_t below = 0;  // wave-uniform
+                for (uint32_t k0 = 0; k0 < m; k0 += 4u * kTailBlock) {
+                    float v[4];
+                    bool in[4];
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) {
+                        const uint32_t k = k0 + (uint32_t)(u * kTailBlock + t);
+                        in[u] = k < m;
+                        v[u] = in[u] ? sel[begin + k] : 0.0f;
+                    }
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) {
+                        const bool lt = in[u] && v[u] < lo, on = in[u] && !(v[u] < lo) && !(v[u] > hi);
+                        below += (uint32_t)__popcll(__ballot(lt));
+                        if (!on) continue;
+                        int bin;
+                        if (!bin_estimate(v[u], lo, scale, lim, bin))
+                            bin = le_cmp ? bin_walk<1>(v[u], lo, hi) : bin_walk<0>(v[u], lo, hi);
+                        atomicAdd(&hist[bin], 1u);
+                    }
+                }
+                if (lane == 0 && below) atomicAdd(&hist[0], below);
+                if (t == 0 && nbelow) atomicAdd(&hist[0], nbelow);  // the keys below the window
+                __syncthreads();
+                if (w == 0) {
+                    const uint4 h4 = reinterpret_cast<const uint4 *>(hist)[lane];
+                    reinterpret_cast<uint4 *>(hist)[lane] = make_uint4(0u, 0u, 0u, 0u);
+                    const uint32_t s0 = h4.x, s1 = s0 + h4.y, s2 = s1 + h4.z, s3 = s2 + h4.w;
+                    const uint32_t base = wave_inclusive_scan(s3) - s3;
+                    const uint32_t pv[4] = {base + s0, base + s1, base + s2, base + s3};
+                    const RoundOut ro = replay_round_lanes(pv, lo, hi, target, passes, lane, trow);
+                    if (lane == 0) {
+                        s_lr[0] = ro.L;
+                        s_lr[1] = ro.R;
+                        s_pf[0] = ro.passes;
+                        s_pf[1] = ro.found ? 1 : 0;
+                    }
+                }
+                __syncthreads();
+                lo = uniform(s_lr[0]);
+                hi = uniform(s_lr[1]);
+                passes = (int32_t)uniform((uint32_t)s_pf[0]);
+                found = uniform((uint32_t)s_pf[1]) != 0u;
+            }
+            const float cut = cell_cut(lo, hi);
+            // ---- stopper masks: a wave per kPer chunks, a word per lane
+            constexpr int kPer = 4;
+            for (uint32_t k0 = (uint32_t)(w * kPer); k0 < nch; k0 += (uint32_t)(kW * kPer)) {
+                uint64_t G[kPer], W[kPer];
+                float v0[kPer];
+                const float *pk[kPer];
+#pragma unroll
+                for (int u = 0; u < kPer; ++u) {
+                    const uint32_t k = k0 + (uint32_t)u < nch ? k0 + (uint32_t)u : nch - 1u;
+                    const uint64_t *mq = masks + (size_t)(f + k) * (2 * kMaskWords);
+                    G[u] = mq[lane];
+                    W[u] = mq[kMaskWords + lane];
+                }
+#pragma unroll
+                for (int u = 0; u < kPer; ++u) {
+                    const uint32_t k = k0 + (uint32_t)u < nch ? k0 + (uint32_t)u : nch - 1u;
+                    const uint32_t cw = (uint32_t)__popcll(W[u]);
+                    const uint32_t ex = wave_inclusive_scan(cw) - cw;
+                    const int q0 = lane & ~15;  // first word of this lane's quarter
+                    const uint32_t rank = ex - (uint32_t)__shfl((int)ex, q0, 64);
+                    pk[u] = pack + begin + k * (uint32_t)kChunk + 64u * (uint32_t)q0 + rank;
+                    v0[u] = W[u] ? *pk[u] : 0.0f;
+                }
+#pragma unroll
+                for (int u = 0; u < kPer; ++u) {
+                    const uint32_t k = k0 + (uint32_t)u;
+                    if (k >= nch) break;  // uniform
+                    const uint32_t p0 = k * (uint32_t)kChunk + 64u * (uint32_t)lane;
+                    const uint64_t valid =
+                        p0 >= n ? 0ull : (n - p0 >= 64u ? ~0ull : (1ull << (n - p0)) - 1ull);
+                    uint64_t L = G[u], R = valid & ~G[u] & ~W[u], wd = W[u];
+                    float vk = v0[u];
+                    const float *at = pk[u];
+                    while (wd) {
+                        const uint32_t bit = (uint32_t)__builtin_ctzll(wd);
+                        wd &= wd - 1ull;
+                        L |= (!(vk < cut) ? 1ull : 0ull) << bit;
+                        R |= (!(vk > cut) ? 1ull : 0ull) << bit;
+                        if (wd) vk = *++at;
+                    }
+                    uint64_t *mq = masks + (size_t)(f + k) * (2 * kMaskWords);
+                    mq[lane] = L;
+                    mq[kMaskWords + lane] = R;
+                    const uint32_t nl = wave_sum((uint32_t)__popcll(L));
+                    const uint32_t nr = wave_sum((uint32_t)__popcll(R));
+                    if (lane == 0) {
+                        preL[k] = nl;
+                        preR[k] = nr;
+                    }
                 }
             }
         }
@@ -3020,6 +3231,14 @@ __global__ __launch_bounds__(kTailBlock) void k_m_tail(
 // ---------------------------------------------------------------------------
 // orchestration
 // ---------------------------------------------------------------------------
+// Rows of weight sums: one a cell (the chunk path), or one a cell and round
+// for levels of few chunks (fewer than kRecsScan cells).
+static size_t hist_w_rows(const Ctx &c)
+{
+    const size_t m = (size_t)c.max_level_cells;
+    return std::max(m, (size_t)kRounds * std::min(m, (size_t)kRecsScan));
+}
+
 static int ensure_state(Ctx &c, int32_t levels_mode, bool *complete)
 {
     if (!c.batched) c.batched = new (std::nothrow) BatchedState;
@@ -3040,8 +3259,10 @@ static int ensure_state(Ctx &c, int32_t levels_mode, bool *complete)
     if (c.trace) ORB_TRY(b.trace.alloc((size_t)c.cap * ORB_MAX_PASSES));
     if (c.weighted) {
         ORB_TRY(b.chunk_hist_w.alloc((size_t)(c.max_chunks + 1) * kBins));
-        if (b.cell_hist_w.n < (size_t)c.max_level_cells * kBins) b.hist_w_clean = false;
-        ORB_TRY(b.cell_hist_w.alloc((size_t)c.max_level_cells * kBins));
+        const size_t rows = hist_w_rows(c);
+        if (b.cell_hist_w.n < rows * kBins) b.hist_w_clean = false;
+        ORB_TRY(b.cell_hist_w.alloc(rows * kBins));
+        ORB_TRY(c.round_state.alloc(4 * 2 * (size_t)kRecsScan));
     }
     if (!c.weighted) ORB_TRY(c.sel.alloc((size_t)c.stride));  // rounds 3 and 4
     // every buffer the launches touch exists before a capture starts
@@ -3083,7 +3304,7 @@ static std::vector<uint64_t> graph_signature(const Ctx &c, const BatchedState &b
                           c.packed.p, c.masks.p, c.cell_cand.p, c.splits.p, c.chunk_comp.p,
                           c.sel.p, c.sel_lists.p, c.swap_plan.p, c.status.p, c.stamps.p, b.level_ids.p, b.heap.p, b.exists.p,
                           b.sub.p, b.chunk_hist.p, b.cell_hist.p, b.trace.p, b.level_passes.p,
-                          c.wt.p, c.wt_tmp.p, b.chunk_hist_w.p, b.cell_hist_w.p, c.hstatus.p, b.hpasses.p};
+                          c.wt.p, c.wt_tmp.p, b.chunk_hist_w.p, b.cell_hist_w.p, c.round_state.p, c.hstatus.p, b.hpasses.p};
     for (const void *p : bufs) s.push_back((uint64_t)(uintptr_t)p);
     s.push_back((uint64_t)c.tune_chunk_blocks.size());
     for (int32_t v : c.tune_chunk_blocks) s.push_back((uint64_t)(int64_t)v);
@@ -3103,8 +3324,8 @@ int enqueue_level(Ctx &c, const LevelEntry *entries, int32_t nCells, orb_cell *h
         return ORB_ERR_STATE;  // rounds 3 and 4 gather into these
     const int32_t sub_max = subtree_max_keys(c);
     const bool use_subtree = any_subtree && c.part == ORB_PART_HOARE && sub_max > 0;
-    if ((kernels.cell_max || kernels.chunks != kChunksAll) && (c.part != ORB_PART_HOARE || c.weighted))
-        return ORB_ERR_STATE;
+    if ((kernels.cell_max || kernels.chunks != kChunksAll) && c.part != ORB_PART_HOARE) return ORB_ERR_STATE;
+    if (c.weighted && kernels.cell_max) return ORB_ERR_STATE;
     const bool mid = kernels.chunks == kChunksMid;
     if (mid && nCells >= kRecsScan) return ORB_ERR_STATE;  // one block fills its tables
     const LevelMode mode{use_subtree ? (uint32_t)sub_max : 0u, kernels.cell_max,
@@ -3202,20 +3423,34 @@ int enqueue_level(Ctx &c, const LevelEntry *entries, int32_t nCells, orb_cell *h
     if (kernels.chunks == kChunksNone) return ORB_OK;
     const unsigned gq = chunk_grid(c);
     if (mid) {
-        const int tb = timing_mark(c);
+        int tb = timing_mark(c);
         unsigned long long *lists = reinterpret_cast<unsigned long long *>(c.sel_lists.p);
-        hipLaunchKernelGGL(le ? k_m_hist<1> : k_m_hist<0>, dim3(gq), dim3(kBlock), 0, c.stream,
-                           c.recs.p, nCells, c.cell_first.p, c.chunk_desc.p, (uint32_t)c.max_chunks,
-                           c.x(), c.y(), c.z(), cell_hist);
-        hipLaunchKernelGGL(k_m_window, dim3(gq), dim3(kBlock), 0, c.stream, c.recs.p, nCells,
-                           c.cell_first.p, c.chunk_desc.p, (uint32_t)c.max_chunks, c.x(), c.y(), c.z(),
-                           cell_hist, c.packed.p, c.masks.p, c.sel.p, lists);
+        RoundState *state = reinterpret_cast<RoundState *>(c.round_state.p);
+        const uint32_t mc = (uint32_t)c.max_chunks;
+        if (c.weighted) {
+            for (int r = 0; r < kRounds; ++r)
+                hipLaunchKernelGGL(le ? k_mw_hist<1> : k_mw_hist<0>, dim3(gq), dim3(kBlock), 0, c.stream,
+                                   c.recs.p, nCells, c.cell_first.p, c.chunk_desc.p, mc, c.x(), c.y(),
+                                   c.z(), c.weights(), r, state, cell_hist_w, trace);
+        } else {
+            hipLaunchKernelGGL(le ? k_m_hist<1> : k_m_hist<0>, dim3(gq), dim3(kBlock), 0, c.stream,
+                               c.recs.p, nCells, c.cell_first.p, c.chunk_desc.p, mc, c.x(), c.y(), c.z(),
+                               cell_hist);
+            hipLaunchKernelGGL(k_m_window, dim3(gq), dim3(kBlock), 0, c.stream, c.recs.p, nCells,
+                               c.cell_first.p, c.chunk_desc.p, mc, c.x(), c.y(), c.z(), cell_hist,
+                               c.packed.p, c.masks.p, c.sel.p, lists);
+        }
         ORB_HIP(hipGetLastError());
         ORB_TRY(timing_pair(c, tb, kTimeCount));
         const int tp = timing_mark(c);
-        hipLaunchKernelGGL(k_m_tail, dim3((unsigned)std::max<int32_t>(nCells, 1)), dim3(kTailBlock), 0,
-                           c.stream, c.recs.p, nCells, c.cell_first.p, cell_hist, c.sel.p, lists,
-                           c.packed.p, c.masks.p, c.chunk_pre.p, c.splits.p,
+        if (c.weighted)
+            hipLaunchKernelGGL(k_mw_masks, dim3(gq), dim3(kBlock), 0, c.stream, c.recs.p, nCells,
+                               c.cell_first.p, c.chunk_desc.p, mc, c.x(), c.y(), c.z(), state, cell_hist_w,
+                               c.masks.p, trace);
+        hipLaunchKernelGGL(c.weighted ? k_m_tail<true> : k_m_tail<false>,
+                           dim3((unsigned)std::max<int32_t>(nCells, 1)), dim3(kTailBlock), 0, c.stream,
+                           c.recs.p, nCells, c.cell_first.p, cell_hist, c.sel.p, lists, c.packed.p, state,
+                           cell_hist_w, c.masks.p, c.chunk_pre.p, c.splits.p,
                            reinterpret_cast<SwapPlan *>(c.swap_plan.p), c.ranges.p, heap, exists, le,
                            trace, level_passes, status);
         ORB_HIP(hipGetLastError());
@@ -3335,7 +3570,13 @@ static LevelKernels level_kernels(const Ctx &c, int32_t level, int32_t cells, in
                                   bool all_sub)
 {
     LevelKernels k;
-    if (c.part != ORB_PART_HOARE || c.weighted || cells <= 0) return k;
+    if (c.part != ORB_PART_HOARE || cells <= 0) return k;
+    const bool few = c.n / kChunk + cells <= kMidLevelChunks && cells < kRecsScan;
+    if (c.weighted) {
+        // sizes below the root follow the weights: twice the even share allowed for
+        if (few && (level == 1 ? hi : 2 * hi) <= (int64_t)kMidChunks * kChunk) k.chunks = kChunksMid;
+        return k;
+    }
     hi += 4 * (int64_t)level;
     lo -= 4 * (int64_t)level;
     if (all_sub) {
@@ -3345,8 +3586,7 @@ static LevelKernels level_kernels(const Ctx &c, int32_t level, int32_t cells, in
     if (lo <= (int64_t)kCellLarge) k.cell_max = hi <= (int64_t)kCellSmall ? kCellSmall : kCellLarge;
     if (hi <= (int64_t)kCellLarge)
         k.chunks = kChunksNone;
-    else if (hi <= (int64_t)kMidChunks * kChunk && c.n / kChunk + cells <= kMidLevelChunks &&
-             cells < kRecsScan)
+    else if (few && hi <= (int64_t)kMidChunks * kChunk)
         k.chunks = kChunksMid;
     return k;
 }
@@ -3374,20 +3614,21 @@ static int enqueue_build(Ctx &c, int32_t levels_mode, bool again)
     // from n and d (orb_level_shape, within the termination rule's +-2 a
     // split).  They give the chunk kernels' grids and the level's kernels;
     // where every cell of a level is expected to finish in the subtree
-    // kernel, the build ends there.  Weighted builds split by weight: unknown.
+    // kernel, the build ends there.  Weighted builds split by weight: their
+    // sizes only choose between the two forms of the chunk path.
     c.level_chunk_hint.assign((size_t)lmax + 2, -1);
     std::vector<LevelKernels> kernels((size_t)lmax + 2);
     int32_t last = lmax;
-    if (!c.weighted && !again) {
+    if (!again) {
         const int32_t sub_max = subtree_max_keys(c);
         for (int32_t l = 1; l <= lmax; ++l) {
             int64_t lo = 0, hi = 0;
             const int cells = orb_level_shape(c.n, c.d, l, &lo, &hi);
             if (cells < 0) break;
             const int64_t max_leaf = ((int64_t)c.d + (int64_t(1) << (l - 1)) - 1) >> (l - 1);
-            const bool all_sub = b.complete && c.part == ORB_PART_HOARE && sub_max > 0 &&
+            const bool all_sub = b.complete && c.part == ORB_PART_HOARE && !c.weighted && sub_max > 0 &&
                                  hi + 4 * l <= sub_max && max_leaf <= kSmallLeaves;
-            c.level_chunk_hint[(size_t)l] = c.n / kChunk + cells + 1;
+            if (!c.weighted) c.level_chunk_hint[(size_t)l] = c.n / kChunk + cells + 1;
             kernels[(size_t)l] = level_kernels(c, l, cells, lo, hi, all_sub);
             if (all_sub) {
                 last = l;
@@ -3442,7 +3683,7 @@ int build_batched(Ctx &c, int32_t levels_mode, orb_build_info *info)
         b.hist_clean = true;
     }
     if (c.weighted && !b.hist_w_clean) {
-        ORB_TRY(launch_zero_u64(c.stream, b.cell_hist_w.p, (size_t)c.max_level_cells * kBins));
+        ORB_TRY(launch_zero_u64(c.stream, b.cell_hist_w.p, hist_w_rows(c) * kBins));
         b.hist_w_clean = true;
     }
     c.trace_weighted = c.weighted;

@@ -89,3 +89,41 @@ def test_larger_than_expected(orb, oracle, n, d, subtree):
     x, y, z = oracle.generate(n)
     x[np.random.default_rng(2).random(n) < 0.7] = np.float32(0.21)
     assert check(orb, oracle, (x, y, z), d, ids=True, subtree=subtree)
+
+
+# weighted builds on levels of few chunks: even weights, many zeros, and a few
+# heavy particles (cells of very uneven sizes; with 3 of them a cell outgrows
+# the tables of a level of few chunks and the levels run again)
+@pytest.mark.parametrize("n,d,kind", [(5121, 2, "even"), (40961, 8, "even"), (150001, 24, "zeros"),
+                                      (150001, 8, "grid"), (1000003, 16, "heavy"), (2000003, 8, "three")])
+@pytest.mark.parametrize("cmp", [0, 1])
+def test_weighted_few_chunks(orb, oracle, n, d, kind, cmp):
+    rng = np.random.default_rng(n)
+    x, y, z = inputs.quantized(n, levels=64, seed=1) if kind == "grid" else oracle.generate(n)
+    w = rng.integers(1, 1000, n).astype(np.uint32)
+    if kind == "zeros":
+        w[rng.random(n) < 0.9] = 0
+    elif kind in ("heavy", "three"):
+        w[:] = 1
+        w[rng.integers(0, n, 3 if kind == "three" else 50)] = 1 << 24
+    with orb.Context(n, d, generate=False) as ctx:
+        ctx.set_semantics(cmp, 0)
+        ctx.set_particles(x, y, z)
+        ctx.enable_ids()
+        ctx.set_weights(w)
+        ctx.enable_trace(True)
+        r = oracle.build(x, y, z, d, levels_mode=1, cmp=cmp, ids=True, weights=w, pass_weights=True)
+        try:
+            info = ctx.build(orb.FORM_BATCHED, orb.LEVELS_FULL)
+        except orb.OrbError as e:
+            assert (e.code, e.error_cell) == (r.rc, r.error_cell)
+            return
+        assert r.rc == 0
+        assert info["level_passes"] == list(r.level_passes)
+        assert_heaps_equal(ctx.heap(), r.heap, r.exists)
+        assert np.array_equal(ctx.ranges(), r.ranges)
+        assert np.array_equal(ctx.pass_weights(), r.pass_weights)
+        for a, b in zip(ctx.get_particles(), (r.x, r.y, r.z)):
+            assert np.array_equal(fbits(a), fbits(b))
+        assert np.array_equal(ctx.ids(), r.ids)
+        assert np.array_equal(ctx.weights(), r.weights)

@@ -108,3 +108,35 @@ def test_rebuild_of_built_order(orb, oracle, form):
     ctx.close()
     g, r = run_both(orb, oracle, bx, by, bz, 256, 1, form=form)
     assert_same_build(g, r)
+
+
+# the stable partition's chunks: one key, partial rows and quarters, a full
+# chunk and one key more, all keys on one side, with and without the payload
+@pytest.mark.parametrize("n", [1, 63, 65, 1023, 1025, 4095, 4096, 4097, 12289])
+@pytest.mark.parametrize("side", ["both", "left", "right"])
+@pytest.mark.parametrize("ids,weights", [(False, False), (True, False), (False, True), (True, True)])
+def test_stable_chunk_edges(orb, n, side, ids, weights):
+    rng = np.random.default_rng(n)
+    xyz = [rng.random(n).astype(np.float32) - np.float32(0.5) for _ in range(3)]
+    w = rng.integers(1, 99, n).astype(np.uint32)
+    cell = np.zeros(1, orb.CELL_DTYPE)
+    cell["nLeafCells"], cell["cutAxis"] = 2, 1
+    cut = {"both": 0.1, "left": 0.75, "right": -0.75}[side]
+    cell["cutMarginLeft"] = cell["cutMarginRight"] = cut
+    cell["lower"], cell["upper"] = -0.5, 0.5
+    with orb.Context(n, 2, generate=False) as ctx:
+        ctx.set_particles(*xyz)
+        if ids:
+            ctx.enable_ids()
+        if weights:
+            ctx.set_weights(w)
+        ctx.partition_gpu(cell)
+        left = xyz[1] <= np.float32(cut)
+        order = np.concatenate([np.nonzero(left)[0], np.nonzero(~left)[0]])
+        for a, b in zip(ctx.get_particles(), xyz):
+            assert np.array_equal(a, b[order])
+        assert ctx.ranges()[1:].tolist() == [[0, int(left.sum())], [int(left.sum()), n]]
+        if ids:
+            assert np.array_equal(ctx.ids(), order)
+        if weights:
+            assert np.array_equal(ctx.weights(), w[order])

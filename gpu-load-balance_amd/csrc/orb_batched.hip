@@ -183,10 +183,10 @@ __global__ void k_b_done(const int32_t *status, const int32_t *level_passes, int
 // most sub_max keys (and kSmallLeaves leaves) go to the subtree kernel, cells
 // of at most cell_max keys to k_b_cell (0: not launched), cells of at most
 // chunk_max keys to the chunk kernels.  A level whose kernels do not take
-// every size (chosen from the sizes the host expects) leaves a larger cell
-// alone and counts it in the build's pass counter 0; the host then runs the
-// levels again with the chunk path (again = 1), which skips the cells that
-// are split already.
+// every size, or after which the build ends (both chosen from the sizes the
+// host expects), leaves a larger cell alone and counts it in the build's pass
+// counter 0; the host then runs the levels again with the chunk path (again =
+// 1), which skips the cells that are split already.
 struct LevelMode {
     uint32_t sub_max, cell_max, chunk_max;
     int32_t again;
@@ -228,9 +228,9 @@ __device__ inline uint32_t level_rec(const LevelEntry *entries, int32_t i, const
         r.flags = 1;
     } else if (mode.sub_max && en.sub_ok && n <= mode.sub_max && cl.nLeafCells <= kSmallLeaves) {
         r.flags = 2;
-    } else if (mode.cell_max && n <= mode.cell_max) {
+    } else if (mode.cell_max && n <= mode.cell_max && !en.last) {
         r.flags = kFlagBlock;
-    } else if (n <= mode.chunk_max) {
+    } else if (n <= mode.chunk_max && !en.last) {
         r.flags = 0;
     } else {
         r.flags = 1;
@@ -3560,34 +3560,58 @@ int enqueue_level(Ctx &c, const LevelEntry *entries, int32_t nCells, orb_cell *h
     return ORB_OK;
 }
 
-// The kernels of a level whose cells are expected to hold lo to hi keys
-// (counts within the termination rule's +-2 a split of the exact shares, four
-// a level allowed for).  k_b_cell takes a level of cells that fit its
+// Adds a build's level; returns whether the build is expected to end there
+// (every cell of it finishes in the subtree kernel).
+bool LevelShape::add(const Ctx &c, int64_t n, int32_t d, int32_t level, bool complete)
+{
+    int64_t l = 0, h = 0;
+    const int32_t m = orb_level_shape(n, d, level, &l, &h);
+    if (m <= 0) {  // unknown
+        known = false;
+        return false;
+    }
+    // counts within the termination rule's +-2 a split of the exact shares,
+    // four a level allowed for
+    h += 4 * (int64_t)level;
+    l -= 4 * (int64_t)level;
+    const int32_t sub_max = subtree_max_keys(c);
+    const int64_t max_leaf = ((int64_t)d + (int64_t(1) << (level - 1)) - 1) >> (level - 1);
+    const bool subtree = complete && c.part == ORB_PART_HOARE && !c.weighted && sub_max > 0 &&
+                         h <= sub_max && max_leaf <= kSmallLeaves;
+    // sizes below the root follow the weights: twice the even share allowed for
+    if (c.weighted && level > 1) h *= 2;
+    if (!subtree) {
+        lo = cells_above ? std::min(lo, l) : l;
+        hi = std::max(hi, h);
+        cells_above += m;
+    }
+    cells += m;
+    keys += n;
+    return subtree;
+}
+
+// The kernels of a level of that shape.  k_b_cell takes cells that fit its
 // registers in two launches where the chunk path needs sixteen and reads the
 // keys once, not twice; a level whose every cell fits it or the subtree kernel
-// goes without the chunk kernels.
-static LevelKernels level_kernels(const Ctx &c, int32_t level, int32_t cells, int64_t lo, int64_t hi,
-                                  bool all_sub)
+// goes without the chunk kernels.  The lines: a block a cell holds 40960
+// keys; a level of few chunks (kMidLevelChunks) is bound by its launches.
+LevelKernels level_kernels(const Ctx &c, const LevelShape &s)
 {
     LevelKernels k;
-    if (c.part != ORB_PART_HOARE || cells <= 0) return k;
-    const bool few = c.n / kChunk + cells <= kMidLevelChunks && cells < kRecsScan;
-    if (c.weighted) {
-        // sizes below the root follow the weights: twice the even share allowed for
-        if (few && (level == 1 ? hi : 2 * hi) <= (int64_t)kMidChunks * kChunk) k.chunks = kChunksMid;
-        return k;
-    }
-    hi += 4 * (int64_t)level;
-    lo -= 4 * (int64_t)level;
-    if (all_sub) {
+    if (c.part != ORB_PART_HOARE || !s.known) return k;
+    if (s.cells_above == 0) {  // subtree cells only
         k.chunks = kChunksNone;
         return k;
     }
-    if (lo <= (int64_t)kCellLarge) k.cell_max = hi <= (int64_t)kCellSmall ? kCellSmall : kCellLarge;
-    if (hi <= (int64_t)kCellLarge)
-        k.chunks = kChunksNone;
-    else if (few && hi <= (int64_t)kMidChunks * kChunk)
-        k.chunks = kChunksMid;
+    const bool few = s.keys / kChunk + s.cells <= kMidLevelChunks && s.cells < kRecsScan;
+    if (!c.weighted) {
+        if (s.lo <= (int64_t)kCellLarge) k.cell_max = s.hi <= (int64_t)kCellSmall ? kCellSmall : kCellLarge;
+        if (s.hi <= (int64_t)kCellLarge) {
+            k.chunks = kChunksNone;
+            return k;
+        }
+    }
+    if (few && s.hi <= (int64_t)kMidChunks * kChunk) k.chunks = kChunksMid;
     return k;
 }
 
@@ -3620,17 +3644,13 @@ static int enqueue_build(Ctx &c, int32_t levels_mode, bool again)
     std::vector<LevelKernels> kernels((size_t)lmax + 2);
     int32_t last = lmax;
     if (!again) {
-        const int32_t sub_max = subtree_max_keys(c);
         for (int32_t l = 1; l <= lmax; ++l) {
-            int64_t lo = 0, hi = 0;
-            const int cells = orb_level_shape(c.n, c.d, l, &lo, &hi);
-            if (cells < 0) break;
-            const int64_t max_leaf = ((int64_t)c.d + (int64_t(1) << (l - 1)) - 1) >> (l - 1);
-            const bool all_sub = b.complete && c.part == ORB_PART_HOARE && !c.weighted && sub_max > 0 &&
-                                 hi + 4 * l <= sub_max && max_leaf <= kSmallLeaves;
-            if (!c.weighted) c.level_chunk_hint[(size_t)l] = c.n / kChunk + cells + 1;
-            kernels[(size_t)l] = level_kernels(c, l, cells, lo, hi, all_sub);
-            if (all_sub) {
+            LevelShape shape;
+            const bool ends = shape.add(c, c.n, c.d, l, b.complete);
+            if (!shape.known) break;
+            if (!c.weighted) c.level_chunk_hint[(size_t)l] = c.n / kChunk + shape.cells + 1;
+            kernels[(size_t)l] = level_kernels(c, shape);
+            if (ends) {
                 last = l;
                 break;
             }

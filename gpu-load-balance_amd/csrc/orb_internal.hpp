@@ -419,7 +419,8 @@ struct LevelEntry {
     int32_t st;       // status pair index: 2 * build slot
     int32_t lmax;     // last level of the build
     int32_t sub_ok;   // the build's schedule lets a subtree finish in LDS
-    int32_t pad;
+    int32_t last;     // no level of the build follows: a cell the subtree kernel does not
+                      // take is left alone and counted (LevelMode)
 };
 
 // Cut and axis a cell's per-chunk counts were taken at (axis -1: none).
@@ -663,6 +664,15 @@ struct LevelKernels {
     uint32_t cell_max = 0;
     bool again = false;
 };
+// What the host expects of a level's cells: their number, the particles of
+// their builds, and the fewest and most keys of those above the subtree kernel.
+struct LevelShape {
+    bool known = true;
+    int64_t lo = 0, hi = 0, keys = 0;
+    int32_t cells = 0, cells_above = 0;
+    bool add(const Ctx &c, int64_t n, int32_t d, int32_t level, bool complete);
+};
+LevelKernels level_kernels(const Ctx &c, const LevelShape &s);
 // one level step of the batched form over `entries` (device array)
 // (chunk_hist_w, cell_hist_w: the weighted rounds' rows, when c.weighted;
 // fin_in: the previous level's due row swaps, run in this level's first

@@ -10,9 +10,8 @@
 // pass counter and status slot (LevelEntry).  A cell's result depends only on
 // its own particles and Cell, so a build's result is the same alone and in
 // any mix.  When a build's last level is enqueued, its particles, ranges,
-// heap and counters are copied to server-owned pinned buffers and its pool
-// ranges are released at once (later uploads are stream-ordered after the
-// copies).
+// heap and counters go to server-owned pinned buffers, and its pool
+// ranges are released once they are done.
 #include <chrono>
 #include <deque>
 #include <map>
@@ -144,6 +143,7 @@ struct Request {
     bool complete = true;
     int32_t lmax = 0;
     int32_t next_level = 1;
+    bool again = false;          // its levels run again (a level left cells alone)
     int state = kPending;
     int error = 0;
     int32_t error_cell = -1;
@@ -189,21 +189,116 @@ struct Server {
     orb_server_stats stats{};
 };
 
-__global__ void k_s_init(orb_cell *heap, uint8_t *exists, uint8_t *sub, uint32_t *ranges,
-                         int64_t hb, int64_t cap, orb_cell root, uint32_t pb, uint32_t n,
-                         int32_t *passes, int32_t *status)
+// Admission of one request in one launch (three copies, a check and an init
+// before): its particles into the pool (src: a device request's arrays, or
+// the pool itself where a copy from the host went before), the NaN check
+// (kErrInputWord into the status pair) and its fresh heap.  Blocks
+// [0, heap_blocks) take the heap, the others the particles, kAdmitPer a
+// thread.  The slot's counters and status pair are zero: k_s_finish leaves
+// them so.
+constexpr int kAdmitPer = 8;
+__global__ __launch_bounds__(kBlock) void k_s_admit(
+    const float *sx, const float *sy, const float *sz, float *dx, float *dy, float *dz, uint32_t n,
+    uint32_t heap_blocks, orb_cell *heap, uint8_t *exists, uint8_t *sub, uint32_t *ranges, int64_t hb,
+    int64_t cap, orb_cell root, uint32_t pb, int32_t *status)
 {
-    int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t k = i; k < cap; k += stride) {
-        store_root_or_zero(&heap[hb + k], root, k == 0);
-        exists[hb + k] = k == 0 ? 1 : 0;
-        sub[hb + k] = 0;
-        ranges[2 * (hb + k)] = k == 0 ? pb : 0u;
-        ranges[2 * (hb + k) + 1] = k == 0 ? pb + n : 0u;
+    if (blockIdx.x < heap_blocks) {  // uniform
+        for (int64_t k = (int64_t)blockIdx.x * kBlock + threadIdx.x; k < cap;
+             k += (int64_t)heap_blocks * kBlock) {
+            store_root_or_zero(&heap[hb + k], root, k == 0);
+            exists[hb + k] = k == 0 ? 1 : 0;
+            sub[hb + k] = 0;
+            ranges[2 * (hb + k)] = k == 0 ? pb : 0u;
+            ranges[2 * (hb + k) + 1] = k == 0 ? pb + n : 0u;
+        }
+        return;
     }
-    if (i < 64) passes[i] = 0;
-    if (i < 2) status[i] = 0;
+    const bool copy = sx != dx;
+    const uint32_t i0 = (blockIdx.x - heap_blocks) * (uint32_t)(kBlock * kAdmitPer) + threadIdx.x;
+    float v[3][kAdmitPer];
+#pragma unroll
+    for (int u = 0; u < kAdmitPer; ++u) {
+        const uint32_t i = i0 + (uint32_t)(u * kBlock);
+        v[0][u] = i < n ? sx[i] : 0.0f;
+        v[1][u] = i < n ? sy[i] : 0.0f;
+        v[2][u] = i < n ? sz[i] : 0.0f;
+    }
+    bool any = false;
+#pragma unroll
+    for (int u = 0; u < kAdmitPer; ++u) {
+        const uint32_t i = i0 + (uint32_t)(u * kBlock);
+        any = any || isnan(v[0][u]) || isnan(v[1][u]) || isnan(v[2][u]);
+        if (copy && i < n) {
+            dx[i] = v[0][u];
+            dy[i] = v[1][u];
+            dz[i] = v[2][u];
+        }
+    }
+    if (__ballot(any) != 0ull && (threadIdx.x & 63) == 0)
+        atomicMax(reinterpret_cast<unsigned long long *>(status), (unsigned long long)kErrInputWord);
+}
+
+// The results of one request in one launch (eight copies before): its ranges,
+// heap, flags, counters and status into its pinned block, a device request's
+// particles back into the caller's arrays; the slot's counters and status are
+// cleared.  A request of which a level left cells alone (counter 0, LevelMode)
+// gets its counters only: the host runs its levels again.
+__global__ __launch_bounds__(kBlock) void k_s_finish(
+    const float *sx, const float *sy, const float *sz, float *dx, float *dy, float *dz, uint32_t n,
+    uint32_t tree_blocks, const uint32_t *ranges, const uint32_t *heap, const uint8_t *exists,
+    int64_t cap, uint32_t *hranges, uint32_t *hheap, uint8_t *hexists, int32_t *passes,
+    int32_t *status, int32_t *hcounters)
+{
+    const bool whole = *((volatile int32_t *)passes) == 0;  // counter 0
+    if (blockIdx.x < tree_blocks) {  // uniform
+        const int64_t i0 = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+        const int64_t step = (int64_t)tree_blocks * kBlock;
+        if (blockIdx.x == 0) {
+            if (threadIdx.x < 64) {
+                hcounters[threadIdx.x] = passes[threadIdx.x];
+                if (whole) passes[threadIdx.x] = 0;
+            } else if (threadIdx.x < 66) {
+                hcounters[threadIdx.x] = status[threadIdx.x - 64];
+                if (whole) status[threadIdx.x - 64] = 0;
+            }
+        }
+        if (!whole) return;
+        constexpr int64_t kWords = sizeof(orb_cell) / 4;
+        for (int64_t k = i0; k < 2 * cap; k += step) hranges[k] = ranges[k];
+        for (int64_t k = i0; k < kWords * cap; k += step) hheap[k] = heap[k];
+        for (int64_t k = i0; k < cap; k += step) hexists[k] = exists[k];
+        return;
+    }
+    if (!whole) return;
+    const uint32_t i0 = (blockIdx.x - tree_blocks) * (uint32_t)(kBlock * kAdmitPer) + threadIdx.x;
+    float v[3][kAdmitPer];
+#pragma unroll
+    for (int u = 0; u < kAdmitPer; ++u) {
+        const uint32_t i = i0 + (uint32_t)(u * kBlock);
+        v[0][u] = i < n ? sx[i] : 0.0f;
+        v[1][u] = i < n ? sy[i] : 0.0f;
+        v[2][u] = i < n ? sz[i] : 0.0f;
+    }
+#pragma unroll
+    for (int u = 0; u < kAdmitPer; ++u) {
+        const uint32_t i = i0 + (uint32_t)(u * kBlock);
+        if (i < n) {
+            dx[i] = v[0][u];
+            dy[i] = v[1][u];
+            dz[i] = v[2][u];
+        }
+    }
+}
+
+// Blocks that share a request's tree words (a word a thread up to 256 blocks).
+static unsigned tree_grid(int64_t cap)
+{
+    const int64_t g = (13 * cap + kBlock - 1) / kBlock;
+    return (unsigned)(g < 1 ? 1 : (g > 256 ? 256 : g));
+}
+static unsigned particle_grid(int64_t n)
+{
+    return (unsigned)((n + kBlock * kAdmitPer - 1) / (kBlock * kAdmitPer));
 }
 
 static int server_alloc(Server &S)
@@ -235,6 +330,8 @@ static int server_alloc(Server &S)
     ORB_TRY(S.hentries[0].alloc((size_t)c.max_level_cells));
     ORB_TRY(S.hentries[1].alloc((size_t)c.max_level_cells));
     ORB_TRY(launch_zero_u32(c.stream, S.cell_hist.p, (size_t)c.max_level_cells * 256));
+    ORB_TRY(launch_zero_u32(c.stream, reinterpret_cast<uint32_t *>(S.level_passes.p), (size_t)slots * 64));
+    ORB_TRY(launch_zero_u32(c.stream, reinterpret_cast<uint32_t *>(S.status.p), (size_t)slots * 2));
     ORB_HIP(hipStreamSynchronize(c.stream));
     S.palloc.init(c.stride);
     S.halloc.init(H);
@@ -259,29 +356,21 @@ static int admit(Server &S)
         r->hb = hb;
         r->slot = S.free_slots.back();
         S.free_slots.pop_back();
-        if (r->n > 0) {
-            const size_t nb = sizeof(float) * (size_t)r->n;
-            float *dst[3] = {c.x() + pb, c.y() + pb, c.z() + pb};
-            for (int a = 0; a < 3; ++a) {
-                if (r->dev[0])
-                    ORB_HIP(hipMemcpyAsync(dst[a], r->dev[a], nb, hipMemcpyDeviceToDevice, c.stream));
-                else
-                    ORB_HIP(hipMemcpyAsync(dst[a], r->xyz + a * r->n, nb, hipMemcpyHostToDevice,
-                                           c.stream));
-            }
+        float *dst[3] = {c.x() + pb, c.y() + pb, c.z() + pb};
+        const float *src[3] = {dst[0], dst[1], dst[2]};
+        for (int a = 0; a < 3 && r->n > 0; ++a) {
+            if (r->dev[0])
+                src[a] = r->dev[a];
+            else
+                ORB_HIP(hipMemcpyAsync(dst[a], r->xyz + a * r->n, sizeof(float) * (size_t)r->n,
+                                       hipMemcpyHostToDevice, c.stream));
         }
-        const orb_cell root = cell_root(r->d);
-        unsigned g = (unsigned)((r->cap + kBlock - 1) / kBlock);
-        if (g > 4096) g = 4096;
-        hipLaunchKernelGGL(k_s_init, dim3(g), dim3(kBlock), 0, c.stream, S.heap.p, S.exists.p,
-                           S.sub.p, c.ranges.p, (int64_t)hb, (int64_t)r->cap, root, (uint32_t)pb,
-                           (uint32_t)r->n, S.level_passes.p + 64 * r->slot,
-                           S.status.p + 2 * r->slot);
+        const unsigned gh = tree_grid(r->cap);
+        hipLaunchKernelGGL(k_s_admit, dim3(gh + particle_grid(r->n)), dim3(kBlock), 0, c.stream, src[0],
+                           src[1], src[2], dst[0], dst[1], dst[2], (uint32_t)r->n, gh, S.heap.p,
+                           S.exists.p, S.sub.p, c.ranges.p, (int64_t)hb, (int64_t)r->cap,
+                           cell_root(r->d), (uint32_t)pb, S.status.p + 2 * r->slot);
         ORB_HIP(hipGetLastError());
-        // a NaN coordinate fails the request with ORB_ERR_ARG (status word
-        // kErrInputWord, above every undefined-cell word)
-        ORB_TRY(launch_find_nan(c.stream, c.x() + pb, c.y() + pb, c.z() + pb, (size_t)r->n,
-                                S.status.p + 2 * r->slot));
         r->state = kActive;
         r->t_admit = now_ms();
         S.active.push_back(r);
@@ -293,32 +382,21 @@ static int admit(Server &S)
 static int finish(Server &S, Request *r)
 {
     Ctx &c = S.c;
-    const size_t n = (size_t)r->n, cap = (size_t)r->cap;
-    if (n > 0) {
-        const float *src[3] = {c.x() + r->pb, c.y() + r->pb, c.z() + r->pb};
-        for (int a = 0; a < 3; ++a) {
-            if (r->dev[0])
-                ORB_HIP(hipMemcpyAsync(r->dev[a], src[a], sizeof(float) * n,
-                                       hipMemcpyDeviceToDevice, c.stream));
-            else
-                ORB_HIP(hipMemcpyAsync(r->xyz + a * n, src[a], sizeof(float) * n,
-                                       hipMemcpyDeviceToHost, c.stream));
-        }
-    }
-    ORB_HIP(hipMemcpyAsync(r->ranges, c.ranges.p + 2 * r->hb, 2 * sizeof(uint32_t) * cap,
-                           hipMemcpyDeviceToHost, c.stream));
-    ORB_HIP(hipMemcpyAsync(r->heap, S.heap.p + r->hb, sizeof(orb_cell) * cap,
-                           hipMemcpyDeviceToHost, c.stream));
-    ORB_HIP(hipMemcpyAsync(r->exists, S.exists.p + r->hb, cap, hipMemcpyDeviceToHost, c.stream));
-    ORB_HIP(hipMemcpyAsync(r->counters, S.level_passes.p + 64 * r->slot, 64 * sizeof(int32_t),
-                           hipMemcpyDeviceToHost, c.stream));
-    ORB_HIP(hipMemcpyAsync(r->counters + 64, S.status.p + 2 * r->slot, 2 * sizeof(int32_t),
-                           hipMemcpyDeviceToHost, c.stream));
+    const bool dev = r->dev[0] != nullptr;
+    const float *src[3] = {c.x() + r->pb, c.y() + r->pb, c.z() + r->pb};
+    const unsigned gt = tree_grid(r->cap);
+    hipLaunchKernelGGL(k_s_finish, dim3(gt + (dev ? particle_grid(r->n) : 0u)), dim3(kBlock), 0, c.stream,
+                       src[0], src[1], src[2], r->dev[0], r->dev[1], r->dev[2], (uint32_t)r->n, gt,
+                       c.ranges.p + 2 * r->hb, reinterpret_cast<const uint32_t *>(S.heap.p + r->hb),
+                       S.exists.p + r->hb, (int64_t)r->cap, r->ranges,
+                       reinterpret_cast<uint32_t *>(r->heap), r->exists, S.level_passes.p + 64 * r->slot,
+                       S.status.p + 2 * r->slot, r->counters);
+    ORB_HIP(hipGetLastError());
+    // (a host request whose levels run again copies its particles again)
+    for (int a = 0; a < 3 && !dev && r->n > 0; ++a)
+        ORB_HIP(hipMemcpyAsync(r->xyz + a * r->n, src[a], sizeof(float) * (size_t)r->n,
+                               hipMemcpyDeviceToHost, c.stream));
     ORB_HIP(hipEventRecord(r->done, c.stream));
-    // later work on these pool ranges is stream-ordered after the copies
-    S.palloc.release(r->pb, r->n > 0 ? r->n : 1);
-    S.halloc.release(r->hb, r->cap);
-    S.free_slots.push_back(r->slot);
     r->state = kFinishing;
     S.finishing.push_back(r);
     return ORB_OK;
@@ -330,6 +408,22 @@ static int poll_finishing(Server &S)
         Request *r = S.finishing[i];
         hipError_t e = hipEventQuery(r->done);
         if (e == hipSuccess) {
+            S.finishing[i] = S.finishing.back();
+            S.finishing.pop_back();
+            if (r->counters[0] > 0) {
+                // a level whose kernels did not take every size left cells
+                // alone: the levels again, with every kernel
+                ORB_TRY(launch_zero_u32(S.c.stream,
+                                        reinterpret_cast<uint32_t *>(S.level_passes.p + 64 * r->slot), 1));
+                r->again = true;
+                r->next_level = 1;
+                r->state = kActive;
+                S.active.push_back(r);
+                continue;
+            }
+            S.palloc.release(r->pb, r->n > 0 ? r->n : 1);
+            S.halloc.release(r->hb, r->cap);
+            S.free_slots.push_back(r->slot);
             r->state = kDone;
             r->t_done = now_ms();
             S.done_ids.push_back(r->id);
@@ -338,8 +432,6 @@ static int poll_finishing(Server &S)
                 r->error = bad < 0 ? ORB_ERR_ARG : ORB_ERR_UB;
             r->error_cell = bad;
             S.stats.completed++;
-            S.finishing[i] = S.finishing.back();
-            S.finishing.pop_back();
         } else if (e == hipErrorNotReady) {
             ++i;
         } else {
@@ -418,13 +510,15 @@ static int submit(Server &S, const float *hx, const float *hy, const float *hz, 
 static int step(Server &S)
 {
     Ctx &c = S.c;
+    ORB_TRY(poll_finishing(S));  // pool ranges back before the next admission
     ORB_TRY(admit(S));
     if (!S.active.empty()) {
         // this step's level of every active build, in one list
         LevelEntry *h = S.hentries[S.flip].p;
         ORB_HIP(hipEventSynchronize(S.ev_entries[S.flip]));  // staging buffer free again
         int64_t m = 0;
-        bool any_sub = false;
+        bool any_sub = false, any_again = false;
+        LevelShape shape;
         std::vector<Request *> stepped;
         for (Request *r : S.active) {
             while (r->next_level <= r->lmax && r->levels[(size_t)r->next_level].empty())
@@ -433,10 +527,14 @@ static int step(Server &S)
             const int32_t l = r->next_level;
             const auto &ids = r->levels[(size_t)l];
             if (m + (int64_t)ids.size() > c.max_level_cells) break;  // next step takes the rest
+            // a level whose cells all fit the subtree kernel is the build's last
+            const bool last = shape.add(c, r->n, r->d, l, r->complete) && !r->again;
             for (int32_t id : ids)
                 h[m++] = LevelEntry{id, (int32_t)r->hb, (int32_t)r->cap, 64 * r->slot + l,
-                                    2 * r->slot, r->lmax, r->complete ? 1 : 0, 0};
+                                    2 * r->slot, r->lmax, r->complete ? 1 : 0, last ? 1 : 0};
             any_sub = any_sub || r->complete;
+            any_again = any_again || r->again;
+            if (last) r->next_level = r->lmax;
             stepped.push_back(r);
         }
         if (m > 0) {
@@ -444,9 +542,15 @@ static int step(Server &S)
                                    hipMemcpyHostToDevice, c.stream));
             ORB_HIP(hipEventRecord(S.ev_entries[S.flip], c.stream));
             S.flip ^= 1;
+            // the kernels the step's cells are expected to need; a request that
+            // runs again gets every kernel
+            LevelKernels kernels = any_again ? LevelKernels() : level_kernels(c, shape);
+            kernels.again = any_again;
+            c.level_chunk_hint.assign(1, shape.keys / kChunk + m + 1);
             ORB_TRY(enqueue_level(c, S.entries.p, (int32_t)m, S.heap.p, S.exists.p, S.sub.p,
                                   S.chunk_hist.p, S.cell_hist.p, nullptr, S.level_passes.p,
-                                  S.status.p, any_sub, false, -1));
+                                  S.status.p, any_sub, false, 0, nullptr, nullptr, nullptr, false,
+                                  kernels));
             S.stats.steps++;
             S.stats.cells_stepped += m;
             if ((int64_t)stepped.size() > S.stats.max_batch) S.stats.max_batch = (int64_t)stepped.size();
@@ -468,6 +572,16 @@ static int step(Server &S)
     }
     ORB_TRY(poll_finishing(S));
     return (int)(S.pending.size() + S.active.size() + S.finishing.size());
+}
+
+// What a caller that only asks for results drives on: requests that are
+// finishing, and the levels of one that runs again.
+static int progress(Server &S)
+{
+    ORB_TRY(poll_finishing(S));
+    for (const Request *r : S.active)
+        if (r->again) return step(S) < 0 ? ORB_ERR_HIP : ORB_OK;
+    return ORB_OK;
 }
 
 }  // namespace orb
@@ -604,7 +718,7 @@ int orb_server_poll(orb_server *o, uint64_t id)
 {
     if (!o) return ORB_ERR_ARG;
     Server &S = o->s;
-    ORB_TRY(poll_finishing(S));
+    ORB_TRY(progress(S));
     auto it = S.all.find(id);
     if (it == S.all.end()) return ORB_ERR_ARG;
     return it->second->state == kDone ? 1 : 0;
@@ -614,7 +728,7 @@ int orb_server_next_done(orb_server *o, uint64_t *id)
 {
     if (!o || !id) return ORB_ERR_ARG;
     Server &S = o->s;
-    ORB_TRY(poll_finishing(S));
+    ORB_TRY(progress(S));
     while (!S.done_ids.empty()) {
         const uint64_t v = S.done_ids.front();
         S.done_ids.pop_front();

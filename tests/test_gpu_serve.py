@@ -118,3 +118,44 @@ def test_serve_device_requests(orb):
         for arr in t:
             arr.free()
     srv.close()
+
+
+# x holds one value in most particles: a cell outgrows what its level expected,
+# and the request's levels run again beside the others'
+@pytest.mark.parametrize("device", [False, True])
+def test_uneven_cells_run_again(orb, oracle, device):
+    reqs = []
+    for k, (n, d) in enumerate([(17000, 4), (75000, 4), (30000, 16), (300007, 4), (9000, 2)]):
+        x, y, z = oracle.generate(n + k)
+        if k % 2 == 0 or n > 200000:
+            x[np.random.default_rng(k).random(n + k) < 0.7] = np.float32(0.21)
+        reqs.append((x, y, z, d))
+    want = [oracle.build(x, y, z, d, levels_mode=1) for x, y, z, d in reqs]
+    with orb.Server(particle_capacity=1 << 20, cell_capacity=1 << 12, max_active=4) as srv:
+        dev, ids = [], []
+        for x, y, z, d in reqs:
+            if device:
+                dev.append([orb.DeviceArray(a) for a in (x, y, z)])
+                ids.append(srv.submit_device(*(a.address for a in dev[-1]), len(x), d))
+            else:
+                ids.append(srv.submit(x, y, z, d))
+        for _ in range(100000):
+            if srv.step() == 0:
+                break
+        for k, (rid, (x, y, z, d)) in enumerate(zip(ids, reqs)):
+            r, got = want[k], srv.fetch(rid, len(x), d)
+            assert got["error"] == r.rc
+            if r.rc:
+                assert got["error_cell"] == r.error_cell
+                continue
+            assert got["level_passes"] == list(r.level_passes)
+            assert np.array_equal(got["exists"], r.exists)
+            assert_heaps_equal(got["heap"], r.heap, r.exists)
+            assert np.array_equal(got["ranges"], r.ranges)
+            for i, a in enumerate((r.x, r.y, r.z)):
+                assert np.array_equal(fbits(got["xyz"[i]]), fbits(a))
+                if device:
+                    assert np.array_equal(fbits(dev[k][i].numpy()), fbits(a))
+        for arrays in dev:
+            for a in arrays:
+                a.free()

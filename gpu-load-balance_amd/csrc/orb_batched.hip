@@ -1706,12 +1706,17 @@ __device__ inline int bin_walk(float v, float lo, float hi)
 // level's cells sit within a few keys of n / 2^(l-1), so the plain
 // capacity stays a little above 8192 for a level of 8192-key cells to
 // qualify whole.
-template <bool IDS, bool W>
+// A block of 512 threads holds half as much (plain particles only): two share
+// a CU, so that one's barriers, replays and children lie under the other's
+// binning; levels of many cells take it.
+template <bool IDS, bool W, int kThreads = 1024>
 struct SubCap {
     static constexpr int value = W ? 5120 : (IDS ? 7680 : 8832);
 };
-constexpr int kSubBlock = 1024;                 // threads of the subtree kernel
-constexpr int kSubWaves = kSubBlock / 64;       // 16 histogram slots
+template <>
+struct SubCap<false, false, 512> {
+    static constexpr int value = 4224;
+};
 
 static int32_t subtree_capacity(const Ctx &c)
 {
@@ -1737,7 +1742,7 @@ static int32_t subtree_capacity(const Ctx &c)
 // IDS: particle ids move with the particles; a 16-bit local index rides along
 // in LDS and the ids are permuted once at the write-back.  W: workload
 // weights ride along in LDS and the histograms sum weights.
-template <bool IDS, bool W>
+template <bool IDS, bool W, int kSubBlock>
 __global__ __launch_bounds__(kSubBlock) void k_b_subtree(const CellRec *recs, int32_t nCells,
                                                          orb_cell *heap, uint8_t *exists,
                                                          uint8_t *sub, uint32_t *ranges, float *x,
@@ -1746,7 +1751,8 @@ __global__ __launch_bounds__(kSubBlock) void k_b_subtree(const CellRec *recs, in
                                                          int32_t *status, uint32_t *pid,
                                                          uint32_t *wgt, int32_t group)
 {
-    constexpr int kCap = SubCap<IDS, W>::value;
+    constexpr int kCap = SubCap<IDS, W, kSubBlock>::value;
+    constexpr int kSubWaves = kSubBlock / 64;  // histogram slots
     using HistWord = typename std::conditional<W, unsigned long long, uint32_t>::type;
     constexpr int kHistWords = W ? kBins : kBins / 2;  // W: a bin per word; else two
     __shared__ float sx[kCap], sy[kCap], sz[kCap];
@@ -2313,7 +2319,7 @@ __global__ __launch_bounds__(kSubBlock) void k_b_subtree(const CellRec *recs, in
 // is the swap's memory traffic on levels that fill the chip (12 B read and
 // written per key, 4 B more for the keys) and its own serial phases on levels
 // of few cells.  Measured: a level of 4096 cells of 16384 keys 451 us (chunk
-// path 530), one of two 32768-key cells 45 us, of four 16384-key cells 34 us
+// path 530), one of 8192 of 8192 keys 433 us, one of two 32768-key cells 45 us, of four 16384-key cells 34 us
 // (chunk path 85).
 //
 // rows is a multiple of 4, so a wave's part is whole 256-key groups; keys
@@ -2321,10 +2327,11 @@ __global__ __launch_bounds__(kSubBlock) void k_b_subtree(const CellRec *recs, in
 // R-stopper) and are masked out of the L-stopper words.
 //
 // Latency decides on levels of few cells: 1024 threads a cell.  Levels that
-// fill the chip take 512-thread blocks of twice the rows, two to a CU, so that
-// one block's barriers and replays lie under the other's traffic.
+// fill the chip take 512-thread blocks of twice the rows, two to a CU (256
+// threads, four to a CU, where the cells allow), so that one block's barriers
+// and replays lie under the others' traffic.
 constexpr int kCellRowsMax = 40;
-constexpr uint32_t kCellSmall = 20u * 1024u, kCellLarge = 40u * 1024u;  // the two capacities
+constexpr uint32_t kCellTiny = 10u * 1024u, kCellSmall = 20u * 1024u, kCellLarge = 40u * 1024u;  // capacities
 constexpr int32_t kCellManyCells = 256;  // more than a cell per CU
 static_assert(kCellRowsMax <= 64 && kCellLarge <= 65536u, "a mask word per lane, 16-bit positions");
 
@@ -3276,6 +3283,19 @@ int32_t subtree_max_keys(const Ctx &c)
     return c.sub_max_keys < 0 ? cap : (c.sub_max_keys > cap ? cap : c.sub_max_keys);
 }
 
+// The subtree kernel's limit on a level of `cells` cells.  A level that gives
+// every CU several takes the half-sized blocks: at 2^26 keys the five levels
+// from 8192-key cells down took 2.37 ms in whole blocks, 1.69 ms and 0.43 ms
+// with the first of them in k_b_cell.  With fewer cells latency decides, and the whole
+// block's levels are the shorter.
+constexpr int32_t kSubManyCells = 1024;
+static int32_t subtree_limit(const Ctx &c, int32_t cells)
+{
+    const int32_t whole = subtree_max_keys(c);
+    return cells > kSubManyCells && !c.track_ids && !c.weighted
+               ? std::min(whole, SubCap<false, false, 512>::value) : whole;
+}
+
 static void drop_graph(BatchedState &b)
 {
     if (b.exec) (void)hipGraphExecDestroy(b.exec);
@@ -3322,7 +3342,8 @@ int enqueue_level(Ctx &c, const LevelEntry *entries, int32_t nCells, orb_cell *h
     if (c.weighted && (!chunk_hist_w || !cell_hist_w)) return ORB_ERR_STATE;
     if (!c.weighted && (c.sel.n < (size_t)c.stride || c.sel_lists.n < (size_t)c.max_chunks + 1))
         return ORB_ERR_STATE;  // rounds 3 and 4 gather into these
-    const int32_t sub_max = subtree_max_keys(c);
+    const int32_t sub_max = kernels.sub_max ? std::min((int32_t)kernels.sub_max, subtree_max_keys(c))
+                                            : subtree_max_keys(c);
     const bool use_subtree = any_subtree && c.part == ORB_PART_HOARE && sub_max > 0;
     if ((kernels.cell_max || kernels.chunks != kChunksAll) && c.part != ORB_PART_HOARE) return ORB_ERR_STATE;
     if (c.weighted && kernels.cell_max) return ORB_ERR_STATE;
@@ -3401,9 +3422,12 @@ int enqueue_level(Ctx &c, const LevelEntry *entries, int32_t nCells, orb_cell *h
         while (group < 64 && (int64_t)group * 2 * 1024 <= (int64_t)nCells) group *= 2;
         const int32_t ngroups = (nCells + group - 1) / group;
         const unsigned gs = (unsigned)(ngroups < sb ? ngroups : sb);
-        auto subtree = c.track_ids ? (c.weighted ? k_b_subtree<true, true> : k_b_subtree<true, false>)
-                                   : (c.weighted ? k_b_subtree<false, true> : k_b_subtree<false, false>);
-        hipLaunchKernelGGL(subtree, dim3(gs), dim3(kSubBlock), 0, c.stream, c.recs.p, nCells, heap,
+        const bool half = !c.track_ids && !c.weighted && sub_max <= SubCap<false, false, 512>::value;
+        auto subtree =
+            half ? k_b_subtree<false, false, 512>
+            : c.track_ids ? (c.weighted ? k_b_subtree<true, true, 1024> : k_b_subtree<true, false, 1024>)
+                          : (c.weighted ? k_b_subtree<false, true, 1024> : k_b_subtree<false, false, 1024>);
+        hipLaunchKernelGGL(subtree, dim3(gs), dim3(half ? 512 : 1024), 0, c.stream, c.recs.p, nCells, heap,
                            exists, sub, c.ranges.p, c.x(), c.y(), c.z(), le, trace, level_passes,
                            status, c.ids(), c.weights(), group);
         ORB_HIP(hipGetLastError());
@@ -3411,11 +3435,13 @@ int enqueue_level(Ctx &c, const LevelEntry *entries, int32_t nCells, orb_cell *h
     if (kernels.cell_max) {
         const bool payload = c.ids() != nullptr;
         const bool large = kernels.cell_max > kCellSmall, many = nCells > kCellManyCells;
+        const bool tiny = kernels.cell_max <= kCellTiny;
         auto cell = large  ? (payload ? k_b_cell<1024, 40, 4> : k_b_cell<1024, 40, 3>)
-                    : many ? (payload ? k_b_cell<512, 40, 4> : k_b_cell<512, 40, 3>)
+                    : many ? (tiny ? (payload ? k_b_cell<256, 40, 4> : k_b_cell<256, 40, 3>)
+                                   : (payload ? k_b_cell<512, 40, 4> : k_b_cell<512, 40, 3>))
                            : (payload ? k_b_cell<1024, 20, 4> : k_b_cell<1024, 20, 3>);
         hipLaunchKernelGGL(cell, dim3((unsigned)std::min<int32_t>(nCells, 65536)),
-                           dim3(!large && many ? 512 : 1024), 0, c.stream, c.recs.p, nCells, heap,
+                           dim3(!large && many ? (tiny ? 256 : 512) : 1024), 0, c.stream, c.recs.p, nCells, heap,
                            exists, c.ranges.p, c.x(), c.y(), c.z(), c.ids(), c.weights(), le, trace,
                            level_passes, status);
         ORB_HIP(hipGetLastError());
@@ -3562,7 +3588,7 @@ int enqueue_level(Ctx &c, const LevelEntry *entries, int32_t nCells, orb_cell *h
 
 // Adds a build's level; returns whether the build is expected to end there
 // (every cell of it finishes in the subtree kernel).
-bool LevelShape::add(const Ctx &c, int64_t n, int32_t d, int32_t level, bool complete)
+bool LevelShape::add(const Ctx &c, int64_t n, int32_t d, int32_t level, bool complete, bool alone)
 {
     int64_t l = 0, h = 0;
     const int32_t m = orb_level_shape(n, d, level, &l, &h);
@@ -3574,7 +3600,8 @@ bool LevelShape::add(const Ctx &c, int64_t n, int32_t d, int32_t level, bool com
     // four a level allowed for
     h += 4 * (int64_t)level;
     l -= 4 * (int64_t)level;
-    const int32_t sub_max = subtree_max_keys(c);
+    sub_max = subtree_limit(c, alone ? m : 0);
+    fewest = cells ? std::min(fewest, l) : l;
     const int64_t max_leaf = ((int64_t)d + (int64_t(1) << (level - 1)) - 1) >> (level - 1);
     const bool subtree = complete && c.part == ORB_PART_HOARE && !c.weighted && sub_max > 0 &&
                          h <= sub_max && max_leaf <= kSmallLeaves;
@@ -3599,13 +3626,16 @@ LevelKernels level_kernels(const Ctx &c, const LevelShape &s)
 {
     LevelKernels k;
     if (c.part != ORB_PART_HOARE || !s.known) return k;
+    k.sub_max = (uint32_t)s.sub_max;
     if (s.cells_above == 0) {  // subtree cells only
         k.chunks = kChunksNone;
         return k;
     }
     const bool few = s.keys / kChunk + s.cells <= kMidLevelChunks && s.cells < kRecsScan;
     if (!c.weighted) {
-        if (s.lo <= (int64_t)kCellLarge) k.cell_max = s.hi <= (int64_t)kCellSmall ? kCellSmall : kCellLarge;
+        if (s.lo <= (int64_t)kCellLarge)
+            k.cell_max = s.hi <= (int64_t)kCellTiny    ? kCellTiny
+                         : s.hi <= (int64_t)kCellSmall ? kCellSmall : kCellLarge;
         if (s.hi <= (int64_t)kCellLarge) {
             k.chunks = kChunksNone;
             return k;
@@ -3642,14 +3672,16 @@ static int enqueue_build(Ctx &c, int32_t levels_mode, bool again)
     // sizes only choose between the two forms of the chunk path.
     c.level_chunk_hint.assign((size_t)lmax + 2, -1);
     std::vector<LevelKernels> kernels((size_t)lmax + 2);
+    std::vector<uint8_t> no_sub((size_t)lmax + 2, 0);  // no cell expected small enough
     int32_t last = lmax;
     if (!again) {
         for (int32_t l = 1; l <= lmax; ++l) {
             LevelShape shape;
-            const bool ends = shape.add(c, c.n, c.d, l, b.complete);
+            const bool ends = shape.add(c, c.n, c.d, l, b.complete, true);
             if (!shape.known) break;
             if (!c.weighted) c.level_chunk_hint[(size_t)l] = c.n / kChunk + shape.cells + 1;
             kernels[(size_t)l] = level_kernels(c, shape);
+            if (!c.weighted) no_sub[(size_t)l] = shape.fewest > shape.sub_max;
             if (ends) {
                 last = l;
                 break;
@@ -3665,11 +3697,11 @@ static int enqueue_build(Ctx &c, int32_t levels_mode, bool again)
         const int tlevel = timing_mark(c);
         // the subtree kernel runs where a cell may be small enough for it:
         // cells split by count, so one with nLeaf leaves holds about
-        // n * nLeaf / d keys; where even the smallest expected cell is several
-        // times the subtree's limit, the launch (and its flags) are left out
-        // -- only a speed choice, every cell is built either way
+        // n * nLeaf / d keys; where even the smallest expected cell is above
+        // the limit (sizes by weight: several times above it), the launch is
+        // left out -- only a speed choice, every cell is built either way
         const int64_t few = c.n * (int64_t)b.level_min_leaf[(size_t)l] / (c.d > 0 ? c.d : 1);
-        const bool may_sub = few <= 4 * (int64_t)subtree_max_keys(c);
+        const bool may_sub = !no_sub[(size_t)l] && few <= 4 * (int64_t)subtree_max_keys(c);
         const LevelEntry *entries = b.level_ids.p + b.level_off[(size_t)l];
         LevelKernels k = kernels[(size_t)l];
         k.again = again;

@@ -662,6 +662,7 @@ enum { kChunksNone = 0, kChunksMid = 1, kChunksAll = 2 };
 struct LevelKernels {
     int32_t chunks = kChunksAll;
     uint32_t cell_max = 0;
+    uint32_t sub_max = 0;  // the subtree kernel's limit (0: its capacity)
     bool again = false;
 };
 // What the host expects of a level's cells: their number, the particles of
@@ -670,7 +671,10 @@ struct LevelShape {
     bool known = true;
     int64_t lo = 0, hi = 0, keys = 0;
     int32_t cells = 0, cells_above = 0;
-    bool add(const Ctx &c, int64_t n, int32_t d, int32_t level, bool complete);
+    int64_t fewest = 0;   // keys of the smallest cell of all
+    int32_t sub_max = 0;  // the subtree kernel's limit
+    // alone: a level of this build only
+    bool add(const Ctx &c, int64_t n, int32_t d, int32_t level, bool complete, bool alone);
 };
 LevelKernels level_kernels(const Ctx &c, const LevelShape &s);
 // one level step of the batched form over `entries` (device array)

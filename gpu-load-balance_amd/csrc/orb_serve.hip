@@ -528,7 +528,7 @@ static int step(Server &S)
             const auto &ids = r->levels[(size_t)l];
             if (m + (int64_t)ids.size() > c.max_level_cells) break;  // next step takes the rest
             // a level whose cells all fit the subtree kernel is the build's last
-            const bool last = shape.add(c, r->n, r->d, l, r->complete) && !r->again;
+            const bool last = shape.add(c, r->n, r->d, l, r->complete, false) && !r->again;
             for (int32_t id : ids)
                 h[m++] = LevelEntry{id, (int32_t)r->hb, (int32_t)r->cap, 64 * r->slot + l,
                                     2 * r->slot, r->lmax, r->complete ? 1 : 0, last ? 1 : 0};

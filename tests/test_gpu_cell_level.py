@@ -65,6 +65,14 @@ def test_every_level(orb, oracle, n, d):
     assert check(orb, oracle, oracle.generate(n), d, ids=True, subtree=0)
 
 
+# the half-sized subtree blocks: their largest cell, a key more, partial
+# 64-key pieces, and cells below
+@pytest.mark.parametrize("n,d", [(4224, 64), (4225, 64), (8440, 32), (4161, 3), (100003, 1000), (513, 8)])
+@pytest.mark.parametrize("cmp", [0, 1])
+def test_half_subtree_blocks(orb, oracle, n, d, cmp):
+    assert check(orb, oracle, inputs.clustered(n, n_spheres=5, a=0.05, seed=n), d, cmp=cmp, subtree=4224)
+
+
 @pytest.mark.parametrize("keys", ["grid", "edges", "one_value", "sorted"])
 @pytest.mark.parametrize("cmp", [0, 1])
 @pytest.mark.parametrize("n", [30011, 150001])

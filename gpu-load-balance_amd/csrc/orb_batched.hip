@@ -47,6 +47,7 @@ struct BatchedState {
     DevBuf<uint64_t> chunk_hist_w;     // weighted builds: [max_chunks][256] weight sums
     DevBuf<uint64_t> cell_hist_w;      // weighted builds: [max_level_cells][256]
     bool hist_w_clean = false;         // cell_hist_w all zero (as cell_hist)
+    bool sample_clean = false;         // sample_hist all zero (as cell_hist)
     DevBuf<uint64_t> trace;            // [cap][32]
     DevBuf<int32_t> level_passes;      // [64]
     PinBuf<int32_t> hpasses;           // [64]
@@ -958,6 +959,46 @@ __device__ inline void finish_round(CellRec r, int32_t c, const RoundOut &ro, in
 }
 
 
+// A predicted window of a cell (large levels, k_p_choose): [lo, hi], its keys
+// in bins 1 to 254 (bin 0: below, 255: above), and the bins [b1, b2] that can
+// hold the cut (k_p_narrow).
+constexpr int kWindowBins = kBins - 2;
+struct Window {
+    float lo, hi, scale;
+    uint32_t b1, b2, pad[3];
+};
+
+// The bin of a key in the window: grows with the key (a difference and a
+// product by a positive number keep order in float32), so keys of smaller
+// bins are smaller.
+__device__ inline uint32_t window_bin(float v, float lo, float scale)
+{
+    return 1u + (uint32_t)__builtin_amdgcn_fmed3f((v - lo) * scale, 0.0f, (float)(kWindowBins - 1));
+}
+
+// The passes of a predicted cell that its window decides: a candidate left of
+// bin b1 (right of b2) has a difference of -3 or less (3 or more).  Stops at
+// the first candidate inside, or at the pass cap.
+__device__ inline void window_passes(const Window &wd, float &L, float &R, int32_t &passes)
+{
+    while (passes < ORB_MAX_PASSES) {
+        const float c = cell_cut(L, R);
+        const uint32_t b = c < wd.lo ? 0u : (c > wd.hi ? (uint32_t)kBins - 1u : window_bin(c, wd.lo, wd.scale));
+        if (b < wd.b1) L = c;
+        else if (b > wd.b2) R = c;
+        else break;
+        ++passes;
+    }
+}
+
+// Whether the final cut lets the window's masks stand (a search that ends at
+// the pass cap may end outside); else the cell is left alone and counted.
+__device__ inline bool window_holds(const Window &wd, float L, float R)
+{
+    const float c = cell_cut(L, R);
+    return !(c < wd.lo) && !(c > wd.hi);
+}
+
 // Rounds 3 and 4 gather a searching cell's keys into up to 64 lists (see
 // k_b_select): list r covers a contiguous range of the cell's chunks.
 constexpr int kSelChunks = 4;  // chunks per wave: a lane per chunk quarter
@@ -1043,7 +1084,9 @@ __global__ __launch_bounds__(kBlock) void k_b_replay(CellRec *recs, int32_t nCel
 // in flight; a wave's keys are usually fewer than 256 and stay in registers
 // between counting and writing (a dense cluster packs a good part of a
 // chunk: few chunks per wave keep such waves short).
-constexpr int kSelBatch = 4;
+// PRED: the keys of the window bins [b1, b2]; the keys left of them are
+// counted already (k_p_narrow).
+template <bool PRED>
 __global__ __launch_bounds__(kBlock) void k_b_select(const CellRec *__restrict__ recs,
                                                      int32_t nCells,
                                                      const uint32_t *__restrict__ first,
@@ -1052,10 +1095,13 @@ __global__ __launch_bounds__(kBlock) void k_b_select(const CellRec *__restrict__
                                                      const float *__restrict__ ckeys,
                                                      const uint32_t *__restrict__ comp,
                                                      float *__restrict__ sel,
-                                                     unsigned long long *__restrict__ sel_lists)
+                                                     unsigned long long *__restrict__ sel_lists,
+                                                     const Window *__restrict__ windows)
 {
     constexpr int kW = kBlock / 64;
     constexpr int kQ = 4 * kSelChunks;  // quarters (lanes) per wave
+    // (8 in flight for the fuller predicted windows: 23 us a level against 20)
+    constexpr int kSelBatch = 4;
     static_assert(kQ <= 64 && (kQ & (kQ - 1)) == 0, "a lane per chunk quarter");
     __shared__ uint32_t s_below[kW][64], s_cnt[kW][64];  // per run of one cell
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, sh = lane & 3;
@@ -1070,16 +1116,21 @@ __global__ __launch_bounds__(kBlock) void k_b_select(const CellRec *__restrict__
         const uint32_t nc0 = comp[8 * (size_t)qr + sh], nb0 = comp[8 * (size_t)qr + 4];
         const uint32_t cell = inq ? d.z : 0xffffffffu;  // runs end at the table's end
         bool live = inq && d.w <= 2u;
-        float lo = 0.0f, hi = 0.0f;
-        uint32_t begin = 0, f = 0, nch = 0;
+        float lo = 0.0f, hi = 0.0f;  // PRED: the window's lower end and scale
+        uint32_t begin = 0, f = 0, nch = 0, bins = 0;
         if (live) {
             const CellRec &r = recs[cell];
             f = first[cell];
             nch = first[cell + 1] - f;
-            live = !r.found;
+            live = !r.found && !r.flags;
             lo = r.margin_l;
             hi = r.margin_r;
             begin = r.begin;
+            if constexpr (PRED) {
+                lo = windows[cell].lo;
+                hi = windows[cell].scale;
+                bins = windows[cell].b1 | (windows[cell].b2 << 16);
+            }
         }
         uint32_t off = 0, cnt = 0;
         if (inq) wave_share(d.x, d.y, sh, off, cnt);
@@ -1093,12 +1144,22 @@ __global__ __launch_bounds__(kBlock) void k_b_select(const CellRec *__restrict__
         s_cnt[w][lane] = 0u;
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
         __builtin_amdgcn_wave_barrier();
-        if (live && sh == 0 && nb0) atomicAdd(&s_below[w][run], nb0);
+        if (!PRED && live && sh == 0 && nb0) atomicAdd(&s_below[w][run], nb0);
         const uint32_t incl = wave_inclusive_scan(nc), ex = incl - nc;
         const uint32_t T = (uint32_t)__shfl((int)incl, 63, 64);
         // key t of the wave: quarter j = the last with ex_j <= t (it holds t)
         float v[kSelBatch], lj[kSelBatch], hj[kSelBatch];
+        uint32_t bj[PRED ? kSelBatch : 1];
         int rj[kSelBatch];
+        // -1: left of what is gathered, 0: gathered, 1: right of it
+        auto side = [&](int u) __attribute__((always_inline)) {
+            if constexpr (PRED) {
+                const uint32_t b = window_bin(v[u], lj[u], hj[u]);
+                return b < (bj[u] & 0xffffu) ? -1 : (b > (bj[u] >> 16) ? 1 : 0);
+            } else {
+                return v[u] < lj[u] ? -1 : (v[u] > hj[u] ? 1 : 0);
+            }
+        };
         auto load_batch = [&](uint32_t t0) __attribute__((always_inline)) {
 #pragma unroll
             for (int u = 0; u < kSelBatch; ++u) {
@@ -1111,6 +1172,7 @@ __global__ __launch_bounds__(kBlock) void k_b_select(const CellRec *__restrict__
                     (uint32_t)__shfl((int)kbase, j, 64) + (t - (uint32_t)__shfl((int)ex, j, 64));
                 lj[u] = __shfl(lo, j, 64);
                 hj[u] = __shfl(hi, j, 64);
+                if constexpr (PRED) bj[u] = (uint32_t)__shfl((int)bins, j, 64);
                 rj[u] = __shfl(run, j, 64);
                 v[u] = t < T ? ckeys[at] : 0.0f;
             }
@@ -1121,8 +1183,9 @@ __global__ __launch_bounds__(kBlock) void k_b_select(const CellRec *__restrict__
 #pragma unroll
             for (int u = 0; u < kSelBatch; ++u) {
                 if (t0 + 64u * (uint32_t)u + (uint32_t)lane < T) {
-                    if (v[u] < lj[u]) atomicAdd(&s_below[w][rj[u]], 1u);
-                    else if (!(v[u] > hj[u])) atomicAdd(&s_cnt[w][rj[u]], 1u);
+                    const int at = side(u);
+                    if (at == 0) atomicAdd(&s_cnt[w][rj[u]], 1u);
+                    else if (!PRED && at < 0) atomicAdd(&s_below[w][rj[u]], 1u);
                 }
             }
         }
@@ -1148,14 +1211,21 @@ __global__ __launch_bounds__(kBlock) void k_b_select(const CellRec *__restrict__
             if (T > kStep) load_batch(t0);  // uniform: one batch is still in registers
 #pragma unroll
             for (int u = 0; u < kSelBatch; ++u) {
-                if (t0 + 64u * (uint32_t)u + (uint32_t)lane < T && !(v[u] < lj[u]) &&
-                    !(v[u] > hj[u]))
+                if (t0 + 64u * (uint32_t)u + (uint32_t)lane < T && side(u) == 0)
                     sel[atomicAdd(&s_cnt[w][rj[u]], 1u)] = v[u];
             }
         }
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
         __builtin_amdgcn_wave_barrier();  // the run tables are cleared for the next chunks
     }
+}
+
+// A predicted cell that its window does not carry: nothing of it is written,
+// the host's second run of the levels builds it.
+__device__ inline void leave_alone(const CellRec &r, int32_t c, CellRec *recs, int32_t *level_passes)
+{
+    recs[c].flags = 1;
+    atomicAdd(&level_passes[r.lp & ~63], 1);
 }
 
 // Rounds 3 and 4 of each searching cell from its gathered keys, a wave per
@@ -1167,15 +1237,18 @@ __global__ __launch_bounds__(kBlock) void k_b_select(const CellRec *__restrict__
 // cut nor reached the pass cap runs round 4 over the same keys with the
 // narrowed margins (the keys that now fall below them join the count
 // below).  The record, heap cell and split are written as after any round.
+// PRED (large levels): the rounds start from the cell's own margins; the
+// passes that the window decides come first.
 constexpr int kFinBatch = 8;  // gathered keys per lane in flight
-template <int LE>
+template <int LE, bool PRED>
 __global__ __launch_bounds__(kBlock) void k_b_finish(CellRec *recs, int32_t nCells,
                                                      const uint32_t *__restrict__ first,
                                                      const float *__restrict__ sel,
                                                      const unsigned long long *__restrict__ sel_lists,
                                                      orb_cell *heap, uint64_t *trace,
                                                      int32_t *level_passes, uint8_t *exists,
-                                                     int32_t *status, int32_t group)
+                                                     int32_t *status, int32_t group,
+                                                     const Window *__restrict__ windows)
 {
     __shared__ float cand[4][kBins + 1];
     __shared__ uint32_t P[4][kBins + 1];
@@ -1206,7 +1279,12 @@ __global__ __launch_bounds__(kBlock) void k_b_finish(CellRec *recs, int32_t nCel
     const uint32_t m = (uint32_t)__shfl((int)lincl, 63, 64);
     const float target = difference_target(r.end - r.begin, r.nLeaf);
     uint64_t *trow = trace ? trace + ((size_t)r.hb + r.id) * ORB_MAX_PASSES : nullptr;
-    for (int round = 0;; ++round) {
+    Window wd{};
+    if constexpr (PRED) {
+        wd = windows[c];
+        window_passes(wd, r.margin_l, r.margin_r, r.passes);
+    }
+    while (true) {
         const float lo = r.margin_l, hi = r.margin_r;
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
         __builtin_amdgcn_wave_barrier();  // the wave's last replay has read the tables
@@ -1246,13 +1324,13 @@ __global__ __launch_bounds__(kBlock) void k_b_finish(CellRec *recs, int32_t nCel
                 }
             }
         }
-        below += wave_sum(bl);
+        const uint32_t left = below + wave_sum(bl);  // every round reads every listed key
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
         __builtin_amdgcn_wave_barrier();
         // P[j] = the keys below the margins + bins < j
         const uint32_t s0 = pw[4 * lane], s1 = s0 + pw[4 * lane + 1];
         const uint32_t s2 = s1 + pw[4 * lane + 2], s3 = s2 + pw[4 * lane + 3];
-        const uint32_t base = below + wave_inclusive_scan(s3) - s3;
+        const uint32_t base = left + wave_inclusive_scan(s3) - s3;
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
         __builtin_amdgcn_wave_barrier();
         pw[4 * lane + 1] = base + s0;
@@ -1263,7 +1341,11 @@ __global__ __launch_bounds__(kBlock) void k_b_finish(CellRec *recs, int32_t nCel
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
         __builtin_amdgcn_wave_barrier();
         const RoundOut ro = replay_round(pw, lo, hi, target, r.passes, lane, trow);
-        if (round == 1 || ro.found || ro.passes >= ORB_MAX_PASSES) {  // uniform
+        if (ro.found || ro.passes >= ORB_MAX_PASSES) {  // uniform
+            if (PRED && !window_holds(wd, ro.L, ro.R)) {
+                if (lane == 0) leave_alone(r, c, recs, level_passes);
+                break;
+            }
             if (lane == 0)
                 finish_round(r, c, ro, found_encoding(ro, lo, hi), recs, heap, level_passes,
                              exists, status, &pm);
@@ -1277,24 +1359,46 @@ __global__ __launch_bounds__(kBlock) void k_b_finish(CellRec *recs, int32_t nCel
     flush_block(pm, level_passes);
 }
 
+// Counts the bins of a wave's keys (those of lanes with `in`): one addition
+// where they share a bin, as keys that tie at a cut do (64 lanes adding to one
+// LDS word wait for each other).
+__device__ inline void count_bin(uint32_t *hist, int bin, bool in)
+{
+    const uint64_t m = __ballot(in);
+    if (!m) return;  // uniform
+    const int src = __builtin_ctzll(m);
+    const int b0 = (int)lane_value((uint32_t)bin, src);
+    if (__ballot(in && bin == b0) == m) {
+        if ((int)(threadIdx.x & 63) == src) atomicAdd(&hist[b0], (uint32_t)__popcll(m));
+    } else if (in) {
+        atomicAdd(&hist[bin], 1u);
+    }
+}
+
 // The same two rounds with a block per cell, for levels of few cells (whose
-// cells hold the most gathered keys): the four waves bin a quarter of the
-// keys each into one LDS histogram, wave 0 prefix-sums and replays, and the
+// cells hold the most gathered keys): the waves bin their shares of the
+// keys into one LDS histogram, wave 0 prefix-sums and replays, and the
 // round's outcome reaches the other waves through LDS.
 constexpr int kFinBlockCells = 1024;  // levels up to this many cells
-template <int LE>
-__global__ __launch_bounds__(kBlock) void k_b_finish_block(CellRec *recs, int32_t nCells,
+// (Sixteen waves, and one addition where a wave's keys share a bin: where many
+// keys tie at the cut, a cell of 2^26 keys on 512 coordinate values lists
+// 131072 of them. Four waves took 962 us a level there over two rounds, these
+// 347 over the predicted window's three or four; 17 us at 2^27 even keys.)
+constexpr int kFinBlock = 1024;
+template <int LE, bool PRED>
+__global__ __launch_bounds__(kFinBlock) void k_b_finish_block(CellRec *recs, int32_t nCells,
                                                            const uint32_t *__restrict__ first,
                                                            const float *__restrict__ sel,
                                                            const unsigned long long *__restrict__ sel_lists,
                                                            orb_cell *heap, uint64_t *trace,
                                                            int32_t *level_passes, uint8_t *exists,
-                                                           int32_t *status)
+                                                           int32_t *status,
+                                                           const Window *__restrict__ windows)
 {
-    static_assert(kBins == kBlock, "a candidate and a bin per thread");
+    constexpr int kW = kFinBlock / 64;
     __shared__ float cand[kBins + 1];
     __shared__ uint32_t hist[kBins], P[kBins + 1];
-    __shared__ uint32_t sm[4];
+    __shared__ uint32_t sm[kW];
     __shared__ float s_lr[2];
     __shared__ int32_t s_pf[2];
     const int t = threadIdx.x, lane = t & 63, w = t >> 6;
@@ -1317,51 +1421,69 @@ __global__ __launch_bounds__(kBlock) void k_b_finish_block(CellRec *recs, int32_
             mr = (uint32_t)e < span ? (uint32_t)e : span;
             bw = (uint32_t)(e >> 32);
         }
-        uint32_t below = wave_sum(bw);
+        const uint32_t below = wave_sum(bw);
         const uint32_t lincl = wave_inclusive_scan(mr), lex = lincl - mr;
         const uint32_t m = (uint32_t)__shfl((int)lincl, 63, 64);
         const float target = difference_target(r.end - r.begin, r.nLeaf);
         uint64_t *trow = trace ? trace + ((size_t)r.hb + r.id) * ORB_MAX_PASSES : nullptr;
-        for (int round = 0;; ++round) {
+        // a batch of the listed keys, all of its loads in flight; a cell of one
+        // batch keeps it in registers for every round
+        constexpr uint32_t kStep = (uint32_t)kFinBlock * kFinBatch;
+        float v[kFinBatch];
+        auto load_batch = [&](uint32_t k0) __attribute__((always_inline)) {
+#pragma unroll
+            for (int u = 0; u < kFinBatch; ++u) {
+                // key k of the cell: list j = the last with lex_j <= k
+                const uint32_t k = k0 + (uint32_t)(kFinBlock * u + t);
+                int j = 0;
+#pragma unroll
+                for (int st = 32; st > 0; st >>= 1)
+                    if ((uint32_t)__shfl((int)lex, j + st, 64) <= k) j += st;
+                const uint32_t at = (uint32_t)__shfl((int)kpos, j, 64) +
+                                    (k - (uint32_t)__shfl((int)lex, j, 64));
+                v[u] = k < m ? sel[at] : 0.0f;
+            }
+        };
+        if (m <= kStep) load_batch(0u);
+        Window wd{};
+        if constexpr (PRED) {
+            wd = windows[c];
+            window_passes(wd, r.margin_l, r.margin_r, r.passes);
+        }
+        while (true) {
             const float lo = r.margin_l, hi = r.margin_r;
             __syncthreads();  // the last round (or cell) has read the tables
-            cand[t] = t ? candidate(t, lo, hi) : -INFINITY;
-            hist[t] = 0u;
+            if (t < kBins) {
+                cand[t] = t ? candidate(t, lo, hi) : -INFINITY;
+                hist[t] = 0u;
+            }
             if (t == 0) cand[kBins] = INFINITY;
             __syncthreads();
             const float width = hi - lo;
             const float scale = width > 0.0f ? (float)kBins / width : 0.0f;
             uint32_t bl = 0;
-            for (uint32_t k0 = 0; k0 < m; k0 += (uint32_t)kBlock * kFinBatch) {
-                float v[kFinBatch];  // all of a batch's loads in flight
+            for (uint32_t k0 = 0; k0 < m; k0 += kStep) {
+                if (m > kStep) load_batch(k0);  // uniform
 #pragma unroll
                 for (int u = 0; u < kFinBatch; ++u) {
-                    // key k of the cell: list j = the last with lex_j <= k
-                    const uint32_t k = k0 + (uint32_t)(kBlock * u + t);
-                    int j = 0;
-#pragma unroll
-                    for (int st = 32; st > 0; st >>= 1)
-                        if ((uint32_t)__shfl((int)lex, j + st, 64) <= k) j += st;
-                    const uint32_t at = (uint32_t)__shfl((int)kpos, j, 64) +
-                                        (k - (uint32_t)__shfl((int)lex, j, 64));
-                    v[u] = k < m ? sel[at] : 0.0f;
-                }
-#pragma unroll
-                for (int u = 0; u < kFinBatch; ++u) {
-                    if (k0 + (uint32_t)(kBlock * u + t) >= m) continue;
-                    if (v[u] < lo) ++bl;
-                    else if (!(v[u] > hi)) {
-                        int tj;
-                        atomicAdd(&hist[bin_of<LE>(cand, v[u], lo, scale, tj)], 1u);
-                    }
+                    const bool on = k0 + (uint32_t)(kFinBlock * u + t) < m;
+                    const bool lt = on && v[u] < lo, in = on && !(v[u] < lo) && !(v[u] > hi);
+                    bl += lt ? 1u : 0u;
+                    int tj, bin = 0;
+                    if (in) bin = bin_of<LE>(cand, v[u], lo, scale, tj);
+                    count_bin(hist, bin, in);
                 }
             }
-            below += block_sum(bl, sm);  // its barriers also complete the binning
+            bl = wave_sum(bl);
+            if (lane == 0) sm[w] = bl;
+            __syncthreads();  // the binning is complete
             if (w == 0) {
+                // every round reads every listed key
+                const uint32_t left = below + wave_sum(lane < kW ? sm[lane] : 0u);
                 // P[j] = the keys below the margins + bins < j
                 const uint32_t s0 = hist[4 * lane], s1 = s0 + hist[4 * lane + 1];
                 const uint32_t s2 = s1 + hist[4 * lane + 2], s3 = s2 + hist[4 * lane + 3];
-                const uint32_t base = below + wave_inclusive_scan(s3) - s3;
+                const uint32_t base = left + wave_inclusive_scan(s3) - s3;
                 P[4 * lane + 1] = base + s0;
                 P[4 * lane + 2] = base + s1;
                 P[4 * lane + 3] = base + s2;
@@ -1384,7 +1506,11 @@ __global__ __launch_bounds__(kBlock) void k_b_finish_block(CellRec *recs, int32_
             ro.passes = s_pf[0];
             ro.found = (s_pf[1] & 1) != 0;
             ro.node = s_pf[1] >> 1;
-            if (round == 1 || ro.found || ro.passes >= ORB_MAX_PASSES) {  // uniform
+            if (ro.found || ro.passes >= ORB_MAX_PASSES) {  // uniform
+                if (PRED && !window_holds(wd, ro.L, ro.R)) {
+                    if (t == 0) leave_alone(r, c, recs, level_passes);
+                    break;
+                }
                 if (t == 0)
                     finish_round(r, c, ro, found_encoding(ro, lo, hi), recs, heap, level_passes,
                                  exists, status, &pm);
@@ -1396,6 +1522,288 @@ __global__ __launch_bounds__(kBlock) void k_b_finish_block(CellRec *recs, int32_
         }
     }
     if (t == 0) pm.flush(level_passes);
+}
+
+// ---------------------------------------------------------------------------
+// large levels: the cut's window from a sample, one pass over the keys
+// ---------------------------------------------------------------------------
+// The rounds above read every key twice: once to find the window that holds
+// the cut, once to count and pack the keys of that window.  Any window will
+// do that the cut lies in, so here a sample of the keys (about 16384 a cell or
+// more) picks it, 6 standard deviations wide each way, and the one full pass
+// counts exactly:
+//   k_p_sample  64-key lines spread over each chunk into the cell's 1024
+//               linear bins
+//   k_p_choose  per cell: the window
+//   k_p_window  as k_b_hist_window: keys below and above the window counted,
+//               its keys packed per chunk quarter and counted in linear bins
+//   (k_b_hist_reduce)
+//   k_p_narrow  per cell: the bins that can hold the cut
+// k_b_select gathers the keys of those bins and k_b_finish runs the
+// controller's rounds on them from the cell's own margins.  Exact: counts
+// grow with the candidate, so a candidate left of the kept bins has at most
+// the keys left of them, whose difference is -3 or less, and the controller
+// goes right there whatever the candidate's own count is; likewise on the
+// other side.  A cell whose counts contradict its window (the sample missed) is
+// left alone, counted, and built by the levels' second run.  Builds with a
+// trace need every pass's count and keep the two full rounds.
+// Measured at 2^27 keys, a level's search (keys read to cut found): 226 us,
+// of it the window pass 147 (5 TB/s counting the swap's lines it waits for),
+// from 296 with two full rounds.  Below kPredKeys a cell's sample would have
+// to be a good part of its keys.
+constexpr int kSampleBins = 1024;
+constexpr int kSampleLines = 64;     // lines (of 64 keys) a block
+constexpr int64_t kPredKeys = 65536;  // smallest expected cell of such a level
+constexpr int64_t kPredLevelKeys = int64_t(1) << 24;  // and keys of the build
+
+// Sample line i of `ls` of chunk q starts here (a multiple of 64; the start
+// moves with the chunk, so that no period of the input meets every line).
+__device__ inline uint32_t sample_line(uint32_t q, uint32_t i, uint32_t ls)
+{
+    const uint32_t span = (uint32_t)kChunk / ls;  // a power of two, at least 64
+    return i * span + ((q * 0x9e3779b1u) >> 20 & (span - 1u) & ~63u);
+}
+
+__global__ __launch_bounds__(kBlock) void k_p_sample(
+    const CellRec *__restrict__ recs, int32_t nCells, const uint32_t *__restrict__ first,
+    const uint4 *__restrict__ chunk_desc, uint32_t max_chunks, const float *__restrict__ x,
+    const float *__restrict__ y, const float *__restrict__ z, uint32_t ls, uint32_t *sample_hist)
+{
+    constexpr int kW = kBlock / 64;
+    constexpr int kPer = kSampleLines / kW;  // 16 lines a wave, all in flight
+    __shared__ uint32_t hist[kSampleBins];
+    const int t = threadIdx.x, lane = t & 63, w = (int)uniform((uint32_t)t >> 6);
+    const uint32_t total = first[nCells];
+    const uint32_t per_block = (uint32_t)kSampleLines / ls;  // chunks a block
+    for (uint32_t q0 = blockIdx.x * per_block; q0 < total; q0 += gridDim.x * per_block) {
+        const uint32_t cell0 = uniform(chunk_record(chunk_desc, q0, max_chunks).z);
+        for (int k = t; k < kSampleBins; k += kBlock) hist[k] = 0u;
+        float v[kPer];
+        uint32_t cell[kPer];
+        bool ok[kPer];
+#pragma unroll
+        for (int j = 0; j < kPer; ++j) {
+            const uint32_t line = (uint32_t)(w * kPer + j);
+            const uint32_t q = q0 + line / ls;
+            const uint4 d = chunk_record(chunk_desc, q, max_chunks);
+            const uint32_t b = uniform(d.x), e = uniform(d.y), axis = uniform(d.w);
+            const uint32_t p = b + sample_line(q, line % ls, ls) + (uint32_t)lane;
+            cell[j] = uniform(d.z);
+            ok[j] = q < total && axis <= 2u && p < e;
+            v[j] = ok[j] ? axis_ptr(x, y, z, (int)axis)[p] : 0.0f;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < kPer; ++j) {
+            if (!__ballot(ok[j])) continue;  // uniform
+            const float lo = uniform(recs[cell[j]].margin_l), hi = uniform(recs[cell[j]].margin_r);
+            const float width = hi - lo, scale = width > 0.0f ? (float)kSampleBins / width : 0.0f;
+            const int bin = (int)__builtin_amdgcn_fmed3f((v[j] - lo) * scale, 0.0f, (float)(kSampleBins - 1));
+            if (ok[j]) {
+                if (cell[j] == cell0) atomicAdd(&hist[bin], 1u);
+                else atomicAdd(&sample_hist[(size_t)cell[j] * kSampleBins + bin], 1u);  // the block's last chunks
+            }
+        }
+        __syncthreads();
+        for (int k = t; k < kSampleBins; k += kBlock)
+            if (hist[k]) atomicAdd(&sample_hist[(size_t)cell0 * kSampleBins + k], hist[k]);
+        __syncthreads();
+    }
+}
+
+// A wave per cell: the window from the sample, and the row cleared.
+__global__ __launch_bounds__(kBlock) void k_p_choose(const CellRec *__restrict__ recs, int32_t nCells,
+                                                     uint32_t *sample_hist, Window *__restrict__ windows)
+{
+    constexpr int kPer = kSampleBins / 64;  // 16 bins a lane
+    const int lane = threadIdx.x & 63;
+    const int32_t c = (int32_t)((blockIdx.x * kBlock + threadIdx.x) >> 6);
+    if (c >= nCells || recs[c].flags) return;  // uniform
+    uint4 *row = reinterpret_cast<uint4 *>(sample_hist + (size_t)c * kSampleBins) + lane * (kPer / 4);
+    uint32_t h[kPer];
+#pragma unroll
+    for (int u = 0; u < kPer / 4; ++u) {
+        const uint4 a = row[u];
+        h[4 * u] = a.x;
+        h[4 * u + 1] = a.y;
+        h[4 * u + 2] = a.z;
+        h[4 * u + 3] = a.w;
+    }
+#pragma unroll
+    for (int u = 0; u < kPer / 4; ++u) row[u] = make_uint4(0u, 0u, 0u, 0u);
+    uint32_t mine = 0;
+#pragma unroll
+    for (int u = 0; u < kPer; ++u) mine += h[u];
+    const uint32_t inc = wave_inclusive_scan(mine);
+    const float s = (float)lane_value(inc, 63);
+    const int32_t nl = recs[c].nLeaf;
+    const float ratio = (float)((nl + 1) / 2) / (float)nl;
+    const float mid = s * ratio, dev = 6.0f * sqrtf(s * ratio * (1.0f - ratio)) + 8.0f;
+    uint32_t below = 0, reach = 0, cum = inc - mine;  // whole bins under each bound
+#pragma unroll
+    for (int u = 0; u < kPer; ++u) {
+        cum += h[u];
+        below += (float)cum < mid - dev ? 1u : 0u;
+        reach += (float)cum < mid + dev ? 1u : 0u;
+    }
+    const uint32_t bl = wave_sum(below), bu = wave_sum(reach) + 1u;
+    if (lane == 0) {
+        const float lo = recs[c].margin_l, hi = recs[c].margin_r, step = (hi - lo) / (float)kSampleBins;
+        const float wl = bl == 0u ? lo : fminf(fmaxf(lo + (float)bl * step, lo), hi);
+        const float wr = bu >= (uint32_t)kSampleBins ? hi : fminf(fmaxf(lo + (float)bu * step, wl), hi);
+        const float width = wr - wl;
+        // (no bins in a window too narrow for a finite scale: one holds its keys)
+        windows[c] = Window{wl, wr, width > 0x1p-100f ? (float)kWindowBins / width : 0.0f, 1u,
+                            (uint32_t)kWindowBins, {0u, 0u, 0u}};
+    }
+}
+
+// Window pass (see k_b_hist_window for its packing and masks).
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_p_window(
+    const Window *__restrict__ windows, int32_t nCells, const uint32_t *__restrict__ first,
+    const uint4 *__restrict__ chunk_desc, uint32_t max_chunks, const float *__restrict__ x,
+    const float *__restrict__ y, const float *__restrict__ z, uint16_t *__restrict__ chunk_hist,
+    float *__restrict__ pack, uint32_t *__restrict__ comp, uint64_t *__restrict__ masks, int rev)
+{
+    constexpr int kW = kBlock / 64;
+    constexpr int kPerWave = kMaskWords / kW;  // 16 loads of 64 keys
+    __shared__ uint32_t hist[kBins];
+    __shared__ uint32_t sm[4];
+    __shared__ float wkeys[kW][kChunk / kW];     // each wave's window keys, packed
+    __shared__ uint64_t words[kW][2][kPerWave];  // each wave's mask words, staged
+    const int t = threadIdx.x, lane = t & 63, w = (int)uniform((uint32_t)t >> 6);
+    const uint64_t lanes_below = lane == 0 ? 0ull : (~0ull >> (64 - lane));
+    const uint32_t total = first[nCells];
+    for (uint32_t q0 = blockIdx.x;; q0 += gridDim.x) {
+        const uint32_t q = rev && q0 < total ? total - 1u - q0 : q0;  // from the last (rev)
+        const uint4 d = chunk_record(chunk_desc, q, max_chunks);
+        const uint32_t b = uniform(d.x), e = uniform(d.y), cell = uniform(d.z);
+        const uint32_t axis = uniform(d.w);
+        keep_values(b, e, cell, axis);  // the whole record, in flight with total
+        if (q >= total) break;
+        if (axis > 2u) continue;  // uniform: the cell is not searched
+        const uint32_t sb = (uint32_t)(w * kPerWave * 64);  // chunk position of the quarter
+        float v[kPerWave];
+        issue_chunk_loads(x, y, z, true, d, sb, lane, v);
+        const float lo = uniform(windows[cell].lo), hi = uniform(windows[cell].hi);
+        const float scale = uniform(windows[cell].scale);
+        hist[t] = 0u;
+        __syncthreads();
+        const uint32_t len = e - b;
+        uint32_t below = 0, packed = 0;  // wave-uniform
+        float *dst = pack + b + sb;
+        float *wk = wkeys[w];
+        auto scan = [&](auto full) __attribute__((always_inline)) {
+            static_for<0, kPerWave>([&](auto jc) __attribute__((always_inline)) {
+                constexpr int j = decltype(jc)::value;
+                uint64_t valid = ~0ull;
+                if constexpr (!decltype(full)::value) {
+                    const uint32_t p0 = sb + 64u * (uint32_t)j;  // chunk position of lane 0
+                    valid = p0 >= len ? 0ull
+                                      : (len - p0 >= 64u ? ~0ull : (1ull << (len - p0)) - 1ull);
+                }
+                const float vj = v[j];
+                const uint64_t mB = __ballot(vj < lo) & valid;
+                const uint64_t mG = __ballot(vj > hi) & valid;
+                const uint64_t mW = valid & ~mB & ~mG;
+                below += (uint32_t)__popcll(mB);
+                if (lane == 0) {  // staged by one lane, as in k_b_hist_window
+                    words[w][0][j] = mG;
+                    words[w][1][j] = mW;
+                }
+                if (mW) {  // wave-uniform
+                    if ((mW >> lane) & 1ull) {
+                        const uint32_t slot = packed + (uint32_t)__popcll(mW & lanes_below);
+                        dst[slot] = vj;
+                        wk[slot] = vj;
+                    }
+                    packed += (uint32_t)__popcll(mW);
+                }
+            });
+        };
+        if (len == (uint32_t)kChunk) scan(std::true_type{});  // uniform
+        else scan(std::false_type{});
+        const uint32_t mine = len > sb ? (len - sb < 1024u ? len - sb : 1024u) : 0u;
+        const uint32_t above = mine - below - packed;
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
+        __builtin_amdgcn_wave_barrier();
+        const uint64_t mineG = lane < kPerWave ? words[w][0][lane] : 0ull;
+        const uint64_t mineW = lane < kPerWave ? words[w][1][lane] : 0ull;
+        for (uint32_t k = (uint32_t)lane; k < packed; k += 64)
+            atomicAdd(&hist[window_bin(wk[k], lo, scale)], 1u);
+        uint64_t *mq = masks + (size_t)q * (2 * kMaskWords) + w * kPerWave;
+        if (lane < kPerWave) {
+            mq[lane] = mineG;
+            mq[kMaskWords + lane] = mineW;
+        }
+        if (lane == 0) {
+            comp[8 * (size_t)q + w] = packed;
+            sm[w] = below | (above << 16);  // each <= 1024
+        }
+        __syncthreads();
+        const uint32_t ba = sm[0] + sm[1] + sm[2] + sm[3];
+        if (t == 0) comp[8 * (size_t)q + 4] = ba & 0xffffu;
+        uint32_t sum = hist[t];
+        if (t == 0) sum += ba & 0xffffu;
+        if (t == kBins - 1) sum += ba >> 16;
+        chunk_hist[(size_t)q * kBins + t] = (uint16_t)sum;
+        __syncthreads();  // the next chunk rewrites hist and sm
+    }
+}
+
+// A wave per cell: from the counts of the window's bins (bin 0: keys below the
+// window, 255: above), the bins [b1, b2] that can hold the cut, and the cell's
+// lists with the keys left of them.  A cell whose counts contradict the window
+// is left alone (see above).
+__global__ __launch_bounds__(kBlock) void k_p_narrow(CellRec *recs, int32_t nCells, uint32_t *cell_hist,
+                                                     Window *__restrict__ windows,
+                                                     const uint32_t *__restrict__ first,
+                                                     unsigned long long *__restrict__ sel_lists,
+                                                     int32_t *level_passes)
+{
+    const int lane = threadIdx.x & 63;
+    const int32_t c = (int32_t)((blockIdx.x * kBlock + threadIdx.x) >> 6);
+    if (c >= nCells || recs[c].flags) return;  // uniform
+    uint4 *row = reinterpret_cast<uint4 *>(cell_hist + (size_t)c * kBins);
+    const uint4 h4 = row[lane];
+    row[lane] = make_uint4(0u, 0u, 0u, 0u);  // the next level adds to zero
+    const uint32_t s0 = h4.x, s1 = s0 + h4.y, s2 = s1 + h4.z, s3 = s2 + h4.w;
+    const uint32_t base = wave_inclusive_scan(s3) - s3;
+    // P[4 lane + 1 + q] (P[j] = keys in bins below j)
+    const uint32_t pv[4] = {base + s0, base + s1, base + s2, base + s3};
+    const float target = difference_target(uniform(recs[c].end) - uniform(recs[c].begin),
+                                           (int32_t)uniform((uint32_t)recs[c].nLeaf));
+    uint32_t left = 0, right = 0;  // j in [1, 255] with difference <= -3, resp. < 3
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const bool in = 4 * lane + 1 + q < kBins;
+        const int32_t df = difference_from_target(pv[q], target);
+        left += (uint32_t)__popcll(__ballot(in && df <= -3));
+        right += (uint32_t)__popcll(__ballot(in && df < 3));
+    }
+    // the last j with difference <= -3 is `left` (differences grow with j),
+    // the first with difference >= 3 is right + 1
+    const Window wd = windows[c];
+    const bool low_ok = left >= 1u || wd.lo == recs[c].margin_l;    // P[1]: the keys below the window
+    const bool high_ok = right < 255u || wd.hi == recs[c].margin_r;  // P[255]: all but those above
+    const uint32_t b1 = left >= 1u ? left : 1u, b2 = right < 255u ? right : 254u;
+    const uint32_t cnt = lane_value(b1 & 3u ? ((b1 & 3u) == 1u ? pv[0] : (b1 & 3u) == 2u ? pv[1] : pv[2]) : pv[3],
+                                    (int)((b1 - 1u) >> 2));  // P[b1]
+    if (!low_ok || !high_ok || b1 > 254u || b2 < 1u) {
+        if (lane == 0) {
+            recs[c].flags = 1;
+            atomicAdd(&level_passes[recs[c].lp & ~63], 1);
+        }
+        return;
+    }
+    const uint32_t f = first[c];
+    const SelLists sl(f, first[c + 1] - f);
+    if ((uint32_t)lane < sl.R)
+        sel_lists[sl.start_chunk((uint32_t)lane)] = lane == 0 ? (unsigned long long)cnt << 32 : 0ull;
+    if (lane == 0) {
+        windows[c].b1 = b1;
+        windows[c].b2 = b2;
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -3032,11 +3440,10 @@ __global__ __launch_bounds__(kTailBlock) void k_m_tail(
                     for (int u = 0; u < 4; ++u) {
                         const bool lt = in[u] && v[u] < lo, on = in[u] && !(v[u] < lo) && !(v[u] > hi);
                         below += (uint32_t)__popcll(__ballot(lt));
-                        if (!on) continue;
-                        int bin;
-                        if (!bin_estimate(v[u], lo, scale, lim, bin))
+                        int bin = 0;
+                        if (on && !bin_estimate(v[u], lo, scale, lim, bin))
                             bin = le_cmp ? bin_walk<1>(v[u], lo, hi) : bin_walk<0>(v[u], lo, hi);
-                        atomicAdd(&hist[bin], 1u);
+                        count_bin(hist, bin, on);
                     }
                 }
                 if (lane == 0 && below) atomicAdd(&hist[0], below);
@@ -3272,6 +3679,13 @@ static int ensure_state(Ctx &c, int32_t levels_mode, bool *complete)
         ORB_TRY(c.round_state.alloc(4 * 2 * (size_t)kRecsScan));
     }
     if (!c.weighted) ORB_TRY(c.sel.alloc((size_t)c.stride));  // rounds 3 and 4
+    if (!c.weighted && c.n >= kPredLevelKeys) {
+        // cells of at least kPredKeys keys (less what a level's sizes vary by)
+        const size_t cells = (size_t)(c.n / (kPredKeys / 2)) + 2;
+        if (c.sample_hist.n < cells * kSampleBins) b.sample_clean = false;
+        ORB_TRY(c.sample_hist.alloc(cells * kSampleBins));
+        ORB_TRY(c.windows.alloc(cells * (sizeof(Window) / 4)));
+    }
     // every buffer the launches touch exists before a capture starts
     ORB_TRY(preallocate_scratch(c));
     return ORB_OK;
@@ -3324,7 +3738,7 @@ static std::vector<uint64_t> graph_signature(const Ctx &c, const BatchedState &b
                           c.packed.p, c.masks.p, c.cell_cand.p, c.splits.p, c.chunk_comp.p,
                           c.sel.p, c.sel_lists.p, c.swap_plan.p, c.status.p, c.stamps.p, b.level_ids.p, b.heap.p, b.exists.p,
                           b.sub.p, b.chunk_hist.p, b.cell_hist.p, b.trace.p, b.level_passes.p,
-                          c.wt.p, c.wt_tmp.p, b.chunk_hist_w.p, b.cell_hist_w.p, c.round_state.p, c.hstatus.p, b.hpasses.p};
+                          c.wt.p, c.wt_tmp.p, b.chunk_hist_w.p, b.cell_hist_w.p, c.round_state.p, c.sample_hist.p, c.windows.p, c.hstatus.p, b.hpasses.p};
     for (const void *p : bufs) s.push_back((uint64_t)(uintptr_t)p);
     s.push_back((uint64_t)c.tune_chunk_blocks.size());
     for (int32_t v : c.tune_chunk_blocks) s.push_back((uint64_t)(int64_t)v);
@@ -3398,7 +3812,7 @@ int enqueue_level(Ctx &c, const LevelEntry *entries, int32_t nCells, orb_cell *h
         const int tb = timing_mark(c);
         const unsigned fill_blocks =
             (unsigned)std::min<int64_t>(16384, std::max<int64_t>(1, (c.max_chunks + kBlock - 1) / kBlock));
-        const unsigned cand_blocks = c.weighted ? 0u : cell_group_blocks(nCells, cgroup);
+        const unsigned cand_blocks = c.weighted || kernels.predict ? 0u : cell_group_blocks(nCells, cgroup);
         hipLaunchKernelGGL(k_b_tables, dim3(fill_blocks + cand_blocks), dim3(kBlock), 0, c.stream,
                            c.cell_first.p, nCells, c.recs.p, c.chunk_cell.p, c.chunk_desc.p,
                            (uint32_t)c.max_chunks, c.cell_cand.p, cgroup, fill_blocks);
@@ -3516,7 +3930,29 @@ int enqueue_level(Ctx &c, const LevelEntry *entries, int32_t nCells, orb_cell *h
         ORB_TRY(timing_pair(c, tp, kTimePartition));
         return ORB_OK;
     }
-    for (int r = 0; r < 2; ++r) {
+    if (kernels.predict) {
+        const int tb = timing_mark(c);
+        Window *windows = reinterpret_cast<Window *>(c.windows.p);
+        const uint32_t mc = (uint32_t)c.max_chunks;
+        const uint32_t ls = kernels.predict, per_block = (uint32_t)kSampleLines / ls;
+        hipLaunchKernelGGL(k_p_sample, dim3((gq + per_block - 1) / per_block), dim3(kBlock), 0, c.stream,
+                           c.recs.p, nCells, c.cell_first.p, c.chunk_desc.p, mc, c.x(), c.y(), c.z(), ls,
+                           c.sample_hist.p);
+        hipLaunchKernelGGL(k_p_choose, dim3(gw), dim3(kBlock), 0, c.stream, c.recs.p, nCells,
+                           c.sample_hist.p, windows);
+        hipLaunchKernelGGL(k_p_window, dim3(gq), dim3(kBlock), 0, c.stream, windows, nCells,
+                           c.cell_first.p, c.chunk_desc.p, mc, c.x(), c.y(), c.z(), later_hist, c.packed.p,
+                           c.chunk_comp.p, c.masks.p, rev);
+        ORB_HIP(hipGetLastError());
+        ORB_TRY(timing_pair(c, tb, kTimeCount));
+        hipLaunchKernelGGL(k_b_hist_reduce, dim3(gr), dim3(kBlock), 0, c.stream, c.recs.p, nCells,
+                           c.cell_first.p, c.chunk_cell.p, later_hist, cell_hist);
+        hipLaunchKernelGGL(k_p_narrow, dim3(gw), dim3(kBlock), 0, c.stream, c.recs.p, nCells, cell_hist,
+                           windows, c.cell_first.p,
+                           reinterpret_cast<unsigned long long *>(c.sel_lists.p), level_passes);
+        ORB_HIP(hipGetLastError());
+    }
+    for (int r = 0; r < 2 && !kernels.predict; ++r) {
         const int tb = timing_mark(c);
         // rounds 1 and 2 over every key of the searching cells; the second
         // also packs the keys inside its margins, per chunk quarter
@@ -3555,20 +3991,24 @@ int enqueue_level(Ctx &c, const LevelEntry *entries, int32_t nCells, orb_cell *h
         const int tb = timing_mark(c);
         const unsigned gs = (gq + 4 * kSelChunks - 1) / (4 * kSelChunks);
         unsigned long long *lists = reinterpret_cast<unsigned long long *>(c.sel_lists.p);
-        hipLaunchKernelGGL(k_b_select, dim3(gs), dim3(kBlock), 0, c.stream, c.recs.p, nCells,
-                           c.cell_first.p, c.chunk_desc.p, (uint32_t)c.max_chunks, c.packed.p,
-                           c.chunk_comp.p, c.sel.p, lists);
+        const bool pred = kernels.predict != 0;
+        const Window *windows = reinterpret_cast<const Window *>(c.windows.p);
+        hipLaunchKernelGGL(pred ? k_b_select<true> : k_b_select<false>, dim3(gs), dim3(kBlock), 0, c.stream,
+                           c.recs.p, nCells, c.cell_first.p, c.chunk_desc.p, (uint32_t)c.max_chunks,
+                           c.packed.p, c.chunk_comp.p, c.sel.p, lists, windows);
         ORB_HIP(hipGetLastError());
         if (nCells <= kFinBlockCells) {  // a block per cell
-            auto finish = le ? k_b_finish_block<1> : k_b_finish_block<0>;
-            hipLaunchKernelGGL(finish, dim3((unsigned)std::max<int32_t>(nCells, 1)), dim3(kBlock), 0,
+            auto finish = pred ? (le ? k_b_finish_block<1, true> : k_b_finish_block<0, true>)
+                               : (le ? k_b_finish_block<1, false> : k_b_finish_block<0, false>);
+            hipLaunchKernelGGL(finish, dim3((unsigned)std::max<int32_t>(nCells, 1)), dim3(kFinBlock), 0,
                                c.stream, c.recs.p, nCells, c.cell_first.p, c.sel.p, lists, heap,
-                               trace, level_passes, exists, status);
+                               trace, level_passes, exists, status, windows);
         } else {
-            auto finish = le ? k_b_finish<1> : k_b_finish<0>;
+            auto finish = pred ? (le ? k_b_finish<1, true> : k_b_finish<0, true>)
+                               : (le ? k_b_finish<1, false> : k_b_finish<0, false>);
             hipLaunchKernelGGL(finish, dim3(cell_group_blocks(nCells, cgroup)), dim3(kBlock), 0,
                                c.stream, c.recs.p, nCells, c.cell_first.p, c.sel.p, lists, heap,
-                               trace, level_passes, exists, status, cgroup);
+                               trace, level_passes, exists, status, cgroup, windows);
         }
         ORB_HIP(hipGetLastError());
         ORB_TRY(timing_pair(c, tb, kTimeCount));
@@ -3580,6 +4020,7 @@ int enqueue_level(Ctx &c, const LevelEntry *entries, int32_t nCells, orb_cell *h
     hc.le = le;
     hc.pack = c.packed.p;
     hc.comp = c.chunk_comp.p;
+    hc.windows_all = kernels.predict ? 1 : 0;
     if (c.part == ORB_PART_HOARE) ORB_TRY(launch_hoare(c, nCells, status, &hc, 0, defer_final));
     else ORB_TRY(launch_stable_le(c, nCells, status, full_cover, &hc));
     ORB_TRY(timing_pair(c, tp, kTimePartition));
@@ -3682,6 +4123,13 @@ static int enqueue_build(Ctx &c, int32_t levels_mode, bool again)
             if (!c.weighted) c.level_chunk_hint[(size_t)l] = c.n / kChunk + shape.cells + 1;
             kernels[(size_t)l] = level_kernels(c, shape);
             if (!c.weighted) no_sub[(size_t)l] = shape.fewest > shape.sub_max;
+            if (!c.weighted && !c.trace && c.part == ORB_PART_HOARE && c.n >= kPredLevelKeys &&
+                kernels[(size_t)l].chunks == kChunksAll && shape.fewest >= kPredKeys) {
+                // sample lines a chunk: at least 256 lines (16384 keys) a cell
+                int32_t ls = 1;
+                while (ls < 16 && ls * (shape.fewest / kChunk) < 256) ls *= 2;
+                kernels[(size_t)l].predict = ls;
+            }
             if (ends) {
                 last = l;
                 break;
@@ -3733,6 +4181,10 @@ int build_batched(Ctx &c, int32_t levels_mode, orb_build_info *info)
     if (!b.hist_clean) {
         ORB_TRY(launch_zero_u32(c.stream, b.cell_hist.p, (size_t)c.max_level_cells * kBins));
         b.hist_clean = true;
+    }
+    if (c.sample_hist.p && !b.sample_clean) {
+        ORB_TRY(launch_zero_u32(c.stream, c.sample_hist.p, c.sample_hist.n));
+        b.sample_clean = true;
     }
     if (c.weighted && !b.hist_w_clean) {
         ORB_TRY(launch_zero_u64(c.stream, b.cell_hist_w.p, hist_w_rows(c) * kBins));
@@ -3787,6 +4239,7 @@ int build_batched(Ctx &c, int32_t levels_mode, orb_build_info *info)
     if (status_error(c.hstatus.p, &info->error_cell)) {
         b.hist_clean = false;  // an aborted subtree may leave rows behind
         b.hist_w_clean = false;
+        b.sample_clean = false;
         return ORB_ERR_UB;
     }
     return ORB_OK;

@@ -516,6 +516,8 @@ struct Ctx {
     DevBuf<uint64_t> sel_lists;      // [max_chunks+1] batched form: count of keys gathered into
                                      // a list of sel | keys below << 32, at the list's first chunk
     DevBuf<SplitRec> splits;         // [cells]
+    DevBuf<uint32_t> sample_hist;    // [cells][1024] large levels: the sample's bins, zero between levels
+    DevBuf<uint32_t> windows;        // [cells][8] large levels: the predicted windows
     DevBuf<uint32_t> round_state;    // [2][cells][4] weighted levels of few chunks: the rounds' margins
     DevBuf<uint4> swap_plan;         // [max_chunks][2] Hoare swap unit of each chunk
     DevBuf<int32_t> status;          // [2]: error flag, failing heap id
@@ -624,6 +626,7 @@ struct HistCounts {
     int le = 0;                       // bins were built with <= (else <)
     const float *pack = nullptr;      // keys packed by the second round, per chunk share
     const uint32_t *comp = nullptr;   // [chunks][8] packed counts per share, keys below
+    int windows_all = 0;              // every cell went through a window pass
 };
 int launch_hoare(Ctx &c, int32_t nCells, int32_t *status = nullptr,
                  const HistCounts *hc = nullptr, int rev = 0, bool defer_final = false);
@@ -664,6 +667,7 @@ struct LevelKernels {
     uint32_t cell_max = 0;
     uint32_t sub_max = 0;  // the subtree kernel's limit (0: its capacity)
     bool again = false;
+    int32_t predict = 0;   // chunk path: sample lines a chunk of a predicted window (0: two full rounds)
 };
 // What the host expects of a level's cells: their number, the particles of
 // their builds, and the fewest and most keys of those above the subtree kernel.

@@ -879,7 +879,7 @@ constexpr int kMasksChunks = 2;  // k_hoare_masks_window: chunks per wave
 __global__ __launch_bounds__(kBlock) void k_hoare_masks_window(
     const CellRec *__restrict__ recs, int32_t nCells, const uint32_t *__restrict__ first,
     const uint4 *__restrict__ chunk_desc, uint32_t max_chunks, const float *x, const float *y,
-    const float *z, const float *pack, uint64_t *masks, uint64_t *chunk_cnt)
+    const float *z, const float *pack, uint64_t *masks, uint64_t *chunk_cnt, int windows_all)
 {
     constexpr int kW = kBlock / 64;
     constexpr int kQuarter = kMaskWords / kW;  // words per packing quarter
@@ -929,7 +929,7 @@ __global__ __launch_bounds__(kBlock) void k_hoare_masks_window(
             v0[i] = W ? pk[rank[i]] : 0.0f;
             const CellRec &r = recs[cell];
             cut[i] = r.cut;
-            win[i] = r.passes > kHistK;
+            win[i] = windows_all || r.passes > kHistK;
         }
 #pragma unroll
         for (int i = 0; i < kPer; ++i) {
@@ -1336,7 +1336,7 @@ int launch_hoare_final(Ctx &c, int32_t nCells)
 __global__ __launch_bounds__(kBlock) void k_b_stopper_counts(
     const CellRec *recs, int32_t nCells, const uint32_t *first, const uint32_t *chunk_cell,
     const float *x, const float *y, const float *z, int le_only, const uint16_t *hist,
-    const uint16_t *tie, int hist_le, const float *pack, const uint32_t *comp,
+    const uint16_t *tie, int hist_le, const float *pack, const uint32_t *comp, int windows_all,
     uint64_t *chunk_cnt)
 {
     constexpr int kW = kBlock / 64;
@@ -1349,7 +1349,7 @@ __global__ __launch_bounds__(kBlock) void k_b_stopper_counts(
         uint32_t e = b + (uint32_t)kChunk;
         if (e > r.end) e = r.end;
         uint32_t lt = 0, le = 0;
-        if (r.passes > kHistK) {
+        if (windows_all || r.passes > kHistK) {
             // the cell went through the packing round: its keys outside the
             // packing window lie below or above every later cut, so the
             // packed keys and the count below decide
@@ -1414,7 +1414,7 @@ int launch_stopper_counts(Ctx &c, int32_t nCells, bool le_only, const HistCounts
         hipLaunchKernelGGL(k_b_stopper_counts, dim3((chunk_grid(c) + 3) / 4), dim3(kBlock), 0, c.stream,
                            c.recs.p, nCells, c.cell_first.p, c.chunk_cell.p, c.x(), c.y(), c.z(),
                            le_only ? 1 : 0, hc->hist, hc->tie, hc->le, hc->pack, hc->comp,
-                           c.chunk_cnt.p);
+                           hc->windows_all, c.chunk_cnt.p);
     else
         hipLaunchKernelGGL(k_stopper_counts, dim3(chunk_grid(c)), dim3(kBlock), 0,
                            c.stream, c.recs.p, nCells, c.cell_first.p, c.chunk_cell.p, c.x(), c.y(),
@@ -1471,7 +1471,7 @@ int launch_hoare(Ctx &c, int32_t nCells, int32_t *status, const HistCounts *hc, 
                            dim3(kBlock), 0, c.stream,
                            c.recs.p, nCells, c.cell_first.p, c.chunk_desc.p,
                            (uint32_t)c.max_chunks, c.x(), c.y(), c.z(), hc->pack, c.masks.p,
-                           c.chunk_cnt.p);
+                           c.chunk_cnt.p, hc->windows_all);
     else
         hipLaunchKernelGGL(k_hoare_masks, dim3(gq), dim3(kBlock), 0, c.stream, c.recs.p, nCells,
                            c.cell_first.p, c.chunk_cell.p, c.x(), c.y(), c.z(), c.masks.p,

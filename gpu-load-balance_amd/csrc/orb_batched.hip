@@ -19,7 +19,11 @@
 //    (the same 8-pass histogram rounds and replay, exact Hoare by ballot
 //    scans) and writes x, y, z back once;
 //  * the partition of the remaining (large) cells uses the same exact Hoare
-//    kernels as the plain form.
+//    kernels as the plain form;
+//  * which kernels a level launches follows from the cell sizes the host
+//    expects (level_kernels): one block a cell with the keys in registers
+//    (k_b_cell), few chunks (k_m_*, k_mw_*), a cut predicted from a sample
+//    (k_p_*), the chunk kernels of every size otherwise.
 #include "orb_device.hpp"
 
 namespace orb {
@@ -3343,9 +3347,14 @@ __global__ __launch_bounds__(kBlock) void k_mw_masks(
 // as in k_b_cell (the crossing chunk, its word, its bit), the children's
 // ranges, and each chunk's swap unit as k_hoare_plan makes it.  WEIGHTED: the
 // search and the masks are done (state, k_mw_masks); the chunks' counts come
-// from the masks.
+// from the masks.  STABLE: the chunks' offsets of the keys going left (<= cut:
+// the R-stoppers) and right, for k_stable_scatter, in place of K, i and the plan.
+// A cell of a stable level is never left alone (where the level's scatter fills
+// the other buffer, all of its cells have to), so its chunks go through the
+// tables kMidChunks at a time.  o=2 builds, host time: 2^16 to 64 leaves 403 ->
+// 234 us, 2^20 to 1024 804 -> 500 us, 500003 with ids and weights 741 -> 422 us.
 constexpr int kTailBlock = 1024;
-template <bool WEIGHTED>
+template <bool WEIGHTED, bool STABLE>
 __global__ __launch_bounds__(kTailBlock) void k_m_tail(
     CellRec *recs, int32_t nCells, const uint32_t *__restrict__ first, uint32_t *cell_hist,
     const float *__restrict__ sel, const unsigned long long *__restrict__ sel_lists,
@@ -3371,7 +3380,7 @@ __global__ __launch_bounds__(kTailBlock) void k_m_tail(
         const uint32_t begin = uniform(rec.begin), n = uniform(rec.end) - begin;
         const int32_t id = (int32_t)uniform((uint32_t)rec.id), hb = (int32_t)uniform((uint32_t)rec.hb);
         const uint32_t f = uniform(first[c]), nch = uniform(first[c + 1]) - f;
-        if (nch > (uint32_t)kMidChunks) {
+        if (!STABLE && nch > (uint32_t)kMidChunks) {
             // the level records hand over at most kMidChunks; refuse anything else
             if (t == 0) {
                 report_error(status + rec.st, rec.lp & 63, kErrSplit, id);
@@ -3398,15 +3407,6 @@ __global__ __launch_bounds__(kTailBlock) void k_m_tail(
             }
             for (int q = t; q < kRounds * kBins; q += kTailBlock)  // the next level adds to zero
                 rows[((size_t)(q / kBins) * (size_t)nCells + c) * kBins + q % kBins] = 0ull;
-            for (uint32_t k = (uint32_t)w; k < nch; k += kW) {
-                const uint64_t *mq = masks + (size_t)(f + k) * (2 * kMaskWords);
-                const uint32_t nl = wave_sum((uint32_t)__popcll(mq[lane]));
-                const uint32_t nr = wave_sum((uint32_t)__popcll(mq[kMaskWords + lane]));
-                if (lane == 0) {
-                    preL[k] = nl;
-                    preR[k] = nr;
-                }
-            }
         } else {
             uint64_t *trow = trace ? trace + ((size_t)hb + id) * ORB_MAX_PASSES : nullptr;
             uint32_t *row = cell_hist + (size_t)c * kBins;
@@ -3469,79 +3469,123 @@ __global__ __launch_bounds__(kTailBlock) void k_m_tail(
                 passes = (int32_t)uniform((uint32_t)s_pf[0]);
                 found = uniform((uint32_t)s_pf[1]) != 0u;
             }
-            const float cut = cell_cut(lo, hi);
-            // ---- stopper masks: a wave per kPer chunks, a word per lane
-            constexpr int kPer = 4;
-            for (uint32_t k0 = (uint32_t)(w * kPer); k0 < nch; k0 += (uint32_t)(kW * kPer)) {
-                uint64_t G[kPer], W[kPer];
-                float v0[kPer];
-                const float *pk[kPer];
-#pragma unroll
-                for (int u = 0; u < kPer; ++u) {
-                    const uint32_t k = k0 + (uint32_t)u < nch ? k0 + (uint32_t)u : nch - 1u;
-                    const uint64_t *mq = masks + (size_t)(f + k) * (2 * kMaskWords);
-                    G[u] = mq[lane];
-                    W[u] = mq[kMaskWords + lane];
-                }
-#pragma unroll
-                for (int u = 0; u < kPer; ++u) {
-                    const uint32_t k = k0 + (uint32_t)u < nch ? k0 + (uint32_t)u : nch - 1u;
-                    const uint32_t cw = (uint32_t)__popcll(W[u]);
-                    const uint32_t ex = wave_inclusive_scan(cw) - cw;
-                    const int q0 = lane & ~15;  // first word of this lane's quarter
-                    const uint32_t rank = ex - (uint32_t)__shfl((int)ex, q0, 64);
-                    pk[u] = pack + begin + k * (uint32_t)kChunk + 64u * (uint32_t)q0 + rank;
-                    v0[u] = W[u] ? *pk[u] : 0.0f;
-                }
-#pragma unroll
-                for (int u = 0; u < kPer; ++u) {
-                    const uint32_t k = k0 + (uint32_t)u;
-                    if (k >= nch) break;  // uniform
-                    const uint32_t p0 = k * (uint32_t)kChunk + 64u * (uint32_t)lane;
-                    const uint64_t valid =
-                        p0 >= n ? 0ull : (n - p0 >= 64u ? ~0ull : (1ull << (n - p0)) - 1ull);
-                    uint64_t L = G[u], R = valid & ~G[u] & ~W[u], wd = W[u];
-                    float vk = v0[u];
-                    const float *at = pk[u];
-                    while (wd) {
-                        const uint32_t bit = (uint32_t)__builtin_ctzll(wd);
-                        wd &= wd - 1ull;
-                        L |= (!(vk < cut) ? 1ull : 0ull) << bit;
-                        R |= (!(vk > cut) ? 1ull : 0ull) << bit;
-                        if (wd) vk = *++at;
-                    }
-                    uint64_t *mq = masks + (size_t)(f + k) * (2 * kMaskWords);
-                    mq[lane] = L;
-                    mq[kMaskWords + lane] = R;
-                    const uint32_t nl = wave_sum((uint32_t)__popcll(L));
-                    const uint32_t nr = wave_sum((uint32_t)__popcll(R));
+        }
+        const float cut = cell_cut(lo, hi);
+        // ---- the chunks' masks and stopper offsets, kMidChunks at a time (a
+        // cell of the stable partition may hold more: its level's other buffer
+        // takes over, so none of its cells can be left alone)
+        uint64_t off = 0ull, all = 0ull;  // this thread's chunk; the chunks so far
+        for (uint32_t tile = 0; tile == 0u || tile < nch; tile += (uint32_t)kMidChunks) {
+            const uint32_t nt = nch - tile < (uint32_t)kMidChunks ? nch - tile : (uint32_t)kMidChunks;
+            if constexpr (WEIGHTED) {
+                for (uint32_t k = (uint32_t)w; k < nt; k += kW) {
+                    const uint64_t *mq = masks + (size_t)(f + tile + k) * (2 * kMaskWords);
+                    const uint32_t nl = wave_sum((uint32_t)__popcll(mq[lane]));
+                    const uint32_t nr = wave_sum((uint32_t)__popcll(mq[kMaskWords + lane]));
                     if (lane == 0) {
                         preL[k] = nl;
                         preR[k] = nr;
                     }
                 }
+            } else {
+                // ---- stopper masks: a wave per kPer chunks, a word per lane
+                constexpr int kPer = 4;
+                for (uint32_t k0 = (uint32_t)(w * kPer); k0 < nt; k0 += (uint32_t)(kW * kPer)) {
+                    uint64_t G[kPer], W[kPer];
+                    float v0[kPer];
+                    const float *pk[kPer];
+#pragma unroll
+                    for (int u = 0; u < kPer; ++u) {
+                        const uint32_t k = tile + (k0 + (uint32_t)u < nt ? k0 + (uint32_t)u : nt - 1u);
+                        const uint64_t *mq = masks + (size_t)(f + k) * (2 * kMaskWords);
+                        G[u] = mq[lane];
+                        W[u] = mq[kMaskWords + lane];
+                    }
+#pragma unroll
+                    for (int u = 0; u < kPer; ++u) {
+                        const uint32_t k = tile + (k0 + (uint32_t)u < nt ? k0 + (uint32_t)u : nt - 1u);
+                        const uint32_t cw = (uint32_t)__popcll(W[u]);
+                        const uint32_t ex = wave_inclusive_scan(cw) - cw;
+                        const int q0 = lane & ~15;  // first word of this lane's quarter
+                        const uint32_t rank = ex - (uint32_t)__shfl((int)ex, q0, 64);
+                        pk[u] = pack + begin + k * (uint32_t)kChunk + 64u * (uint32_t)q0 + rank;
+                        v0[u] = W[u] ? *pk[u] : 0.0f;
+                    }
+#pragma unroll
+                    for (int u = 0; u < kPer; ++u) {
+                        const uint32_t k = tile + k0 + (uint32_t)u;
+                        if (k0 + (uint32_t)u >= nt) break;  // uniform
+                        const uint32_t p0 = k * (uint32_t)kChunk + 64u * (uint32_t)lane;
+                        const uint64_t valid =
+                            p0 >= n ? 0ull : (n - p0 >= 64u ? ~0ull : (1ull << (n - p0)) - 1ull);
+                        uint64_t L = G[u], R = valid & ~G[u] & ~W[u], wd = W[u];
+                        float vk = v0[u];
+                        const float *at = pk[u];
+                        while (wd) {
+                            const uint32_t bit = (uint32_t)__builtin_ctzll(wd);
+                            wd &= wd - 1ull;
+                            L |= (!(vk < cut) ? 1ull : 0ull) << bit;
+                            R |= (!(vk > cut) ? 1ull : 0ull) << bit;
+                            if (wd) vk = *++at;
+                        }
+                        uint64_t *mq = masks + (size_t)(f + k) * (2 * kMaskWords);
+                        mq[lane] = L;
+                        mq[kMaskWords + lane] = R;
+                        const uint32_t nl = wave_sum((uint32_t)__popcll(L));
+                        const uint32_t nr = wave_sum((uint32_t)__popcll(R));
+                        if (lane == 0) {
+                            preL[k - tile] = nl;
+                            preR[k - tile] = nr;
+                        }
+                    }
+                }
             }
+            __syncthreads();
+            uint64_t mine = (uint32_t)t < nt ? (uint64_t)preL[t] | ((uint64_t)preR[t] << 32) : 0ull;
+            if constexpr (STABLE) {
+                // keys going left, and the chunk's others
+                const uint32_t b0 = (tile + (uint32_t)t) * (uint32_t)kChunk;
+                const uint32_t len = n - b0 < (uint32_t)kChunk ? n - b0 : (uint32_t)kChunk;
+                const uint32_t nle = hi32(mine);
+                mine = (uint32_t)t < nt ? (uint64_t)nle | ((uint64_t)(len - nle) << 32) : 0ull;
+            }
+            const uint64_t inc = wave_inclusive_scan(mine);
+            if (lane == 63) s_sum[w] = inc;
+            __syncthreads();
+            const uint64_t ws = lane < kW ? s_sum[lane] : 0ull;
+            const uint64_t wp = wave_inclusive_scan(ws);
+            off = all + inc - mine + lane_value(wp, w) - lane_value(ws, w);
+            all += lane_value(wp, 63);
+            if ((uint32_t)t <= nt && t <= kMidChunks) {
+                preL[t] = lo32(off);
+                preR[t] = hi32(off);
+                chunk_pre[f + (uint32_t)c + tile + (uint32_t)t] = off;
+            }
+            if constexpr (STABLE) __syncthreads();  // the next tile rewrites the tables
         }
-        __syncthreads();
-        // ---- the chunks' stopper offsets, a chunk per thread
-        const uint64_t mine = (uint32_t)t < nch ? (uint64_t)preL[t] | ((uint64_t)preR[t] << 32) : 0ull;
-        const uint64_t inc = wave_inclusive_scan(mine);
-        if (lane == 63) s_sum[w] = inc;
-        __syncthreads();
-        const uint64_t ws = lane < kW ? s_sum[lane] : 0ull;
-        const uint64_t wp = wave_inclusive_scan(ws);
-        const uint64_t all = lane_value(wp, 63);
-        const uint64_t off = inc - mine + lane_value(wp, w) - lane_value(ws, w);
         const uint32_t TL = lo32(all), TR = hi32(all);
-        if ((uint32_t)t <= nch && t <= kMidChunks) {
-            preL[t] = lo32(off);
-            preR[t] = hi32(off);
-            chunk_pre[f + (uint32_t)c + (uint32_t)t] = off;
-        }
         if (t == 64)  // the cell's margins, its passes, its children
             finish_round(rec, c, RoundOut{lo, hi, passes, found, 0}, found ? 1 : 0, recs, heap,
                          level_passes, exists, status);
         const int64_t lid = left_child_id(id), rid = right_child_id(id);
+        if constexpr (STABLE) {
+            // as k_stable_ranges: an empty side is no error
+            if (t == 0) {
+                if (rid >= (int64_t)rec.capr) {
+                    report_error(status + rec.st, rec.lp & 63, kErrPartition, id);
+                } else {
+                    splits[c] = SplitRec{TL, TR, 0u, TL};
+                    const int64_t gl = hb + lid, gr = hb + rid;
+                    ranges[2 * gl] = begin;
+                    ranges[2 * gl + 1] = begin + TL;
+                    ranges[2 * gr] = begin + TL;
+                    ranges[2 * gr + 1] = begin + n;
+                }
+            }
+            // k_stable_scatter reads the cut and the axis of the record
+            __syncthreads();  // the next cell rewrites the tables
+            continue;
+        }
         if (n == 0u || TL == 0u || rid >= (int64_t)(int32_t)uniform((uint32_t)rec.capr)) {
             // empty cell or no key >= cut: the reference's loop leaves the cell
             if (t == 0) {
@@ -3759,13 +3803,12 @@ int enqueue_level(Ctx &c, const LevelEntry *entries, int32_t nCells, orb_cell *h
     const int32_t sub_max = kernels.sub_max ? std::min((int32_t)kernels.sub_max, subtree_max_keys(c))
                                             : subtree_max_keys(c);
     const bool use_subtree = any_subtree && c.part == ORB_PART_HOARE && sub_max > 0;
-    if ((kernels.cell_max || kernels.chunks != kChunksAll) && c.part != ORB_PART_HOARE) return ORB_ERR_STATE;
-    if (c.weighted && kernels.cell_max) return ORB_ERR_STATE;
+    if (kernels.cell_max && (c.part != ORB_PART_HOARE || c.weighted)) return ORB_ERR_STATE;
     const bool mid = kernels.chunks == kChunksMid;
     if (mid && nCells >= kRecsScan) return ORB_ERR_STATE;  // one block fills its tables
     const LevelMode mode{use_subtree ? (uint32_t)sub_max : 0u, kernels.cell_max,
-                         kernels.chunks == kChunksAll ? ~0u
-                                                      : (mid ? (uint32_t)(kMidChunks * kChunk) : 0u),
+                         kernels.chunks == kChunksAll || (mid && c.part == ORB_PART_STABLE_LE) ? ~0u
+                         : mid ? (uint32_t)(kMidChunks * kChunk) : 0u,
                          kernels.again ? 1 : 0};
     const int32_t cgroup = cell_group(nCells);
     // Chunk order: the first round walks the level's chunks from the last, so
@@ -3887,13 +3930,19 @@ int enqueue_level(Ctx &c, const LevelEntry *entries, int32_t nCells, orb_cell *h
             hipLaunchKernelGGL(k_mw_masks, dim3(gq), dim3(kBlock), 0, c.stream, c.recs.p, nCells,
                                c.cell_first.p, c.chunk_desc.p, mc, c.x(), c.y(), c.z(), state, cell_hist_w,
                                c.masks.p, trace);
-        hipLaunchKernelGGL(c.weighted ? k_m_tail<true> : k_m_tail<false>,
+        const bool stable = c.part == ORB_PART_STABLE_LE;
+        hipLaunchKernelGGL(c.weighted ? (stable ? k_m_tail<true, true> : k_m_tail<true, false>)
+                                      : (stable ? k_m_tail<false, true> : k_m_tail<false, false>),
                            dim3((unsigned)std::max<int32_t>(nCells, 1)), dim3(kTailBlock), 0, c.stream,
                            c.recs.p, nCells, c.cell_first.p, cell_hist, c.sel.p, lists, c.packed.p, state,
                            cell_hist_w, c.masks.p, c.chunk_pre.p, c.splits.p,
                            reinterpret_cast<SwapPlan *>(c.swap_plan.p), c.ranges.p, heap, exists, le,
                            trace, level_passes, status);
         ORB_HIP(hipGetLastError());
+        if (stable) {
+            ORB_TRY(launch_stable_scatter(c, nCells, full_cover, true));
+            return timing_pair(c, tp, kTimePartition);
+        }
         ORB_TRY(launch_hoare_swap(c, nCells, 0));
         ORB_TRY(timing_pair(c, tp, kTimePartition));
         return defer_final ? ORB_OK : launch_hoare_final(c, nCells);
@@ -4066,14 +4115,14 @@ bool LevelShape::add(const Ctx &c, int64_t n, int32_t d, int32_t level, bool com
 LevelKernels level_kernels(const Ctx &c, const LevelShape &s)
 {
     LevelKernels k;
-    if (c.part != ORB_PART_HOARE || !s.known) return k;
+    if (!s.known) return k;
     k.sub_max = (uint32_t)s.sub_max;
     if (s.cells_above == 0) {  // subtree cells only
         k.chunks = kChunksNone;
         return k;
     }
     const bool few = s.keys / kChunk + s.cells <= kMidLevelChunks && s.cells < kRecsScan;
-    if (!c.weighted) {
+    if (!c.weighted && c.part == ORB_PART_HOARE) {
         if (s.lo <= (int64_t)kCellLarge)
             k.cell_max = s.hi <= (int64_t)kCellTiny    ? kCellTiny
                          : s.hi <= (int64_t)kCellSmall ? kCellSmall : kCellLarge;

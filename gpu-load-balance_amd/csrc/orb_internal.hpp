@@ -636,6 +636,8 @@ int launch_stopper_counts(Ctx &c, int32_t nCells, bool le_only, const HistCounts
 int invalidate_stamps(Ctx &c, int32_t nCells);
 int launch_stable_le(Ctx &c, int32_t nCells, int32_t *status = nullptr, bool full_cover = false,
                      const HistCounts *hc = nullptr);
+// the scatter from the chunks' offsets in chunk_pre, and the copy back or flip
+int launch_stable_scatter(Ctx &c, int32_t nCells, bool full_cover, bool pre_per_cell);
 int ensure_stable_buffers(Ctx &c);
 int launch_copy_u32(hipStream_t s, const uint32_t *src, uint32_t *dst, size_t n);
 int launch_iota(hipStream_t s, uint32_t *p, size_t n);

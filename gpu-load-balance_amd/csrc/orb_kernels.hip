@@ -1506,7 +1506,7 @@ int launch_hoare(Ctx &c, int32_t nCells, int32_t *status, const HistCounts *hc, 
 // Writing straight from the lanes stored runs of about 32 floats, parts of
 // lines that two waves share: 138 us a level of 2^24 keys against 70 (5.8 TB/s).
 // Bound: memory, 12 B read and written a key.
-template <bool kPayload>
+template <bool kPayload, bool kPerCell>
 __global__ __launch_bounds__(kBlock) void k_stable_scatter(
     const CellRec *__restrict__ recs, int32_t nCells, const uint32_t *__restrict__ first,
     const uint4 *__restrict__ chunk_desc, uint32_t max_chunks, const uint64_t *__restrict__ chunk_pre,
@@ -1547,7 +1547,9 @@ __global__ __launch_bounds__(kBlock) void k_stable_scatter(
         const int axis = (int)uniform((uint32_t)r.axis);
         const uint32_t begin = uniform(r.begin);
         const uint32_t f = uniform(first[cell]), f1 = uniform(first[cell + 1]);
-        const uint64_t pre0 = chunk_pre[f], pre = chunk_pre[q], pre1 = chunk_pre[f1];
+        // a level-wide scan, or a table per cell (one entry longer than its chunks)
+        const uint64_t *pc = chunk_pre + (kPerCell ? cell : 0u);
+        const uint64_t pre0 = pc[f], pre = pc[q], pre1 = pc[f1];
         uint32_t nle = 0;
         uint64_t mine = 0ull;  // row `lane`'s keys going left
         static_for<0, kRows>([&](auto jc) __attribute__((always_inline)) {
@@ -1626,35 +1628,30 @@ __global__ __launch_bounds__(kBlock) void k_stable_scatter(
 
 // The level's ranges back from the other buffer (a level that does not hold
 // every particle cannot flip buffers).
-__device__ inline void k_copy_back_chunk(uint32_t q, const CellRec *recs, int32_t nCells,
-                                         const uint32_t *first, const uint32_t *chunk_cell,
-                                         const float *ox, const float *oy, const float *oz,
-                                         const uint32_t *opid, const uint32_t *ow, float *x,
-                                         float *y, float *z, uint32_t *pid, uint32_t *w)
-{
-    uint32_t cell, b, e;
-    if (!chunk_range(q, first, nCells, chunk_cell, recs, cell, b, e)) return;
-    for (uint32_t p = b + threadIdx.x; p < e; p += kBlock) {
-        x[p] = ox[p];
-        y[p] = oy[p];
-        z[p] = oz[p];
-        if (pid) pid[p] = opid[p];
-        if (w) w[p] = ow[p];
-    }
-}
-
-__global__ __launch_bounds__(kBlock) void k_copy_back(const CellRec *recs, int32_t nCells,
-                                                      const uint32_t *first,
-                                                      const uint32_t *chunk_cell, const float *ox,
-                                                      const float *oy, const float *oz,
-                                                      const uint32_t *opid, const uint32_t *ow,
-                                                      float *x, float *y, float *z, uint32_t *pid,
-                                                      uint32_t *w)
+__global__ __launch_bounds__(kBlock) void k_copy_back(int32_t nCells, const uint32_t *__restrict__ first,
+                                                      const uint4 *__restrict__ chunk_desc,
+                                                      uint32_t max_chunks,
+                                                      const float *__restrict__ ox,
+                                                      const float *__restrict__ oy,
+                                                      const float *__restrict__ oz,
+                                                      const uint32_t *__restrict__ opid,
+                                                      const uint32_t *__restrict__ ow,
+                                                      float *__restrict__ x, float *__restrict__ y,
+                                                      float *__restrict__ z, uint32_t *__restrict__ pid,
+                                                      uint32_t *__restrict__ w)
 {
     const uint32_t total = first[nCells];
-    for (uint32_t q = blockIdx.x; q < total; q += gridDim.x)
-        k_copy_back_chunk(q, recs, nCells, first, chunk_cell, ox, oy, oz, opid, ow, x, y, z, pid,
-                          w);
+    for (uint32_t q = blockIdx.x;; q += gridDim.x) {
+        const uint4 d = chunk_record(chunk_desc, q, max_chunks);
+        if (q >= total) break;
+        for (uint32_t p = d.x + threadIdx.x; p < d.y; p += kBlock) {
+            x[p] = ox[p];
+            y[p] = oy[p];
+            z[p] = oz[p];
+            if (pid) pid[p] = opid[p];
+            if (w) w[p] = ow[p];
+        }
+    }
 }
 
 __global__ void k_stable_ranges(const CellRec *recs, int32_t nCells, const uint32_t *first,
@@ -1681,30 +1678,39 @@ __global__ void k_stable_ranges(const CellRec *recs, int32_t nCells, const uint3
     ranges[2 * gr + 1] = r.end;
 }
 
-int launch_stable_le(Ctx &c, int32_t nCells, int32_t *status, bool full_cover,
-                     const HistCounts *hc)
+int launch_stable_scatter(Ctx &c, int32_t nCells, bool full_cover, bool pre_per_cell)
 {
-    if (!status) status = c.status.p;
     ORB_TRY(ensure_stable_buffers(c));
     const unsigned gq = chunk_grid(c);
-    ORB_TRY(launch_stopper_counts(c, nCells, true, hc));
     float *ob = c.other();
     float *ox = ob, *oy = ob + c.stride, *oz = ob + 2 * c.stride;
-    auto scatter = c.ids() || c.weights() ? k_stable_scatter<true> : k_stable_scatter<false>;
+    const bool payload = c.ids() || c.weights();
+    auto scatter = pre_per_cell ? (payload ? k_stable_scatter<true, true> : k_stable_scatter<false, true>)
+                                : (payload ? k_stable_scatter<true, false> : k_stable_scatter<false, false>);
     hipLaunchKernelGGL(scatter, dim3(gq), dim3(kBlock), 0, c.stream, c.recs.p, nCells,
-                       c.cell_first.p, c.chunk_desc.p, (uint32_t)c.max_chunks, c.chunk_pre.p, c.x(),
-                       c.y(), c.z(), c.ids(), c.weights(), ox, oy, oz, c.other_ids(),
+                       c.cell_first.p, c.chunk_desc.p, (uint32_t)c.max_chunks, c.chunk_pre.p,
+                       c.x(), c.y(), c.z(), c.ids(), c.weights(), ox, oy, oz, c.other_ids(),
                        c.other_weights());
     ORB_HIP(hipGetLastError());
     if (full_cover) {
         // every particle was written to the other buffer: it becomes current
         c.in_tmp = !c.in_tmp;
     } else {
-        hipLaunchKernelGGL(k_copy_back, dim3(gq), dim3(kBlock), 0, c.stream, c.recs.p, nCells,
-                           c.cell_first.p, c.chunk_cell.p, ox, oy, oz, c.other_ids(),
+        hipLaunchKernelGGL(k_copy_back, dim3(gq), dim3(kBlock), 0, c.stream, nCells, c.cell_first.p,
+                           c.chunk_desc.p, (uint32_t)c.max_chunks, ox, oy, oz, c.other_ids(),
                            c.other_weights(), c.x(), c.y(), c.z(), c.ids(), c.weights());
         ORB_HIP(hipGetLastError());
     }
+    return ORB_OK;
+}
+
+int launch_stable_le(Ctx &c, int32_t nCells, int32_t *status, bool full_cover,
+                     const HistCounts *hc)
+{
+    if (!status) status = c.status.p;
+    ORB_TRY(ensure_stable_buffers(c));
+    ORB_TRY(launch_stopper_counts(c, nCells, true, hc));
+    ORB_TRY(launch_stable_scatter(c, nCells, full_cover, false));
     unsigned gc = (unsigned)((nCells + kBlock - 1) / kBlock);
     hipLaunchKernelGGL(k_stable_ranges, dim3(gc), dim3(kBlock), 0, c.stream, c.recs.p, nCells,
                        c.cell_first.p, c.chunk_pre.p, c.splits.p, c.ranges.p, status,

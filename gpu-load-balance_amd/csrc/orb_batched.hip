@@ -3046,11 +3046,16 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4, 4))
 //                        the listed keys, the stopper masks, K, i and the swap plan
 //   k_hoare_swap
 // The same rounds, masks and plan as the chunk path's.  The five top levels of
-// 2^20 keys (1 to 16 cells): 53 us a level, from 89.  Past kMidLevelChunks the
-// atomics on the cells' rows and the chunks each tail block walks grow, and the
-// chunk path's launches are no longer what bounds a level.
+// 2^20 keys (1 to 16 cells): 53 us a level, from 89.  A cell of more chunks keeps
+// one tail block busy for longer than the launches it saves (tables of 1024
+// chunks: 3000001 keys to 500 leaves 638 -> 655 us; of 256: 654).  The level's
+// size matters little: against a line at 2048 chunks, whole builds of 12M keys
+// take 1403 -> 1210 us, 2^24 stable ones 1512 -> 1397, 5e7 tied ones 6870 -> 6030
+// (8192 to 16384) and 5e7 even ones, with predicted windows, 3900 -> 3887.  Past
+// 16384 the one block that fills the chunk table takes longer than the launches
+// saved: with the line at 65536, 2^27 even keys 10046 -> 10217 us.
 constexpr int kMidChunks = 512;         // per cell: k_m_tail's tables
-constexpr int64_t kMidLevelChunks = 2048;
+constexpr int64_t kMidLevelChunks = 16384;
 
 // Round 1 of a chunk's cell from the cell's row of counts (bins of every key
 // of the cell), by a whole wave.
@@ -4111,7 +4116,8 @@ bool LevelShape::add(const Ctx &c, int64_t n, int32_t d, int32_t level, bool com
 // registers in two launches where the chunk path needs sixteen and reads the
 // keys once, not twice; a level whose every cell fits it or the subtree kernel
 // goes without the chunk kernels.  The lines: a block a cell holds 40960
-// keys; a level of few chunks (kMidLevelChunks) is bound by its launches.
+// keys; a level of few chunks a cell (kMidChunks, kMidLevelChunks) is
+// bound by its launches.
 LevelKernels level_kernels(const Ctx &c, const LevelShape &s)
 {
     LevelKernels k;

@@ -135,3 +135,10 @@ def test_weighted_few_chunks(orb, oracle, n, d, kind, cmp):
             assert np.array_equal(fbits(a), fbits(b))
         assert np.array_equal(ctx.ids(), r.ids)
         assert np.array_equal(ctx.weights(), r.weights)
+
+
+# levels of many chunks whose cells still fit the few-chunk kernels' tables
+@pytest.mark.parametrize("n,d", [(9000001, 40), (17000003, 300)])
+@pytest.mark.parametrize("cmp", [0, 1])
+def test_many_chunks(orb, oracle, n, d, cmp):
+    assert check(orb, oracle, inputs.clustered(n, n_spheres=9, a=0.03, seed=d), d, cmp=cmp)

@@ -70,3 +70,10 @@ def test_cell_of_several_tables(orb, oracle):
     w = np.ones(n, np.uint32)
     w[(xyz[0] < np.float32(-0.499))] = 100000
     check(orb, oracle, xyz, 16, w=w)
+
+
+@pytest.mark.parametrize("n,d", [(9000001, 40), (17000003, 300)])
+@pytest.mark.parametrize("weighted", [False, True])
+def test_many_chunks(orb, oracle, n, d, weighted):
+    w = np.random.default_rng(n).integers(1, 9, n).astype(np.uint32) if weighted else None
+    check(orb, oracle, inputs.clustered(n, n_spheres=7, a=0.04, seed=d), d, w=w)

@@ -346,29 +346,46 @@ __device__ inline float candidate(int t, float lo, float hi)
     return cell_cut(lo, hi);
 }
 
+// Exact bin of key v in [lo, hi] among the 255 candidate cuts of the next 8
+// bisection steps, without a table: the walk down the candidate tree
+// computes each midpoint with the cut arithmetic (cell.h:74-76) and counts
+// the candidates at or below v (LE = 0) or below v (LE = 1).  The
+// candidates are sorted, so a node that qualifies takes its whole left
+// subtree with it.
+template <int LE>
+__device__ inline int bin_walk(float v, float lo, float hi)
+{
+    int e = 0;
+#pragma unroll
+    for (int d = 0; d < kHistK; ++d) {
+        const float m = cell_cut(lo, hi);
+        const bool right = LE ? (m < v) : (m <= v);
+        if (right) {
+            e += 1 << (kHistK - 1 - d);
+            lo = m;
+        } else {
+            hi = m;
+        }
+    }
+    return e;
+}
+
 // Bin of key v among the sorted candidates cand[1..255] (cand[0] = -inf,
 // cand[256] = +inf): the number of candidates <= v (LE = 0) or < v (LE = 1).
-// Keys outside the margins [lo, hi] never reach here.  The candidates sit
-// close to lo + j*(hi-lo)/256, so the arithmetic estimate is checked against
-// its two neighbours (one pair of LDS reads); only an estimate that misses
-// (rounding at a bin edge, or a window a few ulps wide) walks, and the walk
-// alone makes the result exact.
+// The candidates sit close to lo + j*(hi-lo)/256, so the arithmetic estimate
+// is checked against its two neighbours (one pair of LDS reads); an estimate
+// that misses (rounding at a bin edge, or a window a few ulps wide) takes the
+// eight steps of the exact walk.  (Stepping along the table instead took up to
+// 255 reads a key where candidates are equal, which is where keys tie: 2^26
+// keys on 256 values, <=, root level 7.26 ms, now 1.21.)
 template <int LE>
-__device__ inline int bin_of(const float *cand, float v, float lo, float scale, int &tie)
+__device__ inline int bin_of(const float *cand, float v, float lo, float hi, float scale, int &tie)
 {
     const float ef = fminf(fmaxf((v - lo) * scale, 0.0f), (float)(kBins - 1));
     int e = (int)ef;
     const float c0 = cand[e], c1 = cand[e + 1];
     const bool ok = LE ? (c0 < v && v <= c1) : (c0 <= v && v < c1);
-    if (__builtin_expect(!ok, 0)) {
-        if (LE) {
-            while (e > 0 && cand[e] >= v) --e;
-            while (e < kBins - 1 && cand[e + 1] < v) ++e;
-        } else {
-            while (e > 0 && cand[e] > v) --e;
-            while (e < kBins - 1 && cand[e + 1] <= v) ++e;
-        }
-    }
+    if (__builtin_expect(!ok, 0)) e = bin_walk<LE>(v, lo, hi);
     // the candidate v equals, if any: cand[e] (<) or cand[e + 1] (<=)
     tie = LE ? (cand[e + 1] == v ? e + 1 : 0) : (cand[e] == v ? e : 0);
     return e;
@@ -543,7 +560,7 @@ __global__ __launch_bounds__(kBlock) void k_b_hist(
                 if (__ballot(ok && slow)) {  // wave-uniform; rare: near a bin edge
                     if (ok && slow) {
                         int tj;
-                        bin = bin_of<LE>(cand, vj, lo, scale, tj);
+                        bin = bin_of<LE>(cand, vj, lo, hi, scale, tj);
                         if (chunk_tie && tj) atomicAdd(&ties[tj], 1u);
                     }
                 }
@@ -667,7 +684,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8, 8))) 
         for (uint32_t k = (uint32_t)lane; k < packed; k += 64) {
             const float vk = wk[k];
             int tj;  // ties: the stopper counts of cells past this round use the packed keys
-            atomicAdd(&hist[bin_of<LE>(cand, vk, lo, scale, tj)], 1u);
+            atomicAdd(&hist[bin_of<LE>(cand, vk, lo, hi, scale, tj)], 1u);
         }
         uint64_t *mq = masks + (size_t)q * (2 * kMaskWords) + w * kPerWave;
         if (lane < kPerWave) {
@@ -1324,7 +1341,7 @@ __global__ __launch_bounds__(kBlock) void k_b_finish(CellRec *recs, int32_t nCel
                 if (v[u] < lo) ++bl;
                 else if (!(v[u] > hi)) {
                     int tj;
-                    atomicAdd(&pw[bin_of<LE>(cw, v[u], lo, scale, tj)], 1u);
+                    atomicAdd(&pw[bin_of<LE>(cw, v[u], lo, hi, scale, tj)], 1u);
                 }
             }
         }
@@ -1474,7 +1491,7 @@ __global__ __launch_bounds__(kFinBlock) void k_b_finish_block(CellRec *recs, int
                     const bool lt = on && v[u] < lo, in = on && !(v[u] < lo) && !(v[u] > hi);
                     bl += lt ? 1u : 0u;
                     int tj, bin = 0;
-                    if (in) bin = bin_of<LE>(cand, v[u], lo, scale, tj);
+                    if (in) bin = bin_of<LE>(cand, v[u], lo, hi, scale, tj);
                     count_bin(hist, bin, in);
                 }
             }
@@ -1833,9 +1850,6 @@ __device__ inline void issue_weight_loads(const uint32_t *wgt, uint4 dd, uint32_
             wr, (int)((sb + (uint32_t)lane) * 4u + 256u * (uint32_t)j), 0, 0);
 }
 
-template <int LE>
-__device__ inline int bin_walk(float v, float lo, float hi);
-
 // A wave's keys and weights into the block's row of weight sums: keys outside
 // the margins add up in registers (as atomics they would share two words) and
 // keys of weight 0, those past the chunk's end among them, add nothing.
@@ -2085,30 +2099,6 @@ __device__ inline int64_t left_difference(uint64_t left, float target)
 {
     if constexpr (W) return difference_from_target_w(left, target);
     else return difference_from_target((uint32_t)left, target);
-}
-
-// Exact bin of key v in [lo, hi] among the 255 candidate cuts of the next 8
-// bisection steps, without a table: the walk down the candidate tree
-// computes each midpoint with the cut arithmetic (cell.h:74-76) and counts
-// the candidates at or below v (LE = 0) or below v (LE = 1).  The
-// candidates are sorted, so a node that qualifies takes its whole left
-// subtree with it.
-template <int LE>
-__device__ inline int bin_walk(float v, float lo, float hi)
-{
-    int e = 0;
-#pragma unroll
-    for (int d = 0; d < kHistK; ++d) {
-        const float m = cell_cut(lo, hi);
-        const bool right = LE ? (m < v) : (m <= v);
-        if (right) {
-            e += 1 << (kHistK - 1 - d);
-            lo = m;
-        } else {
-            hi = m;
-        }
-    }
-    return e;
 }
 
 // The LDS capacity of the subtree kernel (keys of one subtree root) per

@@ -1553,9 +1553,13 @@ __global__ __launch_bounds__(kFinBlock) void k_b_finish_block(CellRec *recs, int
 // do that the cut lies in, so here a sample of the keys (about 16384 a cell or
 // more) picks it, 6 standard deviations wide each way, and the one full pass
 // counts exactly:
-//   k_p_sample  64-key lines spread over each chunk into the cell's 1024
-//               linear bins
-//   k_p_choose  per cell: the window
+//   k_p_sample  16-key segments spread evenly over each chunk into the cell's
+//               1024 linear bins, and how far keys of one segment and of
+//               adjacent ones agree
+//   k_p_choose  per cell: the window.  Neighbours in memory may be neighbours in
+//               space (particles grouped by object or by hash cell): a segment
+//               is then worth as little as one draw, and the deviation grows
+//               with it (sample_spread)
 //   k_p_window  as k_b_hist_window: keys below and above the window counted,
 //               its keys packed per chunk quarter and counted in linear bins
 //   (k_b_hist_reduce)
@@ -1573,16 +1577,19 @@ __global__ __launch_bounds__(kFinBlock) void k_b_finish_block(CellRec *recs, int
 // from 296 with two full rounds.  Below kPredKeys a cell's sample would have
 // to be a good part of its keys.
 constexpr int kSampleBins = 1024;
-constexpr int kSampleLines = 64;     // lines (of 64 keys) a block
+constexpr int kSegment = 16;         // keys of a segment (64 B, a DPP row of lanes)
+constexpr int kSampleRow = kSampleBins + 128;  // the bins, pairs in a segment, pairs across two
+constexpr int kSampleLines = 64;     // lines (of four segments) a block
 constexpr int64_t kPredKeys = 65536;  // smallest expected cell of such a level
 constexpr int64_t kPredLevelKeys = int64_t(1) << 24;  // and keys of the build
 
-// Sample line i of `ls` of chunk q starts here (a multiple of 64; the start
-// moves with the chunk, so that no period of the input meets every line).
-__device__ inline uint32_t sample_line(uint32_t q, uint32_t i, uint32_t ls)
+// Segment i of the 4 ls of chunk q starts here, then at the next multiple of 16
+// in memory (the start moves with the chunk, so that no period of the input
+// meets every segment).
+__device__ inline uint32_t sample_segment(uint32_t q, uint32_t i, uint32_t ls)
 {
-    const uint32_t span = (uint32_t)kChunk / ls;  // a power of two, at least 64
-    return i * span + ((q * 0x9e3779b1u) >> 20 & (span - 1u) & ~63u);
+    const uint32_t span = (uint32_t)kChunk / (4u * ls);  // a power of two, at least 64
+    return i * span + ((q * 0x9e3779b1u) >> 20 & (span - 1u) & ~(uint32_t)(kSegment - 1));
 }
 
 __global__ __launch_bounds__(kBlock) void k_p_sample(
@@ -1592,13 +1599,13 @@ __global__ __launch_bounds__(kBlock) void k_p_sample(
 {
     constexpr int kW = kBlock / 64;
     constexpr int kPer = kSampleLines / kW;  // 16 lines a wave, all in flight
-    __shared__ uint32_t hist[kSampleBins];
+    __shared__ uint32_t hist[kSampleRow];
     const int t = threadIdx.x, lane = t & 63, w = (int)uniform((uint32_t)t >> 6);
     const uint32_t total = first[nCells];
     const uint32_t per_block = (uint32_t)kSampleLines / ls;  // chunks a block
     for (uint32_t q0 = blockIdx.x * per_block; q0 < total; q0 += gridDim.x * per_block) {
         const uint32_t cell0 = uniform(chunk_record(chunk_desc, q0, max_chunks).z);
-        for (int k = t; k < kSampleBins; k += kBlock) hist[k] = 0u;
+        for (int k = t; k < kSampleRow; k += kBlock) hist[k] = 0u;
         float v[kPer];
         uint32_t cell[kPer];
         bool ok[kPer];
@@ -1608,7 +1615,9 @@ __global__ __launch_bounds__(kBlock) void k_p_sample(
             const uint32_t q = q0 + line / ls;
             const uint4 d = chunk_record(chunk_desc, q, max_chunks);
             const uint32_t b = uniform(d.x), e = uniform(d.y), axis = uniform(d.w);
-            const uint32_t p = b + sample_line(q, line % ls, ls) + (uint32_t)lane;
+            const uint32_t off = sample_segment(q, 4u * (line % ls) + (uint32_t)(lane / kSegment), ls);
+            const uint32_t p = ((b + off + (uint32_t)(kSegment - 1)) & ~(uint32_t)(kSegment - 1)) +
+                               (uint32_t)(lane % kSegment);
             cell[j] = uniform(d.z);
             ok[j] = q < total && axis <= 2u && p < e;
             v[j] = ok[j] ? axis_ptr(x, y, z, (int)axis)[p] : 0.0f;
@@ -1616,20 +1625,61 @@ __global__ __launch_bounds__(kBlock) void k_p_sample(
         __syncthreads();
 #pragma unroll
         for (int j = 0; j < kPer; ++j) {
-            if (!__ballot(ok[j])) continue;  // uniform
+            const uint64_t on = __ballot(ok[j]);
+            if (!on) continue;  // uniform
             const float lo = uniform(recs[cell[j]].margin_l), hi = uniform(recs[cell[j]].margin_r);
             const float width = hi - lo, scale = width > 0.0f ? (float)kSampleBins / width : 0.0f;
             const int bin = (int)__builtin_amdgcn_fmed3f((v[j] - lo) * scale, 0.0f, (float)(kSampleBins - 1));
-            if (ok[j]) {
-                if (cell[j] == cell0) atomicAdd(&hist[bin], 1u);
-                else atomicAdd(&sample_hist[(size_t)cell[j] * kSampleBins + bin], 1u);  // the block's last chunks
+            // the block's last chunks may be another cell's (uniform)
+            const bool mine = cell[j] == cell0;
+            auto count = [&](int at) __attribute__((always_inline)) {
+                if (mine) atomicAdd(&hist[at], 1u);
+                else atomicAdd(&sample_hist[(size_t)cell[j] * kSampleRow + at], 1u);
+            };
+            if (ok[j]) count(bin);
+            // every fourth line, if whole, in pairs by the 16-bin group of the larger
+            // key: within a segment (lanes i and 7 - i of every eight, 1 to 7 keys
+            // apart) and with the next segment
+            if (j % 4 == 0 && on == ~0ull) {
+                const int near = (int)dpp_move<0x141, 0xf>((uint32_t)bin), far = __shfl_xor(bin, kSegment, 64);
+                if (!(lane & 4)) count(kSampleBins + ((bin > near ? bin : near) >> 4));
+                if (!(lane & kSegment)) count(kSampleBins + 64 + ((bin > far ? bin : far) >> 4));
             }
         }
         __syncthreads();
-        for (int k = t; k < kSampleBins; k += kBlock)
-            if (hist[k]) atomicAdd(&sample_hist[(size_t)cell0 * kSampleBins + k], hist[k]);
+        for (int k = t; k < kSampleRow; k += kBlock)
+            if (hist[k]) atomicAdd(&sample_hist[(size_t)cell0 * kSampleRow + k], hist[k]);
         __syncthreads();
     }
+}
+
+// The variance of the sample's count below the quantile `mid`, relative to that
+// of independent draws: 1 for keys in no order, up to 16 where each segment lies
+// on one side.  Lane l brings the sample's keys up to the end of its 16-bin group
+// (inc, of s) and the pairs, within a segment and across two, whose larger key
+// lies in it.  With F the share of keys below a bound, A and B the shares of
+// pairs with both below it, within and across, a segment's count varies about
+// its surroundings' by 16 (F - B) + 16 * 15 (A - B): keys that agree over many
+// segments (long runs) are met by each of them and vary less.  A - B counts less
+// two of its standard deviations (even keys stay at 1).  Taken at the bounds of
+// the quantile's group; where neither splits the keys it is unknown: 16.
+__device__ inline float sample_spread(uint32_t inc, float s, float mid, uint32_t in, uint32_t across)
+{
+    const int lane = threadIdx.x & 63;
+    const uint32_t pi = wave_inclusive_scan(in), pa = wave_inclusive_scan(across);
+    const float np = (float)lane_value(pi, 63);  // as many across
+    const float F = s > 0.0f ? (float)inc / s : 0.0f;
+    const float A = np > 0.0f ? (float)pi / np : 0.0f, B = np > 0.0f ? (float)pa / np : 0.0f;
+    const float even = F * (1.0f - F);
+    const bool known = even > 0.05f && np > 0.0f;
+    const float noise = 2.0f * sqrtf((A * (1.0f - A) + B * (1.0f - B)) / np);
+    const float v = known ? (F - B + (float)(kSegment - 1) * fmaxf(A - B - noise, 0.0f)) / even : 0.0f;
+    // the quantile's group, and the bounds at its two ends
+    const int g = __popcll(__ballot((float)inc <= mid));
+    const bool use = known && (lane == g || lane + 1 == g);
+    if (!__ballot(use)) return (float)kSegment;  // uniform
+    const uint32_t m = wave_max(use ? __float_as_uint(fmaxf(v, 0.0f)) : 0u);  // (bits keep the order)
+    return fminf(fmaxf(__uint_as_float(m), 1.0f), (float)kSegment);
 }
 
 // A wave per cell: the window from the sample, and the row cleared.
@@ -1640,7 +1690,11 @@ __global__ __launch_bounds__(kBlock) void k_p_choose(const CellRec *__restrict__
     const int lane = threadIdx.x & 63;
     const int32_t c = (int32_t)((blockIdx.x * kBlock + threadIdx.x) >> 6);
     if (c >= nCells || recs[c].flags) return;  // uniform
-    uint4 *row = reinterpret_cast<uint4 *>(sample_hist + (size_t)c * kSampleBins) + lane * (kPer / 4);
+    uint4 *row = reinterpret_cast<uint4 *>(sample_hist + (size_t)c * kSampleRow) + lane * (kPer / 4);
+    uint32_t *pairs = sample_hist + (size_t)c * kSampleRow + kSampleBins + lane;
+    const uint32_t in = pairs[0], across = pairs[64];
+    pairs[0] = 0u;
+    pairs[64] = 0u;
     uint32_t h[kPer];
 #pragma unroll
     for (int u = 0; u < kPer / 4; ++u) {
@@ -1659,7 +1713,9 @@ __global__ __launch_bounds__(kBlock) void k_p_choose(const CellRec *__restrict__
     const float s = (float)lane_value(inc, 63);
     const int32_t nl = recs[c].nLeaf;
     const float ratio = (float)((nl + 1) / 2) / (float)nl;
-    const float mid = s * ratio, dev = 6.0f * sqrtf(s * ratio * (1.0f - ratio)) + 8.0f;
+    const float mid = s * ratio;
+    const float dev =
+        6.0f * sqrtf(s * ratio * (1.0f - ratio) * sample_spread(inc, s, mid, in, across)) + 8.0f;
     uint32_t below = 0, reach = 0, cum = inc - mine;  // whole bins under each bound
 #pragma unroll
     for (int u = 0; u < kPer; ++u) {
@@ -3721,8 +3777,8 @@ static int ensure_state(Ctx &c, int32_t levels_mode, bool *complete)
     if (!c.weighted && c.n >= kPredLevelKeys) {
         // cells of at least kPredKeys keys (less what a level's sizes vary by)
         const size_t cells = (size_t)(c.n / (kPredKeys / 2)) + 2;
-        if (c.sample_hist.n < cells * kSampleBins) b.sample_clean = false;
-        ORB_TRY(c.sample_hist.alloc(cells * kSampleBins));
+        if (c.sample_hist.n < cells * kSampleRow) b.sample_clean = false;
+        ORB_TRY(c.sample_hist.alloc(cells * kSampleRow));
         ORB_TRY(c.windows.alloc(cells * (sizeof(Window) / 4)));
     }
     // every buffer the launches touch exists before a capture starts

@@ -516,7 +516,7 @@ struct Ctx {
     DevBuf<uint64_t> sel_lists;      // [max_chunks+1] batched form: count of keys gathered into
                                      // a list of sel | keys below << 32, at the list's first chunk
     DevBuf<SplitRec> splits;         // [cells]
-    DevBuf<uint32_t> sample_hist;    // [cells][1024] large levels: the sample's bins, zero between levels
+    DevBuf<uint32_t> sample_hist;    // [cells][1152] large levels: the sample's bins and pairs, zero between levels
     DevBuf<uint32_t> windows;        // [cells][8] large levels: the predicted windows
     DevBuf<uint32_t> round_state;    // [2][cells][4] weighted levels of few chunks: the rounds' margins
     DevBuf<uint4> swap_plan;         // [max_chunks][2] Hoare swap unit of each chunk

@@ -876,6 +876,11 @@ __global__ __launch_bounds__(kBlock) void k_hoare_masks(const CellRec *recs, int
 // skipped: nothing reads their masks, and their count slot is written as
 // zero.
 constexpr int kMasksChunks = 2;  // k_hoare_masks_window: chunks per wave
+// A word with more window keys than this is taken by the whole wave, a key a
+// lane, four words' loads in flight; its own lane takes fewer one by one (2^26
+// keys in runs of 512 neighbours in space, whose words are all in the window or
+// all outside: 52 -> 32 us a level; even keys have a few a word).
+constexpr int kMasksDense = 12;
 __global__ __launch_bounds__(kBlock) void k_hoare_masks_window(
     const CellRec *__restrict__ recs, int32_t nCells, const uint32_t *__restrict__ first,
     const uint4 *__restrict__ chunk_desc, uint32_t max_chunks, const float *x, const float *y,
@@ -953,7 +958,8 @@ __global__ __launch_bounds__(kBlock) void k_hoare_masks_window(
                 const int q0 = lane & ~(kQuarter - 1);
                 const float *pk = pack + b + 64u * (uint32_t)q0;
                 uint32_t rk = rank[i];
-                uint64_t wd = W;
+                uint64_t dense = __ballot((uint32_t)__popcll(W) > (uint32_t)kMasksDense);
+                uint64_t wd = (dense >> lane) & 1ull ? 0ull : W;
                 bool first_bit = true;
                 while (wd) {
                     const uint32_t bit = (uint32_t)__builtin_ctzll(wd);
@@ -963,6 +969,29 @@ __global__ __launch_bounds__(kBlock) void k_hoare_masks_window(
                     first_bit = false;
                     L |= (!(v < c) ? 1ull : 0ull) << bit;
                     R |= (!(v > c) ? 1ull : 0ull) << bit;
+                }
+                while (dense) {  // uniform
+                    float v[4];
+                    int at[4];
+                    uint64_t m[4];
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) {
+                        at[u] = dense ? __builtin_ctzll(dense) : -1;
+                        dense &= dense - 1ull;  // 0 stays 0
+                        m[u] = at[u] >= 0 ? lane_value(W, at[u]) : 0ull;
+                        const uint32_t r0 = at[u] >= 0 ? lane_value(rank[i], at[u]) : 0u;
+                        const uint32_t k = r0 + (uint32_t)__builtin_amdgcn_mbcnt_hi(
+                            (uint32_t)(m[u] >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m[u], 0u));
+                        const float *p = pack + b + 64u * (uint32_t)(at[u] & ~(kQuarter - 1));
+                        v[u] = (m[u] >> lane) & 1ull ? p[k] : 0.0f;
+                    }
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) {
+                        const uint64_t mL = __ballot(!(v[u] < c)) & m[u];
+                        const uint64_t mR = __ballot(!(v[u] > c)) & m[u];
+                        L = lane == at[u] ? mL : L;
+                        R = lane == at[u] ? mR : R;
+                    }
                 }
                 L |= G;
                 R |= valid & ~G & ~W;

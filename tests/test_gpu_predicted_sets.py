@@ -49,3 +49,18 @@ def test_ties_at_the_cut(orb, oracle, cmp):
     even = timed(orb, uniform(N), d, cmp)[1]
     # the root level: 0.40 ms against 0.22; a step a candidate took 1.11 (<) and 1.92 (<=)
     assert ties[0] < 3.0 * even[0], (ties, even)
+
+
+# runs of neighbours in space, in no order (particles grouped by object or by
+# hash cell): consecutive sampled keys say little more than one of them, and a
+# window too narrow misses the cut, which makes the levels run twice
+@pytest.mark.parametrize("run", [16, 64, 4096])
+def test_grouped(orb, oracle, run):
+    d = 128
+    m = (N + run - 1) // run
+    box = np.float32(m ** (-1.0 / 3.0))
+    centres = uniform(m, seed=run)
+    xyz = tuple(np.clip(np.repeat(c, run)[:N] + box * a, np.float32(-0.5), np.float32(0.4999))
+                for c, a in zip(centres, uniform(N, seed=2)))
+    want = oracle.build(*xyz, d, levels_mode=1, threads=8)
+    assert timed(orb, xyz, d, 0, want, reps=1)[0] == timed(orb, uniform(N), d, 0, reps=1)[0]

@@ -522,6 +522,7 @@ int orb_finalize(orb_ctx *ctx)
     c->round_state.release();
     c->sample_hist.release();
     c->windows.release();
+    c->window_bins.release();
     c->chunk_comp.release();
     c->sel.release();
     c->sel_lists.release();

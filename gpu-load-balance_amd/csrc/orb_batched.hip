@@ -981,32 +981,48 @@ __device__ inline void finish_round(CellRec r, int32_t c, const RoundOut &ro, in
 
 
 // A predicted window of a cell (large levels, k_p_choose): [lo, hi], its keys
-// in bins 1 to 254 (bin 0: below, 255: above), and the bins [b1, b2] that can
-// hold the cut (k_p_narrow).
-constexpr int kWindowBins = kBins - 2;
+// in bins 1 to 253 (bin 0: below, 255: above), and the keys [klo, khi] of the bins
+// that can hold the cut (k_p_narrow).  The bins come from the sample's 1024 linear
+// ones over the cell's margins, of which the window takes [bl, bu): each is cut
+// into as many as its share of the window's sample (kSampleBins bytes a cell,
+// the window bins before each), so that keys in a few tight clumps are told
+// apart as well as even ones (two clumps of 0.01, 2^26 keys to 256: 10.1 ms with
+// bins of one width, which a clump falls into one of, now 4.6).
+constexpr int kSampleBins = 1024;
+constexpr int kWindowBins = kBins - 3;
 struct Window {
-    float lo, hi, scale;
-    uint32_t b1, b2, pad[3];
+    float lo, hi, klo, khi;
+    float base, scale;  // sample bin of v: (v - base) * scale
+    uint32_t bl, bu;
 };
 
-// The bin of a key in the window: grows with the key (a difference and a
-// product by a positive number keep order in float32), so keys of smaller
-// bins are smaller.
-__device__ inline uint32_t window_bin(float v, float lo, float scale)
+// Sample bins per unit of a cell's margins (0, one bin, where that is not finite).
+__device__ inline float sample_scale(float width)
 {
-    return 1u + (uint32_t)__builtin_amdgcn_fmed3f((v - lo) * scale, 0.0f, (float)(kWindowBins - 1));
+    return width > 0x1p-100f ? (float)kSampleBins / width : 0.0f;
+}
+
+// The bin of a key in the window (tab: the window bins before each sample bin):
+// grows with the key (a difference, a product by a positive number and their
+// fraction keep order in float32), so keys of smaller bins are smaller.
+__device__ inline uint32_t window_bin(float v, const Window &wd, const uint8_t *tab)
+{
+    const float t = __builtin_amdgcn_fmed3f((v - wd.base) * wd.scale, (float)wd.bl, (float)wd.bu);
+    const uint32_t s = (uint32_t)t < wd.bu ? (uint32_t)t : wd.bu - 1u;
+    const uint32_t b = tab[s], n = (s + 1u < (uint32_t)kSampleBins ? tab[s + 1u] : (uint32_t)kWindowBins) - b;
+    const uint32_t part = (uint32_t)((t - (float)s) * (float)n);
+    return 1u + b + (part < n ? part : n ? n - 1u : 0u);
 }
 
 // The passes of a predicted cell that its window decides: a candidate left of
-// bin b1 (right of b2) has a difference of -3 or less (3 or more).  Stops at
+// klo (right of khi) has a difference of -3 or less (3 or more).  Stops at
 // the first candidate inside, or at the pass cap.
 __device__ inline void window_passes(const Window &wd, float &L, float &R, int32_t &passes)
 {
     while (passes < ORB_MAX_PASSES) {
         const float c = cell_cut(L, R);
-        const uint32_t b = c < wd.lo ? 0u : (c > wd.hi ? (uint32_t)kBins - 1u : window_bin(c, wd.lo, wd.scale));
-        if (b < wd.b1) L = c;
-        else if (b > wd.b2) R = c;
+        if (c < wd.klo) L = c;
+        else if (c > wd.khi) R = c;
         else break;
         ++passes;
     }
@@ -1105,8 +1121,8 @@ __global__ __launch_bounds__(kBlock) void k_b_replay(CellRec *recs, int32_t nCel
 // in flight; a wave's keys are usually fewer than 256 and stay in registers
 // between counting and writing (a dense cluster packs a good part of a
 // chunk: few chunks per wave keep such waves short).
-// PRED: the keys of the window bins [b1, b2]; the keys left of them are
-// counted already (k_p_narrow).
+// PRED: the window's keys in [klo, khi]; the keys left of them are counted
+// already (k_p_narrow).
 template <bool PRED>
 __global__ __launch_bounds__(kBlock) void k_b_select(const CellRec *__restrict__ recs,
                                                      int32_t nCells,
@@ -1137,8 +1153,8 @@ __global__ __launch_bounds__(kBlock) void k_b_select(const CellRec *__restrict__
         const uint32_t nc0 = comp[8 * (size_t)qr + sh], nb0 = comp[8 * (size_t)qr + 4];
         const uint32_t cell = inq ? d.z : 0xffffffffu;  // runs end at the table's end
         bool live = inq && d.w <= 2u;
-        float lo = 0.0f, hi = 0.0f;  // PRED: the window's lower end and scale
-        uint32_t begin = 0, f = 0, nch = 0, bins = 0;
+        float lo = 0.0f, hi = 0.0f;
+        uint32_t begin = 0, f = 0, nch = 0;
         if (live) {
             const CellRec &r = recs[cell];
             f = first[cell];
@@ -1148,9 +1164,8 @@ __global__ __launch_bounds__(kBlock) void k_b_select(const CellRec *__restrict__
             hi = r.margin_r;
             begin = r.begin;
             if constexpr (PRED) {
-                lo = windows[cell].lo;
-                hi = windows[cell].scale;
-                bins = windows[cell].b1 | (windows[cell].b2 << 16);
+                lo = windows[cell].klo;
+                hi = windows[cell].khi;
             }
         }
         uint32_t off = 0, cnt = 0;
@@ -1170,16 +1185,10 @@ __global__ __launch_bounds__(kBlock) void k_b_select(const CellRec *__restrict__
         const uint32_t T = (uint32_t)__shfl((int)incl, 63, 64);
         // key t of the wave: quarter j = the last with ex_j <= t (it holds t)
         float v[kSelBatch], lj[kSelBatch], hj[kSelBatch];
-        uint32_t bj[PRED ? kSelBatch : 1];
         int rj[kSelBatch];
         // -1: left of what is gathered, 0: gathered, 1: right of it
         auto side = [&](int u) __attribute__((always_inline)) {
-            if constexpr (PRED) {
-                const uint32_t b = window_bin(v[u], lj[u], hj[u]);
-                return b < (bj[u] & 0xffffu) ? -1 : (b > (bj[u] >> 16) ? 1 : 0);
-            } else {
-                return v[u] < lj[u] ? -1 : (v[u] > hj[u] ? 1 : 0);
-            }
+            return v[u] < lj[u] ? -1 : (v[u] > hj[u] ? 1 : 0);
         };
         auto load_batch = [&](uint32_t t0) __attribute__((always_inline)) {
 #pragma unroll
@@ -1193,7 +1202,6 @@ __global__ __launch_bounds__(kBlock) void k_b_select(const CellRec *__restrict__
                     (uint32_t)__shfl((int)kbase, j, 64) + (t - (uint32_t)__shfl((int)ex, j, 64));
                 lj[u] = __shfl(lo, j, 64);
                 hj[u] = __shfl(hi, j, 64);
-                if constexpr (PRED) bj[u] = (uint32_t)__shfl((int)bins, j, 64);
                 rj[u] = __shfl(run, j, 64);
                 v[u] = t < T ? ckeys[at] : 0.0f;
             }
@@ -1561,7 +1569,7 @@ __global__ __launch_bounds__(kFinBlock) void k_b_finish_block(CellRec *recs, int
 //               is then worth as little as one draw, and the deviation grows
 //               with it (sample_spread)
 //   k_p_window  as k_b_hist_window: keys below and above the window counted,
-//               its keys packed per chunk quarter and counted in linear bins
+//               its keys packed per chunk quarter and counted in the window's bins
 //   (k_b_hist_reduce)
 //   k_p_narrow  per cell: the bins that can hold the cut
 // k_b_select gathers the keys of those bins and k_b_finish runs the
@@ -1576,7 +1584,6 @@ __global__ __launch_bounds__(kFinBlock) void k_b_finish_block(CellRec *recs, int
 // of it the window pass 147 (5 TB/s counting the swap's lines it waits for),
 // from 296 with two full rounds.  Below kPredKeys a cell's sample would have
 // to be a good part of its keys.
-constexpr int kSampleBins = 1024;
 constexpr int kSegment = 16;         // keys of a segment (64 B, a DPP row of lanes)
 constexpr int kSampleRow = kSampleBins + 128;  // the bins, pairs in a segment, pairs across two
 constexpr int kSampleLines = 64;     // lines (of four segments) a block
@@ -1628,8 +1635,8 @@ __global__ __launch_bounds__(kBlock) void k_p_sample(
             const uint64_t on = __ballot(ok[j]);
             if (!on) continue;  // uniform
             const float lo = uniform(recs[cell[j]].margin_l), hi = uniform(recs[cell[j]].margin_r);
-            const float width = hi - lo, scale = width > 0.0f ? (float)kSampleBins / width : 0.0f;
-            const int bin = (int)__builtin_amdgcn_fmed3f((v[j] - lo) * scale, 0.0f, (float)(kSampleBins - 1));
+            const int bin = (int)__builtin_amdgcn_fmed3f((v[j] - lo) * sample_scale(hi - lo), 0.0f,
+                                                         (float)(kSampleBins - 1));
             // the block's last chunks may be another cell's (uniform)
             const bool mine = cell[j] == cell0;
             auto count = [&](int at) __attribute__((always_inline)) {
@@ -1684,7 +1691,8 @@ __device__ inline float sample_spread(uint32_t inc, float s, float mid, uint32_t
 
 // A wave per cell: the window from the sample, and the row cleared.
 __global__ __launch_bounds__(kBlock) void k_p_choose(const CellRec *__restrict__ recs, int32_t nCells,
-                                                     uint32_t *sample_hist, Window *__restrict__ windows)
+                                                     uint32_t *sample_hist, Window *__restrict__ windows,
+                                                     uint32_t *__restrict__ window_bins)
 {
     constexpr int kPer = kSampleBins / 64;  // 16 bins a lane
     const int lane = threadIdx.x & 63;
@@ -1723,28 +1731,55 @@ __global__ __launch_bounds__(kBlock) void k_p_choose(const CellRec *__restrict__
         below += (float)cum < mid - dev ? 1u : 0u;
         reach += (float)cum < mid + dev ? 1u : 0u;
     }
-    const uint32_t bl = wave_sum(below), bu = wave_sum(reach) + 1u;
+    const uint32_t bl = wave_sum(below), bu0 = wave_sum(reach) + 1u;
+    const uint32_t bu = bu0 < (uint32_t)kSampleBins ? bu0 : (uint32_t)kSampleBins;
+    // the window's share of the sample before each of its bins, as window bins
+    // (no sample in it: by position)
+    uint32_t ca = 0, cb = 0;  // the sample before bl and before bu
+    cum = inc - mine;
+#pragma unroll
+    for (int u = 0; u < kPer; ++u) {
+        const uint32_t bin = (uint32_t)(lane * kPer + u);
+        ca = bin == bl ? cum : ca;
+        cb = bin == bu ? cum : cb;
+        cum += h[u];
+    }
+    ca = lane_value(ca, (int)(bl / kPer));
+    cb = bu < (uint32_t)kSampleBins ? lane_value(cb, (int)(bu / kPer)) : lane_value(inc, 63);
+    const float per = (float)kWindowBins / (float)(cb > ca ? cb - ca : bu - bl);
+    uint32_t packed[kPer / 4] = {};
+    cum = inc - mine;
+#pragma unroll
+    for (int u = 0; u < kPer; ++u) {
+        const uint32_t bin = (uint32_t)(lane * kPer + u);
+        const uint32_t at = cb > ca ? cum - ca : bin - bl;
+        const uint32_t b = bin < bl ? 0u : bin >= bu ? (uint32_t)kWindowBins : (uint32_t)((float)at * per);
+        packed[u / 4] |= (b < (uint32_t)kWindowBins ? b : (uint32_t)kWindowBins) << (8 * (u % 4));
+        cum += h[u];
+    }
+    reinterpret_cast<uint4 *>(window_bins + (size_t)c * (kSampleBins / 4))[lane] =
+        make_uint4(packed[0], packed[1], packed[2], packed[3]);
     if (lane == 0) {
         const float lo = recs[c].margin_l, hi = recs[c].margin_r, step = (hi - lo) / (float)kSampleBins;
         const float wl = bl == 0u ? lo : fminf(fmaxf(lo + (float)bl * step, lo), hi);
         const float wr = bu >= (uint32_t)kSampleBins ? hi : fminf(fmaxf(lo + (float)bu * step, wl), hi);
-        const float width = wr - wl;
-        // (no bins in a window too narrow for a finite scale: one holds its keys)
-        windows[c] = Window{wl, wr, width > 0x1p-100f ? (float)kWindowBins / width : 0.0f, 1u,
-                            (uint32_t)kWindowBins, {0u, 0u, 0u}};
+        windows[c] = Window{wl, wr, wl, wr, lo, sample_scale(hi - lo), bl, bu};
     }
 }
 
 // Window pass (see k_b_hist_window for its packing and masks).
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_p_window(
-    const Window *__restrict__ windows, int32_t nCells, const uint32_t *__restrict__ first,
-    const uint4 *__restrict__ chunk_desc, uint32_t max_chunks, const float *__restrict__ x,
+    const Window *__restrict__ windows, const uint32_t *__restrict__ window_bins, int32_t nCells,
+    const uint32_t *__restrict__ first, const uint4 *__restrict__ chunk_desc, uint32_t max_chunks,
+    const float *__restrict__ x,
     const float *__restrict__ y, const float *__restrict__ z, uint16_t *__restrict__ chunk_hist,
     float *__restrict__ pack, uint32_t *__restrict__ comp, uint64_t *__restrict__ masks, int rev)
 {
     constexpr int kW = kBlock / 64;
     constexpr int kPerWave = kMaskWords / kW;  // 16 loads of 64 keys
     __shared__ uint32_t hist[kBins];
+    __shared__ uint32_t tab[kSampleBins / 4];
+    static_assert(kSampleBins / 4 == kBlock, "a word of the table per thread");
     __shared__ uint32_t sm[4];
     __shared__ float wkeys[kW][kChunk / kW];     // each wave's window keys, packed
     __shared__ uint64_t words[kW][2][kPerWave];  // each wave's mask words, staged
@@ -1760,10 +1795,18 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8, 8))) 
         if (q >= total) break;
         if (axis > 2u) continue;  // uniform: the cell is not searched
         const uint32_t sb = (uint32_t)(w * kPerWave * 64);  // chunk position of the quarter
+        const uint32_t tw = window_bins[(size_t)cell * kBlock + (uint32_t)t];  // issued before the keys
         float v[kPerWave];
         issue_chunk_loads(x, y, z, true, d, sb, lane, v);
-        const float lo = uniform(windows[cell].lo), hi = uniform(windows[cell].hi);
-        const float scale = uniform(windows[cell].scale);
+        Window wd;
+        wd.lo = uniform(windows[cell].lo);
+        wd.hi = uniform(windows[cell].hi);
+        wd.base = uniform(windows[cell].base);
+        wd.scale = uniform(windows[cell].scale);
+        wd.bl = uniform(windows[cell].bl);
+        wd.bu = uniform(windows[cell].bu);
+        const float lo = wd.lo, hi = wd.hi;
+        tab[t] = tw;
         hist[t] = 0u;
         __syncthreads();
         const uint32_t len = e - b;
@@ -1807,7 +1850,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8, 8))) 
         const uint64_t mineG = lane < kPerWave ? words[w][0][lane] : 0ull;
         const uint64_t mineW = lane < kPerWave ? words[w][1][lane] : 0ull;
         for (uint32_t k = (uint32_t)lane; k < packed; k += 64)
-            atomicAdd(&hist[window_bin(wk[k], lo, scale)], 1u);
+            atomicAdd(&hist[window_bin(wk[k], wd, reinterpret_cast<const uint8_t *>(tab))], 1u);
         uint64_t *mq = masks + (size_t)q * (2 * kMaskWords) + w * kPerWave;
         if (lane < kPerWave) {
             mq[lane] = mineG;
@@ -1828,21 +1871,35 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8, 8))) 
     }
 }
 
+// A float32 as an unsigned number of the same order, and back.
+__device__ inline uint32_t ordered(float v)
+{
+    const uint32_t u = __float_as_uint(v);
+    return u & 0x80000000u ? ~u : u | 0x80000000u;
+}
+__device__ inline float from_ordered(uint32_t u)
+{
+    return __uint_as_float(u & 0x80000000u ? u & 0x7fffffffu : ~u);
+}
+
 // A wave per cell: from the counts of the window's bins (bin 0: keys below the
-// window, 255: above), the bins [b1, b2] that can hold the cut, and the cell's
-// lists with the keys left of them.  A cell whose counts contradict the window
+// window, 255: above), the bins [b1, b2] that can hold the cut, the floats
+// [klo, khi] that lie in them, and the cell's lists with the keys left of them.  A cell whose counts contradict the window
 // is left alone (see above).
 __global__ __launch_bounds__(kBlock) void k_p_narrow(CellRec *recs, int32_t nCells, uint32_t *cell_hist,
                                                      Window *__restrict__ windows,
+                                                     const uint32_t *__restrict__ window_bins,
                                                      const uint32_t *__restrict__ first,
                                                      unsigned long long *__restrict__ sel_lists,
                                                      int32_t *level_passes)
 {
-    const int lane = threadIdx.x & 63;
+    __shared__ uint4 tables[kBlock / 64][kSampleBins / 16];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int32_t c = (int32_t)((blockIdx.x * kBlock + threadIdx.x) >> 6);
     if (c >= nCells || recs[c].flags) return;  // uniform
     uint4 *row = reinterpret_cast<uint4 *>(cell_hist + (size_t)c * kBins);
     const uint4 h4 = row[lane];
+    tables[w][lane] = reinterpret_cast<const uint4 *>(window_bins + (size_t)c * (kSampleBins / 4))[lane];
     row[lane] = make_uint4(0u, 0u, 0u, 0u);  // the next level adds to zero
     const uint32_t s0 = h4.x, s1 = s0 + h4.y, s2 = s1 + h4.z, s3 = s2 + h4.w;
     const uint32_t base = wave_inclusive_scan(s3) - s3;
@@ -1877,9 +1934,24 @@ __global__ __launch_bounds__(kBlock) void k_p_narrow(CellRec *recs, int32_t nCel
     const SelLists sl(f, first[c + 1] - f);
     if ((uint32_t)lane < sl.R)
         sel_lists[sl.start_chunk((uint32_t)lane)] = lane == 0 ? (unsigned long long)cnt << 32 : 0ull;
+    // both bins hold keys (their counts decide), so each end lies in the window;
+    // a 64-way search over the floats between, the table in LDS
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
+    __builtin_amdgcn_wave_barrier();
+    const uint8_t *tab = reinterpret_cast<const uint8_t *>(tables[w]);
+    const uint32_t olo = ordered(wd.lo), ohi = ordered(wd.hi) + 1u;
+    float klo = wd.lo, khi = wd.hi;
+    if (window_bin(wd.lo, wd, tab) < b1)  // uniform
+        klo = from_ordered(1u + wave_last_true(olo, ohi, [&](uint32_t k) {
+            return window_bin(from_ordered(k), wd, tab) < b1;
+        }));
+    if (window_bin(wd.hi, wd, tab) > b2)
+        khi = from_ordered(wave_last_true(olo, ohi, [&](uint32_t k) {
+            return window_bin(from_ordered(k), wd, tab) <= b2;
+        }));
     if (lane == 0) {
-        windows[c].b1 = b1;
-        windows[c].b2 = b2;
+        windows[c].klo = klo;
+        windows[c].khi = khi;
     }
 }
 
@@ -3780,6 +3852,7 @@ static int ensure_state(Ctx &c, int32_t levels_mode, bool *complete)
         if (c.sample_hist.n < cells * kSampleRow) b.sample_clean = false;
         ORB_TRY(c.sample_hist.alloc(cells * kSampleRow));
         ORB_TRY(c.windows.alloc(cells * (sizeof(Window) / 4)));
+        ORB_TRY(c.window_bins.alloc(cells * (kSampleBins / 4)));
     }
     // every buffer the launches touch exists before a capture starts
     ORB_TRY(preallocate_scratch(c));
@@ -3833,7 +3906,7 @@ static std::vector<uint64_t> graph_signature(const Ctx &c, const BatchedState &b
                           c.packed.p, c.masks.p, c.cell_cand.p, c.splits.p, c.chunk_comp.p,
                           c.sel.p, c.sel_lists.p, c.swap_plan.p, c.status.p, c.stamps.p, b.level_ids.p, b.heap.p, b.exists.p,
                           b.sub.p, b.chunk_hist.p, b.cell_hist.p, b.trace.p, b.level_passes.p,
-                          c.wt.p, c.wt_tmp.p, b.chunk_hist_w.p, b.cell_hist_w.p, c.round_state.p, c.sample_hist.p, c.windows.p, c.hstatus.p, b.hpasses.p};
+                          c.wt.p, c.wt_tmp.p, b.chunk_hist_w.p, b.cell_hist_w.p, c.round_state.p, c.sample_hist.p, c.windows.p, c.window_bins.p, c.hstatus.p, b.hpasses.p};
     for (const void *p : bufs) s.push_back((uint64_t)(uintptr_t)p);
     s.push_back((uint64_t)c.tune_chunk_blocks.size());
     for (int32_t v : c.tune_chunk_blocks) s.push_back((uint64_t)(int64_t)v);
@@ -4039,8 +4112,8 @@ int enqueue_level(Ctx &c, const LevelEntry *entries, int32_t nCells, orb_cell *h
                            c.recs.p, nCells, c.cell_first.p, c.chunk_desc.p, mc, c.x(), c.y(), c.z(), ls,
                            c.sample_hist.p);
         hipLaunchKernelGGL(k_p_choose, dim3(gw), dim3(kBlock), 0, c.stream, c.recs.p, nCells,
-                           c.sample_hist.p, windows);
-        hipLaunchKernelGGL(k_p_window, dim3(gq), dim3(kBlock), 0, c.stream, windows, nCells,
+                           c.sample_hist.p, windows, c.window_bins.p);
+        hipLaunchKernelGGL(k_p_window, dim3(gq), dim3(kBlock), 0, c.stream, windows, c.window_bins.p, nCells,
                            c.cell_first.p, c.chunk_desc.p, mc, c.x(), c.y(), c.z(), later_hist, c.packed.p,
                            c.chunk_comp.p, c.masks.p, rev);
         ORB_HIP(hipGetLastError());
@@ -4048,7 +4121,7 @@ int enqueue_level(Ctx &c, const LevelEntry *entries, int32_t nCells, orb_cell *h
         hipLaunchKernelGGL(k_b_hist_reduce, dim3(gr), dim3(kBlock), 0, c.stream, c.recs.p, nCells,
                            c.cell_first.p, c.chunk_cell.p, later_hist, cell_hist);
         hipLaunchKernelGGL(k_p_narrow, dim3(gw), dim3(kBlock), 0, c.stream, c.recs.p, nCells, cell_hist,
-                           windows, c.cell_first.p,
+                           windows, c.window_bins.p, c.cell_first.p,
                            reinterpret_cast<unsigned long long *>(c.sel_lists.p), level_passes);
         ORB_HIP(hipGetLastError());
     }

@@ -518,6 +518,7 @@ struct Ctx {
     DevBuf<SplitRec> splits;         // [cells]
     DevBuf<uint32_t> sample_hist;    // [cells][1152] large levels: the sample's bins and pairs, zero between levels
     DevBuf<uint32_t> windows;        // [cells][8] large levels: the predicted windows
+    DevBuf<uint32_t> window_bins;    // [cells][256] and the bins of each (k_p_choose)
     DevBuf<uint32_t> round_state;    // [2][cells][4] weighted levels of few chunks: the rounds' margins
     DevBuf<uint4> swap_plan;         // [max_chunks][2] Hoare swap unit of each chunk
     DevBuf<int32_t> status;          // [2]: error flag, failing heap id

@@ -64,3 +64,20 @@ def test_grouped(orb, oracle, run):
                 for c, a in zip(centres, uniform(N, seed=2)))
     want = oracle.build(*xyz, d, levels_mode=1, threads=8)
     assert timed(orb, xyz, d, 0, want, reps=1)[0] == timed(orb, uniform(N), d, 0, reps=1)[0]
+
+
+# two narrow clumps far apart, even and a little uneven: the window spans the gap
+# between them, and a clump is a small part of it
+@pytest.mark.parametrize("share", [0.5, 0.5005])
+@pytest.mark.parametrize("cmp", [0, 1])
+def test_two_clumps(orb, oracle, share, cmp):
+    d = 64
+    x, y, z = uniform(N)
+    right = np.random.default_rng(3).random(N) >= share
+    x = (np.where(right, np.float32(0.3), np.float32(-0.3)) + np.float32(0.01) * x).astype(np.float32)
+    want = oracle.build(x, y, z, d, levels_mode=1, cmp=cmp, threads=8)
+    clumps = timed(orb, (x, y, z), d, cmp, want)
+    even = timed(orb, uniform(N), d, cmp)
+    assert clumps[0] == even[0]
+    # the root level: 0.25 ms against 0.22; with window bins of one width 1.4 to 1.5
+    assert clumps[1][0] < 2.5 * even[1][0], (clumps, even)

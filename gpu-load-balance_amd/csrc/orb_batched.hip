@@ -47,7 +47,7 @@ struct BatchedState {
     DevBuf<uint8_t> exists;            // [cap]
     DevBuf<uint8_t> sub;               // [cap] cell handled inside a subtree kernel
     DevBuf<uint16_t> chunk_hist;       // [max_chunks][256]
-    DevBuf<uint32_t> cell_hist;        // [max_level_cells][256]
+    DevBuf<uint32_t> cell_hist;        // cell_hist_words
     DevBuf<uint64_t> chunk_hist_w;     // weighted builds: [max_chunks][256] weight sums
     DevBuf<uint64_t> cell_hist_w;      // weighted builds: [max_level_cells][256]
     bool hist_w_clean = false;         // cell_hist_w all zero (as cell_hist)
@@ -279,7 +279,6 @@ __global__ void k_b_recs(const LevelEntry *entries, int32_t nCells, const orb_ce
 // counts into first[] (first[nCells] = the level's chunks), in place of a
 // record launch and a scan launch.  kFill (levels of few chunks): the block
 // also fills the chunk records and clears the cells' key counters.
-constexpr int kRecsScan = 1024;
 template <bool kFill>
 __global__ __launch_bounds__(kRecsScan) void k_b_recs_scan(
     const LevelEntry *__restrict__ entries, int32_t nCells, const orb_cell *__restrict__ heap,
@@ -3153,15 +3152,17 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4, 4))
 // ---------------------------------------------------------------------------
 // A level of at most kMidLevelChunks chunks, its cells at most kMidChunks
 // chunks each, is bound by its launches, not by memory: the chunk path takes
-// 16 of them, 4-7 us each however little they do.  Here it takes five:
+// 16 of them, 4-7 us each however little they do.  Here it takes six:
 //   k_b_recs_scan<true>  cell records, chunk table, the cells' key counters
 //   k_m_hist             round 1 per chunk, added to the cell's row (atomics:
 //                        few blocks share a row)
 //   k_m_window           every block replays round 1 from its cell's row (a
 //                        1 KB read in place of two launches), then takes the
-//                        window pass and appends its window keys to the cell's list
-//   k_m_tail             a block per cell: round 1 again, the later rounds over
-//                        the listed keys, the stopper masks, K, i and the swap plan
+//                        window pass and adds round 2's counts to the cell's second row
+//   k_m_narrow           round 2 likewise; masks, packed keys and the cell's list
+//                        narrowed to its margins
+//   k_m_tail             a block per cell: the later rounds over the listed keys,
+//                        the stopper masks, K, i and the swap plan
 //   k_hoare_swap
 // The same rounds, masks and plan as the chunk path's.  The five top levels of
 // 2^20 keys (1 to 16 cells): 53 us a level, from 89.  A cell of more chunks keeps
@@ -3175,10 +3176,22 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4, 4))
 constexpr int kMidChunks = 512;         // per cell: k_m_tail's tables
 constexpr int64_t kMidLevelChunks = 16384;
 
-// Round 1 of a chunk's cell from the cell's row of counts (bins of every key
-// of the cell), by a whole wave.
-__device__ inline RoundOut replay_row(const uint32_t *row, const CellRec &r, int lane,
-                                      uint64_t *trace_row)
+// A cell's search between the launches of such a level: state[0 .. nCells) after
+// one round, state[nCells ..) after the next (weighted levels take them in turn).
+struct RoundState {
+    float L, R;
+    int32_t passes, found;
+};
+__device__ inline RoundState load_state(const RoundState *p)
+{
+    const RoundState s = *p;
+    return RoundState{uniform(s.L), uniform(s.R), (int32_t)uniform((uint32_t)s.passes),
+                      (int32_t)uniform((uint32_t)s.found)};
+}
+
+// The next round of a cell from its row of counts, by a whole wave.
+__device__ inline RoundState replay_row(const uint32_t *row, const CellRec &r, const RoundState &s, int lane,
+                                        uint64_t *trace_row)
 {
     const uint4 h4 = reinterpret_cast<const uint4 *>(row)[lane];
     const uint32_t s0 = h4.x, s1 = s0 + h4.y, s2 = s1 + h4.z, s3 = s2 + h4.w;
@@ -3187,7 +3200,14 @@ __device__ inline RoundOut replay_row(const uint32_t *row, const CellRec &r, int
     const uint32_t pv[4] = {base + s0, base + s1, base + s2, base + s3};
     const float target = difference_target(uniform(r.end) - uniform(r.begin),
                                            (int32_t)uniform((uint32_t)r.nLeaf));
-    return replay_round_lanes(pv, uniform(r.margin_l), uniform(r.margin_r), target, 0, lane, trace_row);
+    const RoundOut ro = replay_round_lanes(pv, s.L, s.R, target, s.passes, lane, trace_row);
+    return RoundState{uniform(ro.L), uniform(ro.R), ro.passes, ro.found ? 1 : 0};
+}
+
+// Where a cell's passes are traced, for the one wave that traces them.
+__device__ inline uint64_t *trace_of(uint64_t *trace, const CellRec &r, bool mine)
+{
+    return trace && mine ? trace + ((size_t)r.hb + r.id) * ORB_MAX_PASSES : nullptr;
 }
 
 // Round 1: as k_b_hist, without a candidate table (the exact bin of a key
@@ -3244,23 +3264,22 @@ __global__ __launch_bounds__(kBlock) void k_m_hist(const CellRec *__restrict__ r
     }
 }
 
-// Window pass: as k_b_hist_window, from round 1's outcome, without binning:
-// the keys below and above the margins are counted, the keys inside go to the
-// chunk quarter's slots of `pack` (in position order, for the masks) and to
-// the cell's list in `sel` (in any order, for the rounds), whose counter
-// (keys | keys below << 32) takes one atomic a chunk.  A cell whose cut round
-// 1 found has that cut as its window.
+// Window pass: as k_b_hist_window, from round 1's outcome: the keys inside the
+// margins go to the chunk quarter's slots of `pack` (in position order) and are
+// counted for round 2, with the keys below, in the cell's second row.  A cell
+// whose cut round 1 found has that cut as its window.
+template <int LE>
 __global__ __launch_bounds__(kBlock) void k_m_window(
     const CellRec *__restrict__ recs, int32_t nCells, const uint32_t *__restrict__ first,
     const uint4 *__restrict__ chunk_desc, uint32_t max_chunks, const float *__restrict__ x,
-    const float *__restrict__ y, const float *__restrict__ z, const uint32_t *__restrict__ cell_hist,
-    float *__restrict__ pack, uint64_t *__restrict__ masks, float *__restrict__ sel,
-    unsigned long long *__restrict__ sel_lists)
+    const float *__restrict__ y, const float *__restrict__ z, uint32_t *cell_hist,
+    RoundState *__restrict__ state, uint64_t *trace, float *__restrict__ pack,
+    uint64_t *__restrict__ masks)
 {
     constexpr int kW = kBlock / 64;
     constexpr int kPerWave = kMaskWords / kW;
     __shared__ float wkeys[kW][kChunk / kW];  // each wave's window keys, packed
-    __shared__ uint32_t s_n[kW], s_below[kW], s_base;
+    __shared__ uint32_t hist[kBins];
     __shared__ uint64_t words[kW][2][kPerWave];
     const int t = threadIdx.x, lane = t & 63, w = (int)uniform((uint32_t)t >> 6);
     const uint64_t lanes_below = lane == 0 ? 0ull : (~0ull >> (64 - lane));
@@ -3276,10 +3295,15 @@ __global__ __launch_bounds__(kBlock) void k_m_window(
         float v[kPerWave];
         issue_chunk_loads(x, y, z, true, d, sb, lane, v);
         const CellRec &r = recs[cell];
-        const uint32_t begin = uniform(r.begin), f = uniform(first[cell]);
-        const RoundOut ro = replay_row(cell_hist + (size_t)cell * kBins, r, lane, nullptr);
+        hist[t] = 0u;
+        const bool lead = q == uniform(first[cell]);  // the cell's first chunk keeps its state
+        const RoundState ro = replay_row(cell_hist + (size_t)cell * kBins, r,
+                                         RoundState{uniform(r.margin_l), uniform(r.margin_r), 0, 0}, lane,
+                                         trace_of(trace, r, lead && w == 0));
+        if (lead && t == 0) state[cell] = ro;
         const float cut = cell_cut(ro.L, ro.R);
-        const float lo = uniform(ro.found ? cut : ro.L), hi = uniform(ro.found ? cut : ro.R);
+        const float lo = ro.found ? cut : ro.L, hi = ro.found ? cut : ro.R;
+        __syncthreads();  // the row is clear
         const uint32_t len = e - b;
         uint32_t below = 0, packed = 0;  // wave-uniform
         float *dst = pack + b + sb;
@@ -3306,17 +3330,18 @@ __global__ __launch_bounds__(kBlock) void k_m_window(
                 packed += (uint32_t)__popcll(mW);
             }
         });
-        if (lane == 0) {
-            s_n[w] = packed;
-            s_below[w] = below;
-        }
-        __syncthreads();
-        if (t == 0) {
-            const uint32_t ns = s_n[0] + s_n[1] + s_n[2] + s_n[3];
-            const uint32_t nb = s_below[0] + s_below[1] + s_below[2] + s_below[3];
-            s_base = ns || nb ? (uint32_t)atomicAdd(&sel_lists[f], (unsigned long long)ns |
-                                                                       ((unsigned long long)nb << 32))
-                              : 0u;
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
+        __builtin_amdgcn_wave_barrier();
+        if (!ro.found) {  // uniform: round 2's row
+            const float width = hi - lo;
+            const float scale = width > 0.0f ? (float)kBins / width : 0.0f;
+            const float lim = 0.5f - bin_tolerance(lo, hi, scale);
+            for (uint32_t k = (uint32_t)lane; k < packed; k += 64u) {
+                int bin;
+                if (!bin_estimate(wk[k], lo, scale, lim, bin)) bin = bin_walk<LE>(wk[k], lo, hi);
+                atomicAdd(&hist[bin], 1u);
+            }
+            if (lane == 0 && below) atomicAdd(&hist[0], below);
         }
         uint64_t *mq = masks + (size_t)q * (2 * kMaskWords) + w * kPerWave;
         if (lane < kPerWave) {
@@ -3324,11 +3349,138 @@ __global__ __launch_bounds__(kBlock) void k_m_window(
             mq[kMaskWords + lane] = words[w][1][lane];
         }
         __syncthreads();
-        // the cell's list: from its first particle on (it holds at most the cell's keys)
-        uint32_t at = begin + s_base;
-        for (int u = 0; u < w; ++u) at += s_n[u];
-        for (uint32_t k = (uint32_t)lane; k < packed; k += 64u) sel[at + k] = wk[k];
+        if (hist[t]) atomicAdd(&cell_hist[((size_t)nCells + cell) * kBins + (size_t)t], hist[t]);
         __syncthreads();  // the next chunk rewrites the tables
+    }
+}
+
+// Narrows each chunk from round 1's margins to round 2's (1/65536 of the cell's):
+// the packed keys outside them settle their mask bits, those inside are packed
+// again and go to the cell's list in `sel` (in any order, for the later rounds),
+// whose counter (keys | keys below << 32) takes their number.  One tail block a
+// cell then has few keys left, also where the keys lie in a clump that
+// one bin of round 1 holds: without this pass 2^23 keys to 64 leaves, x in a clump
+// of 0.01, took 2577 us, now 960; even keys pay a launch and save a round of the tail.
+// A wave a chunk (a block a chunk replayed the rows in four waves and met at
+// barriers: 21 us at 4096 chunks).
+__global__ __launch_bounds__(kBlock) void k_m_narrow(
+    const CellRec *__restrict__ recs, int32_t nCells, const uint32_t *__restrict__ first,
+    const uint4 *__restrict__ chunk_desc, uint32_t max_chunks, const uint32_t *__restrict__ cell_hist,
+    RoundState *state, uint64_t *trace, float *pack, uint64_t *masks, float *__restrict__ sel,
+    unsigned long long *__restrict__ sel_lists)
+{
+    constexpr int kW = kBlock / 64;
+    constexpr int kQuarter = kMaskWords / kW;  // words per packing quarter
+    constexpr int kBatch = 4;                  // words in flight
+    const int lane = threadIdx.x & 63, w = (int)uniform((uint32_t)threadIdx.x >> 6);
+    const uint32_t total = first[nCells];
+    for (uint32_t q = blockIdx.x * (uint32_t)kW + (uint32_t)w;; q += gridDim.x * (uint32_t)kW) {
+        const uint4 d = chunk_record(chunk_desc, q, max_chunks);
+        const uint32_t b = uniform(d.x), e = uniform(d.y), cell = uniform(d.z);
+        const uint32_t axis = uniform(d.w);
+        keep_values(b, e, cell, axis);
+        if (q >= total) break;
+        if (axis > 2u) continue;  // uniform: the cell is not searched
+        uint64_t *mq = masks + (size_t)q * (2 * kMaskWords);
+        uint64_t G = mq[lane];
+        const uint64_t W = mq[kMaskWords + lane];
+        const CellRec &r = recs[cell];
+        const uint32_t begin = uniform(r.begin), f = uniform(first[cell]);
+        const uint32_t cw = (uint32_t)__popcll(W), in = wave_inclusive_scan(cw);
+        // before this word in its quarter
+        const int quarter = lane & ~(kQuarter - 1);
+        const uint32_t ex = in - cw - (uint32_t)__shfl((int)(in - cw), quarter, 64);
+        float *const keys = pack + b + 64u * (uint32_t)quarter;
+        // a word of few keys by its own lane, their loads in flight with the row;
+        // of more by the wave, a key a lane
+        const bool few = cw <= (uint32_t)kBatch;
+        float own[kBatch];
+#pragma unroll
+        for (int u = 0; u < kBatch; ++u) own[u] = few && (uint32_t)u < cw ? keys[ex + (uint32_t)u] : 0.0f;
+        const bool lead = q == f;
+        RoundState ro = load_state(state + cell);
+        if (!ro.found)  // uniform
+            ro = replay_row(cell_hist + ((size_t)nCells + cell) * kBins, r, ro, lane, trace_of(trace, r, lead));
+        if (lead && lane == 0) state[(size_t)nCells + cell] = ro;
+        const float cut = cell_cut(ro.L, ro.R);
+        const float lo = ro.found ? cut : ro.L, hi = ro.found ? cut : ro.R;
+        uint64_t kept = 0ull;
+        {
+            uint64_t wd = few ? W : 0ull;
+#pragma unroll
+            for (int u = 0; u < kBatch; ++u) {
+                const uint64_t bit = wd & (0ull - wd);  // 0: no key left
+                wd ^= bit;
+                const bool lt = own[u] < lo, gt = own[u] > hi;
+                G |= gt ? bit : 0ull;
+                kept |= lt || gt ? 0ull : bit;
+            }
+        }
+        // word `at` (-1: none) and its keys, a lane each; sub: the keys wanted of them
+        auto load_word = [&](int at, uint64_t sub) {
+            const uint64_t m = at >= 0 ? lane_value(W, at) : 0ull;
+            const uint32_t k = (at >= 0 ? lane_value(ex, at) : 0u) +
+                               (uint32_t)__builtin_amdgcn_mbcnt_hi(
+                                   (uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+            return (m & sub) >> lane & 1ull ? pack[b + 64u * (uint32_t)(at & ~(kQuarter - 1)) + k] : 0.0f;
+        };
+        for (uint64_t todo = __ballot(!few); todo;) {  // uniform
+            float v[kBatch];
+            int at[kBatch];
+#pragma unroll
+            for (int u = 0; u < kBatch; ++u) {
+                at[u] = todo ? __builtin_ctzll(todo) : -1;
+                todo &= todo - 1ull;  // 0 stays 0
+                v[u] = load_word(at[u], ~0ull);
+            }
+#pragma unroll
+            for (int u = 0; u < kBatch; ++u) {
+                const uint64_t mB = __ballot(v[u] < lo), mG = __ballot(v[u] > hi);
+                if (lane == at[u]) {
+                    G |= W & mG;
+                    kept = W & ~mB & ~mG;
+                }
+            }
+        }
+        const uint32_t below = e - b - wave_sum((uint32_t)__popcll(G)) - wave_sum((uint32_t)__popcll(kept));
+        const uint64_t words = __ballot(kept != 0ull);
+        if (words) {  // uniform; rare with even keys
+            const uint32_t ck = (uint32_t)__popcll(kept), ink = wave_inclusive_scan(ck);
+            const uint32_t exk = ink - ck, exq = exk - (uint32_t)__shfl((int)exk, quarter, 64);
+            // (where round 1 or 2 found the cut no later round reads the list)
+            uint32_t slot = 0;
+            if (!ro.found && lane == 0)
+                slot = (uint32_t)atomicAdd(&sel_lists[f], (unsigned long long)lane_value(ink, 63));
+            slot = begin + uniform(slot);
+            for (uint64_t todo = words; todo;) {  // uniform
+                float v[kBatch];
+                int at[kBatch];
+                uint64_t m[kBatch];
+#pragma unroll
+                for (int u = 0; u < kBatch; ++u) {
+                    at[u] = todo ? __builtin_ctzll(todo) : -1;
+                    todo &= todo - 1ull;
+                    m[u] = at[u] >= 0 ? lane_value(kept, at[u]) : 0ull;
+                    v[u] = load_word(at[u], m[u]);
+                }
+#pragma unroll
+                for (int u = 0; u < kBatch; ++u) {
+                    if (at[u] < 0) break;  // uniform
+                    const uint32_t k = (uint32_t)__builtin_amdgcn_mbcnt_hi(
+                        (uint32_t)(m[u] >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m[u], 0u));
+                    const uint32_t to = 64u * (uint32_t)(at[u] & ~(kQuarter - 1)) + lane_value(exq, at[u]) + k;
+                    const uint32_t list = slot + lane_value(exk, at[u]) + k;
+                    if ((m[u] >> lane) & 1ull) {
+                        pack[b + to] = v[u];  // (up to the keys read so far: later words' lie behind)
+                        // the cell's list: from its first particle on (at most the cell's keys)
+                        if (!ro.found) sel[list] = v[u];
+                    }
+                }
+            }
+        }
+        mq[lane] = G;
+        mq[kMaskWords + lane] = kept;
+        if (lane == 0 && below) atomicAdd(&sel_lists[f], (unsigned long long)below << 32);
     }
 }
 
@@ -3343,10 +3495,6 @@ __global__ __launch_bounds__(kBlock) void k_m_window(
 // row to the cell's row of this round: one launch a round where the chunk path
 // takes three.  k_mw_masks replays the last round and writes the stopper
 // masks, k_m_tail<true> takes the split and the plan.
-struct RoundState {
-    float L, R;
-    int32_t passes, found;
-};
 
 // The state after `round` rounds: the state before it and its row.  Every wave
 // that calls it gets it; trace_row (the round's left weights) where wanted.
@@ -3357,9 +3505,7 @@ __device__ inline RoundState weighted_state(const CellRec &r, uint32_t cell, int
     RoundState s{uniform(r.margin_l), uniform(r.margin_r), 0, 0};
     if (round == 0) return s;
     if (round > 1) {
-        const RoundState p = state[(size_t)((round - 1) & 1) * (size_t)nCells + cell];
-        s = RoundState{uniform(p.L), uniform(p.R), (int32_t)uniform((uint32_t)p.passes),
-                       (int32_t)uniform((uint32_t)p.found)};
+        s = load_state(state + (size_t)((round - 1) & 1) * (size_t)nCells + cell);
         if (s.found) return s;
     }
     const uint64_t *row = rows + ((size_t)(round - 1) * (size_t)nCells + cell) * kBins;
@@ -3463,10 +3609,10 @@ __global__ __launch_bounds__(kBlock) void k_mw_masks(
     }
 }
 
-// The rest of a cell's search and its split, a block per cell: round 1's
-// outcome, the later rounds over the listed keys (those inside the margins),
+// The rest of a cell's search and its split, a block per cell: after rounds 1 and
+// 2 (state) the later rounds over the listed keys (those inside the margins),
 // the cell's record and children, the stopper masks of its chunks from the
-// window pass's words and packed keys, the chunks' stopper offsets, K and i
+// narrowed words and packed keys, the chunks' stopper offsets, K and i
 // as in k_b_cell (the crossing chunk, its word, its bit), the children's
 // ranges, and each chunk's swap unit as k_hoare_plan makes it.  WEIGHTED: the
 // search and the masks are done (state, k_mw_masks); the chunks' counts come
@@ -3532,19 +3678,22 @@ __global__ __launch_bounds__(kTailBlock) void k_m_tail(
                 rows[((size_t)(q / kBins) * (size_t)nCells + c) * kBins + q % kBins] = 0ull;
         } else {
             uint64_t *trow = trace ? trace + ((size_t)hb + id) * ORB_MAX_PASSES : nullptr;
-            uint32_t *row = cell_hist + (size_t)c * kBins;
-            const RoundOut r1 = replay_row(row, rec, lane, w == 0 ? trow : nullptr);
-            lo = uniform(r1.L);
-            hi = uniform(r1.R);
-            passes = r1.passes;
-            found = r1.found;
+            // (no chunk carries the rounds of an empty cell: rows of zeros)
+            RoundState r2{lo, hi, 0, 0};
+            if (nch) r2 = load_state(state + (size_t)nCells + c);
+            else r2 = replay_row(cell_hist + (size_t)c * kBins, rec, r2, lane, w == 0 ? trow : nullptr);
+            lo = r2.L;
+            hi = r2.R;
+            passes = r2.passes;
+            found = r2.found != 0;
             const unsigned long long list = n ? sel_lists[f] : 0ull;
             const uint32_t m = uniform((uint32_t)list) < n ? uniform((uint32_t)list) : n;
             const uint32_t nbelow = uniform((uint32_t)(list >> 32));
             const float target = difference_target(n, (int32_t)uniform((uint32_t)rec.nLeaf));
             if (t < kBins) hist[t] = 0u;
-            __syncthreads();  // every wave has read the row
-            if (t < kBins) row[t] = 0u;  // the next level adds to zero
+            __syncthreads();
+            if (t < 2 * kBins)  // the next level adds to zero
+                cell_hist[((size_t)(t / kBins) * (size_t)nCells + c) * kBins + t % kBins] = 0u;
             while (!found && passes < ORB_MAX_PASSES) {
                 const float width = hi - lo;
                 const float scale = width > 0.0f ? (float)kBins / width : 0.0f;
@@ -3570,7 +3719,7 @@ __global__ __launch_bounds__(kTailBlock) void k_m_tail(
                     }
                 }
                 if (lane == 0 && below) atomicAdd(&hist[0], below);
-                if (t == 0 && nbelow) atomicAdd(&hist[0], nbelow);  // the keys below the window
+                if (t == 0 && nbelow) atomicAdd(&hist[0], nbelow);  // the keys below the list's
                 __syncthreads();
                 if (w == 0) {
                     const uint4 h4 = reinterpret_cast<const uint4 *>(hist)[lane];
@@ -3812,6 +3961,14 @@ __global__ __launch_bounds__(kTailBlock) void k_m_tail(
 // ---------------------------------------------------------------------------
 // orchestration
 // ---------------------------------------------------------------------------
+// Words of the cells' rows of counts: a row a cell (the chunk path), or two on
+// levels of few chunks (fewer than kRecsScan cells).
+size_t cell_hist_words(const Ctx &c)
+{
+    const size_t m = (size_t)c.max_level_cells;
+    return std::max(m, 2 * std::min(m, (size_t)kRecsScan)) * kBins;
+}
+
 // Rows of weight sums: one a cell (the chunk path), or one a cell and round
 // for levels of few chunks (fewer than kRecsScan cells).
 static size_t hist_w_rows(const Ctx &c)
@@ -3833,8 +3990,8 @@ static int ensure_state(Ctx &c, int32_t levels_mode, bool *complete)
     ORB_TRY(b.sub.alloc((size_t)c.cap));
     ORB_TRY(b.chunk_hist.alloc(kHistRegions * (size_t)(c.max_chunks + 1) * kBins));
     // a fresh (or grown, hence reallocated) buffer is cleared before use
-    if (b.cell_hist.n < (size_t)c.max_level_cells * kBins) b.hist_clean = false;
-    ORB_TRY(b.cell_hist.alloc((size_t)c.max_level_cells * kBins));
+    if (b.cell_hist.n < cell_hist_words(c)) b.hist_clean = false;
+    ORB_TRY(b.cell_hist.alloc(cell_hist_words(c)));
     ORB_TRY(b.level_passes.alloc(64));
     ORB_TRY(b.hpasses.alloc(64));
     if (c.trace) ORB_TRY(b.trace.alloc((size_t)c.cap * ORB_MAX_PASSES));
@@ -3843,7 +4000,6 @@ static int ensure_state(Ctx &c, int32_t levels_mode, bool *complete)
         const size_t rows = hist_w_rows(c);
         if (b.cell_hist_w.n < rows * kBins) b.hist_w_clean = false;
         ORB_TRY(b.cell_hist_w.alloc(rows * kBins));
-        ORB_TRY(c.round_state.alloc(4 * 2 * (size_t)kRecsScan));
     }
     if (!c.weighted) ORB_TRY(c.sel.alloc((size_t)c.stride));  // rounds 3 and 4
     if (!c.weighted && c.n >= kPredLevelKeys) {
@@ -4043,9 +4199,12 @@ int enqueue_level(Ctx &c, const LevelEntry *entries, int32_t nCells, orb_cell *h
             hipLaunchKernelGGL(le ? k_m_hist<1> : k_m_hist<0>, dim3(gq), dim3(kBlock), 0, c.stream,
                                c.recs.p, nCells, c.cell_first.p, c.chunk_desc.p, mc, c.x(), c.y(), c.z(),
                                cell_hist);
-            hipLaunchKernelGGL(k_m_window, dim3(gq), dim3(kBlock), 0, c.stream, c.recs.p, nCells,
-                               c.cell_first.p, c.chunk_desc.p, mc, c.x(), c.y(), c.z(), cell_hist,
-                               c.packed.p, c.masks.p, c.sel.p, lists);
+            hipLaunchKernelGGL(le ? k_m_window<1> : k_m_window<0>, dim3(gq), dim3(kBlock), 0, c.stream,
+                               c.recs.p, nCells, c.cell_first.p, c.chunk_desc.p, mc, c.x(), c.y(), c.z(),
+                               cell_hist, state, trace, c.packed.p, c.masks.p);
+            hipLaunchKernelGGL(k_m_narrow, dim3((gq + 3) / 4), dim3(kBlock), 0, c.stream, c.recs.p, nCells,
+                               c.cell_first.p, c.chunk_desc.p, mc, cell_hist, state, trace, c.packed.p,
+                               c.masks.p, c.sel.p, lists);
         }
         ORB_HIP(hipGetLastError());
         ORB_TRY(timing_pair(c, tb, kTimeCount));
@@ -4353,7 +4512,7 @@ int build_batched(Ctx &c, int32_t levels_mode, orb_build_info *info)
     c.table_ids.clear();
 
     if (!b.hist_clean) {
-        ORB_TRY(launch_zero_u32(c.stream, b.cell_hist.p, (size_t)c.max_level_cells * kBins));
+        ORB_TRY(launch_zero_u32(c.stream, b.cell_hist.p, cell_hist_words(c)));
         b.hist_clean = true;
     }
     if (c.sample_hist.p && !b.sample_clean) {

@@ -34,6 +34,7 @@ constexpr uint32_t kChunkIdle = 0xffffffffu;  // chunk record axis: no search th
 // batched form, per-chunk 256-bin rows: the first round's bins, the first
 // round's ties (both read again by the partition), the later rounds' bins
 constexpr int kHistRegions = 3;
+constexpr int kRecsScan = 1024;  // a level of fewer cells takes its records in one block
 
 // ---------------------------------------------------------------------------
 // error plumbing
@@ -519,7 +520,7 @@ struct Ctx {
     DevBuf<uint32_t> sample_hist;    // [cells][1152] large levels: the sample's bins and pairs, zero between levels
     DevBuf<uint32_t> windows;        // [cells][8] large levels: the predicted windows
     DevBuf<uint32_t> window_bins;    // [cells][256] and the bins of each (k_p_choose)
-    DevBuf<uint32_t> round_state;    // [2][cells][4] weighted levels of few chunks: the rounds' margins
+    DevBuf<uint32_t> round_state;    // [2][cells][4] levels of few chunks: the rounds' margins
     DevBuf<uint4> swap_plan;         // [max_chunks][2] Hoare swap unit of each chunk
     DevBuf<int32_t> status;          // [2]: error flag, failing heap id
     DevBuf<uint32_t> ids_dev;        // [cells]
@@ -695,6 +696,7 @@ int enqueue_level(Ctx &c, const LevelEntry *entries, int32_t nCells, orb_cell *h
                   uint64_t *cell_hist_w = nullptr, const PendingFinal *fin_in = nullptr,
                   bool defer_final = false, const LevelKernels &kernels = LevelKernels());
 int preallocate_scratch(Ctx &c);
+size_t cell_hist_words(const Ctx &c);  // what enqueue_level's cell_hist holds, zero between levels
 // level tables for nCells cells and (at least) `chunks` chunks
 int ensure_level_capacity(Ctx &c, int64_t nCells, int64_t chunks = 0);
 

@@ -185,6 +185,7 @@ int preallocate_scratch(Ctx &c)
     size_t m = (size_t)c.max_chunks + 1;
     size_t np = (m + kScanTile - 1) / kScanTile;
     ORB_TRY(c.scan_partials.alloc(np));
+    ORB_TRY(c.round_state.alloc(4 * 2 * (size_t)kRecsScan));
     if (c.part == ORB_PART_STABLE_LE) ORB_TRY(ensure_stable_buffers(c));
     return ORB_OK;
 }

@@ -323,13 +323,13 @@ static int server_alloc(Server &S)
     ORB_TRY(S.exists.alloc((size_t)H));
     ORB_TRY(S.sub.alloc((size_t)H));
     ORB_TRY(S.chunk_hist.alloc(kHistRegions * (size_t)(c.max_chunks + 1) * kBins));
-    ORB_TRY(S.cell_hist.alloc((size_t)c.max_level_cells * 256));
+    ORB_TRY(S.cell_hist.alloc(cell_hist_words(c)));
     ORB_TRY(S.level_passes.alloc((size_t)slots * 64));
     ORB_TRY(S.status.alloc((size_t)slots * 2));
     ORB_TRY(S.entries.alloc((size_t)c.max_level_cells));
     ORB_TRY(S.hentries[0].alloc((size_t)c.max_level_cells));
     ORB_TRY(S.hentries[1].alloc((size_t)c.max_level_cells));
-    ORB_TRY(launch_zero_u32(c.stream, S.cell_hist.p, (size_t)c.max_level_cells * 256));
+    ORB_TRY(launch_zero_u32(c.stream, S.cell_hist.p, cell_hist_words(c)));
     ORB_TRY(launch_zero_u32(c.stream, reinterpret_cast<uint32_t *>(S.level_passes.p), (size_t)slots * 64));
     ORB_TRY(launch_zero_u32(c.stream, reinterpret_cast<uint32_t *>(S.status.p), (size_t)slots * 2));
     ORB_HIP(hipStreamSynchronize(c.stream));
@@ -680,6 +680,7 @@ int orb_server_destroy(orb_server *o)
     c.chunk_pre.release();
     c.scan_partials.release();
     c.splits.release();
+    c.round_state.release();
     c.chunk_comp.release();
     c.sel.release();
     c.sel_lists.release();

@@ -15,10 +15,10 @@ def uniform(n, seed=1):
     return tuple((rng.random(n, np.float32) - np.float32(0.5)) for _ in range(3))
 
 
-def timed(orb, xyz, d, cmp=0, want=None, reps=3):
+def timed(orb, xyz, d, cmp=0, want=None, reps=3, partition=0):
     """(search launches, device ms of each level) of a build, the least of `reps`."""
     with orb.Context(len(xyz[0]), d, generate=False) as ctx:
-        ctx.set_semantics(cmp, 0)
+        ctx.set_semantics(cmp, partition)
         ctx.set_particles(*xyz)
         ctx.save_particles()
         ctx.enable_timing()
@@ -81,3 +81,17 @@ def test_two_clumps(orb, oracle, share, cmp):
     assert clumps[0] == even[0]
     # the root level: 0.25 ms against 0.22; with window bins of one width 1.4 to 1.5
     assert clumps[1][0] < 2.5 * even[1][0], (clumps, even)
+
+
+# one clump narrow in x: on the levels of few chunks that cut x, a bin of the
+# first round holds a good part of a cell's keys
+@pytest.mark.parametrize("cmp,partition", [(0, 0), (1, 0), (1, 1)])
+def test_clump_on_few_chunks(orb, oracle, cmp, partition):
+    n, d = 8000009, 64
+    x, y, z = uniform(n)
+    x = (np.float32(0.1) + np.float32(0.01) * x).astype(np.float32)
+    want = oracle.build(x, y, z, d, levels_mode=1, cmp=cmp, partition=partition, threads=8)
+    clump = timed(orb, (x, y, z), d, cmp, want, partition=partition)[1]
+    even = timed(orb, uniform(n), d, cmp, partition=partition)[1]
+    # the longest level took 0.78 ms against 0.17 while the tail had round 1's keys to walk
+    assert clump.max() < 2.5 * even.max(), (clump, even)

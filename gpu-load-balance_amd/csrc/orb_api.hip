@@ -879,12 +879,13 @@ int orb_get_ranges(orb_ctx *ctx, uint32_t *ranges, int64_t cap)
 {
     Ctx *c = C(ctx);
     if (!c || !ranges || cap < c->cap) return ORB_ERR_ARG;
-    // a small tree comes back whole, in one wait
-    if (c->results_on_device && c->cap <= kHostTreeCells) ORB_TRY(batched_pull_results(*c));
+    // a small tree comes back whole, in one wait (a traced one's counts stay)
+    if (c->results_on_device && c->cap <= kWholeTreeCells && !c->trace) ORB_TRY(batched_pull_results(*c));
     if (!c->ranges_on_host) {
         ORB_HIP(hipMemcpyAsync(c->hranges.p, c->ranges.p, 2 * sizeof(uint32_t) * (size_t)c->cap,
                                hipMemcpyDeviceToHost, c->stream));
         ORB_HIP(hipStreamSynchronize(c->stream));
+        c->ranges_on_host = true;
     }
     std::memcpy(ranges, c->hranges.p, 2 * sizeof(uint32_t) * (size_t)c->cap);
     std::memset(ranges + 2 * c->cap, 0, 2 * sizeof(uint32_t) * (size_t)(cap - c->cap));

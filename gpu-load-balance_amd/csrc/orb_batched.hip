@@ -4510,6 +4510,7 @@ int build_batched(Ctx &c, int32_t levels_mode, orb_build_info *info)
     BatchedState &b = *c.batched;
     timing_reset(c);
     c.table_ids.clear();
+    c.ranges_on_host = false;
 
     if (!b.hist_clean) {
         ORB_TRY(launch_zero_u32(c.stream, b.cell_hist.p, cell_hist_words(c)));
@@ -4552,7 +4553,6 @@ int build_batched(Ctx &c, int32_t levels_mode, orb_build_info *info)
     // status and pass counts are in the pinned words once the stream is done
     // (k_b_done); the tree stays in HBM until a getter asks for it
     // (batched_pull_results)
-    c.ranges_on_host = false;
     ORB_HIP(hipStreamSynchronize(c.stream));
     if (b.hpasses.p[0] > 0) {
         // cells larger than their level's kernels expected (keys that tie at
@@ -4587,7 +4587,7 @@ int batched_pull_results(Ctx &c)
     const bool small = c.cap <= kHostTreeCells;
     orb_cell *heap = small ? reinterpret_cast<orb_cell *>(c.hranges.p + 2 * c.cap) : c.heap.data();
     uint8_t *exists = small ? reinterpret_cast<uint8_t *>(heap + c.cap) : c.exists.data();
-    if (small)
+    if (small && !c.ranges_on_host)
         ORB_HIP(hipMemcpyAsync(c.hranges.p, c.ranges.p, 2 * sizeof(uint32_t) * (size_t)c.cap,
                                hipMemcpyDeviceToHost, c.stream));
     ORB_HIP(hipMemcpyAsync(heap, b.heap.p, sizeof(orb_cell) * (size_t)c.cap,

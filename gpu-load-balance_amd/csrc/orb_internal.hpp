@@ -579,6 +579,10 @@ struct Ctx {
 // (61 B a slot, 4 MB at most, allocated with the context): ranges, heap and
 // flags in one wait, where copies into pageable memory wait one by one.
 constexpr int64_t kHostTreeCells = int64_t(1) << 16;
+// Up to this many slots (125 KB) reading the ranges brings the heap and flags
+// too: the bytes cost less than the second wait would.  Above, or with a trace,
+// they come alone (32768 leaves: 250 us with the tree, 1170 with its trace, 50 alone).
+constexpr int64_t kWholeTreeCells = int64_t(1) << 11;
 inline size_t host_tree_words(int64_t cap)
 {
     const size_t n = (size_t)cap;

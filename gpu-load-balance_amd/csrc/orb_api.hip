@@ -519,10 +519,8 @@ int orb_finalize(orb_ctx *ctx)
     c->masks.release();
     c->cell_cand.release();
     c->splits.release();
-    c->round_state.release();
     c->sample_hist.release();
     c->windows.release();
-    c->window_bins.release();
     c->chunk_comp.release();
     c->sel.release();
     c->sel_lists.release();

@@ -3961,6 +3961,13 @@ __global__ __launch_bounds__(kTailBlock) void k_m_tail(
 // ---------------------------------------------------------------------------
 // orchestration
 // ---------------------------------------------------------------------------
+// The most cells of a predicted level: at least kPredKeys keys each (less what a
+// level's sizes vary by).
+static size_t predicted_cells(const Ctx &c)
+{
+    return (size_t)(c.n / (kPredKeys / 2)) + 2;
+}
+
 // Words of the cells' rows of counts: a row a cell (the chunk path), or two on
 // levels of few chunks (fewer than kRecsScan cells).
 size_t cell_hist_words(const Ctx &c)
@@ -4003,12 +4010,10 @@ static int ensure_state(Ctx &c, int32_t levels_mode, bool *complete)
     }
     if (!c.weighted) ORB_TRY(c.sel.alloc((size_t)c.stride));  // rounds 3 and 4
     if (!c.weighted && c.n >= kPredLevelKeys) {
-        // cells of at least kPredKeys keys (less what a level's sizes vary by)
-        const size_t cells = (size_t)(c.n / (kPredKeys / 2)) + 2;
+        const size_t cells = predicted_cells(c);
         if (c.sample_hist.n < cells * kSampleRow) b.sample_clean = false;
         ORB_TRY(c.sample_hist.alloc(cells * kSampleRow));
-        ORB_TRY(c.windows.alloc(cells * (sizeof(Window) / 4)));
-        ORB_TRY(c.window_bins.alloc(cells * (kSampleBins / 4)));
+        ORB_TRY(c.windows.alloc(cells * (sizeof(Window) + kSampleBins) / 4));
     }
     // every buffer the launches touch exists before a capture starts
     ORB_TRY(preallocate_scratch(c));
@@ -4062,7 +4067,7 @@ static std::vector<uint64_t> graph_signature(const Ctx &c, const BatchedState &b
                           c.packed.p, c.masks.p, c.cell_cand.p, c.splits.p, c.chunk_comp.p,
                           c.sel.p, c.sel_lists.p, c.swap_plan.p, c.status.p, c.stamps.p, b.level_ids.p, b.heap.p, b.exists.p,
                           b.sub.p, b.chunk_hist.p, b.cell_hist.p, b.trace.p, b.level_passes.p,
-                          c.wt.p, c.wt_tmp.p, b.chunk_hist_w.p, b.cell_hist_w.p, c.round_state.p, c.sample_hist.p, c.windows.p, c.window_bins.p, c.hstatus.p, b.hpasses.p};
+                          c.wt.p, c.wt_tmp.p, b.chunk_hist_w.p, b.cell_hist_w.p, c.sample_hist.p, c.windows.p, c.hstatus.p, b.hpasses.p};
     for (const void *p : bufs) s.push_back((uint64_t)(uintptr_t)p);
     s.push_back((uint64_t)c.tune_chunk_blocks.size());
     for (int32_t v : c.tune_chunk_blocks) s.push_back((uint64_t)(int64_t)v);
@@ -4188,7 +4193,8 @@ int enqueue_level(Ctx &c, const LevelEntry *entries, int32_t nCells, orb_cell *h
     if (mid) {
         int tb = timing_mark(c);
         unsigned long long *lists = reinterpret_cast<unsigned long long *>(c.sel_lists.p);
-        RoundState *state = reinterpret_cast<RoundState *>(c.round_state.p);
+        static_assert(sizeof(RoundState) == sizeof(SplitRec), "they follow the splits");
+        RoundState *state = reinterpret_cast<RoundState *>(c.splits.p + c.max_level_cells);
         const uint32_t mc = (uint32_t)c.max_chunks;
         if (c.weighted) {
             for (int r = 0; r < kRounds; ++r)
@@ -4265,14 +4271,15 @@ int enqueue_level(Ctx &c, const LevelEntry *entries, int32_t nCells, orb_cell *h
     if (kernels.predict) {
         const int tb = timing_mark(c);
         Window *windows = reinterpret_cast<Window *>(c.windows.p);
+        uint32_t *window_bins = c.windows.p + predicted_cells(c) * (sizeof(Window) / 4);
         const uint32_t mc = (uint32_t)c.max_chunks;
         const uint32_t ls = kernels.predict, per_block = (uint32_t)kSampleLines / ls;
         hipLaunchKernelGGL(k_p_sample, dim3((gq + per_block - 1) / per_block), dim3(kBlock), 0, c.stream,
                            c.recs.p, nCells, c.cell_first.p, c.chunk_desc.p, mc, c.x(), c.y(), c.z(), ls,
                            c.sample_hist.p);
         hipLaunchKernelGGL(k_p_choose, dim3(gw), dim3(kBlock), 0, c.stream, c.recs.p, nCells,
-                           c.sample_hist.p, windows, c.window_bins.p);
-        hipLaunchKernelGGL(k_p_window, dim3(gq), dim3(kBlock), 0, c.stream, windows, c.window_bins.p, nCells,
+                           c.sample_hist.p, windows, window_bins);
+        hipLaunchKernelGGL(k_p_window, dim3(gq), dim3(kBlock), 0, c.stream, windows, window_bins, nCells,
                            c.cell_first.p, c.chunk_desc.p, mc, c.x(), c.y(), c.z(), later_hist, c.packed.p,
                            c.chunk_comp.p, c.masks.p, rev);
         ORB_HIP(hipGetLastError());
@@ -4280,7 +4287,7 @@ int enqueue_level(Ctx &c, const LevelEntry *entries, int32_t nCells, orb_cell *h
         hipLaunchKernelGGL(k_b_hist_reduce, dim3(gr), dim3(kBlock), 0, c.stream, c.recs.p, nCells,
                            c.cell_first.p, c.chunk_cell.p, later_hist, cell_hist);
         hipLaunchKernelGGL(k_p_narrow, dim3(gw), dim3(kBlock), 0, c.stream, c.recs.p, nCells, cell_hist,
-                           windows, c.window_bins.p, c.cell_first.p,
+                           windows, window_bins, c.cell_first.p,
                            reinterpret_cast<unsigned long long *>(c.sel_lists.p), level_passes);
         ORB_HIP(hipGetLastError());
     }

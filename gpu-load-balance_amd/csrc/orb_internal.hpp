@@ -516,11 +516,11 @@ struct Ctx {
                                      // margins after the second round, from the cell's begin
     DevBuf<uint64_t> sel_lists;      // [max_chunks+1] batched form: count of keys gathered into
                                      // a list of sel | keys below << 32, at the list's first chunk
-    DevBuf<SplitRec> splits;         // [cells]
+    DevBuf<SplitRec> splits;         // [cells], then [2][kRecsScan] levels of few chunks: the
+                                     // rounds' margins (one allocation: each costs a new context 0.2 ms)
     DevBuf<uint32_t> sample_hist;    // [cells][1152] large levels: the sample's bins and pairs, zero between levels
-    DevBuf<uint32_t> windows;        // [cells][8] large levels: the predicted windows
-    DevBuf<uint32_t> window_bins;    // [cells][256] and the bins of each (k_p_choose)
-    DevBuf<uint32_t> round_state;    // [2][cells][4] levels of few chunks: the rounds' margins
+    DevBuf<uint32_t> windows;        // [cells][8] large levels: the predicted windows, then
+                                     // [cells][256] the bins of each (k_p_choose)
     DevBuf<uint4> swap_plan;         // [max_chunks][2] Hoare swap unit of each chunk
     DevBuf<int32_t> status;          // [2]: error flag, failing heap id
     DevBuf<uint32_t> ids_dev;        // [cells]

@@ -185,7 +185,6 @@ int preallocate_scratch(Ctx &c)
     size_t m = (size_t)c.max_chunks + 1;
     size_t np = (m + kScanTile - 1) / kScanTile;
     ORB_TRY(c.scan_partials.alloc(np));
-    ORB_TRY(c.round_state.alloc(4 * 2 * (size_t)kRecsScan));
     if (c.part == ORB_PART_STABLE_LE) ORB_TRY(ensure_stable_buffers(c));
     return ORB_OK;
 }
@@ -379,7 +378,7 @@ int ensure_level_capacity(Ctx &c, int64_t nCells, int64_t chunks)
     ORB_TRY(c.chunk_pre.alloc(c.max_chunks + m + 2));  // a level-wide scan, or a table per cell
     ORB_TRY(c.masks.alloc(2 * (size_t)kMaskWords * (size_t)c.max_chunks));
     ORB_TRY(c.cell_cand.alloc((size_t)m * kBins));
-    ORB_TRY(c.splits.alloc(m));
+    ORB_TRY(c.splits.alloc(m + 2 * (size_t)kRecsScan));
     ORB_TRY(c.chunk_comp.alloc(8 * ((size_t)c.max_chunks + 1)));
     ORB_TRY(c.sel_lists.alloc((size_t)c.max_chunks + 1));
     ORB_TRY(c.swap_plan.alloc(2 * (size_t)c.max_chunks));

@@ -680,7 +680,6 @@ int orb_server_destroy(orb_server *o)
     c.chunk_pre.release();
     c.scan_partials.release();
     c.splits.release();
-    c.round_state.release();
     c.chunk_comp.release();
     c.sel.release();
     c.sel_lists.release();

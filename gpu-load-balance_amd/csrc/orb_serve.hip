@@ -507,81 +507,88 @@ static int submit(Server &S, const float *hx, const float *hy, const float *hz, 
     return ORB_OK;
 }
 
-static int step(Server &S)
+// One level of every active build in one list: of those on their first run, or
+// (again) of those that run again, whose levels take every kernel.
+static int advance(Server &S, bool again)
 {
     Ctx &c = S.c;
-    ORB_TRY(poll_finishing(S));  // pool ranges back before the next admission
-    ORB_TRY(admit(S));
-    if (!S.active.empty()) {
-        // this step's level of every active build, in one list
-        LevelEntry *h = S.hentries[S.flip].p;
-        ORB_HIP(hipEventSynchronize(S.ev_entries[S.flip]));  // staging buffer free again
-        int64_t m = 0;
-        bool any_sub = false, any_again = false;
-        LevelShape shape;
-        std::vector<Request *> stepped;
-        for (Request *r : S.active) {
-            while (r->next_level <= r->lmax && r->levels[(size_t)r->next_level].empty())
-                r->next_level++;
-            if (r->next_level > r->lmax) continue;
-            const int32_t l = r->next_level;
-            const auto &ids = r->levels[(size_t)l];
-            if (m + (int64_t)ids.size() > c.max_level_cells) break;  // next step takes the rest
-            // a level whose cells all fit the subtree kernel is the build's last
-            const bool last = shape.add(c, r->n, r->d, l, r->complete, false) && !r->again;
-            for (int32_t id : ids)
-                h[m++] = LevelEntry{id, (int32_t)r->hb, (int32_t)r->cap, 64 * r->slot + l,
-                                    2 * r->slot, r->lmax, r->complete ? 1 : 0, last ? 1 : 0};
-            any_sub = any_sub || r->complete;
-            any_again = any_again || r->again;
-            if (last) r->next_level = r->lmax;
-            stepped.push_back(r);
-        }
-        if (m > 0) {
-            ORB_HIP(hipMemcpyAsync(S.entries.p, h, sizeof(LevelEntry) * (size_t)m,
-                                   hipMemcpyHostToDevice, c.stream));
-            ORB_HIP(hipEventRecord(S.ev_entries[S.flip], c.stream));
-            S.flip ^= 1;
-            // the kernels the step's cells are expected to need; a request that
-            // runs again gets every kernel
-            LevelKernels kernels = any_again ? LevelKernels() : level_kernels(c, shape);
-            kernels.again = any_again;
-            c.level_chunk_hint.assign(1, shape.keys / kChunk + m + 1);
-            ORB_TRY(enqueue_level(c, S.entries.p, (int32_t)m, S.heap.p, S.exists.p, S.sub.p,
-                                  S.chunk_hist.p, S.cell_hist.p, nullptr, S.level_passes.p,
-                                  S.status.p, any_sub, false, 0, nullptr, nullptr, nullptr, false,
-                                  kernels));
-            S.stats.steps++;
-            S.stats.cells_stepped += m;
-            if ((int64_t)stepped.size() > S.stats.max_batch) S.stats.max_batch = (int64_t)stepped.size();
-        }
-        for (Request *r : stepped) r->next_level++;
-        // builds with no level left: results out, pool ranges back
-        for (size_t i = 0; i < S.active.size();) {
-            Request *r = S.active[i];
-            while (r->next_level <= r->lmax && r->levels[(size_t)r->next_level].empty())
-                r->next_level++;
-            if (r->next_level > r->lmax) {
-                ORB_TRY(finish(S, r));
-                S.active[i] = S.active.back();
-                S.active.pop_back();
-            } else {
-                ++i;
-            }
+    bool any = false;
+    for (const Request *r : S.active) any = any || r->again == again;
+    if (!any) return ORB_OK;
+    LevelEntry *h = S.hentries[S.flip].p;
+    ORB_HIP(hipEventSynchronize(S.ev_entries[S.flip]));  // staging buffer free again
+    int64_t m = 0;
+    bool any_sub = false;
+    LevelShape shape;
+    std::vector<Request *> stepped;
+    for (Request *r : S.active) {
+        if (r->again != again) continue;
+        while (r->next_level <= r->lmax && r->levels[(size_t)r->next_level].empty())
+            r->next_level++;
+        if (r->next_level > r->lmax) continue;
+        const int32_t l = r->next_level;
+        const auto &ids = r->levels[(size_t)l];
+        if (m + (int64_t)ids.size() > c.max_level_cells) break;  // next step takes the rest
+        // a level whose cells all fit the subtree kernel is the build's last
+        const bool last = shape.add(c, r->n, r->d, l, r->complete, false) && !again;
+        for (int32_t id : ids)
+            h[m++] = LevelEntry{id, (int32_t)r->hb, (int32_t)r->cap, 64 * r->slot + l,
+                                2 * r->slot, r->lmax, r->complete ? 1 : 0, last ? 1 : 0};
+        any_sub = any_sub || r->complete;
+        if (last) r->next_level = r->lmax;
+        stepped.push_back(r);
+    }
+    if (m > 0) {
+        ORB_HIP(hipMemcpyAsync(S.entries.p, h, sizeof(LevelEntry) * (size_t)m,
+                               hipMemcpyHostToDevice, c.stream));
+        ORB_HIP(hipEventRecord(S.ev_entries[S.flip], c.stream));
+        S.flip ^= 1;
+        // the kernels the cells are expected to need, or every kernel
+        LevelKernels kernels = again ? LevelKernels() : level_kernels(c, shape);
+        kernels.again = again;
+        c.level_chunk_hint.assign(1, shape.keys / kChunk + m + 1);
+        ORB_TRY(enqueue_level(c, S.entries.p, (int32_t)m, S.heap.p, S.exists.p, S.sub.p,
+                              S.chunk_hist.p, S.cell_hist.p, nullptr, S.level_passes.p,
+                              S.status.p, any_sub, false, 0, nullptr, nullptr, nullptr, false,
+                              kernels));
+        S.stats.steps++;
+        S.stats.cells_stepped += m;
+        if ((int64_t)stepped.size() > S.stats.max_batch) S.stats.max_batch = (int64_t)stepped.size();
+    }
+    for (Request *r : stepped) r->next_level++;
+    // builds with no level left: results out, pool ranges back
+    for (size_t i = 0; i < S.active.size();) {
+        Request *r = S.active[i];
+        while (r->next_level <= r->lmax && r->levels[(size_t)r->next_level].empty())
+            r->next_level++;
+        if (r->again == again && r->next_level > r->lmax) {
+            ORB_TRY(finish(S, r));
+            S.active[i] = S.active.back();
+            S.active.pop_back();
+        } else {
+            ++i;
         }
     }
+    return ORB_OK;
+}
+
+static int step(Server &S)
+{
+    ORB_TRY(poll_finishing(S));  // pool ranges back before the next admission
+    ORB_TRY(admit(S));
+    ORB_TRY(advance(S, false));
+    ORB_TRY(advance(S, true));
     ORB_TRY(poll_finishing(S));
     return (int)(S.pending.size() + S.active.size() + S.finishing.size());
 }
 
 // What a caller that only asks for results drives on: requests that are
-// finishing, and the levels of one that runs again.
+// finishing, and those alone that run again (the caller has stepped them to
+// their end).
 static int progress(Server &S)
 {
     ORB_TRY(poll_finishing(S));
-    for (const Request *r : S.active)
-        if (r->again) return step(S) < 0 ? ORB_ERR_HIP : ORB_OK;
-    return ORB_OK;
+    return advance(S, true);
 }
 
 }  // namespace orb

@@ -67,11 +67,13 @@ int orb_server_submit(orb_server *server, const float *x, const float *y, const 
  * valid and untouched until orb_server_poll reports the request done.    */
 int orb_server_submit_device(orb_server *server, float *x, float *y, float *z, int64_t n,
                              int32_t d, uint64_t *request_id);
-/* Admits what fits, launches one level step of every active build, retires
- * finished builds.  Returns the number of requests not yet fetched-ready
+/* Admits what fits, launches one level step of every active build (builds
+ * that run again in a step of their own), retires finished builds.  Returns the number of requests not yet fetched-ready
  * (pending + active + finishing), or an error.                           */
 int orb_server_step(orb_server *server);
-/* 1 when the request's results are ready, 0 otherwise.                   */
+/* 1 when the request's results are ready, 0 otherwise.  (A request whose
+ * cells came out larger than its levels expected runs them again; this and
+ * orb_server_next_done launch those levels, and nothing of other requests.) */
 int orb_server_poll(orb_server *server, uint64_t request_id);
 /* Pops the id of a request that finished since the last call (completion
  * order); returns 1 with *request_id set, 0 when none is waiting.        */

@@ -159,3 +159,32 @@ def test_uneven_cells_run_again(orb, oracle, device):
         for arrays in dev:
             for a in arrays:
                 a.free()
+
+
+# asking for a result drives a request that runs again, and only that one
+@pytest.mark.parametrize("ask", ["poll", "next_done"])
+def test_asking_steps_no_other_request(orb, oracle, ask):
+    n, d = 75000, 4
+    x, y, z = oracle.generate(n)
+    x[np.random.default_rng(2).random(n) < 0.7] = np.float32(0.21)
+    want = oracle.build(x, y, z, d, levels_mode=1)
+    with orb.Server(particle_capacity=1 << 20, cell_capacity=1 << 12, max_active=4) as srv:
+        first = srv.submit(x, y, z, d)
+        srv.step()
+        srv.step()  # its last level; a cell of it is left for the second run
+        second = srv.submit(x, y, z, d)
+        for _ in range(1000000):
+            if srv.poll(first) if ask == "poll" else srv.next_done() == first:
+                break
+        st = srv.stats()
+        assert (st["completed"], st["admitted"], st["pending"], st["active"]) == (1, 1, 1, 0)
+        assert st["steps"] == 4  # two levels, and both again
+        while srv.step():
+            pass
+        for rid in (first, second):
+            got = srv.fetch(rid, n, d)
+            assert got["error"] == want.rc
+            assert np.array_equal(got["ranges"], want.ranges)
+            assert_heaps_equal(got["heap"], want.heap, want.exists)
+            for key, a in zip("xyz", (want.x, want.y, want.z)):
+                assert np.array_equal(fbits(got[key]), fbits(a))

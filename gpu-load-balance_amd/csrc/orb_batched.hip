@@ -3649,13 +3649,29 @@ __global__ __launch_bounds__(kTailBlock) void k_m_tail(
         const uint32_t begin = uniform(rec.begin), n = uniform(rec.end) - begin;
         const int32_t id = (int32_t)uniform((uint32_t)rec.id), hb = (int32_t)uniform((uint32_t)rec.hb);
         const uint32_t f = uniform(first[c]), nch = uniform(first[c + 1]) - f;
-        if (!STABLE && nch > (uint32_t)kMidChunks) {
-            // the level records hand over at most kMidChunks; refuse anything else
+        // the cell's rows: the next level adds to zero
+        auto clear_rows = [&] {
+            if constexpr (WEIGHTED) {
+                for (int q = t; q < kRounds * kBins; q += kTailBlock)
+                    rows[((size_t)(q / kBins) * (size_t)nCells + c) * kBins + q % kBins] = 0ull;
+            } else if (t < 2 * kBins) {
+                cell_hist[((size_t)(t / kBins) * (size_t)nCells + c) * kBins + t % kBins] = 0u;
+            }
+        };
+        // a cell that the swap leaves alone: no split, no unit in its chunks
+        auto idle = [&](int kind) {
             if (t == 0) {
-                report_error(status + rec.st, rec.lp & 63, kErrSplit, id);
+                report_error(status + rec.st, rec.lp & 63, kind, id);
                 splits[c] = SplitRec{0u, 0u, 0u, 0u};
             }
-            continue;
+            for (uint32_t k = (uint32_t)t; k < nch; k += kTailBlock)
+                reinterpret_cast<uint4 *>(plan + f + k)[0] = make_uint4(~0u, 0u, 0u, 0u);
+        };
+        if (!STABLE && nch > (uint32_t)kMidChunks) {
+            // the level records hand over at most kMidChunks; refuse anything else
+            clear_rows();
+            idle(kErrSplit);
+            continue;  // uniform
         }
         float lo = uniform(rec.margin_l), hi = uniform(rec.margin_r);
         int32_t passes = 0;
@@ -3674,8 +3690,7 @@ __global__ __launch_bounds__(kTailBlock) void k_m_tail(
                 found = true;
                 if (trace && t == 0) trace[((size_t)hb + id) * ORB_MAX_PASSES] = 0ull;
             }
-            for (int q = t; q < kRounds * kBins; q += kTailBlock)  // the next level adds to zero
-                rows[((size_t)(q / kBins) * (size_t)nCells + c) * kBins + q % kBins] = 0ull;
+            clear_rows();
         } else {
             uint64_t *trow = trace ? trace + ((size_t)hb + id) * ORB_MAX_PASSES : nullptr;
             // (no chunk carries the rounds of an empty cell: rows of zeros)
@@ -3692,8 +3707,7 @@ __global__ __launch_bounds__(kTailBlock) void k_m_tail(
             const float target = difference_target(n, (int32_t)uniform((uint32_t)rec.nLeaf));
             if (t < kBins) hist[t] = 0u;
             __syncthreads();
-            if (t < 2 * kBins)  // the next level adds to zero
-                cell_hist[((size_t)(t / kBins) * (size_t)nCells + c) * kBins + t % kBins] = 0u;
+            clear_rows();
             while (!found && passes < ORB_MAX_PASSES) {
                 const float width = hi - lo;
                 const float scale = width > 0.0f ? (float)kBins / width : 0.0f;
@@ -3860,12 +3874,7 @@ __global__ __launch_bounds__(kTailBlock) void k_m_tail(
         }
         if (n == 0u || TL == 0u || rid >= (int64_t)(int32_t)uniform((uint32_t)rec.capr)) {
             // empty cell or no key >= cut: the reference's loop leaves the cell
-            if (t == 0) {
-                report_error(status + rec.st, rec.lp & 63, kErrPartition, id);
-                splits[c] = SplitRec{0u, 0u, 0u, 0u};  // the swap skips the cell
-            }
-            for (uint32_t k = (uint32_t)t; k < nch; k += kTailBlock)
-                reinterpret_cast<uint4 *>(plan + f + k)[0] = make_uint4(~0u, 0u, 0u, 0u);
+            idle(kErrPartition);
             __syncthreads();  // the next cell rewrites the tables
             continue;  // uniform
         }

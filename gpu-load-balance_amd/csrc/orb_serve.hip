@@ -148,6 +148,7 @@ struct Request {
     int error = 0;
     int32_t error_cell = -1;
     float *dev[3] = {nullptr, nullptr, nullptr};  // device request: the caller's arrays
+    bool direct = false;         // the kernels reach them
     // pinned blocks: particles (3n floats: in at submit, out at finish; host
     // requests only) and the tree (ranges [cap][2] pool-absolute, heap,
     // exists, 64 level passes + 2 status words)
@@ -191,7 +192,7 @@ struct Server {
 
 // Admission of one request in one launch (three copies, a check and an init
 // before): its particles into the pool (src: a device request's arrays, or
-// the pool itself where a copy from the host went before), the NaN check
+// the pool itself where a copy went before), the NaN check
 // (kErrInputWord into the status pair) and its fresh heap.  Blocks
 // [0, heap_blocks) take the heap, the others the particles, kAdmitPer a
 // thread.  The slot's counters and status pair are zero: k_s_finish leaves
@@ -359,11 +360,12 @@ static int admit(Server &S)
         float *dst[3] = {c.x() + pb, c.y() + pb, c.z() + pb};
         const float *src[3] = {dst[0], dst[1], dst[2]};
         for (int a = 0; a < 3 && r->n > 0; ++a) {
-            if (r->dev[0])
+            if (r->direct)
                 src[a] = r->dev[a];
             else
-                ORB_HIP(hipMemcpyAsync(dst[a], r->xyz + a * r->n, sizeof(float) * (size_t)r->n,
-                                       hipMemcpyHostToDevice, c.stream));
+                ORB_HIP(hipMemcpyAsync(dst[a], r->dev[0] ? r->dev[a] : r->xyz + a * r->n,
+                                       sizeof(float) * (size_t)r->n,
+                                       r->dev[0] ? hipMemcpyDefault : hipMemcpyHostToDevice, c.stream));
         }
         const unsigned gh = tree_grid(r->cap);
         hipLaunchKernelGGL(k_s_admit, dim3(gh + particle_grid(r->n)), dim3(kBlock), 0, c.stream, src[0],
@@ -382,20 +384,20 @@ static int admit(Server &S)
 static int finish(Server &S, Request *r)
 {
     Ctx &c = S.c;
-    const bool dev = r->dev[0] != nullptr;
     const float *src[3] = {c.x() + r->pb, c.y() + r->pb, c.z() + r->pb};
     const unsigned gt = tree_grid(r->cap);
-    hipLaunchKernelGGL(k_s_finish, dim3(gt + (dev ? particle_grid(r->n) : 0u)), dim3(kBlock), 0, c.stream,
+    hipLaunchKernelGGL(k_s_finish, dim3(gt + (r->direct ? particle_grid(r->n) : 0u)), dim3(kBlock), 0, c.stream,
                        src[0], src[1], src[2], r->dev[0], r->dev[1], r->dev[2], (uint32_t)r->n, gt,
                        c.ranges.p + 2 * r->hb, reinterpret_cast<const uint32_t *>(S.heap.p + r->hb),
                        S.exists.p + r->hb, (int64_t)r->cap, r->ranges,
                        reinterpret_cast<uint32_t *>(r->heap), r->exists, S.level_passes.p + 64 * r->slot,
                        S.status.p + 2 * r->slot, r->counters);
     ORB_HIP(hipGetLastError());
-    // (a host request whose levels run again copies its particles again)
-    for (int a = 0; a < 3 && !dev && r->n > 0; ++a)
-        ORB_HIP(hipMemcpyAsync(r->xyz + a * r->n, src[a], sizeof(float) * (size_t)r->n,
-                               hipMemcpyDeviceToHost, c.stream));
+    // (a request whose levels run again copies its particles again)
+    for (int a = 0; a < 3 && !r->direct && r->n > 0; ++a)
+        ORB_HIP(hipMemcpyAsync(r->dev[0] ? r->dev[a] : r->xyz + a * r->n, src[a],
+                               sizeof(float) * (size_t)r->n,
+                               r->dev[0] ? hipMemcpyDefault : hipMemcpyDeviceToHost, c.stream));
     ORB_HIP(hipEventRecord(r->done, c.stream));
     r->state = kFinishing;
     S.finishing.push_back(r);
@@ -452,6 +454,25 @@ static void release_request(Server &S, Request *r)
     r->done = nullptr;
 }
 
+// Whether kernels of this device may read and write the three arrays: its own
+// memory, aligned floats.  Anything else (host memory, a peer's) is left to the
+// runtime's copies, which report what they cannot reach; a kernel would fault.
+static bool kernels_reach(const Ctx &c, float *const (&p)[3])
+{
+    for (const float *a : p) {
+        hipPointerAttribute_t at;
+        std::memset(&at, 0, sizeof at);
+        if (hipPointerGetAttributes(&at, a) != hipSuccess) {
+            (void)hipGetLastError();  // unknown memory: not an error of a later call
+            return false;
+        }
+        if (at.type != hipMemoryTypeDevice || at.device != c.device ||
+            reinterpret_cast<uintptr_t>(a) % alignof(float) != 0)
+            return false;
+    }
+    return true;
+}
+
 static int submit(Server &S, const float *hx, const float *hy, const float *hz, float *dx,
                   float *dy, float *dz, int64_t n, int32_t d, uint64_t *id)
 {
@@ -483,6 +504,7 @@ static int submit(Server &S, const float *hx, const float *hy, const float *hz, 
         r->dev[0] = dx;
         r->dev[1] = dy;
         r->dev[2] = dz;
+        r->direct = kernels_reach(S.c, r->dev);
     } else if (n > 0) {
         r->xyz_bytes = 3 * sizeof(float) * (size_t)n;
         r->xyz = static_cast<float *>(S.pins.get(r->xyz_bytes));

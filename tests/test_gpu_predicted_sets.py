@@ -95,3 +95,48 @@ def test_clump_on_few_chunks(orb, oracle, cmp, partition):
     even = timed(orb, uniform(n), d, cmp, partition=partition)[1]
     # the longest level took 0.78 ms against 0.17 while the tail had round 1's keys to walk
     assert clump.max() < 2.5 * even.max(), (clump, even)
+
+
+# every sampled segment of the root level holds keys far from the rest: the counts
+# contradict the window, the cell is left alone and the levels run again
+def test_sample_misses_runs_again(orb, oracle):
+    d = 64
+    x, y, z = uniform(N)
+    for q in range(N // 4096):
+        h = (((q * 0x9E3779B1) & 0xFFFFFFFF) >> 20) & 1023 & ~15
+        for i in range(4):
+            p = 4096 * q + 1024 * i + h
+            x[p:p + 16] = np.float32(-0.45)
+    want = oracle.build(x, y, z, d, levels_mode=1, threads=8)
+    launches, _ = timed(orb, (x, y, z), d, 0, want, reps=1)
+    assert launches > timed(orb, uniform(N), d, 0, reps=1)[0]  # the second run's
+
+
+# a search that ends at the pass cap a float below its window: the keys around a
+# cell's median tie at the very edge of a sample bin, under <= the search closes in
+# from below, and the last midpoint rounds to the float below (the even one)
+def test_cap_ends_outside_the_window(orb, oracle):
+    F = np.float32
+    d = 16
+    x, y, z = uniform(N)
+    base = oracle.build(x, y, z, d, levels_mode=1, cmp=1, ids=True, threads=8)
+    cell = next(k for k in range(7, 15) if base.heap["cutAxis"][k] == 0)  # depth 3: cut in x again
+    lo, hi = F(base.heap["lower"][cell][0]), F(base.heap["upper"][cell][0])
+    width = F(hi - lo)
+    step, scale = F(width / F(1024)), F(F(1024) / width)
+    b, e = base.ranges[cell]
+    idx = base.ids[b:e]
+    idx = idx[np.argsort(x[idx], kind="stable")]
+    m = len(idx) // 2
+    near = int((x[idx[m]] - lo) * scale)
+    edges = [F(lo + F(F(j) * step)) for j in range(near - 10, near + 10)]
+    v0 = next(v for j, v in zip(range(near - 10, near + 10), edges)
+              if int(F(F(v - lo) * scale)) == j and v.view(np.uint32) & 1)
+    x[idx[m - 126000:m + 126000]] = v0
+    want = oracle.build(x, y, z, d, levels_mode=1, cmp=1, threads=8)
+    # the case is what it is meant to be
+    assert want.heap["lower"][cell][0] == lo and want.heap["upper"][cell][0] == hi
+    L, R = (F(want.heap[k][cell]) for k in ("cutMarginLeft", "cutMarginRight"))
+    assert not want.heap["foundCut"][cell] and F((L + R) / F(2)) < v0
+    launches, _ = timed(orb, (x, y, z), d, 1, want, reps=1)
+    assert launches > timed(orb, uniform(N), d, 1, reps=1)[0]

@@ -1579,9 +1579,9 @@ __global__ __launch_bounds__(kFinBlock) void k_b_finish_block(CellRec *recs, int
 // other side.  A cell whose counts contradict its window (the sample missed) is
 // left alone, counted, and built by the levels' second run.  Builds with a
 // trace need every pass's count and keep the two full rounds.
-// Measured at 2^27 keys, a level's search (keys read to cut found): 226 us,
-// of it the window pass 147 (5 TB/s counting the swap's lines it waits for),
-// from 296 with two full rounds.  Below kPredKeys a cell's sample would have
+// Measured at 2^27 keys, a level's search (keys read to cut found): 230 us,
+// of it the window pass 147 (3.7 TB/s of keys), the sample 25, the gather 20 and
+// the finish 18, from 296 with two full rounds.  Below kPredKeys a cell's sample would have
 // to be a good part of its keys.
 constexpr int kSegment = 16;         // keys of a segment (64 B, a DPP row of lanes)
 constexpr int kSampleRow = kSampleBins + 128;  // the bins, pairs in a segment, pairs across two
@@ -3165,14 +3165,14 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4, 4))
 //                        the stopper masks, K, i and the swap plan
 //   k_hoare_swap
 // The same rounds, masks and plan as the chunk path's.  The five top levels of
-// 2^20 keys (1 to 16 cells): 53 us a level, from 89.  A cell of more chunks keeps
-// one tail block busy for longer than the launches it saves (tables of 1024
-// chunks: 3000001 keys to 500 leaves 638 -> 655 us; of 256: 654).  The level's
-// size matters little: against a line at 2048 chunks, whole builds of 12M keys
-// take 1403 -> 1210 us, 2^24 stable ones 1512 -> 1397, 5e7 tied ones 6870 -> 6030
-// (8192 to 16384) and 5e7 even ones, with predicted windows, 3900 -> 3887.  Past
-// 16384 the one block that fills the chunk table takes longer than the launches
-// saved: with the line at 65536, 2^27 even keys 10046 -> 10217 us.
+// 2^20 keys (1 to 16 cells): 52 us of kernels a level, from 89.  The line at 512
+// chunks a cell: the tables of one tail block (of 256: 3000001 keys to 500 leaves
+// 588 -> 607 us, 2^24 stable ones to 256 1350 -> 1370; of 1024, before k_m_narrow,
+// 638 -> 655).  The level's size matters little: against a line at 2048 chunks,
+// whole builds of 12M keys take 1347 -> 1165 us, 2^24 stable ones 1458 -> 1350,
+// 5e7 even ones, with predicted windows, 4317 -> 4310 and 5e7 tied ones 3121 ->
+// 3167.  Past 16384 the one block that fills the chunk table takes longer than the
+// launches saved: with the line at 65536, 2^27 even keys 10033 -> 10236 us.
 constexpr int kMidChunks = 512;         // per cell: k_m_tail's tables
 constexpr int64_t kMidLevelChunks = 16384;
 

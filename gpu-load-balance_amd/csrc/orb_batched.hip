@@ -1037,24 +1037,17 @@ __device__ inline bool window_holds(const Window &wd, float L, float R)
 
 // Rounds 3 and 4 gather a searching cell's keys into up to 64 lists (see
 // k_b_select): list r covers a contiguous range of the cell's chunks.
-constexpr int kSelChunks = 4;  // chunks per wave: a lane per chunk quarter
 constexpr int kSelLists = 64;
 struct SelLists {
-    uint32_t f, g0, S, R;  // first chunk, first group, groups per list, lists
+    uint32_t f, S, R;  // first chunk, chunks per list, lists
     __device__ SelLists(uint32_t first_chunk, uint32_t nch)
     {
         f = first_chunk;
-        g0 = f / kSelChunks;
-        const uint32_t ng = nch ? (f + nch - 1u) / kSelChunks - g0 + 1u : 0u;
-        S = (ng + kSelLists - 1u) / kSelLists;
-        R = S ? (ng + S - 1u) / S : 0u;
+        S = (nch + kSelLists - 1u) / kSelLists;
+        R = S ? (nch + S - 1u) / S : 0u;
     }
-    __device__ uint32_t list_of_group(uint32_t g) const { return (g - g0) / S; }
-    __device__ uint32_t start_chunk(uint32_t r) const
-    {
-        const uint32_t q = (g0 + r * S) * kSelChunks;
-        return q > f ? q : f;
-    }
+    __device__ uint32_t list_of_chunk(uint32_t q) const { return (q - f) / S; }
+    __device__ uint32_t start_chunk(uint32_t r) const { return f + r * S; }
 };
 
 // One wave per cell: prefix sums of the cell histogram in registers, then
@@ -1105,21 +1098,19 @@ __global__ __launch_bounds__(kBlock) void k_b_replay(CellRec *recs, int32_t nCel
 // Rounds 3 and 4 read only the keys that the window round packed and that
 // lie inside the margins after round 2 (every later candidate lies inside
 // them).  k_b_select gathers them, per searching cell, into up to 64 lists
-// in `sel`, each over a contiguous range of the cell's chunks (whole
-// kSelChunks-chunk groups, one wave's share): the list fills positions from
-// its range's first particle on, which it cannot outgrow, and its counter
-// (kept at the range's first chunk) takes the atomics of few waves even in
-// a cell of the whole level.
+// in `sel`, each over a contiguous range of the cell's chunks: the list fills
+// positions from its range's first particle on, which it cannot outgrow, and
+// its counter (kept at the range's first chunk) takes the atomics of a 64th of
+// the chunks even in a cell of the whole level.
 
-// Each run of one cell in a wave's chunks counts its packed keys inside the
-// cell's margins and below them (the count below also takes the keys below
-// the window round's margins, which that round counted per chunk), then
-// reserves slots in its list with one 64-bit atomic (keys | below << 32)
-// and writes the keys there.  A wave takes 4 chunks, a lane each quarter,
-// and reads the quarters' packed keys laid end to end, four loads per lane
-// in flight; a wave's keys are usually fewer than 256 and stay in registers
-// between counting and writing (a dense cluster packs a good part of a
-// chunk: few chunks per wave keep such waves short).
+// A wave takes a chunk: it reads the quarters' packed keys laid end to end,
+// four loads per lane in flight, counts those inside the cell's margins and
+// those below (with the keys below the window round's margins, which that
+// round counted per chunk), reserves slots in its list with one 64-bit atomic
+// (keys | below << 32) and writes the keys there.  Up to 256 keys stay in
+// registers in between.  Grouped or clustered keys leave a good part of the chunk
+// in the window, a serial chain for a wave of more chunks: with four a wave
+// 2^26 keys in runs of 512 took 47 us a level, with one 20; 2^27 even keys 20 and 15.
 // PRED: the window's keys in [klo, khi]; the keys left of them are counted
 // already (k_p_narrow).
 template <bool PRED>
@@ -1134,117 +1125,75 @@ __global__ __launch_bounds__(kBlock) void k_b_select(const CellRec *__restrict__
                                                      unsigned long long *__restrict__ sel_lists,
                                                      const Window *__restrict__ windows)
 {
-    constexpr int kW = kBlock / 64;
-    constexpr int kQ = 4 * kSelChunks;  // quarters (lanes) per wave
-    // (8 in flight for the fuller predicted windows: 23 us a level against 20)
+    constexpr uint32_t kW = kBlock / 64;
     constexpr int kSelBatch = 4;
-    static_assert(kQ <= 64 && (kQ & (kQ - 1)) == 0, "a lane per chunk quarter");
-    __shared__ uint32_t s_below[kW][64], s_cnt[kW][64];  // per run of one cell
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, sh = lane & 3;
-    const uint32_t wave = blockIdx.x * (uint32_t)kW + (uint32_t)w;
-    const uint32_t nwaves = gridDim.x * (uint32_t)kW;
+    constexpr uint32_t kStep = 64u * kSelBatch;
+    const int lane = threadIdx.x & 63;
     const uint32_t total = first[nCells];
-    for (uint32_t q0 = wave * kSelChunks; q0 < total; q0 += nwaves * kSelChunks) {
-        const uint32_t q = q0 + (uint32_t)(lane >> 2);
-        const bool inq = lane < kQ && q < total;
-        const uint32_t qr = inq ? q : 0u;  // in-bounds record and counts
-        const uint4 d = chunk_record(chunk_desc, qr, max_chunks);
-        const uint32_t nc0 = comp[8 * (size_t)qr + sh], nb0 = comp[8 * (size_t)qr + 4];
-        const uint32_t cell = inq ? d.z : 0xffffffffu;  // runs end at the table's end
-        bool live = inq && d.w <= 2u;
-        float lo = 0.0f, hi = 0.0f;
-        uint32_t begin = 0, f = 0, nch = 0;
-        if (live) {
-            const CellRec &r = recs[cell];
-            f = first[cell];
-            nch = first[cell + 1] - f;
-            live = !r.found && !r.flags;
-            lo = r.margin_l;
-            hi = r.margin_r;
-            begin = r.begin;
-            if constexpr (PRED) {
-                lo = windows[cell].klo;
-                hi = windows[cell].khi;
-            }
+    for (uint32_t q = uniform(blockIdx.x * kW + (threadIdx.x >> 6)); q < total; q += gridDim.x * kW) {
+        const uint4 d = chunk_record(chunk_desc, q, max_chunks);
+        const uint32_t counts = lane < 5 ? comp[8 * (size_t)q + lane] : 0u;
+        const uint32_t b = uniform(d.x), e = uniform(d.y), cell = uniform(d.z);
+        if (uniform(d.w) > 2u) continue;  // uniform, as below
+        const CellRec &r = recs[cell];
+        if (uniform((uint32_t)(r.found | r.flags))) continue;
+        const float lo = uniform(PRED ? windows[cell].klo : r.margin_l);
+        const float hi = uniform(PRED ? windows[cell].khi : r.margin_r);
+        // key t of the chunk lies at t + at[j] of the last quarter j with ex[j] <= t
+        uint32_t ex[kW + 1] = {0u}, at[kW];
+#pragma unroll
+        for (int j = 0; j < (int)kW; ++j) {
+            uint32_t off, cnt;
+            wave_share(b, e, j, off, cnt);
+            at[j] = b + off - ex[j];
+            ex[j + 1] = ex[j] + lane_value(counts, j);
         }
-        uint32_t off = 0, cnt = 0;
-        if (inq) wave_share(d.x, d.y, sh, off, cnt);
-        const uint32_t nc = live ? nc0 : 0u;
-        const uint32_t kbase = d.x + off;  // the quarter's first packed key
-        const uint32_t prev = (uint32_t)__shfl_up((int)cell, 1, 64);
-        const uint64_t heads = __ballot(lane == 0 || prev != cell);
-        const bool head = (heads >> lane) & 1ull;
-        const int run = __popcll(heads & ((2ull << lane) - 1ull)) - 1;
-        s_below[w][lane] = 0u;
-        s_cnt[w][lane] = 0u;
-        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
-        __builtin_amdgcn_wave_barrier();
-        if (!PRED && live && sh == 0 && nb0) atomicAdd(&s_below[w][run], nb0);
-        const uint32_t incl = wave_inclusive_scan(nc), ex = incl - nc;
-        const uint32_t T = (uint32_t)__shfl((int)incl, 63, 64);
-        // key t of the wave: quarter j = the last with ex_j <= t (it holds t)
-        float v[kSelBatch], lj[kSelBatch], hj[kSelBatch];
-        int rj[kSelBatch];
-        // -1: left of what is gathered, 0: gathered, 1: right of it
-        auto side = [&](int u) __attribute__((always_inline)) {
-            return v[u] < lj[u] ? -1 : (v[u] > hj[u] ? 1 : 0);
-        };
+        const uint32_t T = ex[kW];
+        float v[kSelBatch];
         auto load_batch = [&](uint32_t t0) __attribute__((always_inline)) {
 #pragma unroll
             for (int u = 0; u < kSelBatch; ++u) {
                 const uint32_t t = t0 + 64u * (uint32_t)u + (uint32_t)lane;
-                int j = 0;  // (lanes from kQ on hold no keys: ex = T there)
+                uint32_t a = at[0];
 #pragma unroll
-                for (int st = kQ / 2; st > 0; st >>= 1)
-                    if ((uint32_t)__shfl((int)ex, j + st, 64) <= t) j += st;
-                const uint32_t at =
-                    (uint32_t)__shfl((int)kbase, j, 64) + (t - (uint32_t)__shfl((int)ex, j, 64));
-                lj[u] = __shfl(lo, j, 64);
-                hj[u] = __shfl(hi, j, 64);
-                rj[u] = __shfl(run, j, 64);
-                v[u] = t < T ? ckeys[at] : 0.0f;
+                for (int j = 1; j < (int)kW; ++j) a = t >= ex[j] ? at[j] : a;
+                v[u] = t < T ? ckeys[t + a] : 0.0f;
             }
         };
-        constexpr uint32_t kStep = 64u * kSelBatch;
+        auto kept = [&](uint32_t t0, int u) __attribute__((always_inline)) {
+            return __ballot(t0 + 64u * (uint32_t)u + (uint32_t)lane < T && !(v[u] < lo) && !(v[u] > hi));
+        };
+        uint32_t ns = 0, nb = PRED ? 0u : lane_value(counts, (int)kW);
         for (uint32_t t0 = 0; t0 < T; t0 += kStep) {
             load_batch(t0);
 #pragma unroll
             for (int u = 0; u < kSelBatch; ++u) {
-                if (t0 + 64u * (uint32_t)u + (uint32_t)lane < T) {
-                    const int at = side(u);
-                    if (at == 0) atomicAdd(&s_cnt[w][rj[u]], 1u);
-                    else if (!PRED && at < 0) atomicAdd(&s_below[w][rj[u]], 1u);
-                }
+                ns += (uint32_t)__popcll(kept(t0, u));
+                if (!PRED)
+                    nb += (uint32_t)__popcll(
+                        __ballot(t0 + 64u * (uint32_t)u + (uint32_t)lane < T && v[u] < lo));
             }
         }
-        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
-        __builtin_amdgcn_wave_barrier();
+        if (!(ns | nb)) continue;
+        const uint32_t f = first[cell];
+        const SelLists sl(f, first[cell + 1] - f);
+        const uint32_t qs = sl.start_chunk(sl.list_of_chunk(q));
         uint32_t slot = 0;
-        if (head && live) {
-            const uint32_t ns = s_cnt[w][run], nb = s_below[w][run];
-            const SelLists sl(f, nch);
-            const uint32_t qs = sl.start_chunk(sl.list_of_group(q0 / kSelChunks));
-            const unsigned long long old =
-                ns || nb ? atomicAdd(&sel_lists[qs], (unsigned long long)ns |
-                                                         ((unsigned long long)nb << 32))
-                         : 0ull;
-            slot = begin + (qs - f) * (uint32_t)kChunk + (uint32_t)old;
-        }
-        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
-        __builtin_amdgcn_wave_barrier();
-        if (head) s_cnt[w][run] = slot;  // the run's next free slot in sel
-        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
-        __builtin_amdgcn_wave_barrier();
+        if (lane == 0)
+            slot = (uint32_t)atomicAdd(&sel_lists[qs], (unsigned long long)ns | ((unsigned long long)nb << 32));
+        slot = lane_value(slot, 0) + r.begin + (qs - f) * (uint32_t)kChunk;
+        if (!ns) continue;
         for (uint32_t t0 = 0; t0 < T; t0 += kStep) {
             if (T > kStep) load_batch(t0);  // uniform: one batch is still in registers
 #pragma unroll
             for (int u = 0; u < kSelBatch; ++u) {
-                if (t0 + 64u * (uint32_t)u + (uint32_t)lane < T && side(u) == 0)
-                    sel[atomicAdd(&s_cnt[w][rj[u]], 1u)] = v[u];
+                const uint64_t m = kept(t0, u);
+                if (m >> lane & 1ull)
+                    sel[slot + __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
+                                                         __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u))] = v[u];
+                slot += (uint32_t)__popcll(m);
             }
         }
-        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
-        __builtin_amdgcn_wave_barrier();  // the run tables are cleared for the next chunks
     }
 }
 
@@ -1411,7 +1360,7 @@ constexpr int kFinBlockCells = 1024;  // levels up to this many cells
 // (Sixteen waves, and one addition where a wave's keys share a bin: where many
 // keys tie at the cut, a cell of 2^26 keys on 512 coordinate values lists
 // 131072 of them. Four waves took 962 us a level there over two rounds, these
-// 347 over the predicted window's three or four; 17 us at 2^27 even keys.)
+// 322 over the predicted window's three or four; 18 us at 2^27 even keys.)
 constexpr int kFinBlock = 1024;
 template <int LE, bool PRED>
 __global__ __launch_bounds__(kFinBlock) void k_b_finish_block(CellRec *recs, int32_t nCells,
@@ -1579,8 +1528,8 @@ __global__ __launch_bounds__(kFinBlock) void k_b_finish_block(CellRec *recs, int
 // other side.  A cell whose counts contradict its window (the sample missed) is
 // left alone, counted, and built by the levels' second run.  Builds with a
 // trace need every pass's count and keep the two full rounds.
-// Measured at 2^27 keys, a level's search (keys read to cut found): 230 us,
-// of it the window pass 147 (3.7 TB/s of keys), the sample 25, the gather 20 and
+// Measured at 2^27 keys, a level's search (keys read to cut found): 227 us,
+// of it the window pass 147 (3.7 TB/s of keys), the sample 25, the gather 15 and
 // the finish 18, from 296 with two full rounds.  Below kPredKeys a cell's sample would have
 // to be a good part of its keys.
 constexpr int kSegment = 16;         // keys of a segment (64 B, a DPP row of lanes)
@@ -4337,7 +4286,7 @@ int enqueue_level(Ctx &c, const LevelEntry *entries, int32_t nCells, orb_cell *h
         // rounds 3 and 4 from the packed keys inside the margins, gathered
         // per cell once
         const int tb = timing_mark(c);
-        const unsigned gs = (gq + 4 * kSelChunks - 1) / (4 * kSelChunks);
+        const unsigned gs = (gq + kBlock / 64 - 1) / (kBlock / 64);
         unsigned long long *lists = reinterpret_cast<unsigned long long *>(c.sel_lists.p);
         const bool pred = kernels.predict != 0;
         const Window *windows = reinterpret_cast<const Window *>(c.windows.p);

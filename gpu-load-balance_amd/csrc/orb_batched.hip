@@ -2206,8 +2206,8 @@ static int32_t subtree_capacity(const Ctx &c)
 // x, y, z (and ids' local index, weights) are loaded once, every remaining
 // level is built there, and x, y, z are written back once.
 //
-// A depth's cells are taken up to 16 at a time (a slot each); a slot has
-// 16 / (cells) waves when the depth has fewer than 16 cells.  The bisection
+// A depth's cells are taken up to 16 at a time (a slot each; 8 in a block of
+// 512 threads); a slot has 16 / (cells) waves when the depth has fewer cells.  The bisection
 // controller (orbit.cpp:149-231) runs in rounds of 8 passes, as the chunk
 // path's histogram rounds do: the slot's waves bin the cell's keys over the
 // 255 candidate cuts of its margins into a 256-bin LDS histogram (two 16-bit
